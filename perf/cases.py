@@ -1,0 +1,681 @@
+"""Steps of the engine that are worth timing, from a single decoded token to a long prompt.
+
+A case is one batch through the engine's step function (`ModelRunner.step`, which generation, the scheduler's
+loop and trace replay all go through): `rows` requests that decode one token each behind `context` tokens, and
+`prompts` portions of `prompt` tokens each behind `history` tokens. A pass returns the float32 logits of every
+request's last token. Requests that begin in the step (history 0) are admitted, run and released in every pass,
+as a serving loop does; the others were computed by earlier steps and take the same step again.
+
+Models are random ones of the sizes that the benchmark names, cut to a few layers where a whole one would only
+repeat the same layer; the 0.6B size is whole. Weights are drawn on the device by (seed, tensor name), with
+spreads at which every mechanism of a layer shows in the logits. Nothing is kept between states.
+"""
+import hashlib
+import math
+
+import torch
+
+from dinfer_amd.config import EngineOptions, get_architecture
+from dinfer_amd.engine.batch import Entry
+from dinfer_amd.engine.runner import ModelRunner
+from dinfer_amd.parts import DecoderModel
+
+DEVICE = "cuda"
+PAGE = 16
+BUDGET = 2048           # the engine's default step budget, and the longest piece a history is computed in
+
+
+# ---- models ------------------------------------------------------------------------------------------------------
+def _qwen3(hidden, inter, layers, heads, tied):
+    return dict(architectures=["Qwen3ForCausalLM"], model_type="qwen3", hidden_act="silu", attention_bias=False,
+                vocab_size=151936, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=layers,
+                num_attention_heads=heads, num_key_value_heads=8, head_dim=128, rms_norm_eps=1e-6, rope_theta=1e6,
+                max_position_embeddings=40960, tie_word_embeddings=tied)
+
+
+def _kudurax():
+    """Latent attention of 512 + 64 numbers a token; dense and routed feed-forwards in turn, the third and fourth layer
+    on the second one's cache."""
+    m = dict(heads=16, dim=128, rot_dim=64, vdim=128, kv_rank=512, scale=192 ** -0.5,
+             rot=dict(base=10000.0, dims=64, scaling=dict(factor=40.0, original=4096, fast=32.0, slow=1.0)))
+    dense = dict(kind="dense", ff=8192)
+    moe = dict(kind="moe", router=dict(experts=64, top=6), expert=dict(ff=1408), shared=dict(ff=2816))
+    layers = [dict(type="latent_attention", mixer=dict(m, kv_from=1) if i >= 2 else m, mlp=moe if i % 2 else dense)
+              for i in range(4)]
+    return dict(architecture="Kudurax", vocab=32768, width=2048, embedding=dict(scale=1.0), norm=dict(eps=1e-5), layers=layers)
+
+
+def _karopel():
+    """Windowed attention with sinks and kept first tokens; a narrower windowed attention beside a gated delta rule."""
+    mlp = dict(kind="dense", ff=8192)
+    att = dict(type="attention", mlp=mlp, mixer=dict(
+        heads=16, kv_heads=4, dim=128, vdim=128, scale=128 ** -0.5, mask=dict(size=1024, keep_first=4),
+        rot=dict(base=1000000.0, dims=128, scaling=dict(factor=4.0, low=1.0, high=8.0, original=4096))))
+    par = dict(type="parallel", mlp=mlp, mixer=dict(
+        left=dict(heads=8, kv_heads=2, dim=128, vdim=128, scale=128 ** -0.5, mask=dict(size=512)),
+        right=dict(heads=16, kv_heads=8, dim=128, vdim=128, conv=4), left_scale=0.5, right_scale=0.5))
+    return dict(architecture="Karopel", vocab=32768, width=2048, residual_mult=0.5, logit_scale=1.0, norm=dict(eps=1e-6),
+                loop=None, layers=[att, par, par, att])
+
+
+def _fanulix():
+    """Four residual streams; a softmax attention with a sink beside a retention, a state-space layer, routed experts."""
+    moe = dict(kind="moe", router=dict(experts=64, top=6), expert=dict(ff=1408), shared=dict(ff=2816))
+    par = dict(type="parallel", mlp=moe, mixer=dict(
+        left=dict(heads=16, kv_heads=4, dim=128, vdim=128, scale=128 ** -0.5, q_temp=dict(coef=0.1, every=1024)),
+        right=dict(heads=16, dim=128, vdim=128, decay=[1.0 - 2.0 ** (-5 - 3 * i / 16) for i in range(16)],
+                   rot=dict(base=1000000.0, dims=128)),
+        left_scale=0.5, right_scale=0.5))
+    ssm = dict(type="mamba2", mlp=moe, mixer=dict(heads=64, vdim=64, state=128, groups=8, conv=4, norm_groups=8))
+    return dict(architecture="Fanulix", vocab=32768, width=2048, logit_scale=1.0, streams=4, norm=dict(eps=1e-5),
+                layers=[par, ssm, par, par])
+
+
+MODELS = {
+    "qwen3-0.6b": lambda: _qwen3(1024, 3072, 28, 16, True),         # whole
+    "qwen3-8b": lambda: _qwen3(4096, 12288, 8, 32, False),          # 8 layers of 36
+    "qwen3-14b": lambda: _qwen3(5120, 17408, 8, 40, False),         # 8 layers of 40
+    "kudurax-2k": _kudurax,
+    "karopel-2k": _karopel,
+    "fanulix-2k": _fanulix,
+}
+
+
+# ---- cases -------------------------------------------------------------------------------------------------------
+def _case(model, rows=0, context=0, prompts=0, prompt=0, history=0, ragged=False, dtype="bfloat16", **named):
+    return dict(named, model=model, dtype=dtype, rows=rows, context=context, prompts=prompts, prompt=prompt,
+                history=history, ragged=ragged)
+
+
+def listed():
+    return [
+        # one user, a short chat with the smallest model: bound by the number of launches
+        _case("qwen3-0.6b", rows=1, context=250, name="0.6b, 1 token"),
+        # a burst of short requests at a small model: time to the first token
+        _case("qwen3-0.6b", prompts=8, prompt=150, ragged=True, name="0.6b, 8 prompts of about 130"),
+        # the headline decode steps: 8 and 64 requests behind prompts of 2,048 tokens
+        _case("qwen3-8b", rows=8, context=2048, name="8b, 8 tokens"),
+        _case("qwen3-8b", rows=64, context=2048, name="8b, 64 tokens"),
+        # the headline prefill
+        _case("qwen3-8b", prompts=1, prompt=2048, name="8b, prompt of 2,048"),
+        # a document of 30,000 tokens read in portions: the portion that ends it
+        _case("qwen3-8b", prompts=1, prompt=2001, history=28000, name="8b, portion behind 28,000"),
+        # the serving workload: a portion of 512 beside requests that decode
+        _case("qwen3-14b", rows=31, context=3072, prompts=1, prompt=512, history=1024, ragged=True, name="14b, portion of 512 beside 31"),
+        # trace replay and scoring on the 32-bit path
+        _case("qwen3-0.6b", prompts=1, prompt=500, dtype="float32", name="0.6b in 32 bits, prompt of 500"),
+        # latent attention and routed experts: portions of many prompts in one step
+        _case("kudurax-2k", prompts=16, prompt=256, history=1000, name="kudurax, 16 portions of 256"),
+        # one long prompt through a gated delta rule
+        _case("karopel-2k", prompts=1, prompt=2048, name="karopel, prompt of 2,048"),
+        # retention, state space, routed experts: a few prompts at once, and decoding
+        _case("fanulix-2k", prompts=4, prompt=600, ragged=True, name="fanulix, 4 prompts of about 530"),
+        _case("fanulix-2k", rows=64, context=2048, ragged=True, name="fanulix, 64 tokens"),
+    ]
+
+
+def draw(rng):
+    def between(lo, hi):
+        return min(hi, max(lo, round(math.exp(rng.uniform(math.log(lo), math.log(hi + 0.5))))))
+
+    model = rng.choice(["qwen3-0.6b", "qwen3-8b", "qwen3-8b", "qwen3-14b", "kudurax-2k", "karopel-2k", "fanulix-2k"])
+    kind = rng.choice(["decode", "decode", "prompt", "prompt", "mixed"])
+    ragged = rng.random() < 0.6
+    if model == "qwen3-0.6b" and rng.random() < 0.3:
+        if kind == "decode":
+            return _case(model, rows=between(1, 8), context=between(16, 700), ragged=ragged, dtype="float32")
+        return _case(model, prompts=1, prompt=between(16, 600), dtype="float32")
+    if kind == "decode":
+        rows = between(1, 64)
+        return _case(model, rows=rows, context=between(33, min(8192, 131072 // rows)), ragged=ragged)
+    if kind == "prompt":
+        prompts = between(1, 16)
+        prompt = between(17, max(32, 4096 // prompts))
+        history = rng.choice([0, 0, between(16, min(12000, 24000 // prompts))])
+        return _case(model, prompts=prompts, prompt=prompt, history=history, ragged=ragged and prompts > 1)
+    rows = between(1, 48)
+    return _case(model, rows=rows, context=between(65, min(4096, 65536 // rows)), prompts=1, prompt=between(16, 1024),
+                 history=rng.choice([0, between(16, 2048)]), ragged=ragged)
+
+
+def _lengths(case):
+    """[(computed before, tokens in the step)] of every request; ragged: down to three quarters, by the request's number."""
+    def cut(n, i):
+        return n - (i * 37 + 11) * n // 512 % (n // 4 + 1) if case["ragged"] else n
+
+    out = [(cut(case["context"], i), 1) for i in range(case["rows"])]
+    if case["prompts"] == 1:
+        return out + [(case["history"], case["prompt"])]
+    return out + [(cut(case["history"], i), cut(case["prompt"], i + 3)) for i in range(case["prompts"])]
+
+
+def _tokens(case, seed):
+    """Per request all its token ids, those computed before and those of the step."""
+    cfg = MODELS[case["model"]]()
+    g = torch.Generator().manual_seed(_number(seed, "tokens"))
+    vocab = cfg["vocab_size"] if "vocab_size" in cfg else cfg["vocab"]
+    return [torch.randint(0, vocab, (before + new,), generator=g).tolist() for before, new in _lengths(case)]
+
+
+# ---- weights -----------------------------------------------------------------------------------------------------
+def _number(seed, name):
+    return int.from_bytes(hashlib.sha256(f"{seed}:{name}".encode()).digest()[:7], "little")
+
+
+def _weight(seed, name, shape, family):
+    """One tensor in bfloat16 (what a weight file holds). Products keep their operands' spread; routers are decisive, as
+    trained ones are (few tokens stand between two experts, where one rounding chooses)."""
+    g = torch.Generator(device=DEVICE).manual_seed(_number(seed, name))
+    x = torch.randn(shape, generator=g, device=DEVICE, dtype=torch.float32)
+    last = name.rsplit(".", 1)[-1]
+    if last == "b" and len(shape) == 1:
+        t = 0.1 * x
+    elif family == "karopel" and (last in ("norm1", "norm1b", "norm2", "norm2b") or name == "final.norm"):
+        t = 0.1 * x                                     # stored as the distance from one
+    elif len(shape) == 1 and ("norm" in name.rsplit(".", 2)[-2] + last):
+        t = 1.0 + 0.1 * x
+    elif ".hc" in name:
+        t = {"in": 0.25 + 0.1 * x, "out": 0.7 + 0.2 * x}[last] if len(shape) == 1 else 0.05 + 0.05 * x + 0.8 * torch.eye(shape[0], device=DEVICE)
+    elif last == "A_log":
+        t = 0.5 * x
+    elif last == "dt_bias":
+        t = x - 2.0
+    elif last in ("D", "sink"):
+        t = 1.0 + 0.3 * x
+    elif last == "conv":
+        t = 0.5 * x
+    elif name in ("embed", "model.embed_tokens.weight"):
+        t = x * (1.0 if family != "qwen3" else 0.5)
+    elif last == "router":
+        t = 4.0 * x / math.sqrt(shape[-1])
+    else:
+        t = x / math.sqrt(shape[-1])
+    return t.to(torch.bfloat16)
+
+
+class _Weights:
+    """A model's tensors by name, drawn when they are asked for."""
+
+    def __init__(self, seed, family, dtype):
+        self.seed, self.family, self.dtype, self.shapes = seed, family, dtype, {}
+
+    def check(self, expected, optional=frozenset()):
+        self.shapes = {n: tuple(s.shape) for n, s in expected.items()}
+
+    def has(self, name):
+        return name in self.shapes
+
+    def fetch(self, name, *, compute=False):
+        return _weight(self.seed, name, self.shapes[name], self.family).to(self.dtype)
+
+
+# ---- the step ----------------------------------------------------------------------------------------------------
+def prepare(case, seed):
+    cfg = MODELS[case["model"]]()
+    name = cfg.get("architecture") or cfg["architectures"][0]
+    arch = get_architecture(name)
+    tokens, lengths = _tokens(case, seed), _lengths(case)
+    longest = -(-max(len(t) for t in tokens) // 256) * 256
+    options = EngineOptions(
+        dtype=case["dtype"], max_model_len=longest, max_num_seqs=len(tokens), block_size=PAGE,
+        max_num_batched_tokens=max(BUDGET, sum(n for _, n in lengths)), num_blocks=sum(-(-len(t) // PAGE) for t in tokens) + 2 * BUDGET // PAGE)
+    device = torch.device(DEVICE, torch.cuda.current_device())
+    model = DecoderModel(arch.build_spec(arch.config_class.from_dict(cfg)))
+    model.load(_Weights(seed, _family(case), getattr(torch, case["dtype"])))
+    runner = ModelRunner(model, options, device)
+    # what earlier steps computed
+    for i, (toks, (before, _)) in enumerate(zip(tokens, lengths)):
+        for start in range(0, before, BUDGET):
+            n = min(BUDGET, before - start)
+            _reserve(runner, i, start, n)
+            runner.step([Entry(i, toks[start:start + n], start, [])])
+            runner.advance(i, start + n)
+    entries = [Entry(i, toks[before:], before, [new - 1]) for i, (toks, (before, new)) in enumerate(zip(tokens, lengths))]
+    for e in entries:
+        if e.start > 0:
+            _reserve(runner, e.req_id, e.start, len(e.tokens))
+    return dict(runner=runner, entries=entries, begins=[e for e in entries if e.start == 0])
+
+
+def _reserve(runner, req_id, start, n):
+    if not runner.reserve(req_id, start, n):
+        raise RuntimeError("the cache has no pages left")
+
+
+def run(state):
+    runner = state["runner"]
+    for e in state["begins"]:
+        _reserve(runner, e.req_id, 0, len(e.tokens))
+    logits = runner.step(state["entries"])
+    for e in state["begins"]:
+        runner.finish(e.req_id)
+    return logits
+
+
+# ---- what a pass cannot do without -------------------------------------------------------------------------------
+def _family(case):
+    return case["model"].split("-")[0]
+
+
+def _visible(lengths, window=None, keep=0):
+    """(pairs of a query and a key it sees, keys read) over all requests."""
+    pairs = keys = 0
+    for before, new in lengths:
+        n = before + new
+        if window is None:
+            pairs += new * before + new * (new + 1) // 2
+            keys += n
+        else:
+            pairs += sum(min(p + 1, window) + (min(keep, p + 1 - window) if p + 1 > window else 0) for p in range(before, n))
+            first = max(0, before - window + 1)
+            keys += n - first + min(keep, first)
+    return pairs, keys
+
+
+def work(case):
+    """Every weight that is used read once, the cache of the live requests read once and its new part written, state in
+    and out, logits out; multiply-adds of the products, of attention and of the recurrences."""
+    cfg, lengths = MODELS[case["model"]](), _lengths(case)
+    T, R = sum(n for _, n in lengths), len(lengths)
+    size = 4 if case["dtype"] == "float32" else 2
+    width = cfg["hidden_size"] if "hidden_size" in cfg else cfg["width"]
+    vocab = cfg["vocab_size"] if "vocab_size" in cfg else cfg["vocab"]
+    weights, macs, cache = width * vocab, width * vocab * R, 0      # numbers read, multiply-adds, bytes
+    resumed = sum(1 for before, _ in lengths if before)
+
+    def dense(n):
+        nonlocal weights, macs
+        weights, macs = weights + n, macs + n * T
+
+    def attention(heads, kv, dk, dv, window=None, keep=0, values=True):
+        nonlocal macs, cache
+        pairs, keys = _visible(lengths, window, keep)
+        macs += pairs * heads * (dk + dv)
+        cache += (keys + T) * kv * (dk + (dv if values else 0)) * size
+
+    def state(numbers, per_token):
+        nonlocal macs, cache
+        cache += (R + resumed) * numbers * 4
+        macs += T * per_token
+
+    def routed(f, products):
+        nonlocal weights, macs
+        E, k, n = f["router"]["experts"], f["router"]["top"], products * width * f["expert"]["ff"]
+        weights += E * width + n * E * (1 - (1 - k / E) ** T)
+        macs += T * (E * width + n * k)
+        dense(products * width * f["shared"]["ff"])
+
+    fam = _family(case)
+    for layer in cfg["layers"] if "layers" in cfg else range(cfg["num_hidden_layers"]):
+        if fam == "qwen3":
+            H, G, D = cfg["num_attention_heads"], cfg["num_key_value_heads"], cfg["head_dim"]
+            dense(width * D * (2 * H + 2 * G) + 3 * width * cfg["intermediate_size"])
+            attention(H, G, D, D)
+            continue
+        m, f = layer["mixer"], layer["mlp"]
+        if layer["type"] == "latent_attention":
+            H, d, r, v, rank = m["heads"], m["dim"], m["rot_dim"], m["vdim"], m["kv_rank"]
+            dense(width * (H * (d + r) + H + H * v) + H * (d + v) * rank)
+            if "kv_from" not in m:
+                dense(width * (rank + r))
+            pairs, keys = _visible(lengths)
+            macs += pairs * H * (d + r + v)
+            cache += (keys + (T if "kv_from" not in m else 0)) * (rank + r) * size
+        elif layer["type"] == "attention":
+            H, G, D = m["heads"], m["kv_heads"], m["dim"]
+            dense(width * D * (2 * H + 2 * G))
+            attention(H, G, D, D, m["mask"]["size"], m["mask"]["keep_first"])
+        elif layer["type"] == "mamba2":
+            inner, N, H = m["heads"] * m["vdim"], m["state"], m["heads"]
+            dense(width * (3 * inner + 2 * m["groups"] * N + H) + (inner + 2 * m["groups"] * N) * m["conv"])
+            state(inner * N, 2 * inner * N)
+        else:
+            a, b = m["left"], m["right"]
+            H, G, D = a["heads"], a["kv_heads"], a["dim"]
+            if fam == "karopel":
+                dense(width * D * (2 * H + G))
+                attention(H, G, D, D, a["mask"]["size"], values=False)
+                H, G, D, V = b["heads"], b["kv_heads"], b["dim"], b["vdim"]
+                dense(width * (2 * G * D + 3 * H * V + 2 * H) + (2 * G * D + H * V) * b["conv"])
+                state(H * D * V, 3 * H * D * V)
+            else:
+                dense(width * D * (3 * H + 2 * G))
+                attention(H, G, D, D)
+                H, D, V = b["heads"], b["dim"], b["vdim"]
+                dense(width * H * (2 * D + 3 * V))
+                state(H * D * V, 2 * H * D * V)
+        if f["kind"] == "moe":
+            routed(f, 3 if fam == "kudurax" else 2)
+        else:
+            dense((2 if fam == "kudurax" else 3) * width * f["ff"])
+    return {"bytes": weights * size + cache + T * width * size + R * vocab * 4, "flops": 2.0 * macs}
+
+
+def tolerance(case):
+    if case["dtype"] == "float32":
+        return {"rel": 2e-5, "max": 2e-4}       # measured against 64 bits: 3e-6 to 4e-6
+    # measured against 64 bits: 0.011 to 0.017 at the dense models' 8 and 28 layers, 0.005 to 0.010 at the others' four;
+    # two correct forms differ by up to the sum of their errors
+    return {"rel": 0.03 if _family(case) == "qwen3" else 0.025, "max": 0.5}
+
+
+# ---- the same logits in 64 bits ----------------------------------------------------------------------------------
+F = torch.float64
+
+
+class _Sequences:
+    """All requests' tokens end to end, each from its first one: row ranges, positions."""
+
+    def __init__(self, tokens):
+        self.n = [len(t) for t in tokens]
+        self.at = [sum(self.n[:i]) for i in range(len(self.n))]
+        self.ids = torch.tensor([t for ts in tokens for t in ts], device=DEVICE)
+        self.pos = torch.cat([torch.arange(n, device=DEVICE) for n in self.n])
+
+    def __iter__(self):
+        return (slice(a, a + n) for a, n in zip(self.at, self.n))
+
+    @property
+    def last(self):
+        return torch.tensor([a + n - 1 for a, n in zip(self.at, self.n)], device=DEVICE)
+
+    def padded(self, x):
+        """[requests, longest, ...] with zeros behind the shorter ones."""
+        out = torch.zeros((len(self.n), max(self.n)) + x.shape[1:], dtype=x.dtype, device=x.device)
+        for i, s in enumerate(self):
+            out[i, :self.n[i]] = x[s]
+        return out
+
+    def packed(self, x):
+        return torch.cat([x[i, :n] for i, n in enumerate(self.n)])
+
+
+def _in_pieces(fn, x, rows=8192):
+    return torch.cat([fn(x[i:i + rows]) for i in range(0, x.shape[0], rows)])
+
+
+def _rms(x, eps):
+    return x * torch.rsqrt((x * x).mean(-1, keepdim=True) + eps)
+
+
+def _layer_norm(x, w, b, eps):
+    x = x - x.mean(-1, keepdim=True)
+    return _rms(x, eps) * w + b
+
+
+def _silu(x):
+    return x * torch.sigmoid(x)
+
+
+def _turn(x, pos, freq, factor=1.0, neighbours=False):
+    """Pairs of the last axis turned by position times frequency: (2i, 2i + 1), or (i, i + half)."""
+    half = freq.numel()
+    angle = pos.to(F)[:, None, None] * freq
+    c, s = angle.cos() * factor, angle.sin() * factor
+    a, b = (x[..., 0::2], x[..., 1::2]) if neighbours else (x[..., :half], x[..., half:])
+    a, b = a * c - b * s, b * c + a * s
+    return torch.stack([a, b], -1).flatten(-2) if neighbours else torch.cat([a, b], -1)
+
+
+def _powers(base, dims):
+    return base ** (-2.0 * torch.arange(dims // 2, dtype=F, device=DEVICE) / dims)
+
+
+def _attend(seqs, q, k, v, scale, window=None, keep=0, sink=None, slope=None):
+    """q [T, H, D], k [T, G, D], v [T, G, V] -> [T, H V]. sink: a score a head that only joins the denominator; slope:
+    taken off a head's scores for every position between query and key."""
+    H, G = q.shape[1], k.shape[1]
+    out = torch.empty(q.shape[0], H, v.shape[2], dtype=F, device=DEVICE)
+    for s in seqs:
+        n = s.stop - s.start
+        kk, vv = k[s].transpose(0, 1).contiguous(), v[s].transpose(0, 1).contiguous()          # [G, n, D]
+        step = max(16, (1 << 28) // (H * n))
+        for r in range(0, n, step):
+            e = min(n, r + step)
+            qq = q[s][r:e].view(e - r, G, H // G, -1).permute(1, 2, 0, 3).reshape(G, -1, q.shape[2])
+            z = torch.matmul(qq, kk[:, :e].transpose(1, 2).contiguous()).view(G, H // G, e - r, e).mul_(scale)
+            i, j = torch.arange(r, e, device=DEVICE)[:, None], torch.arange(e, device=DEVICE)[None, :]
+            if slope is not None:
+                z -= slope.view(G, H // G, 1, 1) * (i - j)
+            hidden = j > i
+            if window is not None:
+                hidden = hidden | ((i - j >= window) & (j >= keep))
+            z.masked_fill_(hidden, float("-inf"))
+            if sink is not None:
+                extra = sink.view(G, H // G, 1, 1).expand(G, H // G, e - r, 1)
+                z = torch.cat([z, extra], -1).softmax(-1)[..., :-1]
+            else:
+                z = z.softmax(-1)
+            o = torch.matmul(z.reshape(G, -1, e).contiguous(), vv[:, :e]).view(G, H // G, e - r, -1)
+            out[s.start + r:s.start + e] = o.permute(2, 0, 1, 3).reshape(e - r, H, -1)
+    return out.flatten(1)
+
+
+def _recur(seqs, q, k, v, decay, beta=None, gain=None):
+    """S <- decay S + k u^T, o = S^T q over every request from its start; u = gain v, or with beta (the delta rule)
+    beta (v - (decay S)^T k). q, k [T, H, N], v [T, H, P], decay, beta, gain [T, H]."""
+    q, k, v, decay = (seqs.padded(t) for t in (q, k, v, decay))
+    beta = seqs.padded(beta) if beta is not None else None
+    gain = seqs.padded(gain) if gain is not None else None
+    S = torch.zeros(q.shape[0], q.shape[2], q.shape[3], v.shape[3], dtype=F, device=DEVICE)
+    out = torch.empty_like(v)
+    for t in range(q.shape[1]):
+        S *= decay[:, t, :, None, None]
+        u = v[:, t]
+        if beta is not None:
+            u = (u - (k[:, t, :, None] @ S).squeeze(2)) * beta[:, t, :, None]
+        elif gain is not None:
+            u = u * gain[:, t, :, None]
+        S += k[:, t, :, :, None] * u[:, :, None, :]
+        out[:, t] = (q[:, t, :, None] @ S).squeeze(2)
+    return seqs.packed(out)
+
+
+def _conv(seqs, x, taps):
+    """Causal convolution of every channel over a request's tokens; the last tap is the current token's."""
+    y = torch.zeros_like(x)
+    K = taps.shape[1]
+    for s in seqs:
+        a, b = x[s], y[s]
+        for j in range(K):
+            b[j:] += a[:a.shape[0] - j] * taps[:, K - 1 - j]
+    return y
+
+
+def _routed(h, w, p, f, expert):
+    """The k largest of all scores, their softmax as weights."""
+    z = h @ w(p + "router", f["router"]["experts"], h.shape[1]).T
+    top, idx = z.topk(f["router"]["top"], dim=-1)
+    share = top.softmax(-1)
+    out = torch.zeros_like(h)
+    for e in range(f["router"]["experts"]):
+        rows, slot = (idx == e).nonzero(as_tuple=True)
+        if rows.numel():
+            out[rows] += expert(h[rows], f"{p}e{e}.", f["expert"]["ff"]) * share[rows, slot][:, None]
+    return out
+
+
+def _qwen3_exact(cfg, w, seqs):
+    Hd, H, G, D, I, eps = (cfg[k] for k in ("hidden_size", "num_attention_heads", "num_key_value_heads", "head_dim",
+                                            "intermediate_size", "rms_norm_eps"))
+    freq = _powers(cfg["rope_theta"], D)
+    x = w("model.embed_tokens.weight", cfg["vocab_size"], Hd, rows=seqs.ids)
+    for l in range(cfg["num_hidden_layers"]):
+        p = f"model.layers.{l}."
+        a, m = p + "self_attn.", p + "mlp."
+        h = _rms(x, eps) * w(p + "input_layernorm.weight", Hd)
+        q, k, v = (h @ w(f"{a}{n}_proj.weight", heads * D, Hd).T for n, heads in (("q", H), ("k", G), ("v", G)))
+        q = _turn(_rms(q.view(-1, H, D), eps) * w(a + "q_norm.weight", D), seqs.pos, freq)
+        k = _turn(_rms(k.view(-1, G, D), eps) * w(a + "k_norm.weight", D), seqs.pos, freq)
+        x = x + _attend(seqs, q, k, v.view(-1, G, D), D ** -0.5) @ w(a + "o_proj.weight", Hd, H * D).T
+        del q, k, v
+        gain, g, u, d = w(p + "post_attention_layernorm.weight", Hd), w(m + "gate_proj.weight", I, Hd), w(m + "up_proj.weight", I, Hd), w(m + "down_proj.weight", Hd, I)
+
+        def mlp(r):
+            h = _rms(r, eps) * gain
+            return r + (_silu(h @ g.T) * (h @ u.T)) @ d.T
+
+        x = _in_pieces(mlp, x)
+    x = _rms(x[seqs.last], eps) * w("model.norm.weight", Hd)
+    return x @ w("model.embed_tokens.weight" if cfg["tie_word_embeddings"] else "lm_head.weight", cfg["vocab_size"], Hd).T
+
+
+def _kudurax_exact(cfg, w, seqs):
+    W, eps = cfg["width"], cfg["norm"]["eps"]
+
+    def norm(x, name):
+        return _layer_norm(x, w(name, W), w(name + ".b", W), eps)
+
+    def gated(h, p, n):
+        return (_silu(h @ w(p + "gate", n, W).T) * (h @ w(p + "up", n, W).T)) @ w(p + "down", W, n).T
+
+    x = w("embed", cfg["vocab"], W, rows=seqs.ids) * cfg["embedding"]["scale"]
+    latents = {}
+    for i, layer in enumerate(cfg["layers"]):
+        p, m, f = f"l{i}.", layer["mixer"], layer["mlp"]
+        H, d, r, dv, R = m["heads"], m["dim"], m["rot_dim"], m["vdim"], m["kv_rank"]
+        # long wavelengths are slowed by the factor, short ones stay, a ramp between
+        sc, base = m["rot"]["scaling"], m["rot"]["base"]
+        at = [r * math.log(sc["original"] / (2 * math.pi * turns)) / (2 * math.log(base)) for turns in (sc["fast"], sc["slow"])]
+        lo, hi = max(math.floor(at[0]), 0), min(math.ceil(at[1]), r - 1)
+        ramp = ((torch.arange(r // 2, dtype=F, device=DEVICE) - lo) / max(hi - lo, 0.001)).clamp(0, 1)
+        freq = _powers(base, r) * (ramp / sc["factor"] + 1 - ramp)
+        turn = dict(freq=freq, factor=0.1 * math.log(sc["factor"]) + 1, neighbours=True)
+        h = norm(x, p + "norm1")
+        if "kv_from" not in m:
+            c = h @ w(p + "mix.dkv", R + r, W).T
+            latents[i] = _rms(c[:, :R], eps) * w(p + "mix.dkv.norm", R), _turn(c[:, None, R:], seqs.pos, **turn)
+        c, kr = latents[m.get("kv_from", i)]
+        q = (h @ w(p + "mix.q", H * (d + r), W).T).view(-1, H, d + r)
+        q = torch.cat([q[..., :d], _turn(q[..., d:], seqs.pos, **turn)], -1)
+        k = torch.cat([(c @ w(p + "mix.uk", H * d, R).T).view(-1, H, d), kr.expand(-1, H, r)], -1)
+        v = (c @ w(p + "mix.uv", H * dv, R).T).view(-1, H, dv)
+        gate = torch.sigmoid(h @ w(p + "mix.g", H, W).T)
+        o = _attend(seqs, q, k, v, m["scale"]).view(-1, H, dv) * gate[:, :, None]
+        x = x + o.flatten(1) @ w(p + "mix.o", W, H * dv).T
+        h = norm(x, p + "norm2")
+        p += "mlp."
+        if f["kind"] == "dense":
+            x = x + torch.relu(h @ w(p + "up", f["ff"], W).T) ** 2 @ w(p + "down", W, f["ff"]).T
+        else:
+            x = x + _routed(h, w, p, f, gated) + gated(h, p + "shared.", f["shared"]["ff"]) * torch.sigmoid(h @ w(p + "shared.sg", 1, W).T)
+    return norm(x[seqs.last], "final.norm") @ w("head", cfg["vocab"], W).T
+
+
+def _karopel_exact(cfg, w, seqs):
+    W, eps = cfg["width"], cfg["norm"]["eps"]
+
+    def norm(x, name):
+        return _rms(x, eps) * (1 + w(name, W))
+
+    x = w("embed", cfg["vocab"], W, rows=seqs.ids)
+    for i, layer in enumerate(cfg["layers"]):
+        p, m, ff = f"l{i}.", layer["mixer"], layer["mlp"]["ff"]
+        h = norm(x, p + "norm1")
+        if layer["type"] == "attention":
+            H, G, D = m["heads"], m["kv_heads"], m["dim"]
+            sc, freq = m["rot"]["scaling"], _powers(m["rot"]["base"], D)
+            # three zones by wavelength: kept, slowed, and a mixture between
+            s = ((sc["original"] * freq / (2 * math.pi) - sc["low"]) / (sc["high"] - sc["low"])).clamp(0, 1)
+            freq = freq * (s + (1 - s) / sc["factor"])
+            q, k, v = (h @ w(f"{p}mix.{n}", heads * D, W).T for n, heads in (("q", H), ("k", G), ("v", G)))
+            q = _turn(_rms(q.view(-1, H, D), eps) * w(p + "mix.q.norm", D), seqs.pos, freq, neighbours=True)
+            k = _turn(_rms(k.view(-1, G, D), eps) * w(p + "mix.k.norm", D), seqs.pos, freq, neighbours=True)
+            y = _attend(seqs, q, k, v.view(-1, G, D), m["scale"], m["mask"]["size"], m["mask"]["keep_first"], w(p + "mix.sink", H))
+            y = y @ w(p + "mix.o", W, H * D).T
+        else:
+            a, b = m["left"], m["right"]
+            H, G, D, n = a["heads"], a["kv_heads"], a["dim"], p + "mix.left."
+            q, k = (h @ w(n + "q", H * D, W).T).view(-1, H, D), (h @ w(n + "k", G * D, W).T).view(-1, G, D)
+            slope = 2.0 ** (-8.0 * (torch.arange(H, dtype=F, device=DEVICE) + 1) / H)
+            left = _attend(seqs, q, k, k, a["scale"], a["mask"]["size"], slope=slope) @ w(n + "o", W, H * D).T
+            H, G, D, V, K, n = b["heads"], b["kv_heads"], b["dim"], b["vdim"], b["conv"], p + "mix.right."
+            q, k, v = (_silu(_conv(seqs, h @ w(n + t, c, W).T, w(f"{n}{t}.conv", c, K))).view(-1, heads, c // heads)
+                       for t, c, heads in (("q", G * D, G), ("k", G * D, G), ("v", H * V, H)))
+            q = q * torch.rsqrt((q * q).sum(-1, keepdim=True) + 1e-6) * D ** -0.5
+            k = k * torch.rsqrt((k * k).sum(-1, keepdim=True) + 1e-6)
+            q, k = (t.repeat_interleave(H // G, dim=1) for t in (q, k))
+            beta = torch.sigmoid(h @ w(n + "b", H, W).T)
+            decay = torch.exp(-torch.exp(w(n + "A_log", H)) * torch.nn.functional.softplus(h @ w(n + "a", H, W).T + w(n + "dt_bias", H)))
+            o = _recur(seqs, q, k, v, decay, beta=beta)
+            o = _rms(o, eps) * w(n + "norm", V) * _silu(h @ w(n + "g", H * V, W).T).view(-1, H, V)
+            y = m["left_scale"] * left + m["right_scale"] * (o.flatten(1) @ w(n + "o", W, H * V).T)
+        x = x + cfg["residual_mult"] * norm(y, p + "norm1b")
+        h = norm(x, p + "norm2")
+        y = (_silu(h @ w(p + "mlp.gate", ff, W).T) * (h @ w(p + "mlp.up", ff, W).T)) @ w(p + "mlp.down", W, ff).T
+        x = x + cfg["residual_mult"] * norm(y, p + "norm2b")
+    return norm(x[seqs.last], "final.norm") @ w("head", cfg["vocab"], W).T * cfg["logit_scale"]
+
+
+def _fanulix_exact(cfg, w, seqs):
+    W, eps, n_streams = cfg["width"], cfg["norm"]["eps"], cfg["streams"]
+
+    def norm(x, name):
+        return _layer_norm(x, w(name, W), w(name + ".b", W), eps)
+
+    def expert(h, p, n):
+        return torch.nn.functional.gelu(h @ w(p + "up", n, W).T) @ w(p + "down", W, n).T
+
+    def parallel(h, p, m):
+        a, b = m["left"], m["right"]
+        H, G, D, n = a["heads"], a["kv_heads"], a["dim"], p + "left."
+        q, k, v = ((h @ w(n + t, heads * D, W).T + w(f"{n}{t}.b", heads * D)).view(-1, heads, D) for t, heads in (("q", H), ("k", G), ("v", G)))
+        steps = torch.div(seqs.pos + 1, a["q_temp"]["every"], rounding_mode="floor").to(F)
+        q = _rms(q, eps) * (1 + a["q_temp"]["coef"] * torch.log(steps + 1))[:, None, None]
+        o = _attend(seqs, q, _rms(k, eps), v, a["scale"], sink=torch.zeros(H, dtype=F, device=DEVICE))
+        left = (o * torch.sigmoid(h @ w(n + "g", H * D, W).T)) @ w(n + "o", W, H * D).T
+        H, D, V, n = b["heads"], b["dim"], b["vdim"], p + "right."
+        freq = _powers(b["rot"]["base"], b["rot"]["dims"])
+        q, k = (_turn((h @ w(n + t, H * D, W).T).view(-1, H, D), seqs.pos, freq) for t in "qk")
+        v = (h @ w(n + "v", H * V, W).T).view(-1, H, V)
+        decay = torch.tensor(b["decay"], dtype=F, device=DEVICE).expand(h.shape[0], H)
+        o = _rms(_recur(seqs, q, k * D ** -0.5, v, decay), eps).flatten(1)
+        right = (o * _silu(h @ w(n + "g", H * V, W).T)) @ w(n + "o", W, H * V).T
+        return m["left_scale"] * left + m["right_scale"] * right
+
+    def state_space(h, p, m):
+        H, P, N, G, K = m["heads"], m["vdim"], m["state"], m["groups"], m["conv"]
+        inner, mixed = H * P, H * P + 2 * G * N
+        z, x, dt = (h @ w(p + "in", inner + mixed + H, W).T).split([inner, mixed, H], -1)
+        x = _silu(_conv(seqs, x, w(p + "conv", mixed, K)) + w(p + "conv.b", mixed))
+        v, k, q = x.split([inner, G * N, G * N], -1)
+        v = v.reshape(-1, H, P)
+        k, q = (t.reshape(-1, G, N).repeat_interleave(H // G, dim=1) for t in (k, q))
+        dt = torch.nn.functional.softplus(dt + w(p + "dt_bias", H))
+        y = _recur(seqs, q, k, v, torch.exp(-torch.exp(w(p + "A_log", H)) * dt), gain=dt) + w(p + "D", H)[:, None] * v
+        y = y.flatten(1) * _silu(z)
+        y = _rms(y.view(-1, m["norm_groups"], inner // m["norm_groups"]), eps).flatten(1) * w(p + "norm", inner)
+        return y @ w(p + "o", W, inner).T
+
+    streams = [w("embed", cfg["vocab"], W, rows=seqs.ids)] * n_streams
+
+    def sublayer(streams, name, fn):
+        read, mix, write = w(name + ".in", n_streams), w(name + ".mix", n_streams, n_streams), w(name + ".out", n_streams)
+        y = fn(sum(s * c for s, c in zip(streams, read)))
+        return [sum(s * mix[j, i] for j, s in enumerate(streams)) + write[i] * y for i in range(n_streams)]
+
+    for i, layer in enumerate(cfg["layers"]):
+        p, f = f"l{i}.", layer["mlp"]
+        mixer = parallel if layer["type"] == "parallel" else state_space
+        streams = sublayer(streams, p + "hc1", lambda u: mixer(norm(u, p + "norm1"), p + "mix.", layer["mixer"]))
+
+        def feed(u):
+            h = norm(u, p + "norm2")
+            return _routed(h, w, p + "mlp.", f, expert) + expert(h, p + "mlp.shared.", f["shared"]["ff"])
+
+        streams = sublayer(streams, p + "hc2", feed)
+    x = norm(sum(s[seqs.last] for s in streams), "final.norm")
+    return x @ w("embed", cfg["vocab"], W).T * cfg["logit_scale"]
+
+
+def exact(case, seed):
+    """The logits in 64 bits: every request as one whole sequence from its first token."""
+    cfg, fam = MODELS[case["model"]](), _family(case)
+
+    def w(name, *shape, rows=None):
+        t = _weight(seed, name, shape, fam)
+        return (t if rows is None else t[rows]).to(F)
+
+    of = {"qwen3": _qwen3_exact, "kudurax": _kudurax_exact, "karopel": _karopel_exact, "fanulix": _fanulix_exact}[fam]
+    with torch.no_grad():
+        return of(cfg, w, _Sequences(_tokens(case, seed)))
