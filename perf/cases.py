@@ -90,27 +90,27 @@ def _case(model, rows=0, context=0, prompts=0, prompt=0, history=0, ragged=False
 def listed():
     return [
         # one user, a short chat with the smallest model: bound by the number of launches
-        _case("qwen3-0.6b", rows=1, context=250, name="0.6b, 1 token"),
+        _case("qwen3-0.6b", rows=1, context=250, name="0.6b-1-token"),
         # a burst of short requests at a small model: time to the first token
-        _case("qwen3-0.6b", prompts=8, prompt=150, ragged=True, name="0.6b, 8 prompts of about 130"),
+        _case("qwen3-0.6b", prompts=8, prompt=150, ragged=True, name="0.6b-8-prompts"),
         # the headline decode steps: 8 and 64 requests behind prompts of 2,048 tokens
-        _case("qwen3-8b", rows=8, context=2048, name="8b, 8 tokens"),
-        _case("qwen3-8b", rows=64, context=2048, name="8b, 64 tokens"),
+        _case("qwen3-8b", rows=8, context=2048, name="8b-8-tokens"),
+        _case("qwen3-8b", rows=64, context=2048, name="8b-64-tokens"),
         # the headline prefill
-        _case("qwen3-8b", prompts=1, prompt=2048, name="8b, prompt of 2,048"),
+        _case("qwen3-8b", prompts=1, prompt=2048, name="8b-prompt-2048"),
         # a document of 30,000 tokens read in portions: the portion that ends it
-        _case("qwen3-8b", prompts=1, prompt=2001, history=28000, name="8b, portion behind 28,000"),
+        _case("qwen3-8b", prompts=1, prompt=2001, history=28000, name="8b-portion-behind-28000"),
         # the serving workload: a portion of 512 beside requests that decode
-        _case("qwen3-14b", rows=31, context=3072, prompts=1, prompt=512, history=1024, ragged=True, name="14b, portion of 512 beside 31"),
+        _case("qwen3-14b", rows=31, context=3072, prompts=1, prompt=512, history=1024, ragged=True, name="14b-portion-beside-31"),
         # trace replay and scoring on the 32-bit path
-        _case("qwen3-0.6b", prompts=1, prompt=500, dtype="float32", name="0.6b in 32 bits, prompt of 500"),
+        _case("qwen3-0.6b", prompts=1, prompt=500, dtype="float32", name="0.6b-32-bit-prompt"),
         # latent attention and routed experts: portions of many prompts in one step
-        _case("kudurax-2k", prompts=16, prompt=256, history=1000, name="kudurax, 16 portions of 256"),
+        _case("kudurax-2k", prompts=16, prompt=256, history=1000, name="kudurax-16-portions"),
         # one long prompt through a gated delta rule
-        _case("karopel-2k", prompts=1, prompt=2048, name="karopel, prompt of 2,048"),
+        _case("karopel-2k", prompts=1, prompt=2048, name="karopel-prompt-2048"),
         # retention, state space, routed experts: a few prompts at once, and decoding
-        _case("fanulix-2k", prompts=4, prompt=600, ragged=True, name="fanulix, 4 prompts of about 530"),
-        _case("fanulix-2k", rows=64, context=2048, ragged=True, name="fanulix, 64 tokens"),
+        _case("fanulix-2k", prompts=4, prompt=600, ragged=True, name="fanulix-4-prompts"),
+        _case("fanulix-2k", rows=64, context=2048, ragged=True, name="fanulix-64-tokens"),
     ]
 
 
