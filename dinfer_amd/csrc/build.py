@@ -31,6 +31,7 @@ SOURCES = {
     "attention": "attention.hip",
     "attention_ext": "attention_ext.hip",
     "gemm_ref": "gemm_ref.hip",
+    "f32": "f32.hip",
     "gemm": "gemm.hip",
     "gemm_mid": "gemm_mid.hip",
     "gemm_wide": "gemm_wide.hip",

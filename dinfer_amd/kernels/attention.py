@@ -1,6 +1,7 @@
 """Chooses the attention kernels for a step.
 
-float32 storage: always the plain kernel (fixed key order, any sizes).
+float32 storage: the 32-bit matrix-core kernel for the head sizes it is built for, the plain kernel for all others; a
+row's keys are visited in an order fixed by their positions in both.
 bfloat16 storage: MFMA kernels where the geometry fits them (head size from the
 instantiated list, page size a multiple of 8): split-K decode for the requests that
 bring one row, flash for the others; the plain kernel otherwise.
@@ -32,6 +33,7 @@ class Workspace:
         # keys: 1.17 -> 1.0x ms a step at one request)
         self.max_splits = max(1, min(self.max_splits, -(-longest // SHORTEST_PART)))
         self.mfma = (ctx.dtype == torch.bfloat16 and ops.attn_mfma_supports(head_dim, ctx.page_size, heads, kv_heads))
+        self.f32 = ctx.dtype == torch.float32 and ops.attn_f32_supports(head_dim, ctx.page_size, heads, kv_heads)
         self.split_k = self.mfma and heads // kv_heads <= 16
         self.part = None
         self.kv_heads = kv_heads
@@ -61,6 +63,8 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k_cache, v_cache, batc
     geo = dict(scale=scale, window=window, heads=heads, kv_heads=kv_heads, head_dim=head_dim, page_size=page_size)
     bt = batch.block_table[group]
     B, T = batch.num_reqs, batch.num_tokens
+    if ws.f32 and all(t.stride(0) % 4 == 0 and t.data_ptr() % 16 == 0 for t in (qkv, out)):
+        return ops.attn_f32(qkv, out, k_cache, v_cache, bt, batch.cu_seqlens, batch.seq_lens, B, T, batch.max_q_len, **geo)
     if not ws.mfma:
         return ops.attn_paged_ref(qkv, out, k_cache, v_cache, bt, batch.cu_seqlens, batch.seq_lens, B, T, **geo)
     singles = batch.num_singles if ws.split_k else 0

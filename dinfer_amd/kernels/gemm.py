@@ -1,7 +1,8 @@
 """Matrix products out = a . w^T.
 
-float32 operands: the vector-ALU kernel with a fixed summation order (the true
-32-bit path). bfloat16 operands: up to 32 rows the hand-written MFMA kernel that
+float32 operands (the true 32-bit path): the matrix cores' 32-bit instruction with
+a summation order fixed by k alone, or, for rows that are no whole 16-byte pieces,
+the vector-ALU kernel with an order as fixed. bfloat16 operands: up to 32 rows the hand-written MFMA kernel that
 streams the weight once (decode, LM head); beyond, the vendor library, where the
 reference uses a library too (crates/kernels/src/gemm.rs:605-647): hipBLASLt
 called directly with the algorithm measured per shape (blaslt.py); a shape it
@@ -91,7 +92,7 @@ def matmul_nt(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, may_p
     if m <= 0:
         return out
     if a.dtype == torch.float32:
-        return ops.gemm_ref(a, w, out, m)
+        return ops.gemm_f32(a, w, out, m) if ops.gemm_f32_supports(a, w) else ops.gemm_ref(a, w, out, m)
     if not a.is_cuda:
         raise RuntimeError("matrix products run on the GPU only")
     n, k = w.shape

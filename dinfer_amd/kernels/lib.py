@@ -119,6 +119,10 @@ SIGNATURES = {
         [_P, _P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _L, _P, _I, _I, _F, _I, _I, _I, _I, _I, _P, _P, _F, _F, _P, _P,
          _P, _P],
     ),
+    "dinfer_gemm_f32_supports": ("f32", [_P, _L, _P, _L, _L]),
+    "dinfer_gemm_f32": ("f32", [_P, _L, _P, _L, _P, _L, _L, _L, _L, _P]),
+    "dinfer_attn_f32_supports": ("f32", [_I, _I, _I, _I]),
+    "dinfer_attn_f32": ("f32", [_P, _L, _P, _L, _P, _P, _P, _L, _P, _P, _I, _I, _F, _I, _I, _I, _I, _I, _P]),
     "dinfer_gemm_ref": ("gemm_ref", [_I, _I, _P, _L, _P, _L, _P, _L, _L, _L, _L, _P]),
     "dinfer_gemm_small_m": ("gemm", [_I, _P, _L, _P, _L, _P, _L, _L, _L, _L, _I, _I, _P]),
     "dinfer_gemm_small_m_gated": ("gemm", [_P, _L, _P, _L, _P, _L, _L, _L, _L, _I, _P]),

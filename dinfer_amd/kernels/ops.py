@@ -1271,6 +1271,47 @@ def gemm_ref(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int) -> tor
     return out
 
 
+def gemm_f32_supports(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether gemm_f32 takes the operands: float32, 16-byte pieces along k."""
+    return (a.dtype == w.dtype == torch.float32 and a.is_cuda
+            and bool(lib.get("dinfer_gemm_f32_supports")(a.data_ptr(), _rows(a), w.data_ptr(), _rows(w), w.shape[1])))
+
+
+def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int) -> torch.Tensor:
+    """out[:m] = a[:m] @ w.T, float32 throughout, on the matrix cores' 32-bit instruction; a row's sum is the same
+    whatever m is."""
+    _need_gpu(a, w, out)
+    n, k = w.shape
+    assert a.dtype == w.dtype == out.dtype == torch.float32 and a.shape[1] == k and out.shape[1] == n
+    assert a.shape[0] >= m and out.shape[0] >= m
+    lib.call("dinfer_gemm_f32", a.data_ptr(), _rows(a), w.data_ptr(), _rows(w), out.data_ptr(), _rows(out), m, n, k, _stream())
+    return out
+
+
+def attn_f32_supports(head_dim: int, page_size: int, heads: int, kv_heads: int) -> bool:
+    return bool(lib.get("dinfer_attn_f32_supports")(head_dim, page_size, heads, kv_heads))
+
+
+def attn_f32(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
+             cu_seqlens: torch.Tensor, seq_lens: torch.Tensor, num_reqs: int, tokens: int, max_q_len: int, *, scale: float,
+             window: int, heads: int, kv_heads: int, head_dim: int, page_size: int) -> torch.Tensor:
+    """Paged attention in 32 bits on the matrix cores (sizes of attn_f32_supports); a row's result is the same however
+    the step was cut. max_q_len: at least the longest portion of the step."""
+    _need_gpu(q, out, k_cache, v_cache, block_table, cu_seqlens, seq_lens)
+    assert q.dtype == out.dtype == k_cache.dtype == v_cache.dtype == torch.float32
+    assert block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.is_contiguous()
+    assert block_table.shape[0] >= num_reqs
+    assert cu_seqlens.dtype == torch.int32 and cu_seqlens.numel() >= num_reqs + 1
+    assert seq_lens.dtype == torch.int32 and seq_lens.numel() >= num_reqs
+    _check_pages(k_cache, v_cache, kv_heads, head_dim, page_size)
+    assert q.shape[1] >= heads * head_dim and out.shape[1] >= heads * head_dim
+    assert q.shape[0] >= tokens and out.shape[0] >= tokens
+    lib.call("dinfer_attn_f32", q.data_ptr(), _rows(q), out.data_ptr(), _rows(out), k_cache.data_ptr(), v_cache.data_ptr(),
+             block_table.data_ptr(), block_table.shape[1], cu_seqlens.data_ptr(), seq_lens.data_ptr(), num_reqs, max_q_len,
+             float(scale), int(window), heads, kv_heads, head_dim, page_size, _stream())
+    return out
+
+
 def gemm_small_m(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, *, row_tiles: int = 0,
                  waves: int = 0) -> torch.Tensor:
     """out[:m] = a[:m] @ w.T for m <= 64, bf16 operands, weight streamed once (MFMA, split-K in the workgroup)."""
