@@ -18,7 +18,7 @@
 // Float operands run on the vector ALUs, every output element summed over k in ascending order by one thread (the
 // true 32-bit path; a row's result does not depend on which tile or group size it met). bf16 operands run on the
 // matrix cores, operands read straight from memory in the MFMA's own order (8 consecutive k a lane), in two forms:
-// tiles of 128 rows (a wave 64 x 64 outputs) and tiles of 16 rows whose waves split k (see the kernels).
+// tiles of 128 rows and tiles of 16 rows whose waves split k (see the kernels).
 //
 //   moe_route    two kernels: router logits in float (a wave an expert, a router row read once per 8 tokens), then per
 //                token the `top` largest (lowest index first among equals), the softmax over the chosen and the shared
@@ -38,6 +38,8 @@ struct Groups {
   void* C; int64_t ldc, c_zs;
   int M, N, K;
   const int32_t* tiles;     // experts: [max_tiles][2]
+  int max_tiles;
+  int64_t entries;          // experts: at most so many rows in all
   const int32_t* offsets;   // experts: [G + 1]
   const int32_t* perm;      // experts: sorted place -> entry
   int a_div;                // experts: > 0: A row = perm[i] / a_div; 0: A row = i
@@ -45,7 +47,7 @@ struct Groups {
   const void* gate; int64_t ld_gate;   // heads: optional
   int gate_entries;         // heads: the gate has a column an entry of C's rows (else one a head)
   int gate_n;               // GATED: rows of each half of W_g
-  int tm;                   // rows of a tile: 64 on the vector ALUs, 16 or 128 on the matrix cores
+  int tm;                   // rows of a tile: 64 on the vector ALUs; on the matrix cores 16 or 128
   int act;                  // not GATED: 0 nothing, 1 silu, 2 gelu (error function), 3 the square of relu on every result
   const float* row_scale;   // experts: a factor an entry on its row of A, or null
   int clamped; float limit, slope;     // GATED: the form with clamps
@@ -60,11 +62,15 @@ __device__ __forceinline__ float plain_act(float x, int act) {
   return x;
 }
 
+template <bool CLAMPED>
 __device__ __forceinline__ float gated_value(const Groups& p, float g, float u) {
-  if (!p.clamped) return silu(g) * u;
+  if (!CLAMPED) return silu(g) * u;
   g = fminf(g, p.limit);
   u = fminf(fmaxf(u, -p.limit), p.limit);
   return g * sigmoid(p.slope * g) * (u + 1.f);
+}
+__device__ __forceinline__ float gated_value(const Groups& p, float g, float u) {
+  return p.clamped ? gated_value<true>(p, g, u) : gated_value<false>(p, g, u);
 }
 // what entry n of row `row` of head z's block is multiplied by
 template <class S>
@@ -78,19 +84,20 @@ constexpr int BM = 64, BN = 64, BK = 16;
 struct Tile {
   int z, m0, rows;
   const int32_t* perm; int a_div, c_to_perm, base;
-  __device__ __forceinline__ bool init(const Groups& p) {
+  __device__ __forceinline__ bool init(const Groups& p) { return init(p, blockIdx.y); }
+  __device__ __forceinline__ bool init(const Groups& p, int at) {   // at: the tile's place
     const int tm = p.tm;   // rows a tile
     if (p.tiles) {
-      z = p.tiles[2 * blockIdx.y];
+      z = p.tiles[2 * at];
       if (z < 0) return false;
-      base = p.tiles[2 * blockIdx.y + 1];
+      base = p.tiles[2 * at + 1];
       m0 = 0;
       const int end = p.offsets[z + 1];
       rows = end - base < tm ? end - base : tm;
       perm = p.perm; a_div = p.a_div; c_to_perm = p.c_to_perm;
     } else {
       z = blockIdx.z;
-      m0 = blockIdx.y * tm;
+      m0 = at * tm;
       rows = p.M - m0 < tm ? p.M - m0 : tm;
       perm = nullptr; a_div = 0; c_to_perm = 0; base = m0;
     }
@@ -179,173 +186,498 @@ __global__ void __launch_bounds__(256) grouped_valu_kernel(Groups p) {
 // starting at 8 (l / 16); of the result it holds column l % 16, rows 4 (l / 16) .. + 3. Operands are read straight from
 // memory in that order (16 bytes a lane).
 //
-// Many rows (tiles of 128): a workgroup takes 128 rows x 128 columns (gated: 64 columns of each half), its waves
-// 2 x 2, a wave 64 x 64. Both operands are staged through LDS 64 k at a time (16-byte pieces, read from memory by
-// the whole workgroup once, rows gathered through the tile's row list on the way), the next step's pieces are loaded
-// into registers while this step is multiplied; four row fragments and four column fragments feed sixteen MFMAs per
-// 32 k. Every output element is still summed over ascending k by one lane.
+// Many rows a head (tiles of 128): a workgroup's four waves stand side by side over the columns, a wave 128 rows x 64
+// columns; products of up to 128 columns have them 2 x 2, a wave 64 x 64. The rows of A are staged in LDS for all waves,
+// 64 k at a time in two buffers; a wave's columns are its own, so the weights go past LDS straight into registers in the
+// MFMA's order, a step ahead. Blocks of 64 rows beyond M are skipped. The weight is the MFMA's first operand and its rows are
+// dealt so that a lane ends up with 16 consecutive columns of a row: 16-byte stores instead of 2-byte ones, which is what
+// these products are bound by (4,096 rows, 16 heads, 128 -> 512 columns each: 81 -> 31 us for 84 MB; 512 -> 128: 33 -> 26).
+// Every output element is summed over ascending k by one lane.
 constexpr int TM_BIG = 128, TM_SMALL = 16;
 
-constexpr int BIG_K = 64;            // k a step
-constexpr int BIG_LD = BIG_K + 8;    // row of a staged tile in LDS, padded: rows 16 bytes apart in the banks
+constexpr int BIG_K = 64;            // k a step; a staged row is 128 bytes, its 16-byte pieces exchanged by the row's bits 1..3
 
-template <class O, bool GATED>
-__global__ void __launch_bounds__(256) grouped_mfma_big_kernel(Groups p) {
+// LDS is written and read around this; loads from memory stay in flight across it (__syncthreads would wait for them)
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// what becomes of a sum: an instance each (with all of them in one, the 128 results of a lane are 25,000 instructions)
+enum : int { END_PLAIN, END_SILU, END_GELU, END_RELU2, END_HEAD_GATE, END_ENTRY_GATE, END_GATED, END_GATED_CLAMPED };
+
+// A wave's block of 64 rows (from row m0 of the tile on): lane l holds, of rows 16 i + l % 16, the 16 columns from
+// c0 + 16 (l / 16) on.
+template <class O, int END>
+__device__ __forceinline__ void store_block(const Groups& p, const Tile& tl, O* C, int m0, int c0, const f32x4 (&acc)[4][4]) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, kq = lane >> 4;
+  const int n = c0 + kq * 16;   // a lane's first column
+  const bool pieces = sizeof(O) == 2 && p.ldc % 8 == 0 && ((uintptr_t)C & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = m0 + i * 16 + lr;
+    if (row >= tl.rows || n >= p.N) continue;
+    const int64_t cr = tl.c_row(row);
+    const float g1 = END == END_HEAD_GATE ? head_gate<bf16>(p, cr, tl.z, 0) : 1.f;
+    O* c = C + cr * p.ldc + n;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {   // 8 columns at a time
+      if (n + 8 * e >= p.N) continue;
+      float v[8];
+#pragma unroll
+      for (int x = 0; x < 8; ++x) {
+        v[x] = acc[i][2 * e + (x >> 2)][x & 3] * g1;
+        if (END == END_ENTRY_GATE) v[x] *= n + 8 * e + x < p.N ? head_gate<bf16>(p, cr, tl.z, n + 8 * e + x) : 0.f;
+      }
+      if (pieces && n + 8 * e + 8 <= p.N) {
+        bf16x8 o;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) o[x] = (bf16)v[x];
+        *(bf16x8*)(c + 8 * e) = o;
+      } else {
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+          if (n + 8 * e + x < p.N) c[8 * e + x] = from_f32<O>(v[x]);
+      }
+    }
+  }
+}
+
+template <class O, int END, int WM>
+__global__ void __launch_bounds__(256, 2) grouped_mfma_big_kernel(Groups p) {
+  constexpr int WN = 4 / WM, HALVES = 2 / WM;   // waves side by side; blocks of 64 rows a wave
+  constexpr int COLS = 64;                      // columns of C a wave
   __shared__ int64_t arow[TM_BIG];
-  __shared__ __attribute__((aligned(16))) bf16 As[TM_BIG * BIG_LD];
-  __shared__ __attribute__((aligned(16))) bf16 Ws[128 * BIG_LD];
+  __shared__ __attribute__((aligned(16))) bf16 As[2][TM_BIG * BIG_K];
   Tile tl;
   if (!tl.init(p)) return;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int n0 = blockIdx.x * (GATED ? 64 : 128);
-  const bool experts = p.tiles != nullptr;
-  const bf16* A = (const bf16*)p.A + (experts ? 0 : (int64_t)tl.z * p.a_zs);
+  const int wm = wave / WN, wn = wave % WN;
+  const int lr = lane & 15, kq = lane >> 4;
+  const int c0 = (blockIdx.x * WN + wn) * COLS;   // this wave's first column
+  const bf16* A = (const bf16*)p.A + (int64_t)tl.z * p.a_zs;
   const bf16* W = (const bf16*)p.W + (int64_t)tl.z * p.w_zs;
-  if (threadIdx.x < TM_BIG) arow[threadIdx.x] = threadIdx.x < tl.rows ? tl.a_row(threadIdx.x) : -1;
+  const int K = p.K;   // a multiple of 8 (checked on the host)
+  if (threadIdx.x < TM_BIG) arow[threadIdx.x] = tl.a_row(threadIdx.x < tl.rows ? threadIdx.x : 0);   // rows beyond: computed, not stored
   __syncthreads();
-  // staging: a tile is 128 rows x 64 k = 1,024 pieces of 16 bytes, four a thread for each operand; piece q of a thread
-  // is row (q * 256 + thread) / 8, k piece (thread % 8)
+
+  // staging: 128 rows x 64 k = 1,024 pieces of 16 bytes, four a thread; piece q of a thread is row (q * 256 + thread) / 8
   const int sp = threadIdx.x & 7;
   const bf16* ag[4];
-  const bf16* wg[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int row = (q * 256 + threadIdx.x) >> 3;
-    const int64_t ar = arow[row];
-    ag[q] = ar >= 0 ? A + ar * p.lda + sp * 8 : nullptr;
-    // row of the weight behind row `row` of the staged tile; gated: 64 gate rows, then the 64 up rows of the same numbers
-    const int gn = GATED ? n0 + (row & 63) : n0 + row;
-    const int64_t wrow = GATED && row >= 64 ? gn + p.gate_n : gn;
-    wg[q] = gn < p.N ? W + wrow * p.ldw + sp * 8 : nullptr;
-  }
+  for (int q = 0; q < 4; ++q) ag[q] = A + arow[(q * 256 + threadIdx.x) >> 3] * p.lda;
+  bf16x8 an[4];
   bf16x8 zero;
 #pragma unroll
   for (int i = 0; i < 8; ++i) zero[i] = (bf16)0.f;
-  const int K = p.K;   // a multiple of 8 (checked on the host)
-  bf16x8 an[4], wn_[4];
-  auto fetch = [&](int k0) {
-    const bool in = k0 + sp * 8 < K;
+  auto fetch = [&](int k0) {   // (pieces past K are read at K - 8 and cleared on their way into LDS)
+    const int k = min(k0 + sp * 8, K - 8);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      an[q] = (ag[q] && in) ? *(const bf16x8*)(ag[q] + k0) : zero;
-      wn_[q] = (wg[q] && in) ? *(const bf16x8*)(wg[q] + k0) : zero;
-    }
+    for (int q = 0; q < 4; ++q) an[q] = *(const bf16x8*)(ag[q] + k);
   };
-  const int lr = lane & 15, kq = lane >> 4;
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += BIG_K) {
-    __syncthreads();      // the step before has read the tiles
+  auto put = [&](int buf, int k0) {
+    const bool tail = k0 + BIG_K > K, in = k0 + sp * 8 < K;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int row = (q * 256 + threadIdx.x) >> 3;
-      *(bf16x8*)(As + row * BIG_LD + sp * 8) = an[q];
-      *(bf16x8*)(Ws + row * BIG_LD + sp * 8) = wn_[q];
+      if (tail) an[q] = in ? an[q] : zero;
+      *(bf16x8*)(As[buf] + row * BIG_K + ((sp ^ (row >> 1)) & 7) * 8) = an[q];
     }
-    __syncthreads();
-    if (k0 + BIG_K < K) fetch(k0 + BIG_K);    // the next step's pieces travel while this one is multiplied
+  };
+  // the weight's row behind row lr of tile j: a lane's results of all tiles are consecutive columns
+  const bf16* wrow[4];
 #pragma unroll
-    for (int kk = 0; kk < BIG_K; kk += 32) {
-      bf16x8 a[4], w[4];
+  for (int j = 0; j < 4; ++j) {
+    const int n = c0 + (lr >> 2) * 16 + j * 4 + (lr & 3);
+    wrow[j] = W + (int64_t)min(n, p.N - 1) * p.ldw;
+  }
+  bf16x8 w[2][2][4];   // [step's parity][32 k][tile]
+  auto weights = [&](int k0, bf16x8(&f)[2][4]) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = *(const bf16x8*)(As + (wm * 64 + i * 16 + lr) * BIG_LD + kk + kq * 8);
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        // gated: fragments 0, 1 are gate columns, 2, 3 the up columns of the same numbers
-        const int row = GATED ? (j >> 1) * 64 + wn * 32 + (j & 1) * 16 + lr : wn * 64 + j * 16 + lr;
-        w[j] = *(const bf16x8*)(Ws + row * BIG_LD + kk + kq * 8);
+      for (int kk = 0; kk < 2; ++kk) f[kk][j] = *(const bf16x8*)(wrow[j] + min(k0 + kk * 32 + kq * 8, K - 8));
+  };
+  f32x4 acc[HALVES][4][4];
+#pragma unroll
+  for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[h][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int live = c0 < p.N ? (tl.rows - wm * 64 * HALVES + 63) / 64 : 0;   // blocks of 64 rows that hold any
+
+  fetch(0);
+  weights(0, w[0]);
+  put(0, 0);
+  lds_barrier();
+  for (int k0 = 0; k0 < K; k0 += 2 * BIG_K) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int k = k0 + b * BIG_K;
+      if (k >= K) break;
+      fetch(k + BIG_K);
+      weights(k + BIG_K, w[b ^ 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (k + BIG_K > K) {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[b][kk][j] = k + kk * 32 + kq * 8 < K ? w[b][kk][j] : zero;
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int h = 0; h < HALVES; ++h) {
+        if (h >= live) continue;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], w[j], acc[i][j], 0, 0, 0);
+        for (int kk = 0; kk < 2; ++kk) {
+          bf16x8 a[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            a[i] = *(const bf16x8*)(As[b] + ((wm * HALVES + h) * 64 + i * 16 + lr) * BIG_K + (((kk * 4 + kq) ^ (lr >> 1)) & 7) * 8);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              acc[h][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[b][kk][j], a[i], acc[h][i][j], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (k + BIG_K < K) put(b ^ 1, k + BIG_K);
+      lds_barrier();
     }
   }
-  O* C = (O*)p.C + (experts ? 0 : (int64_t)tl.z * p.c_zs);
+  O* C = (O*)p.C + (int64_t)tl.z * p.c_zs;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int h = 0; h < HALVES; ++h)
+    if (h < live) store_block<O, END>(p, tl, C, (wm * HALVES + h) * 64, c0, acc[h]);
+}
+
+// Many rows an expert (tiles of 128): a workgroup's four waves stand side by side over the columns, a wave all 128 rows x
+// 64 columns (gated: 32 of each half) in v_mfma_f32_32x32x16_bf16, which the matrix cores take at 2.0 PFLOP/s where the
+// 16 x 16 form, two instructions for as much, is bound by their issue at 1.35. The rows of A, gathered through the tile's
+// row list, go through registers into two LDS buffers for all waves; the wave's own weights past LDS straight into
+// registers; both a step of 64 k ahead. Blocks of 32 rows that a tile does not fill are skipped. Two workgroups a CU: with
+// tiles of 256 rows and everything two steps ahead, one workgroup a CU, a workgroup's beginning and end stood alone (106 us
+// of 484) and loads, LDS and MFMAs added up.
+//
+// Four lanes that follow each other read 64 bytes of a weight row in one piece (in the MFMA's own order, a row a lane, each
+// lane's 16 bytes are an access of the load path), so a tile of 32 weight rows x 64 k arrives as four instructions of
+// 8 rows x 128 bytes: instruction r, lane (g b1 b0 h c1 c0) holds piece 4 g + c of the row numbered (b h r) in the MFMA. Two
+// exchanges of a lane bit with a bit of the register's number turn that into MFMA c's operand, lane (g b1 b0 h r1 r0). The
+// weight is the MFMA's first operand and its row (b h r) is column 16 h + 4 b + r: a lane ends up with 16 consecutive
+// columns of a row, 16-byte stores.
+//
+// 64 experts of 1,408 in a width of 2,048, 6 a token: gate/up of 4,096 tokens 586 -> 442 us (641 TFLOP/s), down 366 -> 245;
+// one product of 2,023 tokens 213 -> 160, down 207 -> 127; of 512 tokens 128 -> 97 (the form before: both operands through one
+// LDS buffer, 16 x 16 MFMAs, 2-byte stores). Loads alone take 195 of the 442 us, the MFMAs alone about 230: the two waves of
+// a SIMD overlap them in part.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+template <bool SECOND>   // lane bit 0 (SECOND: bit 1) changes places with the choice between x0 and x1
+__device__ __forceinline__ void swap_in_quads(u32x4& x0, u32x4& x1) {
+  u32x4 y0, y1;
+  // v_cndmask: the second source where vcc is set, else the first, which the DPP takes from the partner lane
+#define DINFER_QUADS(perm, even, odd)                                                                      \
+  asm("s_mov_b32 vcc_lo, " even "\n\ts_mov_b32 vcc_hi, " even "\n\ts_nop 1\n\t"                           \
+      "v_cndmask_b32_dpp %0, %12, %8, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"               \
+      "v_cndmask_b32_dpp %1, %13, %9, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"               \
+      "v_cndmask_b32_dpp %2, %14, %10, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"              \
+      "v_cndmask_b32_dpp %3, %15, %11, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"              \
+      "s_mov_b32 vcc_lo, " odd "\n\ts_mov_b32 vcc_hi, " odd "\n\t"                                        \
+      "v_cndmask_b32_dpp %4, %8, %12, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"               \
+      "v_cndmask_b32_dpp %5, %9, %13, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"               \
+      "v_cndmask_b32_dpp %6, %10, %14, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"              \
+      "v_cndmask_b32_dpp %7, %11, %15, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\ts_nop 1"       \
+      : "=&v"(y0[0]), "=&v"(y0[1]), "=&v"(y0[2]), "=&v"(y0[3]), "=&v"(y1[0]), "=&v"(y1[1]), "=&v"(y1[2]),  \
+        "=&v"(y1[3])                                                                                       \
+      : "v"(x0[0]), "v"(x0[1]), "v"(x0[2]), "v"(x0[3]), "v"(x1[0]), "v"(x1[1]), "v"(x1[2]), "v"(x1[3])     \
+      : "vcc")
+  if (SECOND) DINFER_QUADS("[2,3,0,1]", "0x33333333", "0xcccccccc");
+  else DINFER_QUADS("[1,0,3,2]", "0x55555555", "0xaaaaaaaa");
+#undef DINFER_QUADS
+  x0 = y0;
+  x1 = y1;
+}
+
+// 32 rows of a wave (from row m0 of the tile on): a lane holds, of row m0 + lane % 32, 16 columns from n0 + 16 (lane / 32)
+// on of the wave's two tiles of columns (gated: of the same columns of both halves).
+template <class O, int END>
+__device__ __forceinline__ void store_rows(const Groups& p, const Tile& tl, int m0, int c0, const f32x16 (&acc)[2]) {
+  constexpr bool GATED = END >= END_GATED;
+  const int lane = threadIdx.x & 63, row = m0 + (lane & 31);
+  if (row >= tl.rows) return;
+  const float rs = tl.scale_of(p, row);
+  O* c = (O*)p.C + tl.c_row(row) * p.ldc;
+  const bool pieces = sizeof(O) == 2 && p.ldc % 8 == 0 && ((uintptr_t)p.C & 15) == 0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = wm * 64 + i * 16 + kq * 4 + r;
-      if (row >= tl.rows) continue;
-      const int64_t cr = tl.c_row(row);
-      const float g1 = p.gate_entries ? 1.f : head_gate<bf16>(p, cr, tl.z, 0);
-      const float rs = tl.scale_of(p, row);
+  for (int j = 0; j < (GATED ? 1 : 2); ++j)
 #pragma unroll
-      for (int j = 0; j < (GATED ? 2 : 4); ++j) {
-        const int gn = GATED ? n0 + wn * 32 + j * 16 + lr : n0 + wn * 64 + j * 16 + lr;
-        if (gn < p.N) {
-          const float v = GATED ? gated_value(p, acc[i][j][r] * rs, acc[i][(j + 2) & 3][r] * rs) : plain_act(acc[i][j][r] * rs, p.act);
-          C[cr * p.ldc + gn] = from_f32<O>(v * (p.gate_entries ? head_gate<bf16>(p, cr, tl.z, gn) : g1));
-        }
+    for (int e = 0; e < 2; ++e) {   // 8 columns at a time
+      const int n = c0 + 32 * j + 16 * (lane >> 5) + 8 * e;
+      if (n >= p.N) continue;
+      float v[8];
+#pragma unroll
+      for (int x = 0; x < 8; ++x)
+        v[x] = GATED ? gated_value<END == END_GATED_CLAMPED>(p, acc[0][8 * e + x] * rs, acc[1][8 * e + x] * rs)
+                     : plain_act(acc[j][8 * e + x] * rs, END);
+      if (pieces && n + 8 <= p.N) {
+        bf16x8 o;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) o[x] = (bf16)v[x];
+        *(bf16x8*)(c + n) = o;
+      } else {
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+          if (n + x < p.N) c[n + x] = from_f32<O>(v[x]);
       }
     }
 }
 
-// Few rows (tiles of 16: steps of single tokens): time is the time to stream the weights, so a workgroup takes only 16
-// columns (gated: of each half) and its four waves take a quarter of k each; their partial sums meet in LDS and are
-// added in wave order.
-template <class O, bool GATED>
-__global__ void __launch_bounds__(256) grouped_mfma_small_kernel(Groups p) {
-  __shared__ int64_t arow[TM_SMALL];
-  __shared__ float part[4][GATED ? 2 : 1][16][17];
+template <class O, int END>
+__global__ void __launch_bounds__(256, 2) grouped_mfma_experts_kernel(Groups p) {
+  constexpr bool GATED = END >= END_GATED;
+  constexpr int COLS = GATED ? 32 : 64, PIECES = TM_BIG / 32, BLOCKS = TM_BIG / 32;
+  __shared__ int64_t arow[TM_BIG];
+  __shared__ __attribute__((aligned(16))) bf16 As[2][TM_BIG * BIG_K];
+  // An XCD (the workgroups of one linear id modulo 8) walks its own run of the sorted tiles, four at a time with the
+  // columns outside: tiles of one expert that run together read its weights once from memory and then from L2.
+  int bx, by;
+  {
+    const int nx = gridDim.x, id = blockIdx.y * nx + blockIdx.x, slot = id >> 3, r = slot % (4 * nx);
+    bx = r >> 2;
+    by = (slot / (4 * nx) * 4 + (r & 3)) * 8 + (id & 7);
+    if (by >= p.max_tiles) return;
+  }
   Tile tl;
-  if (!tl.init(p)) return;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int n0 = blockIdx.x * 16;
-  const bool experts = p.tiles != nullptr;
-  const bf16* A = (const bf16*)p.A + (experts ? 0 : (int64_t)tl.z * p.a_zs);
+  if (!tl.init(p, by)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;   // (scalar: offsets and branches that depend on it)
+  const int c0 = (bx * 4 + wave) * COLS;        // this wave's first column
+  const bf16* A = (const bf16*)p.A;
   const bf16* W = (const bf16*)p.W + (int64_t)tl.z * p.w_zs;
-  if (threadIdx.x < TM_SMALL) arow[threadIdx.x] = threadIdx.x < tl.rows ? tl.a_row(threadIdx.x) : -1;
+  const int K = p.K;   // a multiple of 8 (checked on the host)
+  if (threadIdx.x < TM_BIG) arow[threadIdx.x] = tl.a_row(threadIdx.x < tl.rows ? threadIdx.x : 0);   // rows beyond: computed, not stored
   __syncthreads();
-  const int lr = lane & 15, kq = lane >> 4;
-  const int64_t ar = arow[lr];
-  const int gn = n0 + lr;
-  const bf16* ap = ar >= 0 ? A + ar * p.lda + kq * 8 : nullptr;
-  const bf16* wp = gn < p.N ? W + (int64_t)gn * p.ldw + kq * 8 : nullptr;
-  const bf16* up = (GATED && gn < p.N) ? W + (int64_t)(gn + p.gate_n) * p.ldw + kq * 8 : nullptr;
+
+  // staging: 256 rows x 64 k = 2,048 pieces of 16 bytes, eight a thread; piece q of a thread is row (q * 256 + thread) / 8.
+  // A staged row is 128 bytes, its pieces exchanged by bits 1..3 of the row's number: no bank is met twice
+  const int sp = threadIdx.x & 7;
+  const bf16* ag[PIECES];
+#pragma unroll
+  for (int q = 0; q < PIECES; ++q) ag[q] = A + arow[(q * 256 + threadIdx.x) >> 3] * p.lda;
   bf16x8 zero;
 #pragma unroll
   for (int i = 0; i < 8; ++i) zero[i] = (bf16)0.f;
-  const int K = p.K;
-  const int steps = (K + 31) / 32, per = (steps + 3) / 4;
-  const int k_lo = wave * per * 32, k_hi = (wave + 1) * per * 32 < K ? (wave + 1) * per * 32 : K;
-  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f}, acu = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int k0 = k_lo; k0 < k_hi; k0 += 32) {
-    const bool in = k0 + kq * 8 < K;
-    const bf16x8 a = (ap && in) ? *(const bf16x8*)(ap + k0) : zero;
-    const bf16x8 w = (wp && in) ? __builtin_nontemporal_load((const bf16x8*)(wp + k0)) : zero;
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w, acc, 0, 0, 0);
-    if (GATED) {
-      const bf16x8 u = (up && in) ? __builtin_nontemporal_load((const bf16x8*)(up + k0)) : zero;
-      acu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, u, acu, 0, 0, 0);
+  bf16x8 an[PIECES];
+  auto fetch = [&](int k0, bf16x8(&f)[PIECES]) {   // (pieces past K are read at K - 8 and cleared on their way into LDS)
+    const int k = min(k0 + sp * 8, K - 8);
+#pragma unroll
+    for (int q = 0; q < PIECES; ++q) f[q] = *(const bf16x8*)(ag[q] + k);
+  };
+  auto put = [&](int buf, int k0, bf16x8(&f)[PIECES]) {
+    if (k0 + BIG_K > K) {
+      const bool in = k0 + sp * 8 < K;
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q) f[q] = in ? f[q] : zero;
+    }
+#pragma unroll
+    for (int q = 0; q < PIECES; ++q) {
+      const int row = (q * 256 + threadIdx.x) >> 3;
+      *(bf16x8*)(As[buf] + row * BIG_K + ((sp ^ (row >> 1)) & 7) * 8) = f[q];
+    }
+  };
+  // (buffer loads: a row's offset is one register, what lies beyond the expert's rows reads as zero)
+  const __amdgpu_buffer_rsrc_t wd = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, (int)(p.w_zs * 2), 0x00020000);
+  const int w_lane = (16 * ((lane >> 2) & 1) + 4 * ((lane >> 3) & 3)) * (int)p.ldw * 2 + ((lane >> 5) * 4 + (lane & 3)) * 16;
+  u32x4 w[2][2][4];   // [step's parity][tile of 32 columns][instruction, then MFMA]
+  auto weights = [&](int k0, u32x4(&f)[2][4]) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = c0 + (GATED ? j * p.gate_n : 32 * j) + r;
+        f[j][r] = __builtin_amdgcn_raw_buffer_load_b128(wd, w_lane, (n * (int)p.ldw + k0) * 2, 0);
+      }
+  };
+  auto order = [&](u32x4(&f)[4], int step) {   // four parts of a tile's way into the MFMA's order
+    if (step == 0) swap_in_quads<false>(f[0], f[1]);
+    if (step == 1) swap_in_quads<false>(f[2], f[3]);
+    if (step == 2) swap_in_quads<true>(f[0], f[2]);
+    if (step == 3) swap_in_quads<true>(f[1], f[3]);
+  };
+  f32x16 acc[BLOCKS][2];
+#pragma unroll
+  for (int h = 0; h < BLOCKS; ++h)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[h][j][i] = 0.f;
+  const int live = c0 < p.N ? (tl.rows + 31) / 32 : 0;   // blocks of 32 rows that hold any
+
+  fetch(0, an);
+  weights(0, w[0]);
+  put(0, 0, an);
+#pragma unroll
+  for (int x = 0; x < 8; ++x) order(w[0][x >> 2], x & 3);
+  lds_barrier();
+  for (int k0 = 0; k0 < K; k0 += 2 * BIG_K) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int k = k0 + b * BIG_K;
+      if (k >= K) break;
+      // block h's fragments: rows 32 h + lane % 32, MFMA t's piece 4 (lane / 32) + t
+      auto rows = [&](int h, bf16x8(&f)[4]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          f[t] = *(const bf16x8*)(As[b] + (h * 32 + (lane & 31)) * BIG_K + ((((lane >> 5) * 4 + t) ^ (lane >> 1)) & 7) * 8);
+      };
+      fetch(k + BIG_K, an);
+      weights(k + BIG_K, w[b ^ 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (k + BIG_K > K) {   // what lies past K
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[b][j][t][i] = k + ((lane >> 5) * 4 + t) * 8 < K ? w[b][j][t][i] : 0u;
+      }
+#pragma unroll
+      for (int h = 0; h < BLOCKS; ++h) {
+        if (h >= live) break;
+        bf16x8 a[4];
+        rows(h, a);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[h][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[b][j][t]), a[t], acc[h][j], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (k + BIG_K < K) put(b ^ 1, k + BIG_K, an);
+#pragma unroll
+      for (int x = 0; x < 8; ++x) order(w[b ^ 1][x >> 2], x & 3);
+      lds_barrier();
     }
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    part[wave][0][kq * 4 + r][lr] = acc[r];
-    if (GATED) part[wave][GATED ? 1 : 0][kq * 4 + r][lr] = acu[r];
-  }
-  __syncthreads();
-  const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
-  if (row >= tl.rows || n0 + col >= p.N) return;
-  float v = 0.f, u = 0.f;
+  for (int h = 0; h < BLOCKS; ++h)
+    if (h < live) store_rows<O, END>(p, tl, h * 32, c0, acc[h]);
+}
+
+// Few rows (tiles of 16: steps of single tokens): time is the time to stream the weights, so a workgroup takes only 32
+// columns (gated: of each half) and its four waves deal the steps of 64 k among themselves; their partial sums meet in LDS
+// and are added in wave order. Both operands come in whole 128-byte lines, eight rows an instruction, and reach the MFMA's
+// order as the weights above do (in that order from the start, 16 bytes a lane each from a row of its own, the load path
+// took 64 accesses an instruction and gave 3.5 TB/s); DEPTH steps are in flight. The tile's rows are the even columns of the
+// 32-wide MFMA, so that their two instructions r = 0, 2 bring them (the odd columns compute nothing of use: the matrix
+// cores idle here). All 64 experts of 1,408 in a width of 2,048 at 64 tokens: one
+// product 101 -> 65 us (5.7 TB/s), 106 -> 67, gate/up 209 -> 113 (6.5 TB/s); at 8 tokens 53 -> 39 and 113 -> 67; at one token,
+// 6 experts, 13.7 -> 14.5, 11.4 -> 11.2 and 25.7 -> 20.0 (a step less in flight 68 us at 64 tokens, one more 78: registers for
+// a wave a SIMD fewer).
+template <class O, bool GATED, int NW>
+__global__ void __launch_bounds__(NW * 64) grouped_mfma_small_kernel(Groups p) {
+  constexpr int HALVES = GATED ? 2 : 1, DEPTH = GATED || NW == 8 ? 2 : 3, COLS = 32;
+  __shared__ int64_t arow[TM_SMALL];
+  __shared__ float part[NW][HALVES][TM_SMALL][COLS + 1];
+  Tile tl;
+  if (!tl.init(p)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int n0 = blockIdx.x * COLS;
+  const bool experts = p.tiles != nullptr;
+  const bf16* A = (const bf16*)p.A + (experts ? 0 : (int64_t)tl.z * p.a_zs);
+  const bf16* W = (const bf16*)p.W + (int64_t)tl.z * p.w_zs;
+  const int K = p.K, piece = (lane >> 5) * 4 + (lane & 3);
+  const bf16 *ap[2], *wp[HALVES][4];
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    v += part[w][0][row][col];
-    if (GATED) u += part[w][GATED ? 1 : 0][row][col];
+  for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      wp[h][r] = W + (int64_t)(min(n0 + 16 * ((lane >> 2) & 1) + 4 * ((lane >> 3) & 3) + r, p.N - 1) + h * p.gate_n) * p.ldw;
+  if (threadIdx.x < TM_SMALL) arow[threadIdx.x] = tl.a_row(min((int)threadIdx.x, tl.rows - 1));   // rows beyond: computed, not stored
+  __syncthreads();
+  // MFMA column 4 * (lane bits 4..2) + r holds row column / 2 of the tile
+#pragma unroll
+  for (int r = 0; r < 2; ++r) ap[r] = A + arow[2 * ((lane >> 2) & 7) + r] * p.lda;
+  const u32x4 none = {0u, 0u, 0u, 0u};
+  u32x4 a[DEPTH][2], w[DEPTH][HALVES][4];
+  auto fetch = [&](int step, int d) {   // (pieces past K are read at K - 8 and cleared when they are used)
+    const int k = min(step * 64 + piece * 8, K - 8);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) a[d][r] = *(const u32x4*)(ap[r] + k);
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) w[d][h][r] = __builtin_nontemporal_load((const u32x4*)(wp[h][r] + k));
+  };
+  auto order = [&](u32x4(&f)[4]) {
+    swap_in_quads<false>(f[0], f[1]);
+    swap_in_quads<false>(f[2], f[3]);
+    swap_in_quads<true>(f[0], f[2]);
+    swap_in_quads<true>(f[1], f[3]);
+  };
+  f32x16 acc[HALVES];
+#pragma unroll
+  for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[h][i] = 0.f;
+  const int steps = (K + 63) / 64, per = (steps + NW - 1) / NW;
+  const int lo = wave * per, hi = min(lo + per, steps);
+  if (lo < hi) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) fetch(min(lo + d, hi - 1), d);
+    for (int s0 = lo; s0 < hi; s0 += DEPTH) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        const int s = s0 + d;
+        if (s >= hi) break;
+        u32x4 fa[4] = {a[d][0], none, a[d][1], none}, fw[HALVES][4];
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) fw[h][r] = w[d][h][r];
+        if (s * 64 + 64 > K && s * 64 + piece * 8 >= K) {
+          fa[0] = fa[2] = none;
+#pragma unroll
+          for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) fw[h][r] = none;
+        }
+        order(fa);
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) order(fw[h]);
+        if (s + DEPTH < hi) fetch(s + DEPTH, d);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int h = 0; h < HALVES; ++h)
+            acc[h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fw[h][t]), __builtin_bit_cast(bf16x8, fa[t]), acc[h], 0, 0, 0);
+      }
+    }
   }
-  const int64_t cr = tl.c_row(row);
-  const float g = head_gate<bf16>(p, cr, tl.z, n0 + col);
+  if (!(lane & 1))   // an even column: row (lane % 32) / 2, columns 16 (lane / 32) + i
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) part[wave][h][(lane & 31) >> 1][16 * (lane >> 5) + i] = acc[h][i];
+  __syncthreads();
   O* C = (O*)p.C + (experts ? 0 : (int64_t)tl.z * p.c_zs);
-  const float rs = tl.scale_of(p, row);
-  C[cr * p.ldc + n0 + col] = from_f32<O>((GATED ? gated_value(p, v * rs, u * rs) : plain_act(v * rs, p.act)) * g);
+#pragma unroll
+  for (int e = 0; e < 8 / NW; ++e) {
+    const int row = e * 2 * NW + (threadIdx.x >> 5), col = threadIdx.x & 31;
+    if (row >= tl.rows || n0 + col >= p.N) continue;
+    float v = 0.f, u = 0.f;
+#pragma unroll
+    for (int x = 0; x < NW; ++x) {
+      v += part[x][0][row][col];
+      if (GATED) u += part[x][HALVES - 1][row][col];
+    }
+    const int64_t cr = tl.c_row(row);
+    const float g = head_gate<bf16>(p, cr, tl.z, n0 + col);
+    const float rs = tl.scale_of(p, row);
+    C[cr * p.ldc + n0 + col] = from_f32<O>((GATED ? gated_value(p, v * rs, u * rs) : plain_act(v * rs, p.act)) * g);
+  }
 }
 
 // ---- routing ---------------------------------------------------------------------------------------------------
@@ -525,10 +857,15 @@ __global__ void __launch_bounds__(1024) moe_scatter_kernel(const int32_t* __rest
   }
   __syncthreads();
   for (int e = threadIdx.x; e <= E; e += blockDim.x) offsets[e] = off[e];
+  // tiles of many rows: the list is dealt to the eight XCDs in runs of the sorted tiles, run c at places c, c + 8, ...: the
+  // first `rest` runs hold q + 1 tiles, the others q (tiles of few rows, mostly one an expert, stay in order)
+  const int runs = tile_rows == TM_BIG ? 8 : 1;
+  const int q = tbase[E] / runs, rest = tbase[E] % runs, long_end = rest * (q + 1);
   for (int e = threadIdx.x; e < E; e += blockDim.x) {
     const int n = tbase[e + 1] - tbase[e];
     for (int k = 0; k < n; ++k) {
-      const int at = tbase[e] + k;
+      const int t = tbase[e] + k;
+      const int at = runs * (t < long_end ? t % (q + 1) : (t - long_end) % max(q, 1)) + (t < long_end ? t / (q + 1) : rest + (t - long_end) / max(q, 1));
       if (at < max_tiles) { tiles[2 * at] = e; tiles[2 * at + 1] = off[e] + k * tile_rows; }
     }
     cnt[e] = 0;   // now the cursor
@@ -566,7 +903,6 @@ inline bool mfma_fits(int dtype, const Groups& p) {
          ((uintptr_t)p.A % 16) == 0 && ((uintptr_t)p.W % 16) == 0;
 }
 
-// grid.x is set here from the kernel's columns a workgroup; grid.y / z arrive from the caller (tiles, groups).
 // bf16 rows whose width is a multiple of 8: a thread takes 8 consecutive entries of every chosen expert's row.
 __global__ void __launch_bounds__(256) moe_combine_bf16x8_kernel(const bf16* __restrict__ y, int64_t ld_y,
                                                                  const float* __restrict__ share, int top,
@@ -600,16 +936,44 @@ __global__ void __launch_bounds__(256) moe_combine_bf16x8_kernel(const bf16* __r
   }
 }
 
+// grid.y arrives from the caller (tiles or blocks of rows), grid.z too (groups); grid.x is set here from the kernel's
+// columns a workgroup.
+template <int END>
+void launch_experts(const Groups& p, unsigned gy, hipStream_t stream) {
+  const int cols = END >= END_GATED ? 128 : 256;
+  gy = (gy + 31) / 32 * 32;   // eight XCDs, four tiles at a time
+  grouped_mfma_experts_kernel<bf16, END><<<dim3((unsigned)((p.N + cols - 1) / cols), gy), 256, 0, stream>>>(p);
+}
+template <int END>
+void launch_big(const Groups& p, unsigned gy, unsigned gz, hipStream_t stream) {
+  // up to 128 columns four waves side by side would leave half of them without any
+  if (p.N > 128)
+    grouped_mfma_big_kernel<bf16, END, 1><<<dim3((unsigned)((p.N + 255) / 256), gy, gz), 256, 0, stream>>>(p);
+  else
+    grouped_mfma_big_kernel<bf16, END, 2><<<dim3(1, gy, gz), 256, 0, stream>>>(p);
+}
+
 template <bool GATED>
 int launch_groups(int dtype, Groups p, unsigned gy, unsigned gz, hipStream_t stream) {
   if (dtype != DT_F32 && dtype != DT_BF16) return ERR_BAD_DTYPE;
   if (mfma_fits(dtype, p) && p.tm == TM_SMALL) {
-    const dim3 grid((unsigned)((p.N + 15) / 16), gy, gz);
-    grouped_mfma_small_kernel<bf16, GATED><<<grid, 256, 0, stream>>>(p);
-  } else if (mfma_fits(dtype, p) && p.tm == TM_BIG) {
-    const int cols = GATED ? 64 : 128;
-    const dim3 grid((unsigned)((p.N + cols - 1) / cols), gy, gz);
-    grouped_mfma_big_kernel<bf16, GATED><<<grid, 256, 0, stream>>>(p);
+    const dim3 grid((unsigned)((p.N + 31) / 32), gy, gz);
+    // fewer than two workgroups a CU: eight waves share a workgroup's k (one token, 6 experts: 14.8 -> 14.5, 12.5 -> 11.2 us)
+    if (!GATED && p.tiles && p.entries * grid.x < 512) grouped_mfma_small_kernel<bf16, GATED, 8><<<grid, 512, 0, stream>>>(p);
+    else grouped_mfma_small_kernel<bf16, GATED, 4><<<grid, 256, 0, stream>>>(p);
+  } else if (mfma_fits(dtype, p) && p.tiles && p.tm == TM_BIG) {
+    switch (GATED ? (p.clamped ? END_GATED_CLAMPED : END_GATED) : p.act) {
+      case END_PLAIN: launch_experts<END_PLAIN>(p, gy, stream); break;
+      case END_SILU: launch_experts<END_SILU>(p, gy, stream); break;
+      case END_GELU: launch_experts<END_GELU>(p, gy, stream); break;
+      case END_RELU2: launch_experts<END_RELU2>(p, gy, stream); break;
+      case END_GATED: launch_experts<END_GATED>(p, gy, stream); break;
+      default: launch_experts<END_GATED_CLAMPED>(p, gy, stream); break;
+    }
+  } else if (mfma_fits(dtype, p) && !p.tiles && p.tm == TM_BIG) {
+    if (!p.gate) launch_big<END_PLAIN>(p, gy, gz, stream);
+    else if (!p.gate_entries) launch_big<END_HEAD_GATE>(p, gy, gz, stream);
+    else launch_big<END_ENTRY_GATE>(p, gy, gz, stream);
   } else {
     if (p.tm > BM) return ERR_UNSUPPORTED;
     const dim3 grid((unsigned)((p.N + BN - 1) / BN), gy, gz);
@@ -644,20 +1008,21 @@ extern "C" int dinfer_heads_nt(int dtype, const void* A, int64_t lda, int64_t a_
 extern "C" int dinfer_experts_nt(int dtype, int gated, const void* A, int64_t lda, const void* W, int64_t ldw,
                                  int64_t w_zs, void* C, int64_t ldc, int64_t N, int64_t K, const int32_t* tiles,
                                  int64_t max_tiles, int tile_rows, const int32_t* offsets, const int32_t* perm, int a_div,
-                                 int c_to_perm, const float* row_scale, float limit, float slope, hipStream_t stream) {
+                                 int c_to_perm, const float* row_scale, float limit, float slope, int64_t entries, hipStream_t stream) {
   if (N <= 0 || max_tiles <= 0) return OK;
   if (K <= 0 || ldw < K || lda < K || ldc < N || N > 0x7fffffff || K > 0x7fffffff || max_tiles > 65535 || !tiles ||
       !offsets || !perm || tile_rows <= 0)
     return ERR_BAD_SHAPE;
   Groups p{};
   p.A = A; p.lda = lda; p.W = W; p.ldw = ldw; p.w_zs = w_zs; p.C = C; p.ldc = ldc;
-  p.N = (int)N; p.K = (int)K; p.tiles = tiles; p.offsets = offsets; p.perm = perm; p.a_div = a_div;
+  p.N = (int)N; p.K = (int)K; p.tiles = tiles; p.max_tiles = (int)max_tiles; p.entries = entries; p.offsets = offsets; p.perm = perm; p.a_div = a_div;
   p.c_to_perm = c_to_perm; p.gate_n = (int)N; p.tm = tile_rows;
   p.row_scale = row_scale;
   p.clamped = gated == 1 && limit > 0.f; p.limit = limit; p.slope = slope;
   if (gated < 0 || gated > 4) return ERR_UNSUPPORTED;
   p.act = gated >= 2 ? gated - 1 : 0;
   if (!mfma_fits(dtype, p) && tile_rows > BM) return ERR_UNSUPPORTED;
+  if (tile_rows == TM_BIG && w_zs > 0x30000000) return ERR_UNSUPPORTED;   // 32-bit offsets into an expert's weights
   return gated == 1 ? launch_groups<true>(dtype, p, (unsigned)max_tiles, 1, stream)
                : launch_groups<false>(dtype, p, (unsigned)max_tiles, 1, stream);
 }

@@ -942,7 +942,7 @@ def experts_nt(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, entries: int
     lib.call("dinfer_experts_nt", dtype_code(a.dtype), 1 if gated else EXPERT_ACTS[act] if act else 0, a.data_ptr(), _rows(a), w.data_ptr(), k,
              rows * k, out.data_ptr(), _rows(out), n, k, tiles.data_ptr(), moe_max_tiles(entries, experts, tile_rows),
              int(tile_rows), offsets.data_ptr(), perm.data_ptr(), int(a_div), 1 if c_to_perm else 0, _ptr(row_scale),
-             float(clamp[0]) if clamp else 0.0, float(clamp[1]) if clamp else 0.0, _stream())
+             float(clamp[0]) if clamp else 0.0, float(clamp[1]) if clamp else 0.0, entries, _stream())
     return out
 
 

@@ -1,0 +1,131 @@
+"""The experts' and heads' products of many rows (csrc/grouped.hip) at the edges of their tiles, against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def act(z, name):
+    return {None: lambda x: x, "silu": lambda x: x * torch.sigmoid(x), "relu2": lambda x: torch.relu(x) ** 2,
+            "gelu": lambda x: torch.nn.functional.gelu(x)}[name](z)
+
+
+def close(out, want):
+    """bfloat16 results of float sums: half a unit of 2^-8 of the value, and sums of K products of size one that carry at
+    most K 2^-24 each, far below."""
+    err = (out.double() - want).abs()
+    assert (err <= 2.0 ** -8 * want.abs() + 2e-3).all(), f"off by {err.max().item()}"
+
+
+# rows an expert gets: none, one, the edges of blocks of 32 and of tiles of 128
+COUNTS = [0, 1, 31, 32, 33, 64, 65, 96, 127, 0, 128, 129, 160, 300]
+
+
+def sorted_entries(counts, top, tokens, seed):
+    """A list of choices in which expert e is chosen counts[e] times, in a random order; entry i belongs to token i // top."""
+    flat = torch.tensor([e for e, c in enumerate(counts) for _ in range(c)], dtype=torch.int32)
+    g = torch.Generator().manual_seed(seed)
+    return flat[torch.randperm(flat.numel(), generator=g)]
+
+
+# columns: fewer than a wave's, two waves beside two, a last wave in part, no whole 16-byte pieces, several workgroups
+# K: one piece, a step and a piece, whole steps, a part of a step
+@pytest.mark.parametrize("N,K,kind", [(40, 8, None), (128, 72, "silu"), (130, 64, "gelu"), (256, 136, "relu2"), (300, 128, None),
+                                      (1408, 256, "gelu"), (24, 64, "gated"), (64, 200, "gated"), (72, 64, "gated"), (132, 328, "gated")])
+def test_experts_of_many_rows(N, K, kind):
+    from dinfer_amd.kernels import ops
+    E, n = len(COUNTS), sum(COUNTS)
+    top = 3
+    idx = sorted_entries(COUNTS, top, n, N)
+    tokens = -(-n // top)
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    x = torch.randn(tokens, K, generator=g, device=DEV).to(torch.bfloat16)
+    gated = kind == "gated"
+    w = (torch.randn(E, 2 * N if gated else N, K, generator=g, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    perm, offsets, tiles = torch.zeros(n, **i32), torch.zeros(E + 1, **i32), torch.zeros((ops.moe_max_tiles(n, E, 16), 2), **i32)
+    rows = ops.moe_tile_rows(torch.bfloat16, n, E, K, K)
+    assert rows == 128
+    ops.moe_scatter(idx.to(DEV), n, E, offsets, perm, tiles, rows)
+    scale = torch.rand(n, generator=g, device=DEV) + 0.5
+    for row_scale in (None, scale):
+        for to_perm in (True, False):
+            out = torch.full((n, N), 7.0, dtype=torch.bfloat16, device=DEV)
+            ops.experts_nt(x, w, out, n, tiles, offsets, perm, gated=gated, a_div=top, c_to_perm=to_perm, tile_rows=rows,
+                           act=None if gated else kind, row_scale=row_scale)
+            e = idx.to(DEV).long()
+            y = torch.empty(n, w.shape[1], dtype=torch.float64, device=DEV)
+            for k in range(E):
+                at = (e == k).nonzero().flatten()
+                y[at] = x[at // top].double() @ w[k].double().T
+            if row_scale is not None:
+                y = y * row_scale.double()[:, None]
+            want = act(y[:, :N], "silu") * y[:, N:] if gated else act(y, kind)
+            close(out, want if to_perm else want[perm.long()])
+    # the second product's form: the rows of A are the sorted places themselves
+    if not gated:
+        out = torch.full((n, N), 7.0, dtype=torch.bfloat16, device=DEV)
+        a = torch.randn(n, K, generator=g, device=DEV).to(torch.bfloat16)
+        ops.experts_nt(a, w, out, n, tiles, offsets, perm, gated=False, a_div=0, c_to_perm=True, tile_rows=rows)
+        for k in range(E):
+            places = slice(int(offsets[k]), int(offsets[k + 1]))
+            close(out[perm[places].long()], a[places].double() @ w[k].double().T)
+
+
+@pytest.mark.parametrize("gate", [None, "head", "entry"])
+@pytest.mark.parametrize("M,N,K,extra", [(17, 128, 64, 0), (128, 512, 128, 0), (129, 96, 40, 8), (300, 260, 72, 0), (64, 33, 8, 5)])
+def test_heads_of_many_rows(M, N, K, extra, gate):
+    from dinfer_amd.kernels import ops
+    H = 3
+    g = torch.Generator(device=DEV).manual_seed(M)
+    a = torch.randn(M, H * K + 8, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(H, N, K, generator=g, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    out = torch.full((M, H * (N + extra)), 7.0, dtype=torch.bfloat16, device=DEV)
+    gates = torch.randn(M, H * N, generator=g, device=DEV).to(torch.bfloat16)
+    ops.heads_nt(a, 8, K, w, out, 0, N + extra, M, **({} if gate is None else dict(gate=gates, gate_entries=gate == "entry")))
+    for h in range(H):
+        want = a[:, 8 + h * K:8 + (h + 1) * K].double() @ w[h].double().T
+        if gate == "head":
+            want = want * torch.sigmoid(gates[:, h:h + 1].double())
+        elif gate == "entry":
+            want = want * torch.sigmoid(gates[:, h * N:(h + 1) * N].double())
+        close(out[:, h * (N + extra):h * (N + extra) + N], want)
+        assert (out[:, h * (N + extra) + N:(h + 1) * (N + extra)] == 7.0).all()
+
+
+# few rows: up to 16 an expert (full tiles, one row, none), columns in part of a workgroup's 32, k in part of a step and in
+# more steps than are in flight
+@pytest.mark.parametrize("N,K,kind", [(32, 8, None), (33, 64, "silu"), (40, 72, "gelu"), (96, 520, "relu2"), (1408, 2048, None),
+                                      (24, 64, "gated"), (70, 200, "gated"), (64, 1408, "gated")])
+def test_experts_of_few_rows(N, K, kind):
+    from dinfer_amd.kernels import ops
+    counts = [0, 1, 16, 15, 2, 0, 9, 17, 3, 1]
+    E, n, top = len(counts), sum(counts), 3
+    idx = sorted_entries(counts, top, n, N)
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    x = torch.randn(-(-n // top), K, generator=g, device=DEV).to(torch.bfloat16)
+    gated = kind == "gated"
+    w = (torch.randn(E, 2 * N if gated else N, K, generator=g, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    perm, offsets, tiles = torch.zeros(n, **i32), torch.zeros(E + 1, **i32), torch.zeros((ops.moe_max_tiles(n, E, 16), 2), **i32)
+    rows = ops.moe_tile_rows(torch.bfloat16, n, E, K, K)
+    assert rows == 16
+    ops.moe_scatter(idx.to(DEV), n, E, offsets, perm, tiles, rows)
+    out = torch.full((n, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.experts_nt(x, w, out, n, tiles, offsets, perm, gated=gated, a_div=top, c_to_perm=True, tile_rows=rows, act=None if gated else kind)
+    e = idx.to(DEV).long()
+    y = torch.stack([w[int(e[i])].double() @ x[i // top].double() for i in range(n)])
+    close(out, act(y[:, :N], "silu") * y[:, N:] if gated else act(y, kind))
+
+
+@pytest.mark.parametrize("M", [1, 5, 16])
+def test_heads_of_few_rows(M):
+    from dinfer_amd.kernels import ops
+    H, N, K = 3, 72, 136
+    g = torch.Generator(device=DEV).manual_seed(M)
+    a = torch.randn(M, H * K, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(H, N, K, generator=g, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    out = torch.full((M, H * N), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.heads_nt(a, 0, K, w, out, 0, N, M)
+    close(out, torch.cat([a[:, h * K:(h + 1) * K].double() @ w[h].double().T for h in range(H)], dim=1))
