@@ -182,6 +182,9 @@ __global__ void __launch_bounds__(WAVES * 64) latent_attn_ref_kernel(
 
 
 // ---- attention over the latent pages on the matrix cores --------------------------------------------------------
+// LDS is written and read around this; loads from memory, those that write LDS among them, stay in flight across it (a fence
+// on LDS would wait for the latter)
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 constexpr float LOG2E = 1.4426950408889634f;
 
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
@@ -637,6 +640,267 @@ __global__ void __launch_bounds__(256) latent_attn_lds_kernel(
     }
 }
 
+// Steps with prompt portions at latents of 128, 256 or 512 entries and key rows of whole chunks of 32: a workgroup of eight
+// waves owns 64 rows (token, head) of a request and walks its keys in blocks of 32, each brought into LDS once for all of
+// them and one block ahead (global loads that write LDS: no register between; two buffers, objects of their own so that a
+// read of one does not wait for the loads into the other).
+//   scores  waves 2 r and 2 r + 1 take row tile r, half of the contraction each (their queries stay in registers, 40 a lane);
+//           the halves meet through LDS (16 KB a block), both waves then hold the tile's scores
+//   values  the weights pass through LDS (4 KB), and wave w takes an eighth of the latent entries for all 64 rows: a fragment
+//           of the values read from LDS feeds four MFMAs, where a wave that keeps to its rows reads all of them for one each
+// LDS rows are unpadded, their 16-byte pieces exchanged by the row's bits 1..3 (keys) or 2..3 (values), which the loads do by
+// asking for another piece: no bank is met twice. A block moves 310 KB through LDS, 2,400 cycles, beside 1,090 of MFMAs a
+// SIMD: LDS bounds it. 16 heads of 512 + 64: 16 portions of 256 tokens behind 1,000 each 1,099 -> 435 us (370
+// TFLOP/s), a prompt of 2,048 493 -> 185, 2,048 tokens behind 6,144 3,076 -> 1,070 (a wave that keeps its 16 rows, one workgroup
+// of four waves a CU, keys, values and queries in padded rows of LDS: 87 KB read a wave and block, and two more barriers).
+template <int DT, int KPS>   // R = 64 DT; pieces of a key row's place in LDS, at least (R + dr) / 8
+__global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
+    const bf16* __restrict__ qa, int64_t ld_qa, bf16* __restrict__ out, int64_t ld_out, const bf16* __restrict__ cache,
+    const bf16* __restrict__ cache_t, const int32_t* __restrict__ block_table, int64_t max_blocks,
+    const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ seq_lens, int num_reqs, float scale_log2,
+    int window, int H, int dr, int page_shift) {
+  constexpr int R = 64 * DT, NC = KPS / 8, TW = DT / 2;   // a wave's chunks of the contraction, its tiles of the latent
+  __shared__ __attribute__((aligned(16))) bf16 K0[32 * KPS * 8], K1[32 * KPS * 8];   // [32][8 KPS]
+  __shared__ __attribute__((aligned(16))) bf16 V0[R * 32], V1[R * 32];               // [R][32]
+  __shared__ __attribute__((aligned(16))) bf16x8 Ps[4][64];      // [row tile][lane]
+  __shared__ __attribute__((aligned(16))) f32x4 Ss[8][2][64];    // [wave][key tile][lane]
+  __shared__ float alphas[64];
+  __shared__ int moved[4];
+  const int DK = R + dr, kp = DK >> 3, chunks = DK >> 5;
+  // which request and which of its groups of 64 rows; the last groups of a prompt walk the most keys and start first
+  int grp = (int)gridDim.x - 1 - (int)blockIdx.x, b = -1, q_len = 0;
+  {
+    const int ln = threadIdx.x & 63;
+    for (int b0 = 0; b0 < num_reqs && b < 0; b0 += 64) {
+      const int mine = b0 + ln < num_reqs ? cu_seqlens[b0 + ln + 1] - cu_seqlens[b0 + ln] : 0;
+      int upto = (mine * H + 63) >> 6;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(upto, o, 64);
+        if (ln >= o) upto += v;
+      }
+      const unsigned long long holds = __ballot(grp < upto);
+      if (holds) {
+        const int at = __ffsll((long long)holds) - 1;
+        b = b0 + at;
+        q_len = __shfl(mine, at, 64);
+        grp -= at ? __shfl(upto, at - 1, 64) : 0;
+      } else {
+        grp -= __shfl(upto, 63, 64);
+      }
+    }
+  }
+  if (b < 0) return;   // (the whole workgroup: every wave counts the same)
+  b = __builtin_amdgcn_readfirstlane(b);
+  grp = __builtin_amdgcn_readfirstlane(grp);
+  q_len = __builtin_amdgcn_readfirstlane(q_len);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
+  const int rt = wave >> 1, half = wave & 1;     // this wave's row tile and half of the scores' contraction
+  const int t0 = cu_seqlens[b], start = seq_lens[b] - q_len, all_rows = q_len * H;
+  const int row0 = grp * 64 + rt * 16;
+  const int nrows = min(all_rows - row0, 16);    // <= 0: none
+  const bool rv = lr < nrows;
+  const int tok = rv ? (row0 + lr) / H : 0, head = rv ? (row0 + lr) % H : 0;
+  const int p = rv ? start + tok : -1;
+  const int my_last = nrows > 0 ? start + (row0 + nrows - 1) / H : -1, my_first = start + row0 / H;
+  const int lowest = window > 0 ? max(p - window + 1, 0) : 0;
+  // the workgroup's keys
+  const int p_first = start + grp * 64 / H, p_last = start + (min(all_rows, grp * 64 + 64) - 1) / H;
+  const int first = window > 0 ? max(p_first - window + 1, 0) : 0;
+  const int page = 1 << page_shift, pmask = page - 1, page_lo = first >> page_shift, page_hi = p_last >> page_shift;
+  const int32_t* bt = block_table + (int64_t)b * max_blocks;
+
+  bf16x8 qf[NC];
+  {
+    const bf16* qrow = qa + (int64_t)(t0 + tok) * ld_qa + (int64_t)head * DK + 8 * g;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int ch = half * NC + c;   // (chunks past the row's end: zeros of the query meet the row's last chunk)
+      qf[c] = *(const bf16x8*)(qrow + 32 * min(ch, chunks - 1));
+      if (ch >= chunks)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) qf[c][i] = (bf16)0.f;
+    }
+  }
+  f32x4 o[TW][4];   // latent entries 16 (TW wave + t) + 4 g + i of row lr of row tile r
+#pragma unroll
+  for (int t = 0; t < TW; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[t][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+
+  // A block's way into LDS: an instruction brings 64 pieces to 1 KB in a row. Where a lane's piece lies inside its page, and
+  // in which of the block's pages (blocks begin at multiples of 32: several where pages are shorter, else one and an offset
+  // that all lanes share), is the same for every block and worked out here: done a block at a time it was 400 instructions a
+  // wave, as long as all the rest.
+  constexpr int KU = (KPS / 2 + 7) / 8, VU = R / 128;
+  int k_off[KU], v_off[VU], k_page = 0, v_page = 0;   // bytes inside the page; two bits an instruction: which page
+  const int in_block = min(page, 32) - 1;
+#pragma unroll
+  for (int u = 0; u < KU; ++u) {
+    const int q = min(u * 8 + wave, KPS / 2 - 1) * 64 + lane, row = q / KPS, slot = q - row * KPS;
+    k_off[u] = ((row & in_block) * DK + min((slot & ~7) | ((slot ^ (row >> 1)) & 7), kp - 1) * 8) * 2;
+    k_page |= (page < 32 ? row >> page_shift : 0) << (2 * u);
+  }
+#pragma unroll
+  for (int u = 0; u < VU; ++u) {
+    const int q = (u * 8 + wave) * 64 + lane, d = q >> 2, key = 8 * ((q ^ (d >> 2)) & 3);
+    v_off[u] = ((d << page_shift) + (key & in_block)) * 2;
+    v_page |= (page < 32 ? key >> page_shift : 0) << (2 * u);
+  }
+  // (a page beyond the request's keys is replaced by its last one, whose rows exist: what they hold is masked)
+  auto load = [&](int kb, bf16* Ks, bf16* Vs) {
+    uint32_t pid[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pid[j] = __builtin_amdgcn_readfirstlane(bt[min(max((kb + (j << page_shift)) >> page_shift, page_lo), page_hi)]);
+    asm volatile("" : "+s"(pid[0]), "+s"(pid[1]), "+s"(pid[2]), "+s"(pid[3]));   // (or each choice below becomes a branch around a load)
+    auto of = [&](int j) {
+      const uint32_t even = j & 2 ? pid[2] : pid[0], odd = j & 2 ? pid[3] : pid[1];
+      return j & 1 ? odd : even;
+    };
+    const int kbm = kb & pmask;   // (0 where pages are no longer than a block)
+    const char* kbase = (const char*)cache + (int64_t)kbm * DK * 2;
+    const char* vbase = (const char*)cache_t + kbm * 2;
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+      if (u * 8 + wave < KPS / 2)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kbase + ((uint64_t)of((k_page >> (2 * u)) & 3) * (uint32_t)(DK * 2 << page_shift) + (uint32_t)k_off[u])),
+                                         (__attribute__((address_space(3))) void*)(Ks + (u * 8 + wave) * 512), 16, 0, 0);
+#pragma unroll
+    for (int u = 0; u < VU; ++u)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vbase + ((uint64_t)of((v_page >> (2 * u)) & 3) * (uint32_t)(R * 2 << page_shift) + (uint32_t)v_off[u])),
+                                       (__attribute__((address_space(3))) void*)(Vs + (u * 8 + wave) * 512), 16, 0, 0);
+  };
+  // row lr of key tile t stands for key 8 (lr / 4) + 4 t + lr % 4 of the block, so that a lane's eight weights belong to the
+  // eight consecutive keys 8 g .. + 7: the operand of the product with the values
+  const int kofs = 8 * (lr >> 2) + (lr & 3);
+  const int kb0 = first & ~31, nblk = (p_last - kb0) / 32 + 1;
+  auto block = [&](int kb, const bf16* Ks, const bf16* Vs) {
+    const bool busy = kb <= my_last;
+    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    if (busy) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int piece = 4 * min(half * NC + c, chunks - 1) + g;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int row = kofs + 4 * t;
+          s[t] = mfma16(*(const bf16x8*)(Ks + (row * KPS + (piece & ~7) + ((piece ^ (row >> 1)) & 7)) * 8), qf[c], s[t]);
+        }
+      }
+      Ss[wave][0][lane] = s[0];
+      Ss[wave][1][lane] = s[1];
+    }
+    lds_barrier();
+    if (busy) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) s[t] += Ss[wave ^ 1][t][lane];
+      // a block that every row of the tile sees whole needs no mask (most blocks of a long prompt)
+      const bool whole = nrows == 16 && kb + 31 <= my_first && (window == 0 || kb >= my_last - window + 1);
+      float mx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = kb + 8 * g + 4 * t + i;
+          const float v = s[t][i] * scale_log2;
+          s[t][i] = whole | ((key <= p) & (key >= lowest)) ? v : -INFINITY;
+          mx = fmaxf(mx, s[t][i]);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      // The running maximum follows the scores only when one of the tile's rows has outgrown it by more than 2^8 (or has
+      // none yet): the weights may then exceed 1, up to 256, which float sums and bf16 weights hold without loss. Both waves
+      // of a tile come to the same numbers.
+      const bool rescale = __any(mx > m + 8.f);
+      float alpha = 1.f;
+      if (rescale) {
+        const float m_new = fmaxf(m, mx);
+        alpha = m == -INFINITY ? 0.f : exp2_of(m - m_new);
+        l *= alpha;
+        m = m_new;
+      }
+      bf16x8 pb;
+      float psum = 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float pv = s[t][i] == -INFINITY ? 0.f : exp2_of(s[t][i] - m);
+          psum += pv;
+          pb[4 * t + i] = (bf16)pv;
+        }
+      l += psum;
+      if (half == 0) {
+        Ps[rt][lane] = pb;
+        if (g == 0) alphas[rt * 16 + lr] = alpha;
+        if (lane == 0) moved[rt] = rescale;
+      }
+    } else if (half == 0) {
+      bf16x8 pb;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pb[i] = (bf16)0.f;
+      Ps[rt][lane] = pb;
+      if (g == 0) alphas[rt * 16 + lr] = 1.f;
+      if (lane == 0) moved[rt] = 0;
+    }
+    lds_barrier();
+    bf16x8 pr[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) pr[r] = Ps[r][lane];
+    if (moved[0] | moved[1] | moved[2] | moved[3]) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float a = alphas[r * 16 + lr];
+#pragma unroll
+        for (int t = 0; t < TW; ++t) o[t][r] = o[t][r] * a;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+      const int d = 16 * (TW * wave + t) + lr;
+      const bf16x8 v = *(const bf16x8*)(Vs + d * 32 + ((g ^ (lr >> 2)) & 3) * 8);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[t][r] = mfma16(v, pr[r], o[t][r]);
+    }
+  };
+  // this wave's loads into LDS have landed (a barrier alone does not wait for them), then everybody's; and everybody has read
+  // the other buffer
+  auto ready = [&]() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  load(kb0, K0, V0);
+  for (int blk = 0; blk < nblk; blk += 2) {
+    const int kb = kb0 + blk * 32;
+    ready();
+    if (blk + 1 < nblk) load(kb + 32, K1, V1);
+    block(kb, K0, V0);
+    if (blk + 1 >= nblk) break;
+    ready();
+    if (blk + 2 < nblk) load(kb + 64, K0, V0);
+    block(kb + 32, K1, V1);
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  lds_barrier();
+  if (g == 0 && half == 0) alphas[rt * 16 + lr] = l > 0.f ? 1.f / l : 0.f;
+  lds_barrier();
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = grp * 64 + 16 * r + lr;
+    if (row >= all_rows) continue;
+    const float inv = alphas[16 * r + lr];
+    bf16* orow = out + (int64_t)(t0 + row / H) * ld_out + (int64_t)(row % H) * R + 16 * TW * wave + 4 * g;
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+      bf16x4 y;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = (bf16)(o[t][r][i] * inv);
+      *(bf16x4*)(orow + 16 * t) = y;
+    }
+  }
+}
+
 // One workgroup per (token, head) row: the parts' (max, sum, output) become the row's output. A part is R + 4 floats
 // (output, max, sum, two unused), so its rows are read 16 bytes a lane.
 __global__ void __launch_bounds__(128) latent_attn_merge_kernel(const float* __restrict__ part, bf16* __restrict__ out,
@@ -746,6 +1010,22 @@ extern "C" int dinfer_latent_attn_mfma(const void* qa, int64_t ld_qa, void* out,
   const int64_t tiles = (tokens * heads + 15) / 16 + num_reqs;
   if (tiles > 0x7fffffff || splits > 65535) return ERR_UNSUPPORTED;
   const bool solo = tokens != num_reqs;      // some request brings more than one row
+  // latents of 128, 256 or 512 with whole chunks of 32 in a key row, two blocks of which fit LDS: the kernel whose waves share
+  // their rows' weights
+  if (solo && (page_size & (page_size - 1)) == 0 && dr % 32 == 0 && (R == 128 || R == 256 || (R == 512 && dr <= 64))) {
+    const int64_t groups = (tokens * heads + 63) / 64 + num_reqs;
+    if (groups > 0x7fffffff) return ERR_UNSUPPORTED;
+    const int page_shift = __builtin_ctz(page_size);
+#define SHARED_LAUNCH(DT, KPS)                                                                                         \
+  latent_attn_shared_kernel<DT, KPS><<<(unsigned)groups, 512, 0, stream>>>(                                            \
+      (const bf16*)qa, ld_qa, (bf16*)out, ld_out, (const bf16*)cache, (const bf16*)cache_t, block_table, max_blocks,   \
+      cu_seqlens, seq_lens, num_reqs, scale * LOG2E, window, heads, dr, page_shift)
+    if (R == 128) SHARED_LAUNCH(2, 32);
+    else if (R == 256) SHARED_LAUNCH(4, 48);
+    else SHARED_LAUNCH(8, 72);
+#undef SHARED_LAUNCH
+    return launch_status();
+  }
   // keys, 4 x 16 queries and values of a block in LDS: where that fits (and pages are a power of two) prompt portions
   // take the kernel that shares them; else every wave walks its own keys
   const size_t bytes = ((size_t)(32 + 64) * (R + dr + 8) + (size_t)R * 40) * sizeof(bf16);

@@ -1,0 +1,49 @@
+"""Latent attention over prompt portions at the sizes of the kernel that shares a block of keys among 64 rows, against
+float64: edges of its row groups and key blocks, histories, windows, short pages."""
+import math
+
+import pytest
+import torch
+
+from test_gpu_kudurax import latent_case, latent_plain
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # seqs, q_lens, H, R, dr, page, window, far (request, token, head, key it looks at)
+    ([300], [300], 4, 128, 32, 8, 0, (0, 299, 2, 3)),                   # pages shorter than a block; tails of both
+    ([33, 64, 31, 1], [33, 64, 31, 1], 16, 128, 0, 16, 0, (1, 63, 7, 0)),  # no rotated part; a prompt of one token among others
+    ([500, 64, 33], [37, 1, 33], 16, 256, 64, 32, 0, (0, 36, 9, 0)),    # histories; a single row
+    ([200, 90], [64, 2], 3, 128, 96, 64, 50, (0, 10, 1, 200 - 64 + 10 - 49)),   # a window: the oldest key a row still sees
+    ([200, 90], [64, 2], 3, 128, 96, 64, 50, (0, 10, 1, 200 - 64 + 10 - 50)),   # ... and the first it does not; rows of 28 pieces
+    ([150, 70], [150, 3], 5, 512, 64, 16, 0, (0, 149, 1, 5)),           # the widest rows
+    ([700], [130], 16, 512, 64, 16, 0, (0, 129, 15, 31)),               # several groups behind a history
+    ([70] * 66, [2] * 66, 16, 128, 32, 16, 0, (65, 1, 3, 64)),          # more requests than a wave counts at once
+]
+
+
+@pytest.mark.parametrize("case_no", range(len(CASES)))
+def test_latent_prompt_portions(case_no):
+    from dinfer_amd.kernels import ops
+    seqs, q_lens, H, R, dr, page, window, far = CASES[case_no]
+    case = latent_case(seqs, q_lens, H, R, dr, page, 500 + case_no, torch.bfloat16, far)
+    scale = 0.7 / math.sqrt(R + dr)
+    want = latent_plain(case, q_lens, seqs, H, R, dr, scale, window)
+    dev = {k: v.cuda() for k, v in case.items() if k != "keys"}
+    if window:      # what lies behind every row's window has been given back
+        for b, (s, n) in enumerate(zip(seqs, q_lens)):
+            dev["bt"][b, :max(0, s - n - window + 1) // page] = -1
+    T, B = sum(q_lens), len(seqs)
+    out = torch.zeros(T, H * R, dtype=torch.bfloat16, device="cuda")
+    cache_t = dev["cache"][:, :, :R].transpose(1, 2).contiguous()
+    part = torch.zeros(T * H * (R + 4), dtype=torch.float32, device="cuda")
+    ops.latent_attn_mfma(dev["qa"], out, dev["cache"], cache_t, dev["bt"], dev["cu"], dev["seq"], B, T, 1, part, scale=scale,
+                         window=window, heads=H, rank=R, rot_dim=dr, page_size=page)
+    got = out.double().cpu()
+    # weights and results rounded to 2^-9 each, values of size one: a few times that of the largest
+    assert (got - want).abs().max().item() < 0.015 * max(1.0, want.abs().max().item())
+    b, i, h, j = far
+    t, p = sum(q_lens[:b]) + i, seqs[b] - q_lens[b] + i
+    seen = j <= p and (not window or j > p - window)
+    close = (got[t, h * R:(h + 1) * R] - case["keys"][b][j][:R].double()).abs().max().item()
+    assert (close < 0.1) == seen
