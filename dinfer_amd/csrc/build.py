@@ -32,6 +32,7 @@ SOURCES = {
     "attention_ext": "attention_ext.hip",
     "gemm_ref": "gemm_ref.hip",
     "f32": "f32.hip",
+    "chunked": "chunked.hip",
     "gemm": "gemm.hip",
     "gemm_mid": "gemm_mid.hip",
     "gemm_wide": "gemm_wide.hip",

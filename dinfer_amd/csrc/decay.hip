@@ -16,7 +16,8 @@
 //   decay_recurrence   token by token, one request, one head and 8 columns of S a workgroup: the 32 lanes of half a wave
 //                      share a column and own a strip of its rows; 16 tokens' operands wait in LDS while the next 16 are
 //                      on their way in registers. Serves single decoded rows (the whole state in and out once) and
-//                      prompt portions of any length
+//                      prompt portions of any length; long ones go chunk by chunk instead where the sizes allow it
+//                      (chunked.hip)
 //   gated_group_norm   (y + skip_h x) * silu(z), then divided by the root mean square of its group of columns, times a
 //                      gain a column; or the gate after the norm; one workgroup a (token, group)
 //
@@ -257,7 +258,7 @@ __global__ void __launch_bounds__(256) decay_recurrence_kernel(Operands p, float
                                                                const int32_t* __restrict__ cu,
                                                                const int32_t* __restrict__ seq_lens,
                                                                float* __restrict__ out, int64_t ld_out, int G, int H,
-                                                               int D, int V) {
+                                                               int D, int V, int below) {
   constexpr int DP = 32 * RPT;
   __shared__ __attribute__((aligned(16))) float ks[CH][DP];
   __shared__ __attribute__((aligned(16))) float qs[CH][DP];
@@ -270,6 +271,7 @@ __global__ void __launch_bounds__(256) decay_recurrence_kernel(Operands p, float
   const int rg = tid & 31, cj = tid >> 5;
   const int j = cb * COLS + cj;
   const int t0 = cu[b], n = cu[b + 1] - t0;
+  if (n >= below) return;   // (taken by the chunked form)
   const int start = seq_lens[b] - n;
   const int g = h / (H / G);
   const bool col_ok = j < V;
@@ -599,14 +601,15 @@ extern "C" int dinfer_decay_recurrence(const float* q, int64_t ldq, const float*
                                        int64_t ldv, const float* decay, int64_t ld_decay, const float* gain,
                                        int64_t ld_gain, float* state, const int32_t* state_slots,
                                        const int32_t* cu_seqlens, const int32_t* seq_lens, float* out, int64_t ld_out,
-                                       int num_reqs, int G, int H, int D, int V, hipStream_t stream) {
+                                       int num_reqs, int G, int H, int D, int V, int below,
+                                       hipStream_t stream) {
   if (num_reqs <= 0) return OK;
   if (G <= 0 || H <= 0 || H % G || D <= 0 || V <= 0 || num_reqs > 65535 || H > 65535 || !decay) return ERR_BAD_SHAPE;
   if (D > 256) return ERR_UNSUPPORTED;
   Operands p{q, ldq, k, ldk, v, ldv, decay, ld_decay, gain, ld_gain};
   const dim3 grid((unsigned)((V + COLS - 1) / COLS), (unsigned)H, (unsigned)num_reqs);
 #define DECAY_REC(R_) \
-  decay_recurrence_kernel<R_><<<grid, 256, 0, stream>>>(p, state, state_slots, cu_seqlens, seq_lens, out, ld_out, G, H, D, V)
+  decay_recurrence_kernel<R_><<<grid, 256, 0, stream>>>(p, state, state_slots, cu_seqlens, seq_lens, out, ld_out, G, H, D, V, below)
   if (D <= 32) DECAY_REC(1);
   else if (D <= 64) DECAY_REC(2);
   else if (D <= 128) DECAY_REC(4);

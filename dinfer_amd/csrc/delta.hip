@@ -19,7 +19,8 @@
 // S is stored transposed, [slot][head][V][D]: a thread's strip is contiguous, a wave reads and writes 2 KB to 8 KB in
 // one piece, which is what a decode step (one token a request: all of S in and out) is made of.
 // A request whose step starts at position 0 starts from S = 0 and zero stored inputs, whatever its slot held.
-// Nothing depends on how a request's tokens were cut into steps: every token does the same arithmetic in the same order.
+// Here nothing depends on how a request's tokens were cut into steps: every token does the same arithmetic in the same
+// order. (Requests of many rows in a step go chunk by chunk instead, chunked.hip: the same sums in another order.)
 #include "common.cuh"
 
 using namespace dinfer;
@@ -235,7 +236,7 @@ template <int RPT>
 __global__ void __launch_bounds__(256) delta_recurrence_kernel(
     const float* __restrict__ work, int64_t ldw, float* __restrict__ state, const int32_t* __restrict__ slots,
     const int32_t* __restrict__ cu, const int32_t* __restrict__ seq_lens, float* __restrict__ out, int64_t ld_out,
-    int G, int H, int D, int V) {
+    int G, int H, int D, int V, int below) {
   constexpr int DP = 32 * RPT;
   __shared__ __attribute__((aligned(16))) float ks[CH][DP];
   __shared__ __attribute__((aligned(16))) float qs[CH][DP];
@@ -248,6 +249,7 @@ __global__ void __launch_bounds__(256) delta_recurrence_kernel(
   const int rg = tid & 31, cj = tid >> 5;
   const int j = cb * COLS + cj;
   const int t0 = cu[b], n = cu[b + 1] - t0;
+  if (n >= below) return;   // (taken by the chunked form)
   const int start = seq_lens[b] - n;
   const int g = h / (H / G);
   const int gd = 2 * G * D;
@@ -608,14 +610,15 @@ extern "C" int dinfer_delta_conv_update(int dtype, const void* proj, int64_t ld,
 // state [slots, H, V, D] float (S transposed); out [T, ld_out] float, head h at column h V.
 extern "C" int dinfer_delta_recurrence(const float* work, int64_t ldw, float* state, const int32_t* state_slots,
                                        const int32_t* cu_seqlens, const int32_t* seq_lens, float* out, int64_t ld_out,
-                                       int num_reqs, int G, int H, int D, int V, hipStream_t stream) {
+                                       int num_reqs, int G, int H, int D, int V, int below,
+                                       hipStream_t stream) {
   if (num_reqs <= 0) return OK;
   if (G <= 0 || H <= 0 || H % G || D <= 0 || V <= 0 || num_reqs > 65535 || H > 65535) return ERR_BAD_SHAPE;
   if (D > 256) return ERR_UNSUPPORTED;
   const dim3 grid((unsigned)((V + COLS - 1) / COLS), (unsigned)H, (unsigned)num_reqs);
 #define DELTA_REC(R_)                                                                                               \
   delta_recurrence_kernel<R_><<<grid, 256, 0, stream>>>(work, ldw, state, state_slots, cu_seqlens, seq_lens, out, \
-                                                        ld_out, G, H, D, V)
+                                                        ld_out, G, H, D, V, below)
   if (D <= 32) DELTA_REC(1);
   else if (D <= 64) DELTA_REC(2);
   else if (D <= 128) DELTA_REC(4);

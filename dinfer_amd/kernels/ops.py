@@ -397,17 +397,61 @@ def delta_conv_update(proj: torch.Tensor, *, qkv_off: int, conv_state: torch.Ten
 
 def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor, *, state_slots: torch.Tensor,
                      cu_seqlens: torch.Tensor, seq_lens: torch.Tensor, num_reqs: int, qk_heads: int, heads: int,
-                     dim: int, vdim: int) -> torch.Tensor:
+                     dim: int, vdim: int, tokens: int | None = None, scratch: torch.Tensor | None = None) -> torch.Tensor:
     """The recurrence over each request's rows of the step. state [slots, heads, vdim, dim] float32 (a head's matrix
-    transposed), updated in place; out [T, heads * vdim] float32."""
+    transposed), updated in place; out [T, heads * vdim] float32. tokens, scratch: the step's rows and a buffer of
+    chunk_scratch's size; with them requests of CHUNKED_ROWS rows or more go chunk by chunk."""
     _need_gpu(work, state, out, state_slots, cu_seqlens, seq_lens)
     assert work.dtype == state.dtype == out.dtype == torch.float32 and state.is_contiguous()
     assert tuple(state.shape[1:]) == (heads, vdim, dim) and out.shape[1] >= heads * vdim
     assert work.shape[1] >= delta_work_columns(qk_heads, heads, dim, vdim)
-    lib.call("dinfer_delta_recurrence", work.data_ptr(), _rows(work), state.data_ptr(), state_slots.data_ptr(),
-             cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs, qk_heads, heads, dim, vdim,
-             _stream())
+    qk, v_end = qk_heads * dim, 2 * qk_heads * dim + heads * vdim
+    below = _chunked(True, work, work[:, qk:], work[:, 2 * qk:], work[:, v_end + heads:], work[:, v_end:], state, out,
+                     state_slots, cu_seqlens, seq_lens, num_reqs, qk_heads, heads, dim, vdim, tokens, scratch)
+    if below > 0:
+        lib.call("dinfer_delta_recurrence", work.data_ptr(), _rows(work), state.data_ptr(), state_slots.data_ptr(),
+                 cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs, qk_heads, heads, dim,
+                 vdim, below, _stream())
     return out
+
+
+# A request of this many rows in a step goes chunk by chunk, the others token by token. One request, delta rule 16 x 128 x 128,
+# decays 16 x 128 x 128 and 64 x 128 x 64: at 96 rows 29, 17 and 20 us token by token against 32, 21 and 23 in chunks; at 128
+# 37, 21 and 25 against 32, 21 and 25; at 256 70, 43 and 49 against 39, 27 and 33; at 2,048 545, 322 and 364 against 128,
+# 115 and 130.
+CHUNKED_ROWS = 128
+CHUNK = 64              # tokens of a chunk (chunked.hip)
+CHUNKS_AT_ONCE = 64     # chunks that a scratch buffer holds at most: longer steps go through it in turns
+
+
+def chunk_scratch(delta: bool, groups: int, heads: int, dim: int, vdim: int, max_tokens: int, max_reqs: int):
+    """(rows, columns) of the float32 scratch for delta_recurrence or decay_recurrence of these sizes and at most
+    max_tokens rows a step; None where they always go token by token."""
+    if dim not in (64, 128) or vdim % 16 or vdim > 1024 or heads > 4096 or max_tokens < CHUNKED_ROWS:
+        return None
+    floats = 2 * groups * CHUNK * dim + heads * ((CHUNK * dim if delta else 0) + 10 * 256 + 3 * CHUNK)
+    most = (max_tokens + (CHUNK - 1) * min(max_reqs, max_tokens // CHUNKED_ROWS)) // CHUNK
+    return min(most, CHUNKS_AT_ONCE), floats
+
+
+def _chunked(delta, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens, num_reqs, groups, heads, dim,
+             vdim, tokens, scratch) -> int:
+    """Runs the chunked form of a recurrence for the requests it takes, if the step may have any. Returns the rows below
+    which a request is left to the token-by-token kernel; 0: none is left."""
+    everything = 2 ** 31 - 1
+    # (every request of a step has a row at least: none has more than this)
+    if scratch is None or tokens is None or num_reqs <= 0 or tokens - num_reqs + 1 < CHUNKED_ROWS:
+        return everything
+    if q.stride(0) % 4 or k.stride(0) % 4 or (q.data_ptr() | k.data_ptr() | state.data_ptr()) % 16:
+        return everything
+    floats = lib.get("dinfer_chunk_floats")(int(delta), groups, heads, dim, vdim)
+    assert scratch.dtype == torch.float32 and scratch.is_contiguous() and floats > 0 and scratch.shape[1] >= floats
+    assert tokens <= q.shape[0] and tokens <= out.shape[0]
+    lib.call("dinfer_chunked_recurrence", int(delta), q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v),
+             decay.data_ptr(), 0 if decay.dim() == 1 else _rows(decay), _ptr(gain), _rows(gain) if gain is not None else 0,
+             state.data_ptr(), state_slots.data_ptr(), cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out),
+             scratch.data_ptr(), scratch.shape[0], tokens, num_reqs, CHUNKED_ROWS, groups, heads, dim, vdim, _stream())
+    return 0 if num_reqs == 1 else CHUNKED_ROWS
 
 
 def delta_out(o: torch.Tensor, proj: torch.Tensor, g_off: int, weight: torch.Tensor, out: torch.Tensor, tokens: int, *,
@@ -514,10 +558,13 @@ def conv_silu(proj: torch.Tensor, tokens: int, *, x_off: int, dt_off: int, taps:
 
 def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, gain: torch.Tensor | None,
                      state: torch.Tensor, out: torch.Tensor, *, state_slots: torch.Tensor, cu_seqlens: torch.Tensor,
-                     seq_lens: torch.Tensor, num_reqs: int, groups: int, heads: int, dim: int, vdim: int) -> torch.Tensor:
+                     seq_lens: torch.Tensor, num_reqs: int, groups: int, heads: int, dim: int, vdim: int,
+                     tokens: int | None = None, scratch: torch.Tensor | None = None) -> torch.Tensor:
     """Per request and head, token by token: S <- decay S + gain k v^T, out = S^T q. q, k: float32 views [T, groups dim]
     (head h reads group h // (heads / groups)); v [T, heads vdim]; decay [T, heads], or [heads] for one decay a head;
-    gain [T, heads] or None. state [slots, heads, vdim, dim] float32, updated in place; out [T, >= heads vdim] float32."""
+    gain [T, heads] or None. state [slots, heads, vdim, dim] float32, updated in place; out [T, >= heads vdim] float32.
+    tokens, scratch: the step's rows and a buffer of chunk_scratch's size; with them requests of CHUNKED_ROWS rows or
+    more go chunk by chunk."""
     _need_gpu(q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens)
     tensors = [q, k, v, decay, state, out] + ([gain] if gain is not None else [])
     assert all(t.dtype == torch.float32 for t in tensors) and state.is_contiguous()
@@ -530,10 +577,13 @@ def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: t
         assert decay.shape[1] >= heads
         ldd = _rows(decay)
     assert gain is None or gain.shape[1] >= heads
-    lib.call("dinfer_decay_recurrence", q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v),
-             decay.data_ptr(), ldd, _ptr(gain), _rows(gain) if gain is not None else 0, state.data_ptr(),
-             state_slots.data_ptr(), cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs,
-             groups, heads, dim, vdim, _stream())
+    below = _chunked(False, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens, num_reqs, groups, heads,
+                     dim, vdim, tokens, scratch)
+    if below > 0:
+        lib.call("dinfer_decay_recurrence", q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v),
+                 decay.data_ptr(), ldd, _ptr(gain), _rows(gain) if gain is not None else 0, state.data_ptr(),
+                 state_slots.data_ptr(), cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs,
+                 groups, heads, dim, vdim, below, _stream())
     return out
 
 

@@ -11,6 +11,7 @@ from typing import Callable
 
 import torch
 
+from ..kernels import ops
 from .spec import CacheSpec, TensorSpec
 
 
@@ -52,6 +53,11 @@ class BuildContext:
         self.max_seq_len = max_seq_len
         self.workspace = Workspace(device, dtype, max_tokens)
         self._shared: dict = {}
+
+    def chunk_scratch(self, delta: bool, groups: int, heads: int, dim: int, vdim: int) -> torch.Tensor | None:
+        """The scratch of ops.delta_recurrence or ops.decay_recurrence; None for sizes that need none."""
+        size = ops.chunk_scratch(delta, groups, heads, dim, vdim, self.max_tokens, self.max_reqs)
+        return size and self.workspace.buffer("chunks", size[1], dtype=torch.float32, rows=size[0])
 
     def share(self, key, make):
         """One object for all parts that ask under the same key (a table every layer would otherwise build for itself)."""

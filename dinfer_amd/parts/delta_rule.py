@@ -112,6 +112,7 @@ class GatedDeltaRule(Mixer):
         self.work = ws.buffer("delta_work", ops.delta_work_columns(self.qk_heads, self.heads, self.dim, self.vdim),
                               dtype=torch.float32)
         self.o_buf = ws.buffer("delta_o", self.v_size, dtype=torch.float32)
+        self.chunks = ctx.chunk_scratch(True, self.qk_heads, self.heads, self.dim, self.vdim)
 
     def forward(self, x, batch, cache: CacheView):
         T = batch.num_tokens
@@ -130,6 +131,6 @@ class GatedDeltaRule(Mixer):
                        eps=self.unit_eps, q_scale=self.dim ** -0.5, taps_t=self.conv_taps_t, **common, **sizes)
         if cache.owner:
             ops.delta_conv_update(proj_buf, qkv_off=col, conv_state=cache.conv, **common)
-        ops.delta_recurrence(self.work, cache.state, self.o_buf, **common, **sizes)
+        ops.delta_recurrence(self.work, cache.state, self.o_buf, tokens=T, scratch=self.chunks, **common, **sizes)
         ops.delta_out(self.o_buf, proj_buf, col + self.g_off, self.norm_weight, gated_buf, T, heads=self.heads,
                       vdim=self.vdim, eps=self.norm_eps, col_off=out_col, out_scale=self.out_scale)

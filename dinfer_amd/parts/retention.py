@@ -98,6 +98,7 @@ class Retention(Mixer):
         self.position.bind(ctx)
         self.work = ws.buffer("retention_work", 2 * self.qk_size + self.v_size, dtype=torch.float32)
         self.o_buf = ws.buffer("retention_o", self.v_size, dtype=torch.float32)
+        self.chunks = ctx.chunk_scratch(False, self.heads, self.heads, self.dim, self.vdim)
 
     def forward(self, x, batch, cache: CacheView):
         T = batch.num_tokens
@@ -116,6 +117,7 @@ class Retention(Mixer):
         w = self.work
         ops.decay_recurrence(w[:, :qk], w[:, qk:2 * qk], w[:, 2 * qk:], self.decay_vec, None, cache.state, self.o_buf,
                              state_slots=batch.state_slots, cu_seqlens=batch.cu_seqlens, seq_lens=batch.seq_lens,
-                             num_reqs=batch.num_reqs, groups=self.heads, heads=self.heads, dim=self.dim, vdim=self.vdim)
+                             num_reqs=batch.num_reqs, groups=self.heads, heads=self.heads, dim=self.dim, vdim=self.vdim,
+                             tokens=T, scratch=self.chunks)
         ops.gated_group_norm(self.o_buf, proj_buf, col + self.g_off, gated_buf, T, groups=self.heads, group=self.vdim,
                              eps=self.norm_eps, col_off=out_col, out_scale=self.out_scale, gate_first=False)

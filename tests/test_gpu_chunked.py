@@ -1,0 +1,99 @@
+"""Recurrences over prompt portions in chunks of 64 tokens (chunked.hip) against the recurrence token by token in 64 bits, and
+beside the token-by-token kernels of the same sums in 32 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def plain(q, k, v, decay, gain, delta, S):
+    """One request in 64 bits: q, k [n, H, D], v [n, H, V], decay and gain [n, H], S [H, D, V]."""
+    out = torch.empty_like(v)
+    for t in range(q.shape[0]):
+        S = decay[t, :, None, None] * S
+        u = v[t] - (k[t, :, None] @ S)[:, 0] if delta else v[t]
+        S = S + k[t, :, :, None] * (gain[t, :, None] * u)[:, None]
+        out[t] = (q[t, :, None] @ S)[:, 0]
+    return out, S
+
+
+# delta, groups, heads, dim, vdim, rows a request, rows before (0: from nothing), chunks of scratch, one decay a head
+CASES = [
+    (True, 2, 2, 128, 128, [128], [0], 64, False),              # the fewest rows, whole chunks
+    (True, 1, 2, 64, 48, [129, 1, 191, 64], [5, 3, 0, 0], 64, False),    # ragged ends, rows that go token by token between
+    (True, 2, 4, 128, 16, [500, 300], [0, 7], 3, False),        # a scratch that the step goes through in turns
+    (True, 1, 1, 64, 64, [256] + [1] * 70, [0] * 71, 64, False),   # more requests than a wave has lanes
+    (False, 2, 2, 128, 128, [128], [0], 64, True),
+    (False, 1, 3, 64, 48, [129, 1, 191, 64], [5, 3, 0, 0], 64, False),
+    (False, 2, 8, 128, 64, [500, 300], [0, 7], 3, False),
+    (False, 1, 16, 64, 16, [4500], [9], 64, False),             # more chunks than a buffer; heads that share k . q
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_against_token_by_token(case):
+    from dinfer_amd.kernels import ops
+    delta, G, H, D, V, new, before, chunks, fixed = case
+    g = torch.Generator().manual_seed(sum(new) + D)
+    T, B = sum(new), len(new)
+    cu = [0]
+    for n in new:
+        cu.append(cu[-1] + n)
+    unit = torch.nn.functional.normalize
+    # neighbouring keys alike, so that the triangular system is far from the identity; a decay of zero, and some of one
+    k = torch.randn(T, G, D, generator=g)
+    k[1::2] = k[0::2][:k[1::2].shape[0]] + 0.5 * k[1::2]
+    k, q = unit(k, dim=-1), unit(torch.randn(T, G, D, generator=g), dim=-1)
+    v = torch.randn(T, H, V, generator=g)
+    gain = torch.rand(T, H, generator=g)
+    decay = 1 - 0.2 * torch.rand(T, H, generator=g) ** 2
+    if fixed:
+        decay = torch.tensor([1.0, 0.97]).expand(T, H).contiguous()
+        gain = torch.ones(T, H)
+    else:
+        decay[T // 2, 0] = 0.0
+        decay[T // 3:T // 3 + 20] = 1.0
+    slots = torch.randperm(B + 2, generator=g)[:B]
+    state0 = torch.randn(B + 2, H, V, D, generator=g)
+    cols = ops.delta_work_columns(G, H, D, V)
+    work = torch.cat([q.reshape(T, -1), k.reshape(T, -1), v.reshape(T, -1), gain, decay], dim=1)
+    work = torch.nn.functional.pad(work, (0, -(-cols // 4) * 4 - cols)).cuda()
+    size = ops.chunk_scratch(delta, G, H, D, V, T, B)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    common = dict(state_slots=slots.to(**i32), cu_seqlens=torch.tensor(cu, **i32),
+                  seq_lens=torch.tensor([a + b for a, b in zip(new, before)], **i32), num_reqs=B, heads=H, dim=D, vdim=V)
+    got = {}
+    for chunked in (False, True):
+        state = state0.cuda()
+        out = torch.full((T + 1, H * V), 7.0, device="cuda")
+        more = dict(tokens=T, scratch=torch.full((min(size[0], chunks), size[1]), float("nan"), device="cuda")) if chunked else {}
+        if delta:
+            ops.delta_recurrence(work, state, out, qk_heads=G, **common, **more)
+        else:
+            qk, ve = G * D, 2 * G * D + H * V
+            ops.decay_recurrence(work[:, :qk], work[:, qk:2 * qk], work[:, 2 * qk:ve],
+                                 decay[0].cuda() if fixed else work[:, ve + H:ve + 2 * H],
+                                 None if fixed else work[:, ve:ve + H], state, out, groups=G, **common, **more)
+        torch.cuda.synchronize()
+        assert (out[T] == 7.0).all()
+        got[chunked] = out[:T].double().cpu(), state.double().cpu()
+    rep = H // G
+    q, k = q.double().repeat_interleave(rep, 1), k.double().repeat_interleave(rep, 1)
+    v, gain, decay = v.double(), gain.double(), decay.double()
+    want, want_state = torch.empty(T, H * V, dtype=torch.float64), state0.double()
+    for b in range(B):
+        s = slice(cu[b], cu[b + 1])
+        S = state0[slots[b]].double().transpose(1, 2) if before[b] else torch.zeros(H, D, V, dtype=torch.float64)
+        o, S = plain(q[s], k[s], v[s], decay[s], gain[s], delta, S)
+        want[s] = o.reshape(-1, H * V)
+        want_state[slots[b]] = S.transpose(1, 2)
+    for i, w in ((0, want), (1, want_state)):
+        # both forms round each product and each partial sum to 2^-24 of itself: some 2 log2(D) roundings of a sum over D in
+        # trees, as many of a sum over a chunk; and the chunked form is to be no further off than the other
+        top = w.abs().max().item()
+        worst, rms = {}, {}
+        for c in got:
+            e = (got[c][i] - w) / top
+            worst[c], rms[c] = e.abs().max().item(), e.pow(2).mean().sqrt().item()
+        assert worst[True] < 4 * (7 + 6) * 2.0 ** -24, (worst, rms)
+        assert rms[True] <= 1.02 * rms[False], (worst, rms)
