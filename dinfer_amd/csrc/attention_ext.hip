@@ -22,32 +22,35 @@ struct Args {
   FlashExt ext;
 };
 
-template <int DT, int DV, int KIND, int QT>
+template <int DT, int DV, int KIND, int QT, bool HEADS = false>
 int launch_rows(const Args& p, hipStream_t stream) {
-  const int tiles = (p.max_q_len + 16 * QT - 1) / (16 * QT);
-  const int64_t blocks = (int64_t)tiles * p.H * p.num_reqs;
+  const int tiles = HEADS ? 1 : (p.max_q_len + 16 * QT - 1) / (16 * QT);
+  const int64_t blocks = (int64_t)tiles * (HEADS ? p.Hkv : p.H) * p.num_reqs;
   if (blocks > 0x7fffffff) return ERR_UNSUPPORTED;
   // page sizes that are no powers of two: only where keys and values are of one size, under a softmax
   constexpr bool ANY_PAGE = KIND == OPTIONS && DT == DV;
-  auto kernel = attn_flash_kernel<DT, QT, true, KIND, DV>;
+  auto kernel = attn_flash_kernel<DT, QT, true, KIND, DV, HEADS>;
   if constexpr (ANY_PAGE) {
-    if (p.ps & (p.ps - 1)) kernel = attn_flash_kernel<DT, QT, false, KIND, DV>;
+    if (p.ps & (p.ps - 1)) kernel = attn_flash_kernel<DT, QT, false, KIND, DV, HEADS>;
   } else if (p.ps & (p.ps - 1)) {
     return ERR_UNSUPPORTED;
   }
-  const size_t lds = (size_t)3 * QT * 64 * (sizeof(f32x4) * DV + 2 * sizeof(float));
+  constexpr int waves = flash_waves(HEADS);
+  const size_t lds = (size_t)(waves - 1) * QT * 64 * (sizeof(f32x4) * DV + 2 * sizeof(float));
   // (more than the 64 KB of LDS a launch may ask for without saying so)
   if (lds > 65536 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return ERR_LAUNCH;
-  kernel<<<(unsigned)blocks, 256, lds, stream>>>(p.q, p.ld_q, p.out, p.ld_out, p.kc, p.vc, p.bt, p.max_blocks, p.cu, p.sl, tiles,
+  kernel<<<(unsigned)blocks, 64 * waves, lds, stream>>>(p.q, p.ld_q, p.out, p.ld_out, p.kc, p.vc, p.bt, p.max_blocks, p.cu, p.sl, tiles,
                                                 p.ext.scale * LOG2E, p.window, p.H, p.Hkv, p.ps, 0, p.ext);
   return launch_status();
 }
 
 // Rows a workgroup takes: 48 at heads of 128 where the rows make several rounds of workgroups over the chip (rows of at
-// most two tiles a request never fill the third), 32 where portions are longer than one tile, else 16.
+// most two tiles a request never fill the third), 32 where portions are longer than one tile, else 16. Steps of single rows:
+// the heads of a group instead of rows, where they fit a tile.
 template <int DT, int DV, int KIND>
 int launch(const Args& p, hipStream_t stream) {
+  if (p.max_q_len == 1 && p.H / p.Hkv <= 16) return launch_rows<DT, DV, KIND, 1, true>(p, stream);
   if constexpr (DT == 8 && DV == 8) {
     if (p.max_q_len > 32 && (int64_t)((p.max_q_len + 47) / 48) * p.H * p.num_reqs >= 2000) return launch_rows<DT, DV, KIND, 3>(p, stream);
   }

@@ -377,22 +377,32 @@ struct FlashExt {
   int chunk;            // > 0: keys of the row's own chunk of positions only
 };
 
-template <int DT, int QT, bool P2, int KIND = PLAIN, int DV = DT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) attn_flash_kernel(
+//
+// HEADS (steps of single rows): the columns of the tile are the heads of a group instead of rows, at most 16, so a kv
+// head's keys are read once instead of once a head, and eight waves share them. Bound by memory from some 64 rows on: 64
+// rows behind 4,200 keys each, 16 heads over 4 kv heads of 128, 241 -> 115 us (4.8 TB/s); 32 heads over 2, 2,100 keys,
+// 157 -> 27 us; below that by the walk of one wave over its run of keys, which is as long as before (8 rows: 42 us both ways).
+constexpr int flash_waves(bool heads) { return heads ? 8 : 4; }
+
+template <int DT, int QT, bool P2, int KIND = PLAIN, int DV = DT, bool HEADS = false>
+__global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu_waves_per_eu(2, 8))) attn_flash_kernel(
     const bf16* __restrict__ q, int64_t ld_q, bf16* __restrict__ out, int64_t ld_out, const bf16* __restrict__ kc,
     const bf16* __restrict__ vc, const int32_t* __restrict__ block_table, int64_t max_blocks,
     const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ seq_lens, int tiles_x, float scale_log2e,
     int window, int H, int Hkv, int ps, int skip_single, FlashExt ext = FlashExt{}) {
   constexpr bool EXT = KIND != PLAIN;
+  constexpr int WAVES = flash_waves(HEADS), PARTS = WAVES - 1;
+  constexpr int AT_ONCE = HEADS ? 1 : PARTS;   // parts joined at once: seven would not fit the registers
+  static_assert(!HEADS || QT == 1, "one tile of heads");
   constexpr int D = DT * 16;
   constexpr int KS = (DT + 1) / 2;
   constexpr int QW = 16 * QT;  // query rows per workgroup
-  // what waves 1..3 hand to wave 0 (dynamic: three row tiles of head size 128 need more than the 64 KB a kernel
-  // may declare): part_o[3][QT][DV][64] of f32x4, then part_m and part_l [3][QT][64] of float
+  // what the other waves hand to wave 0 (dynamic: three row tiles of head size 128 need more than the 64 KB a kernel
+  // may declare): part_o[PARTS][QT][DV][64] of f32x4, then part_m and part_l [PARTS][QT][64] of float
   extern __shared__ __attribute__((aligned(16))) char flash_smem[];
   f32x4* const part_o_ = (f32x4*)flash_smem;
-  float* const part_m_ = (float*)(flash_smem + sizeof(f32x4) * 3 * QT * DV * 64);
-  float* const part_l_ = part_m_ + 3 * QT * 64;
+  float* const part_m_ = (float*)(flash_smem + sizeof(f32x4) * PARTS * QT * DV * 64);
+  float* const part_l_ = part_m_ + PARTS * QT * 64;
   auto part_o = [&](int r, int t, int d) -> f32x4& { return part_o_[((r * QT + t) * DV + d) * 64 + lane_of()]; };
   auto part_m = [&](int r, int t) -> float& { return part_m_[(r * QT + t) * 64 + lane_of()]; };
   auto part_l = [&](int r, int t) -> float& { return part_l_[(r * QT + t) * 64 + lane_of()]; };
@@ -400,14 +410,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
   // workgroups an XCD receives (linear id modulo 8) share kv heads, and with them the L2 lines
   // of K and V. Late query tiles (most keys) are issued first.
   const int L = blockIdx.x;
-  const int e = L % H, rest = L / H;
-  const int tile = tiles_x - 1 - rest % tiles_x, b = rest / tiles_x;
+  const int e = HEADS ? L % Hkv : L % H, rest = HEADS ? L / Hkv : L / H;
+  const int tile = HEADS ? 0 : tiles_x - 1 - rest % tiles_x, b = HEADS ? rest : rest / tiles_x;
   const int G = H / Hkv;
-  const int hk = e % Hkv, h = hk * G + e / Hkv;
+  const int hk = e % Hkv;
   const int q_begin = cu_seqlens[b];
   const int q_len = cu_seqlens[b + 1] - q_begin;
   const int hist = seq_lens[b] - q_len;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i16 = lane & 15, g4 = lane >> 4;
+  // HEADS: the lane's column is a head (columns past the group's last do that one's work once more, never stored)
+  const int h = hk * G + (HEADS ? min(i16, G - 1) : e / Hkv);
   const int q0 = tile * QW;
   if (q0 >= q_len) return;                // the whole workgroup: nobody is left waiting at the barrier below
   if (skip_single && q_len == 1) return;  // single rows go to the split-K kernel
@@ -425,7 +437,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
   int col_lo[QT], col_hi[QT];
 #pragma unroll
   for (int t = 0; t < QT; ++t) {
-    const int row = q0 + t * 16 + i16;
+    const int row = HEADS ? 0 : q0 + t * 16 + i16;
     const int rc = row < q_len ? row : q_len - 1;  // rows past the end compute something harmless, never stored
     const bf16* qp = q + (int64_t)(q_begin + rc) * ld_q + (int64_t)h * D;
 #pragma unroll
@@ -439,11 +451,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
   }
   // the keys any row of the tile sees, and this wave's run of 32-key blocks among them
   const int p_first = hist + q0;
-  const int p_last = hist + (q0 + QW < q_len ? q0 + QW : q_len) - 1;
+  const int p_last = HEADS ? hist : hist + (q0 + QW < q_len ? q0 + QW : q_len) - 1;
   const int all_hi = p_last + 1;
   const int all_lo = low_of(p_first), last_lo = low_of(p_last);
   const int blk_first = all_lo >> 5, blk_end = (all_hi + 31) >> 5;
-  const int per = (blk_end - blk_first + 3) >> 2;
+  const int per = (blk_end - blk_first + PARTS) / WAVES;
   const int blk0 = blk_first + wave * per;
   const int blk1 = blk0 + per < blk_end ? blk0 + per : blk_end;
   const int k_lo = blk0 * 32 > all_lo ? blk0 * 32 : all_lo;
@@ -489,26 +501,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
     // o = sum_r 2^(c (m_r - M)) o_r, likewise l (still a partial over the lane's keys)
     float inv;
     if constexpr (KIND == SIGMOID) {      // weights against no reference: the parts simply add up
-#pragma unroll
-      for (int r = 0; r < 3; ++r)
+#pragma unroll AT_ONCE
+      for (int r = 0; r < PARTS; ++r)
 #pragma unroll
         for (int d = 0; d < DV; ++d) tl.o[t][d] += part_o(r, t, d);
       inv = ext.out_scale;
     } else {
-      float mr[3], M = tl.m[t];
+      float M = tl.m[t];
 #pragma unroll
-      for (int r = 0; r < 3; ++r) {
-        mr[r] = part_m(r, t);
-        M = fmaxf(M, mr[r]);
-      }
+      for (int r = 0; r < PARTS; ++r) M = fmaxf(M, part_m(r, t));
       const float mc = (M == -INFINITY ? 0.f : M) * scale_log2e;
       const float a0 = exp2_raw(fmaf(tl.m[t], scale_log2e, -mc));  // an empty part has m = -inf: weight 0
       float lsum = tl.l[t] * a0;
 #pragma unroll
       for (int d = 0; d < DV; ++d) tl.o[t][d] *= a0;
-#pragma unroll
-      for (int r = 0; r < 3; ++r) {
-        const float ar = exp2_raw(fmaf(mr[r], scale_log2e, -mc));
+#pragma unroll AT_ONCE
+      for (int r = 0; r < PARTS; ++r) {
+        const float ar = exp2_raw(fmaf(part_m(r, t), scale_log2e, -mc));
         lsum += part_l(r, t) * ar;
 #pragma unroll
         for (int d = 0; d < DV; ++d) tl.o[t][d] += part_o(r, t, d) * ar;
@@ -532,8 +541,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
         inv = lt > 0.f ? 1.f / lt : 0.f;
       }
     }
-    const int row = q0 + t * 16 + i16;
-    if (row < q_len) {
+    const int row = HEADS ? 0 : q0 + t * 16 + i16;
+    if (HEADS ? i16 < G : row < q_len) {
       bf16* op = out + (int64_t)(q_begin + row) * ld_out + (int64_t)h * (DV * 16) + 4 * g4;
 #pragma unroll
       for (int d = 0; d < DV; ++d) {
