@@ -838,22 +838,53 @@ __global__ void __launch_bounds__(256) moe_topk_kernel(const float* __restrict__
 // One workgroup. entries = tokens * top.
 // Experts from `real` on have no weights (their output is their input): their entries are sorted like the others', but
 // no tile is made for them.
+// Bound by latencies: the entries are read eight at once (one after the other a load's latency each), the counts are
+// summed up by a wave (one thread: 64 times LDS's latency). 64 experts, 6 a token: 2,023 tokens 13.0 -> 9.1 us, 4,096
+// 19.5 -> 15.6, 64 7.6 -> 5.5.
 __global__ void __launch_bounds__(1024) moe_scatter_kernel(const int32_t* __restrict__ idx, int entries, int E, int tile_rows,
                                                            int32_t* __restrict__ offsets, int32_t* __restrict__ perm,
                                                            int32_t* __restrict__ tiles, int max_tiles, int real) {
   __shared__ int cnt[MAX_EXPERTS], off[MAX_EXPERTS + 1], tbase[MAX_EXPERTS + 1];
+  auto each_entry = [&](auto fn) {
+    constexpr int AT_ONCE = 8;
+    for (int i0 = threadIdx.x; i0 < entries; i0 += AT_ONCE * 1024) {
+      int e[AT_ONCE];
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k) e[k] = idx[min(i0 + k * 1024, entries - 1)];
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k)
+        if (i0 + k * 1024 < entries) fn(i0 + k * 1024, e[k]);
+    }
+  };
   for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < entries; i += blockDim.x) atomicAdd(&cnt[idx[i]], 1);
+  each_entry([&](int, int e) { atomicAdd(&cnt[e], 1); });
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
     int o = 0, tb = 0;
-    for (int e = 0; e < E; ++e) {
-      off[e] = o; tbase[e] = tb;
-      o += cnt[e];
-      if (e < real) tb += (cnt[e] + tile_rows - 1) / tile_rows;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane, c = e < E ? cnt[e] : 0, n = e < real ? (c + tile_rows - 1) / tile_rows : 0;
+      int co = c, cn = n;      // summed up to this lane
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int a = __shfl_up(co, d, 64), b = __shfl_up(cn, d, 64);
+        if (lane >= d) {
+          co += a;
+          cn += b;
+        }
+      }
+      if (e < E) {
+        off[e] = o + co - c;
+        tbase[e] = tb + cn - n;
+      }
+      o += __shfl(co, 63, 64);
+      tb += __shfl(cn, 63, 64);
     }
-    off[E] = o; tbase[E] = tb;
+    if (lane == 0) {
+      off[E] = o;
+      tbase[E] = tb;
+    }
   }
   __syncthreads();
   for (int e = threadIdx.x; e <= E; e += blockDim.x) offsets[e] = off[e];
@@ -872,10 +903,7 @@ __global__ void __launch_bounds__(1024) moe_scatter_kernel(const int32_t* __rest
   }
   for (int at = tbase[E] + threadIdx.x; at < max_tiles; at += blockDim.x) { tiles[2 * at] = -1; tiles[2 * at + 1] = 0; }
   __syncthreads();
-  for (int i = threadIdx.x; i < entries; i += blockDim.x) {
-    const int e = idx[i];
-    perm[off[e] + atomicAdd(&cnt[e], 1)] = i;
-  }
+  each_entry([&](int i, int e) { perm[off[e] + atomicAdd(&cnt[e], 1)] = i; });
 }
 
 template <class S>

@@ -129,3 +129,23 @@ def test_heads_of_few_rows(M):
     out = torch.full((M, H * N), 7.0, dtype=torch.bfloat16, device=DEV)
     ops.heads_nt(a, 0, K, w, out, 0, N, M)
     close(out, torch.cat([a[:, h * K:(h + 1) * K].double() @ w[h].double().T for h in range(H)], dim=1))
+
+
+@pytest.mark.parametrize("entries,experts,real,tile_rows", [(1, 1, 1, 128), (63, 64, 64, 16), (1024, 65, 60, 128), (8193, 130, 130, 128), (20000, 200, 190, 32)])
+def test_entries_are_sorted_by_expert(entries, experts, real, tile_rows):
+    from dinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(entries)
+    idx = (torch.rand(entries, generator=g) ** 2 * experts).to(torch.int32)
+    most = -(-entries // tile_rows) + experts
+    offsets, perm, tiles = (torch.full((n,), -7, dtype=torch.int32, device=DEV) for n in (experts + 1, entries + 1, 2 * most))
+    ops.lib.call("dinfer_moe_scatter", idx.to(DEV).data_ptr(), entries, experts, tile_rows, offsets.data_ptr(), perm.data_ptr(),
+                 tiles.data_ptr(), most, real, ops._stream())
+    counts = torch.bincount(idx.long(), minlength=experts)
+    off = torch.cat([torch.zeros(1, dtype=torch.long), counts.cumsum(0)])
+    assert torch.equal(offsets.cpu().long(), off) and perm[entries].item() == -7
+    p = perm[:entries].cpu().long()
+    assert torch.equal(p.sort().values, torch.arange(entries))
+    assert torch.equal(idx[p].long(), torch.arange(experts).repeat_interleave(counts))
+    want = sorted((e, int(off[e]) + r) for e in range(real) for r in range(0, int(counts[e]), tile_rows))
+    got = [tuple(t) for t in tiles.cpu().view(-1, 2).tolist()]
+    assert sorted(t for t in got if t[0] >= 0) == want and len(got) == most
