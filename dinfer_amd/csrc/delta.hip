@@ -348,6 +348,55 @@ __global__ void __launch_bounds__(256) delta_recurrence_kernel(
   }
 }
 
+// Steps of single rows (decoding), D a multiple of 4 from 68 to 128: the whole state in and out once. A thread holds 4 rows of
+// SINGLE_COLS columns, all on their way at once, and reads its part of k and q itself: nothing waits at a barrier. The
+// arithmetic of the kernel above, bit by bit. Bound by memory: 64 requests of 16 heads of 128 x 128 (134 MB) 45.9 -> 21.8 us, 8 requests 7.9 -> 4.3.
+constexpr int SINGLE_COLS = 4;
+__global__ void __launch_bounds__(256) delta_single_kernel(const float* __restrict__ work, int64_t ldw, float* __restrict__ state,
+                                                           const int32_t* __restrict__ slots, const int32_t* __restrict__ cu,
+                                                           const int32_t* __restrict__ seq_lens, float* __restrict__ out,
+                                                           int64_t ld_out, int G, int H, int D, int V) {
+  const int b = blockIdx.z, h = blockIdx.y;
+  const int rg = threadIdx.x & 31, j0 = blockIdx.x * 8 * SINGLE_COLS + (threadIdx.x >> 5);
+  const int64_t t = cu[b];
+  const bool fresh = seq_lens[b] <= 1;
+  const int g = h / (H / G), gd = 2 * G * D;
+  const bool row_ok = rg * 4 < D;
+  float* sp = state + (((int64_t)slots[b] * H + h) * V + j0) * D + rg * 4;
+  const float* row = work + t * ldw;
+  f32x4 S[SINGLE_COLS], k = {0.f, 0.f, 0.f, 0.f}, q = k;
+#pragma unroll
+  for (int c = 0; c < SINGLE_COLS; ++c) {
+    S[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (!fresh && row_ok && j0 + 8 * c < V) S[c] = *(const f32x4*)(sp + (int64_t)8 * c * D);
+  }
+  if (row_ok) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      q[i] = row[g * D + rg * 4 + i];
+      k[i] = row[G * D + g * D + rg * 4 + i];
+    }
+  }
+  const float bt = row[gd + H * V + h], gt = row[gd + H * V + H + h];
+  float v[SINGLE_COLS];
+#pragma unroll
+  for (int c = 0; c < SINGLE_COLS; ++c) v[c] = j0 + 8 * c < V ? row[gd + h * V + j0 + 8 * c] : 0.f;
+  // two chains a sum, as above
+  auto dot = [](const f32x4& x, const f32x4& y) {
+    return __builtin_fmaf(x[2], y[2], __builtin_fmaf(x[0], y[0], 0.f)) + __builtin_fmaf(x[3], y[3], __builtin_fmaf(x[1], y[1], 0.f));
+  };
+  const float kq = half_wave_sum(dot(k, q));
+#pragma unroll
+  for (int c = 0; c < SINGLE_COLS; ++c) {
+    const float a = half_wave_sum(dot(S[c], k)), bq = half_wave_sum(dot(S[c], q));
+    const float u = bt * (v[c] - gt * a);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[c][i] = __builtin_fmaf(k[i], u, gt * S[c][i]);
+    if (row_ok && j0 + 8 * c < V) *(f32x4*)(sp + (int64_t)8 * c * D) = S[c];
+    if (rg == 0 && j0 + 8 * c < V) out[t * ld_out + h * V + j0 + 8 * c] = __builtin_fmaf(kq, u, gt * bq);
+  }
+}
+
 template <class S>
 __global__ void __launch_bounds__(WAVES * 64) delta_out_kernel(const float* __restrict__ o, int64_t ld_o,
                                                                const S* __restrict__ proj, int64_t ld, int64_t g_off,
@@ -610,12 +659,18 @@ extern "C" int dinfer_delta_conv_update(int dtype, const void* proj, int64_t ld,
 // state [slots, H, V, D] float (S transposed); out [T, ld_out] float, head h at column h V.
 extern "C" int dinfer_delta_recurrence(const float* work, int64_t ldw, float* state, const int32_t* state_slots,
                                        const int32_t* cu_seqlens, const int32_t* seq_lens, float* out, int64_t ld_out,
-                                       int num_reqs, int G, int H, int D, int V, int below,
+                                       int num_reqs, int G, int H, int D, int V, int below, int single,
                                        hipStream_t stream) {
   if (num_reqs <= 0) return OK;
   if (G <= 0 || H <= 0 || H % G || D <= 0 || V <= 0 || num_reqs > 65535 || H > 65535) return ERR_BAD_SHAPE;
   if (D > 256) return ERR_UNSUPPORTED;
   const dim3 grid((unsigned)((V + COLS - 1) / COLS), (unsigned)H, (unsigned)num_reqs);
+  if (single && D > 64 && D <= 128 && D % 4 == 0 && (uintptr_t)state % 16 == 0) {
+    const int cols = 8 * SINGLE_COLS;
+    delta_single_kernel<<<dim3((unsigned)((V + cols - 1) / cols), (unsigned)H, (unsigned)num_reqs), 256, 0, stream>>>(
+        work, ldw, state, state_slots, cu_seqlens, seq_lens, out, ld_out, G, H, D, V);
+    return launch_status();
+  }
 #define DELTA_REC(R_)                                                                                               \
   delta_recurrence_kernel<R_><<<grid, 256, 0, stream>>>(work, ldw, state, state_slots, cu_seqlens, seq_lens, out, \
                                                         ld_out, G, H, D, V, below)

@@ -84,7 +84,7 @@ SIGNATURES = {
     "dinfer_delta_prep": ("delta", [_I, _P, _L, _L, _L, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _L, _I, _I, _I,
                                     _I, _I, _F, _F, _P]),
     "dinfer_delta_conv_update": ("delta", [_I, _P, _L, _L, _P, _P, _P, _P, _I, _I, _I, _P]),
-    "dinfer_delta_recurrence": ("delta", [_P, _L, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P]),
+    "dinfer_delta_recurrence": ("delta", [_P, _L, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _I, _P]),
     "dinfer_delta_out": ("delta", [_I, _P, _L, _P, _L, _L, _P, _P, _L, _L, _L, _I, _I, _F, _F, _I, _I, _P]),
     "dinfer_channel_delta_prep": ("delta", [_I, _P, _L, _L, _L, _L, _L, _L, _P, _P, _P, _I, _P, _L, _L, _I, _I, _F, _F, _P, _L,
                                             _P]),
@@ -94,7 +94,7 @@ SIGNATURES = {
     "dinfer_rot_widen": ("decay", [_I, _P, _L, _L, _L, _L, _P, _P, _I, _F, _P, _L, _L, _I, _I, _I, _P]),
     "dinfer_conv_silu": ("decay", [_I, _P, _L, _L, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _L, _I, _I, _I, _P]),
     "dinfer_decay_recurrence": ("decay", [_P, _L, _P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I,
-                                          _I, _I, _P]),
+                                          _I, _I, _I, _P]),
     "dinfer_chunk_floats": ("chunked", [_I, _I, _I, _I, _I]),
     "dinfer_chunked_recurrence": ("chunked", [_I, _P, _L, _P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _P, _L, _P, _I, _I,
                                               _I, _I, _I, _I, _I, _I, _P]),

@@ -399,8 +399,8 @@ def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor,
                      cu_seqlens: torch.Tensor, seq_lens: torch.Tensor, num_reqs: int, qk_heads: int, heads: int,
                      dim: int, vdim: int, tokens: int | None = None, scratch: torch.Tensor | None = None) -> torch.Tensor:
     """The recurrence over each request's rows of the step. state [slots, heads, vdim, dim] float32 (a head's matrix
-    transposed), updated in place; out [T, heads * vdim] float32. tokens, scratch: the step's rows and a buffer of
-    chunk_scratch's size; with them requests of CHUNKED_ROWS rows or more go chunk by chunk."""
+    transposed), updated in place; out [T, heads * vdim] float32. tokens, scratch: the step's rows (one a request at
+    least) and a buffer of chunk_scratch's size; with them requests of CHUNKED_ROWS rows or more go chunk by chunk."""
     _need_gpu(work, state, out, state_slots, cu_seqlens, seq_lens)
     assert work.dtype == state.dtype == out.dtype == torch.float32 and state.is_contiguous()
     assert tuple(state.shape[1:]) == (heads, vdim, dim) and out.shape[1] >= heads * vdim
@@ -411,7 +411,7 @@ def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor,
     if below > 0:
         lib.call("dinfer_delta_recurrence", work.data_ptr(), _rows(work), state.data_ptr(), state_slots.data_ptr(),
                  cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs, qk_heads, heads, dim,
-                 vdim, below, _stream())
+                 vdim, below, int(tokens == num_reqs), _stream())
     return out
 
 
@@ -563,8 +563,8 @@ def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: t
     """Per request and head, token by token: S <- decay S + gain k v^T, out = S^T q. q, k: float32 views [T, groups dim]
     (head h reads group h // (heads / groups)); v [T, heads vdim]; decay [T, heads], or [heads] for one decay a head;
     gain [T, heads] or None. state [slots, heads, vdim, dim] float32, updated in place; out [T, >= heads vdim] float32.
-    tokens, scratch: the step's rows and a buffer of chunk_scratch's size; with them requests of CHUNKED_ROWS rows or
-    more go chunk by chunk."""
+    tokens, scratch: the step's rows (one a request at least) and a buffer of chunk_scratch's size; with them requests of
+    CHUNKED_ROWS rows or more go chunk by chunk."""
     _need_gpu(q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens)
     tensors = [q, k, v, decay, state, out] + ([gain] if gain is not None else [])
     assert all(t.dtype == torch.float32 for t in tensors) and state.is_contiguous()
@@ -583,7 +583,7 @@ def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: t
         lib.call("dinfer_decay_recurrence", q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v),
                  decay.data_ptr(), ldd, _ptr(gain), _rows(gain) if gain is not None else 0, state.data_ptr(),
                  state_slots.data_ptr(), cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs,
-                 groups, heads, dim, vdim, below, _stream())
+                 groups, heads, dim, vdim, below, int(tokens == num_reqs), _stream())
     return out
 
 

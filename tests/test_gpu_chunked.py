@@ -97,3 +97,29 @@ def test_against_token_by_token(case):
             worst[c], rms[c] = e.abs().max().item(), e.pow(2).mean().sqrt().item()
         assert worst[True] < 4 * (7 + 6) * 2.0 ** -24, (worst, rms)
         assert rms[True] <= 1.02 * rms[False], (worst, rms)
+
+
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("G,H,D,V,B", [(1, 2, 128, 128, 3), (2, 4, 68, 40, 1), (1, 3, 100, 9, 70), (2, 2, 128, 33, 5), (1, 1, 64, 32, 2)])
+def test_single_rows_have_the_same_bits(delta, G, H, D, V, B):
+    """A step of single rows, told so, against the kernel for any rows: the same arithmetic, so the same bits; columns that fill
+    no workgroup, heads that fill no half wave, a request that starts from nothing."""
+    from dinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(D + V)
+    cols = ops.delta_work_columns(G, H, D, V) + 3
+    work = torch.rand(B, cols, generator=g).cuda()
+    state0 = torch.randn(B + 2, H, V, D, generator=g)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    common = dict(state_slots=torch.randperm(B + 2, generator=g)[:B].to(**i32), cu_seqlens=torch.arange(B + 1, **i32),
+                  seq_lens=torch.tensor([1 + b % 3 for b in range(B)], **i32), num_reqs=B, heads=H, dim=D, vdim=V)
+    got = []
+    for told in (dict(), dict(tokens=B)):
+        state, out = state0.cuda(), torch.full((B + 1, H * V), 7.0, device="cuda")
+        if delta:
+            ops.delta_recurrence(work, state, out, qk_heads=G, **common, **told)
+        else:
+            qk, ve = G * D, 2 * G * D + H * V
+            ops.decay_recurrence(work[:, :qk], work[:, qk:2 * qk], work[:, 2 * qk:ve], work[:, ve + H:ve + 2 * H], work[:, ve:ve + H],
+                                 state, out, groups=G, **common, **told)
+        got.append((out, state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
