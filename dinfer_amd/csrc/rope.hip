@@ -312,14 +312,14 @@ __device__ __forceinline__ void v_write_transposed(const bf16* __restrict__ qkv,
   }
 }
 
-// bf16, whole-head neox rotation, D in {64, 128, 256}: LPH = D / 8 lanes share a head, each with 8
-// consecutive dims in one 16-byte load; the partner of a pair sits LPH / 2 lanes away and comes by a
-// cross-lane read. A wave covers 64 / LPH heads of one token per instruction, an order of magnitude
+// bf16, rotation of the whole head, D in {64, 128, 256}: LPH = D / 8 lanes share a head, each with 8
+// consecutive dims in one 16-byte load; the partner of a pair (i, i + D / 2) sits LPH / 2 lanes away and comes by a
+// cross-lane read, pairs (2i, 2i + 1) (NEIGHBOURS) lie in the lane itself. A wave covers 64 / LPH heads of one token per instruction, an order of magnitude
 // fewer memory instructions than 2-byte accesses.
 // gather_v > 0: V is not written by the heads' lanes; the workgroups from blockIdx.x = `tokens` on (gather_v of them,
 // one per kv head and run of 8 * WAVES tokens) gather it into its transposed pages, in the same launch (a kernel of
 // its own for that cost a prefill layer 5.7 us, a step of prompt portions beside decoding requests 7.8).
-template <int LPH>
+template <int LPH, bool NEIGHBOURS>
 __global__ void __launch_bounds__(WAVES * 64) qkv_post_vec_kernel(
     bf16* __restrict__ qkv, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, const void* __restrict__ wq,
     const void* __restrict__ wk, int wf32, float eps, float w_offset, const int32_t* __restrict__ pos,
@@ -354,10 +354,15 @@ __global__ void __launch_bounds__(WAVES * 64) qkv_post_vec_kernel(
     return item < H ? row + q_off + (int64_t)item * D
                     : item < H + Hkv ? row + k_off + (int64_t)(item - H) * D : row + v_off + (int64_t)(item - H - Hkv) * D;
   };
-  // angles of this lane's dims: the pair index of dim d is d mod D/2
+  // angles of this lane's dims: the pair index of dim d is d mod D/2, or d / 2
   float c[8], sn[8];
-  const int pi = d0 % HALF;
-  if (cos_sin) {
+  const int pi = NEIGHBOURS ? d0 / 2 : d0 % HALF;
+  if (cos_sin && NEIGHBOURS) {
+    const float* cs = cos_sin + (int64_t)pos[t] * D;
+    const f32x4 c0 = *(const f32x4*)(cs + pi), s0 = *(const f32x4*)(cs + HALF + pi);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { c[e] = c0[e]; sn[e] = s0[e]; }
+  } else if (cos_sin) {
     const float* cs = cos_sin + (int64_t)pos[t] * D;
     const f32x4 c0 = *(const f32x4*)(cs + pi), c1 = *(const f32x4*)(cs + pi + 4);
     const f32x4 s0 = *(const f32x4*)(cs + HALF + pi), s1 = *(const f32x4*)(cs + HALF + pi + 4);
@@ -439,17 +444,27 @@ __global__ void __launch_bounds__(WAVES * 64) qkv_post_vec_kernel(
     // a query grows with its position: 1 + coef ln(floor((p + 1) / every) + 1)
     if (is_q && w && temp_every > 0) inv *= 1.f + temp_coef * logf((float)((pos[t] + 1) / temp_every) + 1.f);
     if (is_q && w && head_scale) inv *= head_scale[item];
-    float y[8], other[8];
+    float y[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) y[e] = (qk && w) ? x[e] * inv * g[e] : x[e];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) other[e] = __shfl_xor(y[e], LPH / 2, 64);
-    if (!qk) continue;
-    const bool first = l < LPH / 2;  // this lane holds the first elements of its pairs
     bf16x8 r;
+    if constexpr (NEIGHBOURS) {
+      if (!qk) continue;
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      r[e] = (bf16)(first ? rotated_first(y[e], other[e], c[e], sn[e]) : rotated_second(other[e], y[e], c[e], sn[e]));
+      for (int e = 0; e < 8; e += 2) {
+        r[e] = (bf16)rotated_first(y[e], y[e + 1], c[e / 2], sn[e / 2]);
+        r[e + 1] = (bf16)rotated_second(y[e], y[e + 1], c[e / 2], sn[e / 2]);
+      }
+    } else {
+      float other[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) other[e] = __shfl_xor(y[e], LPH / 2, 64);
+      if (!qk) continue;
+      const bool first = l < LPH / 2;  // this lane holds the first elements of its pairs
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        r[e] = (bf16)(first ? rotated_first(y[e], other[e], c[e], sn[e]) : rotated_second(other[e], y[e], c[e], sn[e]));
+    }
     if (is_q || !slots) {
       *(bf16x8*)(src + d0) = r;
     } else if (slot >= 0) {
@@ -757,7 +772,11 @@ extern "C" int dinfer_qkv_post(int dtype, void* qkv, int64_t tokens, int64_t ld,
                       ((uintptr_t)q_gain % 16) == 0 && ((uintptr_t)k_gain % 16) == 0 && ((uintptr_t)cos_sin % 16) == 0 &&
                       ((uintptr_t)k_cache % 16) == 0 && ((uintptr_t)bias % 16) == 0 &&
                       (!v_first || (((uintptr_t)v_first % 16) == 0 && ld_v_first % 8 == 0));
-  if (whole_head_neox && vec_ok) {
+  // pairs (2i, 2i + 1) of whole heads: 27.9 us by the general kernel (a wave a head, 2-byte stores) at 2,048 rows of 24 heads of
+  // 128, 10.3 by this one (1 row 3.7, 3.3). Without a table nothing is rotated and both styles are one.
+  const bool whole_head = style == 0 ? whole_head_neox
+                                     : (!cos_sin || rotary_dim == head_dim) && v_dim == head_dim && (v_cache || !slot_mapping);
+  if (whole_head && vec_ok) {
     const int lph = head_dim / 8, hpw = 64 / lph;
     // many tokens fill the chip with one workgroup each; few tokens spread their heads over several
     // many tokens: V goes to its transposed pages through workgroups that gather it (16-byte stores)
@@ -766,8 +785,9 @@ extern "C" int dinfer_qkv_post(int dtype, void* qkv, int64_t tokens, int64_t ld,
     if (tokens + gather_v > 0x7fffffff) return ERR_BAD_SHAPE;
     const dim3 vgrid((unsigned)(tokens + gather_v),
                      tokens >= 512 ? 1u : (unsigned)((items + WAVES * hpw - 1) / (WAVES * hpw)));
+    const bool pairs = style == 1 && cos_sin;
 #define DINFER_QKV_VEC(LPH_)                                                                                          \
-  qkv_post_vec_kernel<LPH_><<<vgrid, WAVES * 64, 0, stream>>>(                                                         \
+  (pairs ? qkv_post_vec_kernel<LPH_, true> : qkv_post_vec_kernel<LPH_, false>)<<<vgrid, WAVES * 64, 0, stream>>>(      \
       (bf16*)qkv, ld, q_off, k_off, v_off, q_gain, k_gain, w_f32, eps, w_offset, positions, cos_sin, (bf16*)k_cache, \
       (bf16*)v_cache, slot_mapping, heads, kv_heads, page_size, (int)tokens, (int)gather_v, bias, temp_coef,       \
       temp_every, head_scale, mix)
