@@ -405,9 +405,11 @@ def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor,
     assert work.dtype == state.dtype == out.dtype == torch.float32 and state.is_contiguous()
     assert tuple(state.shape[1:]) == (heads, vdim, dim) and out.shape[1] >= heads * vdim
     assert work.shape[1] >= delta_work_columns(qk_heads, heads, dim, vdim)
-    qk, v_end = qk_heads * dim, 2 * qk_heads * dim + heads * vdim
-    below = _chunked(True, work, work[:, qk:], work[:, 2 * qk:], work[:, v_end + heads:], work[:, v_end:], state, out,
-                     state_slots, cu_seqlens, seq_lens, num_reqs, qk_heads, heads, dim, vdim, tokens, scratch)
+    below = EVERY_ROW
+    if _may_be_long(tokens, num_reqs, scratch):
+        qk, v_end = qk_heads * dim, 2 * qk_heads * dim + heads * vdim
+        below = _chunked(True, work, work[:, qk:], work[:, 2 * qk:], work[:, v_end + heads:], work[:, v_end:], state, out,
+                         state_slots, cu_seqlens, seq_lens, num_reqs, qk_heads, heads, dim, vdim, tokens, scratch)
     if below > 0:
         lib.call("dinfer_delta_recurrence", work.data_ptr(), _rows(work), state.data_ptr(), state_slots.data_ptr(),
                  cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs, qk_heads, heads, dim,
@@ -420,6 +422,7 @@ def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor,
 # 37, 21 and 26 against 27, 21 and 21; at 256 70, 43 and 50 against 33, 24 and 30; at 2,048 546, 323 and 362 against 128,
 # 117 and 125.
 CHUNKED_ROWS = 128
+EVERY_ROW = 2 ** 31 - 1     # (no request has as many)
 CHUNK = 64              # tokens of a chunk (chunked.hip)
 CHUNKS_AT_ONCE = 64     # chunks that a scratch buffer holds at most: longer steps go through it in turns
 
@@ -434,16 +437,17 @@ def chunk_scratch(delta: bool, groups: int, heads: int, dim: int, vdim: int, max
     return min(most, CHUNKS_AT_ONCE), floats
 
 
+def _may_be_long(tokens: int | None, num_reqs: int, scratch: torch.Tensor | None) -> bool:
+    """Whether a request of the step may have CHUNKED_ROWS rows: every one has a row at least."""
+    return scratch is not None and tokens is not None and num_reqs > 0 and tokens - num_reqs + 1 >= CHUNKED_ROWS
+
+
 def _chunked(delta, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens, num_reqs, groups, heads, dim,
              vdim, tokens, scratch) -> int:
-    """Runs the chunked form of a recurrence for the requests it takes, if the step may have any. Returns the rows below
-    which a request is left to the token-by-token kernel; 0: none is left."""
-    everything = 2 ** 31 - 1
-    # (every request of a step has a row at least: none has more than this)
-    if scratch is None or tokens is None or num_reqs <= 0 or tokens - num_reqs + 1 < CHUNKED_ROWS:
-        return everything
+    """Runs the chunked form of a recurrence for the requests it takes. Returns the rows below which a request is left to
+    the token-by-token kernel; 0: none is left."""
     if q.stride(0) % 4 or k.stride(0) % 4 or (q.data_ptr() | k.data_ptr() | state.data_ptr()) % 16:
-        return everything
+        return EVERY_ROW
     floats = lib.get("dinfer_chunk_floats")(int(delta), groups, heads, dim, vdim)
     assert scratch.dtype == torch.float32 and scratch.is_contiguous() and floats > 0 and scratch.shape[1] >= floats
     assert tokens <= q.shape[0] and tokens <= out.shape[0]
@@ -577,8 +581,10 @@ def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: t
         assert decay.shape[1] >= heads
         ldd = _rows(decay)
     assert gain is None or gain.shape[1] >= heads
-    below = _chunked(False, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens, num_reqs, groups, heads,
-                     dim, vdim, tokens, scratch)
+    below = EVERY_ROW
+    if _may_be_long(tokens, num_reqs, scratch):
+        below = _chunked(False, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens, num_reqs, groups, heads,
+                         dim, vdim, tokens, scratch)
     if below > 0:
         lib.call("dinfer_decay_recurrence", q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v),
                  decay.data_ptr(), ldd, _ptr(gain), _rows(gain) if gain is not None else 0, state.data_ptr(),
