@@ -434,6 +434,22 @@ __device__ __forceinline__ void store_rows(const Groups& p, const Tile& tl, int 
     }
 }
 
+// Tile j of the wave whose first column is c0 holds the expert's rows from weights_row on, weights_bytes of them: 32 rows, fewer
+// or none where the columns end. (Gated: j is the half, N rows each.)
+__host__ __device__ __forceinline__ int64_t weights_row(bool gated, int N, int c0, int j) {
+  return (int64_t)c0 + (gated ? (int64_t)j * N : 32 * j);
+}
+__host__ __device__ __forceinline__ uint32_t weights_bytes(bool gated, int N, int64_t ldw, int c0, int j) {
+  const int rows = N - c0 - (gated ? 0 : 32 * j);
+  return (uint32_t)(rows <= 0 ? 0 : rows < 32 ? rows : 32) * (uint32_t)ldw * 2u;
+}
+// The byte of a tile at which a lane's 16 begin in instruction r (pieces past K are those at K - 8, cleared before they are used).
+__host__ __device__ __forceinline__ uint32_t weights_at(int lane, int r, int64_t ldw, int K, int k0) {
+  const int row = 16 * ((lane >> 2) & 1) + 4 * ((lane >> 3) & 3) + r, k = k0 + ((lane >> 5) * 4 + (lane & 3)) * 8;
+  return ((uint32_t)row * (uint32_t)ldw + (uint32_t)(k < K - 8 ? k : K - 8)) * 2u;
+}
+constexpr int64_t WEIGHTS_K = (1 << 26) - 1;   // the widest row that 32 of fit such an offset
+
 template <class O, int END>
 __global__ void __launch_bounds__(256, 2) grouped_mfma_experts_kernel(Groups p) {
   constexpr bool GATED = END >= END_GATED;
@@ -486,18 +502,22 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_experts_kernel(Groups p) 
       *(bf16x8*)(As[buf] + row * BIG_K + ((sp ^ (row >> 1)) & 7) * 8) = f[q];
     }
   };
-  // (buffer loads: a row's offset is one register, what lies beyond the expert's rows reads as zero)
-  const __amdgpu_buffer_rsrc_t wd = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, (int)(p.w_zs * 2), 0x00020000);
-  const int w_lane = (16 * ((lane >> 2) & 1) + 4 * ((lane >> 3) & 3)) * (int)p.ldw * 2 + ((lane >> 5) * 4 + (lane & 3)) * 16;
+  // Buffer loads: what lies past the last column reads as zero. The bounds check of such a load is promised for a lane's
+  // offset alone, not for the scalar one: each tile has a descriptor that begins at its own first row, the rest of the
+  // address is the lane's.
+  __amdgpu_buffer_rsrc_t wd[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    wd[j] = __builtin_amdgcn_make_buffer_rsrc((void*)(W + weights_row(GATED, p.N, c0, j) * p.ldw), 0,
+                                              (int)weights_bytes(GATED, p.N, p.ldw, c0, j), 0x00020000);
   u32x4 w[2][2][4];   // [step's parity][tile of 32 columns][instruction, then MFMA]
   auto weights = [&](int k0, u32x4(&f)[2][4]) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int r = 0; r < 4; ++r) {
+      const int at = (int)weights_at(lane, r, p.ldw, K, k0);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = c0 + (GATED ? j * p.gate_n : 32 * j) + r;
-        f[j][r] = __builtin_amdgcn_raw_buffer_load_b128(wd, w_lane, (n * (int)p.ldw + k0) * 2, 0);
-      }
+      for (int j = 0; j < 2; ++j) f[j][r] = __builtin_amdgcn_raw_buffer_load_b128(wd[j], at, 0, 0);
+    }
   };
   auto order = [&](u32x4(&f)[4], int step) {   // four parts of a tile's way into the MFMA's order
     if (step == 0) swap_in_quads<false>(f[0], f[1]);
@@ -1050,9 +1070,16 @@ extern "C" int dinfer_experts_nt(int dtype, int gated, const void* A, int64_t ld
   if (gated < 0 || gated > 4) return ERR_UNSUPPORTED;
   p.act = gated >= 2 ? gated - 1 : 0;
   if (!mfma_fits(dtype, p) && tile_rows > BM) return ERR_UNSUPPORTED;
-  if (tile_rows == TM_BIG && w_zs > 0x30000000) return ERR_UNSUPPORTED;   // 32-bit offsets into an expert's weights
+  if (tile_rows == TM_BIG && (w_zs > 0x30000000 || ldw > WEIGHTS_K)) return ERR_UNSUPPORTED;   // 32-bit offsets into an expert's weights
   return gated == 1 ? launch_groups<true>(dtype, p, (unsigned)max_tiles, 1, stream)
                : launch_groups<false>(dtype, p, (unsigned)max_tiles, 1, stream);
+}
+
+// Where the experts' product of many rows reads: the byte of an expert's weights (the gate and up rows, or N rows, of ldw) at
+// which lane `lane` of the wave whose first column is c0 reads 16 in instruction r of tile j, in the step at k0; -1: nowhere.
+extern "C" int64_t dinfer_experts_weights_byte(int gated, int N, int64_t ldw, int K, int c0, int j, int r, int lane, int k0) {
+  const uint32_t at = weights_at(lane, r, ldw, K, k0);
+  return at < weights_bytes(gated, N, ldw, c0, j) ? weights_row(gated, N, c0, j) * ldw * 2 + at : -1;
 }
 
 // Rows of a tile for a routed layer's two products: the matrix-core kernels take 16 (few rows an expert: the weights
