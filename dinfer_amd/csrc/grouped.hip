@@ -507,9 +507,13 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_experts_kernel(Groups p) 
   // address is the lane's.
   __amdgpu_buffer_rsrc_t wd[2];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
-    wd[j] = __builtin_amdgcn_make_buffer_rsrc((void*)(W + weights_row(GATED, p.N, c0, j) * p.ldw), 0,
-                                              (int)weights_bytes(GATED, p.N, p.ldw, c0, j), 0x00020000);
+  for (int j = 0; j < 2; ++j) {
+    const uint64_t at = (uint64_t)(W + weights_row(GATED, p.N, c0, j) * p.ldw);
+    // (in scalar registers: one that the compiler works out in vector registers costs a loop around every load)
+    const uint64_t base = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    wd[j] = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, __builtin_amdgcn_readfirstlane((int)weights_bytes(GATED, p.N, p.ldw, c0, j)),
+                                              0x00020000);
+  }
   u32x4 w[2][2][4];   // [step's parity][tile of 32 columns][instruction, then MFMA]
   auto weights = [&](int k0, u32x4(&f)[2][4]) {
 #pragma unroll
