@@ -45,12 +45,24 @@ int launch_rows(const Args& p, hipStream_t stream) {
   return launch_status();
 }
 
+// Whether a step of single rows takes the tile of heads, for `rows` = requests x heads. It reads a group's keys once and walks them
+// with eight waves, in fewer and larger workgroups. Measured against the tile of rows at 1 to 64 requests behind 40 to 4,000
+// keys, groups of 1 to 16. Heads of up to 128: as fast behind 300 keys, faster beyond (one request behind 4,000: 24 -> 19 us, 64
+// behind 1,000 in groups of 4: 40 -> 23); groups of one share nothing, so there only while the workgroups leave CUs empty (64 rows
+// behind 4,000: 37 -> 30 us, 256: 93 -> 94, 1,024 behind 40: 8 -> 12). Heads of 256 fill a CU's LDS: from 256 rows in groups of
+// 4 and more (25 -> 20 us; 64 rows behind 4,000: 46 -> 49), from 1,024 in smaller ones (403 -> 362; 256 rows: 105 -> 114).
+bool shares_heads(int group, int64_t rows, bool large) {
+  if (group > 16) return false;
+  if (large) return group >= 4 ? rows >= 256 : group >= 2 && rows >= 1024;
+  return group >= 2 || rows <= 128;
+}
+
 // Rows a workgroup takes: 48 at heads of 128 where the rows make several rounds of workgroups over the chip (rows of at
 // most two tiles a request never fill the third), 32 where portions are longer than one tile, else 16. Steps of single rows:
-// the heads of a group instead of rows, where they fit a tile.
+// the heads of a group instead of rows (shares_heads).
 template <int DT, int DV, int KIND>
 int launch(const Args& p, hipStream_t stream) {
-  if (p.max_q_len == 1 && p.H / p.Hkv <= 16) return launch_rows<DT, DV, KIND, 1, true>(p, stream);
+  if (p.max_q_len == 1 && shares_heads(p.H / p.Hkv, (int64_t)p.H * p.num_reqs, DT > 8)) return launch_rows<DT, DV, KIND, 1, true>(p, stream);
   if constexpr (DT == 8 && DV == 8) {
     if (p.max_q_len > 32 && (int64_t)((p.max_q_len + 47) / 48) * p.H * p.num_reqs >= 2000) return launch_rows<DT, DV, KIND, 3>(p, stream);
   }

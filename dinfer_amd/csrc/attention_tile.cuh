@@ -381,7 +381,9 @@ struct FlashExt {
 // HEADS (steps of single rows): the columns of the tile are the heads of a group instead of rows, at most 16, so a kv
 // head's keys are read once instead of once a head, and eight waves share them. Bound by memory from some 64 rows on: 64
 // rows behind 4,200 keys each, 16 heads over 4 kv heads of 128, 241 -> 115 us (4.8 TB/s); 32 heads over 2, 2,100 keys,
-// 157 -> 27 us; below that by the walk of one wave over its run of keys, which is as long as before (8 rows: 42 us both ways).
+// 157 -> 27 us; below that by the walk of one wave over its run of keys. Fewer than 24 key blocks are dealt to no more waves than
+// runs of three need, and only waves with keys hand a part over: 16 heads over 4 of 128, one row behind 300 keys 6.4 -> 5.8 us
+// with all eight always joined, behind 40 5.3 -> 4.6 (tiles of rows 5.8 and 5.0).
 constexpr int flash_waves(bool heads) { return heads ? 8 : 4; }
 
 template <int DT, int QT, bool P2, int KIND = PLAIN, int DV = DT, bool HEADS = false>
@@ -455,7 +457,9 @@ __global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu
   const int all_hi = p_last + 1;
   const int all_lo = low_of(p_first), last_lo = low_of(p_last);
   const int blk_first = all_lo >> 5, blk_end = (all_hi + 31) >> 5;
-  const int per = (blk_end - blk_first + PARTS) / WAVES;
+  const int blocks = blk_end - blk_first;
+  const int per = HEADS ? max((blocks + PARTS) / WAVES, min(3, (blocks + 3) / 4)) : (blocks + PARTS) / WAVES;
+  const int parts = HEADS ? (blocks - 1) / per : PARTS;   // waves 1 .. parts have keys at all
   const int blk0 = blk_first + wave * per;
   const int blk1 = blk0 + per < blk_end ? blk0 + per : blk_end;
   const int k_lo = blk0 * 32 > all_lo ? blk0 * 32 : all_lo;
@@ -484,7 +488,7 @@ __global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu
     }
   }
 
-  if (wave > 0) {
+  if (wave > 0 && (!HEADS || wave <= parts)) {
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
       part_m(wave - 1, t) = tl.m[t];
@@ -502,21 +506,21 @@ __global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu
     float inv;
     if constexpr (KIND == SIGMOID) {      // weights against no reference: the parts simply add up
 #pragma unroll AT_ONCE
-      for (int r = 0; r < PARTS; ++r)
+      for (int r = 0; r < (HEADS ? parts : PARTS); ++r)
 #pragma unroll
         for (int d = 0; d < DV; ++d) tl.o[t][d] += part_o(r, t, d);
       inv = ext.out_scale;
     } else {
       float M = tl.m[t];
-#pragma unroll
-      for (int r = 0; r < PARTS; ++r) M = fmaxf(M, part_m(r, t));
+#pragma unroll AT_ONCE
+      for (int r = 0; r < (HEADS ? parts : PARTS); ++r) M = fmaxf(M, part_m(r, t));
       const float mc = (M == -INFINITY ? 0.f : M) * scale_log2e;
       const float a0 = exp2_raw(fmaf(tl.m[t], scale_log2e, -mc));  // an empty part has m = -inf: weight 0
       float lsum = tl.l[t] * a0;
 #pragma unroll
       for (int d = 0; d < DV; ++d) tl.o[t][d] *= a0;
 #pragma unroll AT_ONCE
-      for (int r = 0; r < PARTS; ++r) {
+      for (int r = 0; r < (HEADS ? parts : PARTS); ++r) {
         const float ar = exp2_raw(fmaf(part_m(r, t), scale_log2e, -mc));
         lsum += part_l(r, t) * ar;
 #pragma unroll

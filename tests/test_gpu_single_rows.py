@@ -59,3 +59,16 @@ def test_heads_of_a_group_share_the_tile(case):
     for name, got in (("heads", new), ("rows", rows)):
         err = (got.double() - want.double()).abs().max().item()
         assert err < 2.0 ** -7 * top, f"{name}: off by {err} of {top}"
+
+
+@pytest.mark.parametrize("case", [
+    (8, 4, 64, 64, 32, {}, [32 * n - n % 3 for n in range(1, 28)]),     # every count of key blocks up to three a wave and beyond
+    (8, 4, 48, 32, 16, dict(window=250, keep_first=33, sinks=True), list(range(20, 1100, 90))),
+    (16, 4, 256, 256, 16, {}, [40 * n + 1 for n in range(16)]),         # heads of 256: 256 rows in groups of four,
+    (4, 2, 256, 256, 32, dict(slope_exp=8.0), [7 + n % 130 for n in range(256)]),   # 1,024 in groups of two
+    (16, 4, 256, 256, 16, dict(softcap=5.0), [1, 900]),                 # ... and fewer: rows
+    (16, 16, 32, 32, 16, {}, [5, 77, 130, 200, 64, 1, 300, 31]),        # groups of one: 128 rows,
+    (16, 16, 32, 32, 16, {}, [5, 77, 130, 200, 64, 1, 300, 31, 9]),     # and more
+])
+def test_runs_of_keys_and_the_choice_of_the_tile(case):
+    test_heads_of_a_group_share_the_tile(case)
