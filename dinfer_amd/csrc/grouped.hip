@@ -460,7 +460,7 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_experts_kernel(Groups p) 
   // columns outside: tiles of one expert that run together read its weights once from memory and then from L2.
   int bx, by;
   {
-    const int nx = gridDim.x, id = blockIdx.y * nx + blockIdx.x, slot = id >> 3, r = slot % (4 * nx);
+    const int nx = gridDim.x, id = (blockIdx.z * gridDim.y + blockIdx.y) * nx + blockIdx.x, slot = id >> 3, r = slot % (4 * nx);
     bx = r >> 2;
     by = (slot / (4 * nx) * 4 + (r & 3)) * 8 + (id & 7);
     if (by >= p.max_tiles) return;
@@ -993,8 +993,8 @@ __global__ void __launch_bounds__(256) moe_combine_bf16x8_kernel(const bf16* __r
 template <int END>
 void launch_experts(const Groups& p, unsigned gy, hipStream_t stream) {
   const int cols = END >= END_GATED ? 128 : 256;
-  gy = (gy + 31) / 32 * 32;   // eight XCDs, four tiles at a time
-  grouped_mfma_experts_kernel<bf16, END><<<dim3((unsigned)((p.N + cols - 1) / cols), gy), 256, 0, stream>>>(p);
+  // eight XCDs, four tiles at a time (y and z together: the places rounded up may be more than y takes)
+  grouped_mfma_experts_kernel<bf16, END><<<dim3((unsigned)((p.N + cols - 1) / cols), (gy + 31) / 32, 32), 256, 0, stream>>>(p);
 }
 template <int END>
 void launch_big(const Groups& p, unsigned gy, unsigned gz, hipStream_t stream) {

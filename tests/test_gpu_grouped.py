@@ -149,3 +149,24 @@ def test_entries_are_sorted_by_expert(entries, experts, real, tile_rows):
     want = sorted((e, int(off[e]) + r) for e in range(real) for r in range(0, int(counts[e]), tile_rows))
     got = [tuple(t) for t in tiles.cpu().view(-1, 2).tolist()]
     assert sorted(t for t in got if t[0] >= 0) == want and len(got) == most
+
+
+@pytest.mark.parametrize("places", [65504, 65505, 65535])
+def test_work_lists_of_the_longest_length(places):
+    """As many places as a grid has in y, and the last counts before: the tiles named by the last places are worked off."""
+    from dinfer_amd.kernels import ops
+    E, N, K, n = 3, 24, 16, 300
+    g = torch.Generator(device=DEV).manual_seed(places)
+    a = torch.randn(n, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.randn(E, N, K, generator=g, device=DEV).to(torch.bfloat16)
+    out = torch.full((n, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    offsets = torch.tensor([0, 100, 150, n], dtype=torch.int32, device=DEV)
+    perm = torch.arange(n, dtype=torch.int32, device=DEV)
+    tiles = torch.full((places, 2), -1, dtype=torch.int32)
+    for at, tile in ((0, (0, 0)), (places // 2, (1, 100)), (places - 2, (2, 150)), (places - 1, (2, 278))):
+        tiles[at] = torch.tensor(tile, dtype=torch.int32)
+    tiles = tiles.to(DEV)
+    ops.lib.call("dinfer_experts_nt", ops.dtype_code(a.dtype), 0, a.data_ptr(), K, w.data_ptr(), K, N * K, out.data_ptr(), N, N, K,
+                 tiles.data_ptr(), places, 128, offsets.data_ptr(), perm.data_ptr(), 0, 1, 0, 0.0, 0.0, n, ops._stream())
+    for e, (lo, hi) in enumerate(((0, 100), (100, 150), (150, n))):
+        close(out[lo:hi], a[lo:hi].double() @ w[e].double().T)
