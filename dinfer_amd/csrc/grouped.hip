@@ -1074,7 +1074,7 @@ extern "C" int dinfer_experts_nt(int dtype, int gated, const void* A, int64_t ld
   if (gated < 0 || gated > 4) return ERR_UNSUPPORTED;
   p.act = gated >= 2 ? gated - 1 : 0;
   if (!mfma_fits(dtype, p) && tile_rows > BM) return ERR_UNSUPPORTED;
-  if (tile_rows == TM_BIG && (w_zs > 0x30000000 || ldw > WEIGHTS_K)) return ERR_UNSUPPORTED;   // 32-bit offsets into an expert's weights
+  if (tile_rows == TM_BIG && ldw > WEIGHTS_K) return ERR_UNSUPPORTED;   // (dinfer_moe_tile_rows names 16 there)
   return gated == 1 ? launch_groups<true>(dtype, p, (unsigned)max_tiles, 1, stream)
                : launch_groups<false>(dtype, p, (unsigned)max_tiles, 1, stream);
 }
@@ -1087,10 +1087,11 @@ extern "C" int64_t dinfer_experts_weights_byte(int gated, int N, int64_t ldw, in
 }
 
 // Rows of a tile for a routed layer's two products: the matrix-core kernels take 16 (few rows an expert: the weights
-// are streamed) or 128; anything else (float, sizes that are no multiples of 8) runs on the vector ALUs with 64.
+// are streamed) or 128; anything else (float, sizes that are no multiples of 8) runs on the vector ALUs with 64. Rows of
+// weights too wide for the 32-bit offsets of the kernel for 128 (2^26 numbers): 16.
 extern "C" int dinfer_moe_tile_rows(int dtype, int64_t entries, int experts, int64_t k_in, int64_t k_mid) {
   if (dtype != DT_BF16 || k_in % 8 || k_mid % 8) return BM;
-  return entries <= (int64_t)TM_SMALL * experts ? TM_SMALL : TM_BIG;
+  return entries <= (int64_t)TM_SMALL * experts || k_in > WEIGHTS_K || k_mid > WEIGHTS_K ? TM_SMALL : TM_BIG;
 }
 
 

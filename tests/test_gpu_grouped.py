@@ -170,3 +170,38 @@ def test_work_lists_of_the_longest_length(places):
                  tiles.data_ptr(), places, 128, offsets.data_ptr(), perm.data_ptr(), 0, 1, 0, 0.0, 0.0, n, ops._stream())
     for e, (lo, hi) in enumerate(((0, 100), (100, 150), (150, n))):
         close(out[lo:hi], a[lo:hi].double() @ w[e].double().T)
+
+
+@pytest.mark.parametrize("gated", [False, True])
+def test_an_expert_of_more_than_2_gb(gated):
+    from dinfer_amd.kernels import ops
+    E, N, K, n = 2, 280008, 4096, 70
+    g = torch.Generator(device=DEV).manual_seed(3)
+    a = torch.randn(n, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.empty(E, N, K, dtype=torch.bfloat16, device=DEV)
+    for e in range(E):
+        for lo in range(0, N, 20000):
+            w[e, lo:lo + 20000] = torch.randn(min(20000, N - lo), K, generator=g, device=DEV) / K ** 0.5
+    i32 = dict(dtype=torch.int32, device=DEV)
+    idx = (torch.arange(n, **i32) * 7 % 3 > 0).to(torch.int32)
+    perm, offsets, tiles = torch.zeros(n, **i32), torch.zeros(E + 1, **i32), torch.zeros((ops.moe_max_tiles(n, E, 128), 2), **i32)
+    rows = ops.moe_tile_rows(torch.bfloat16, n, E, K, K)
+    assert rows == 128
+    ops.moe_scatter(idx, n, E, offsets, perm, tiles, rows)
+    cols = N // 2 if gated else N
+    out = torch.full((n, cols), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.experts_nt(a, w, out, n, tiles, offsets, perm, gated=gated, a_div=1, c_to_perm=True, tile_rows=rows)
+    pick = torch.cat([torch.arange(300), torch.arange(0, cols, 997), torch.arange(cols - 300, cols)]).to(DEV)
+    for e in range(E):
+        at = (idx == e).nonzero().flatten()
+        y = a[at].double() @ w[e, pick].double().T
+        if gated:
+            y = act(y, "silu") * (a[at].double() @ w[e, pick + cols].double().T)
+        close(out[at][:, pick], y)
+
+
+def test_rows_too_wide_for_32_bit_offsets_take_tiles_of_16():
+    from dinfer_amd.kernels import ops
+    wide = 2 ** 26
+    assert ops.moe_tile_rows(torch.bfloat16, 1000, 2, wide - 8, 64) == 128
+    assert ops.moe_tile_rows(torch.bfloat16, 1000, 2, wide, 64) == 16 and ops.moe_tile_rows(torch.bfloat16, 1000, 2, 64, wide) == 16
