@@ -397,10 +397,12 @@ def delta_conv_update(proj: torch.Tensor, *, qkv_off: int, conv_state: torch.Ten
 
 def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor, *, state_slots: torch.Tensor,
                      cu_seqlens: torch.Tensor, seq_lens: torch.Tensor, num_reqs: int, qk_heads: int, heads: int,
-                     dim: int, vdim: int, tokens: int | None = None, scratch: torch.Tensor | None = None) -> torch.Tensor:
+                     dim: int, vdim: int, tokens: int | None = None, scratch: torch.Tensor | None = None,
+                     one_row_each: bool | None = None) -> torch.Tensor:
     """The recurrence over each request's rows of the step. state [slots, heads, vdim, dim] float32 (a head's matrix
     transposed), updated in place; out [T, heads * vdim] float32. tokens, scratch: the step's rows (one a request at
-    least) and a buffer of chunk_scratch's size; with them requests of CHUNKED_ROWS rows or more go chunk by chunk."""
+    least) and a buffer of chunk_scratch's size; with them requests of CHUNKED_ROWS rows or more go chunk by chunk.
+    one_row_each: whether every request has one row, no more and no less (None: it has if tokens equals num_reqs)."""
     _need_gpu(work, state, out, state_slots, cu_seqlens, seq_lens)
     assert work.dtype == state.dtype == out.dtype == torch.float32 and state.is_contiguous()
     assert tuple(state.shape[1:]) == (heads, vdim, dim) and out.shape[1] >= heads * vdim
@@ -413,7 +415,7 @@ def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor,
     if below > 0:
         lib.call("dinfer_delta_recurrence", work.data_ptr(), _rows(work), state.data_ptr(), state_slots.data_ptr(),
                  cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs, qk_heads, heads, dim,
-                 vdim, below, int(tokens == num_reqs), _stream())
+                 vdim, below, int(tokens == num_reqs if one_row_each is None else one_row_each), _stream())
     return out
 
 
@@ -451,10 +453,12 @@ def _chunked(delta, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, s
     floats = lib.get("dinfer_chunk_floats")(int(delta), groups, heads, dim, vdim)
     assert scratch.dtype == torch.float32 and scratch.is_contiguous() and floats > 0 and scratch.shape[1] >= floats
     assert tokens <= q.shape[0] and tokens <= out.shape[0]
+    # (a lone request is taken however many rows it has: `tokens` may be more than those)
+    shortest = 1 if num_reqs == 1 else CHUNKED_ROWS
     lib.call("dinfer_chunked_recurrence", int(delta), q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v),
              decay.data_ptr(), 0 if decay.dim() == 1 else _rows(decay), _ptr(gain), _rows(gain) if gain is not None else 0,
              state.data_ptr(), state_slots.data_ptr(), cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out),
-             scratch.data_ptr(), scratch.shape[0], tokens, num_reqs, CHUNKED_ROWS, groups, heads, dim, vdim, _stream())
+             scratch.data_ptr(), scratch.shape[0], tokens, num_reqs, shortest, groups, heads, dim, vdim, _stream())
     return 0 if num_reqs == 1 else CHUNKED_ROWS
 
 
@@ -563,12 +567,14 @@ def conv_silu(proj: torch.Tensor, tokens: int, *, x_off: int, dt_off: int, taps:
 def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, gain: torch.Tensor | None,
                      state: torch.Tensor, out: torch.Tensor, *, state_slots: torch.Tensor, cu_seqlens: torch.Tensor,
                      seq_lens: torch.Tensor, num_reqs: int, groups: int, heads: int, dim: int, vdim: int,
-                     tokens: int | None = None, scratch: torch.Tensor | None = None) -> torch.Tensor:
+                     tokens: int | None = None, scratch: torch.Tensor | None = None,
+                     one_row_each: bool | None = None) -> torch.Tensor:
     """Per request and head, token by token: S <- decay S + gain k v^T, out = S^T q. q, k: float32 views [T, groups dim]
     (head h reads group h // (heads / groups)); v [T, heads vdim]; decay [T, heads], or [heads] for one decay a head;
     gain [T, heads] or None. state [slots, heads, vdim, dim] float32, updated in place; out [T, >= heads vdim] float32.
     tokens, scratch: the step's rows (one a request at least) and a buffer of chunk_scratch's size; with them requests of
-    CHUNKED_ROWS rows or more go chunk by chunk."""
+    CHUNKED_ROWS rows or more go chunk by chunk. one_row_each: whether every request has one row, no more and no less (None:
+    it has if tokens equals num_reqs)."""
     _need_gpu(q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens)
     tensors = [q, k, v, decay, state, out] + ([gain] if gain is not None else [])
     assert all(t.dtype == torch.float32 for t in tensors) and state.is_contiguous()
@@ -589,7 +595,7 @@ def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: t
         lib.call("dinfer_decay_recurrence", q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v),
                  decay.data_ptr(), ldd, _ptr(gain), _rows(gain) if gain is not None else 0, state.data_ptr(),
                  state_slots.data_ptr(), cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs,
-                 groups, heads, dim, vdim, below, int(tokens == num_reqs), _stream())
+                 groups, heads, dim, vdim, below, int(tokens == num_reqs if one_row_each is None else one_row_each), _stream())
     return out
 
 

@@ -123,3 +123,39 @@ def test_single_rows_have_the_same_bits(delta, G, H, D, V, B):
                                  state, out, groups=G, **common, **told)
         got.append((out, state))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("rows,tokens", [
+    ([100], 200),            # a lone request of fewer rows than the step is long: it is not left out
+    ([1], 128), ([128], 128), ([70], 4300),
+    ([2, 0, 1], 3),          # as many rows as requests, but not one each
+    ([0, 0, 3, 1, 1], 5),
+])
+def test_steps_longer_than_their_rows(delta, rows, tokens):
+    """`tokens` says how long a step may be; what a request gets follows its own rows."""
+    from dinfer_amd.kernels import ops
+    G, H, D, V, B = 1, 2, 128, 32, len(rows)
+    g = torch.Generator().manual_seed(sum(rows) + tokens)
+    work = torch.rand(tokens, ops.delta_work_columns(G, H, D, V) + 2, generator=g) / 8
+    state0 = torch.randn(B + 1, H, V, D, generator=g)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    cu = torch.tensor([0] + rows).cumsum(0)
+    common = dict(state_slots=torch.arange(B, **i32), cu_seqlens=cu.to(**i32), seq_lens=torch.tensor([9 + n for n in rows], **i32),
+                  num_reqs=B, heads=H, dim=D, vdim=V)
+    size = ops.chunk_scratch(delta, G, H, D, V, 4300, B)
+    got = []
+    for more in (dict(), dict(tokens=tokens, scratch=torch.zeros(size, device="cuda"), one_row_each=False)):
+        w, state, out = work.cuda(), state0.cuda(), torch.full((tokens, H * V), 7.0, device="cuda")
+        w = torch.nn.functional.pad(w, (0, -w.shape[1] % 4))
+        if delta:
+            ops.delta_recurrence(w, state, out, qk_heads=G, **common, **more)
+        else:
+            qk, ve = G * D, 2 * G * D + H * V
+            ops.decay_recurrence(w[:, :qk], w[:, qk:2 * qk], w[:, 2 * qk:ve], w[:, ve + H:ve + 2 * H], w[:, ve:ve + H], state, out, groups=G,
+                                 **common, **more)
+        got.append((out, state))
+    # (both in 32 bits, sums of 128 products in two orders)
+    for a, b in zip(*got):
+        torch.testing.assert_close(b, a, rtol=1e-5, atol=1e-5 * a.abs().max().item())
+    assert (got[1][0][sum(rows):] == 7.0).all()
