@@ -26,6 +26,8 @@
 //                  kernel joins them; the launch shape follows the step's counts alone.
 #include "common.cuh"
 
+#include <type_traits>
+
 using namespace dinfer;
 
 namespace {
@@ -707,6 +709,9 @@ __global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
   // the workgroup's keys
   const int p_first = start + grp * 64 / H, p_last = start + (min(all_rows, grp * 64 + 64) - 1) / H;
   const int first = window > 0 ? max(p_first - window + 1, 0) : 0;
+  int last[4];   // the last key that row tile r sees (tiles without rows: as the others)
+#pragma unroll
+  for (int r = 0; r < 4; ++r) last[r] = min(start + (grp * 64 + 16 * r + 15) / H, p_last);
   const int page = 1 << page_shift, pmask = page - 1, page_lo = first >> page_shift, page_hi = p_last >> page_shift;
   const int32_t* bt = block_table + (int64_t)b * max_blocks;
 
@@ -856,13 +861,19 @@ __global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
         for (int t = 0; t < TW; ++t) o[t][r] = o[t][r] * a;
       }
     }
+    auto values = [&](auto all) {
 #pragma unroll
-    for (int t = 0; t < TW; ++t) {
-      const int d = 16 * (TW * wave + t) + lr;
-      const bf16x8 v = *(const bf16x8*)(Vs + d * 32 + ((g ^ (lr >> 2)) & 3) * 8);
+      for (int t = 0; t < TW; ++t) {
+        const int d = 16 * (TW * wave + t) + lr;
+        const bf16x8 v = *(const bf16x8*)(Vs + d * 32 + ((g ^ (lr >> 2)) & 3) * 8);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[t][r] = mfma16(v, pr[r], o[t][r]);
-    }
+        for (int r = 0; r < 4; ++r)
+          if (decltype(all)::value || kb <= last[r]) o[t][r] = mfma16(v, pr[r], o[t][r]);
+      }
+    };
+    // rows before the block take nothing of it, not 0 times what a later token left there (an infinity or NaN)
+    if (kb <= last[0]) values(std::true_type{});
+    else values(std::false_type{});
   };
   // this wave's loads into LDS have landed (a barrier alone does not wait for them), then everybody's; and everybody has read
   // the other buffer

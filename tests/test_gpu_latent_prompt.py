@@ -47,3 +47,25 @@ def test_latent_prompt_portions(case_no):
     seen = j <= p and (not window or j > p - window)
     close = (got[t, h * R:(h + 1) * R] - case["keys"][b][j][:R].double()).abs().max().item()
     assert (close < 0.1) == seen
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("n,hist,H,R,dr,page,at", [(100, 0, 1, 128, 32, 16, 40), (40, 9, 2, 512, 64, 64, 33), (300, 70, 4, 256, 64, 8, 300)])
+def test_a_bad_key_stays_away_from_rows_before_it(n, hist, H, R, dr, page, at, bad):
+    """An infinity or NaN that a later token left in the cache does not reach a tile of 16 rows that ends before its block of 32 keys."""
+    from dinfer_amd.kernels import ops
+    case = latent_case([hist + n], [n], H, R, dr, page, at, torch.bfloat16)
+    args = lambda c: (c["cache"], c["cache"][:, :, :R].transpose(1, 2).contiguous(), dev["bt"], dev["cu"], dev["seq"], 1, n, 1,
+                      torch.zeros(n * H * (R + 4), device="cuda"))
+    dev = {k: v.cuda() for k, v in case.items() if k != "keys"}
+    got = []
+    for value in (None, bad):
+        c = dict(cache=dev["cache"].clone())
+        if value is not None:
+            c["cache"][int(case["bt"][0, at // page]), at % page, :] = value
+        out = torch.zeros(n, H * R, dtype=torch.bfloat16, device="cuda")
+        ops.latent_attn_mfma(dev["qa"], out, *args(c), scale=0.1, window=0, heads=H, rank=R, rot_dim=dr, page_size=page)
+        got.append(out)
+    safe, sees = (at // 32 * 32 - hist) * H // 16 * 16 // H, at - hist      # tokens of the tiles before the block; the first that sees it
+    assert safe > 0 and torch.equal(got[1][:safe], got[0][:safe])
+    assert torch.isfinite(got[0]).all() and not torch.isfinite(got[1][sees:]).any()
