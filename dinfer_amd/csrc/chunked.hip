@@ -23,7 +23,8 @@
 //   chunk_scan   one workgroup a request, head and 16 columns of S, chunk after chunk: x, o and the next S. Of the eight
 //                waves the first four make the chunk's x, the others its o, and each keeps 16 rows of S as an accumulator.
 //
-// A decay d(t, s) is a product, taken factor by factor, never a quotient: decays of zero are as good as any. Everything
+// A decay d(t, s) is a product, taken factor by factor, never a quotient: decays of zero are as good as any. An infinity or NaN of
+// a token reaches that token and what follows it, as token by token: no row before it multiplies it, not by 0 either. Everything
 // stays in 32 bits, long sums are trees of short chains: about the error that the trees of lanes of
 // the token-by-token kernels leave (x is made from S0 itself, not as a difference of two solutions, for the same reason).
 // An accumulator of the 16 x 16 x 4 instruction holds rows 4 g + i (lane l: g = l / 16, column l % 16) in its register i,
@@ -135,6 +136,7 @@ __global__ void __launch_bounds__(256, 2) chunk_prep_kernel(Rows p, Pieces out, 
   f32x4 (*sys)[64] = (f32x4 (*)[64])&qs[0][0];
   static_assert(sizeof(qs) >= sizeof(blk), "the system's blocks fit where q was");
   __shared__ __attribute__((aligned(16))) float ends[C];
+  __shared__ int odd[5];               // delta rule: whether the system, or the inverses (4), hold an infinity or NaN
   const int h0 = blockIdx.x * heads, chunk = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
@@ -231,28 +233,33 @@ __global__ void __launch_bounds__(256, 2) chunk_prep_kernel(Rows p, Pieces out, 
       }
     }
     __syncthreads();
+    float off = 0.f;   // 0 times every entry of the system
 #pragma unroll
     for (int x = 0; x < MINE; ++x) {
       const int bl = wave + 4 * x;
       if (bl < BLOCKS) {
-        const f32x4 pv = kq[x] * blk[bl][lane];
+        const int i = bl >= 6 ? 3 : bl >= 3 ? 2 : bl >= 1 ? 1 : 0;
+        const bool diagonal = bl == block_of(i, i);
+        f32x4 pv = kq[x] * blk[bl][lane];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) pv[m] = diagonal && 4 * lg + m > lr ? 0.f : pv[m];   // (not 0 times a later token's infinity)
         if (!DELTA) {
           out.p[(ch * BLOCKS + bl) * 64 + lane] = pv;
         } else {
-          const int i = bl >= 6 ? 3 : bl >= 3 ? 2 : bl >= 1 ? 1 : 0;
-          const bool diagonal = bl == block_of(i, i);
           const f32x4 d = sys[bl][lane];
           f32x4 a;
 #pragma unroll
           for (int m = 0; m < 4; ++m) {
             const float c = __shfl(cv, 16 * i + 4 * lg + m, 64);   // (by all lanes)
             a[m] = diagonal && 4 * lg + m <= lr ? 0.f : -c * d[m] * kk[x][m];
+            off = __builtin_fmaf(a[m], 0.f, off);
           }
           blk[bl][lane] = pv;
           sys[bl][lane] = a;
         }
       }
     }
+    if (DELTA) odd[wave] = __any(off != 0.f);
     __syncthreads();
     if constexpr (DELTA) {
       // the inverses of the four diagonal blocks, less the ones on their diagonals, in their place: a lane a block and column
@@ -273,6 +280,10 @@ __global__ void __launch_bounds__(256, 2) chunk_prep_kernel(Rows p, Pieces out, 
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        float off_x = 0.f;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) off_x = __builtin_fmaf(x[t], 0.f, off_x);
+        odd[4] = __any(off_x != 0.f);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           f32x4 o;
@@ -282,6 +293,29 @@ __global__ void __launch_bounds__(256, 2) chunk_prep_kernel(Rows p, Pieces out, 
         }
       }
       __syncthreads();
+      // From a row that is not finite on everything is not (what a token adds to the state goes into all that follows), but the rows
+      // before it must not meet it: as rows of zeros it stays out of their sums. Never taken while a model's numbers are finite.
+      int first_bad = C;
+      if (odd[0] | odd[1] | odd[2] | odd[3] | odd[4]) {
+#pragma unroll 1
+        for (int t = C - 1; t >= 0; --t)
+          for (int j = 0; j <= t >> 4; ++j)
+            if (!(fabsf(((const float*)sys[block_of(t >> 4, j)])[4 * (lr + (t & 12) * 4) + (t & 3)]) < INFINITY)) first_bad = t;
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) first_bad = min(first_bad, __shfl_xor(first_bad, o, 64));
+        __syncthreads();   // (every wave has counted)
+      }
+      if (first_bad < C) {
+#pragma unroll 1
+        for (int bl = wave; bl < BLOCKS; bl += 4) {
+          const int t = 16 * (bl >= 6 ? 3 : bl >= 3 ? 2 : bl >= 1 ? 1 : 0) + 4 * lg;
+          f32x4 a = sys[bl][lane];
+#pragma unroll
+          for (int m = 0; m < 4; ++m) a[m] = t + m >= first_bad ? 0.f : a[m];
+          sys[bl][lane] = a;
+        }
+        __syncthreads();
+      }
       // T^T times 16 columns: entries of k with the decays behind each token, or rows of P; upwards from the last block
 #pragma unroll 1
       for (int ct = wave; ct < KT + 4; ct += 4) {
@@ -305,6 +339,11 @@ __global__ void __launch_bounds__(256, 2) chunk_prep_kernel(Rows p, Pieces out, 
           x[i] += y[0] + (y[1] + y[2]);
           x[i] += mfma_tree<1>([&](int) { return sys[block_of(i, i)][lane]; }, [&](int) { return x[i]; });
         }
+        if (first_bad < C && (ct < KT || 16 * (ct - KT) + lr >= first_bad)) {   // what is added to the state; the later rows of P T
+          const float nan = __builtin_nanf("");
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[i] = f32x4{nan, nan, nan, nan};
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           if (ct < KT) out.w[((ch * KT + ct) * 4 + i) * 64 + lane] = x[i];
@@ -314,6 +353,29 @@ __global__ void __launch_bounds__(256, 2) chunk_prep_kernel(Rows p, Pieces out, 
       __syncthreads();
     }
   }
+}
+
+// A block of x that holds infinities or NaNs, for the product with the rows of its own tokens: those become zeros, and the result is
+// NaN from their row on in their column (lane: column lane % 16, rows 4 (lane / 16) + m, of x and of the result).
+__device__ __forceinline__ f32x4 cut_at_rows(f32x4& x) {
+  const int lane = threadIdx.x & 63;
+  f32x4 y;
+  float sum = 0.f;
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    sum += x[m] * 0.f;
+    y[m] = sum;
+    x[m] = fabsf(x[m]) < INFINITY ? x[m] : 0.f;
+  }
+#pragma unroll
+  for (int o = 16; o < 64; o <<= 1) {
+    const float before = __shfl_up(sum, o, 64);
+    if (lane >= o) sum += before;
+  }
+  const float before = __shfl_up(sum, 16, 64);
+#pragma unroll
+  for (int m = 0; m < 4; ++m) y[m] += lane >= 16 ? before : 0.f;
+  return y;
 }
 
 // A chunk is two rounds of matrix instructions with a barrier between: with S of the chunk's start (waves 0 to 3: x,
@@ -334,6 +396,7 @@ __global__ void __launch_bounds__(512, DELTA ? 2 : 4) chunk_scan_kernel(Rows p, 
   constexpr bool AHEAD = DELTA;
   __shared__ f32x4 s_state[KT][64];
   __shared__ f32x4 s_x[2][4][64];     // x; x times the decay behind it (decay only)
+  __shared__ int s_odd[4];            // whether a block of x holds an infinity or NaN: 0 times it is not 0 for the rows before it
   // the head is the fastest index of the grid: the workgroups of a head's columns, which read the same pieces, share an
   // XCD (consecutive workgroups go to consecutive XCDs) where the heads are a multiple of 8
   const int h = blockIdx.x, cb = blockIdx.y, b = blockIdx.z;
@@ -406,6 +469,8 @@ __global__ void __launch_bounds__(512, DELTA ? 2 : 4) chunk_scan_kernel(Rows p, 
     if (!is_o) {
       x = DELTA ? fa.c * (fa.v - x) : fa.c * fa.v;
       s_x[0][r][lane] = x;
+      const bool odd = !(fabsf(x[0]) < INFINITY && fabsf(x[1]) < INFINITY && fabsf(x[2]) < INFINITY && fabsf(x[3]) < INFINITY);
+      s_odd[r] = __any(odd);
       if (!DELTA) s_x[1][r][lane] = x * fa.end;
     }
     if (!AHEAD && c + 1 < hi) fetch_first(c + 1, fa);
@@ -415,9 +480,11 @@ __global__ void __launch_bounds__(512, DELTA ? 2 : 4) chunk_scan_kernel(Rows p, 
     }
     if (is_o) {
       f32x4 y = zero;
+      f32x4 own = s_x[0][r][lane];
+      if (__builtin_amdgcn_readfirstlane(s_odd[r])) y = cut_at_rows(own);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (j <= r) y += mfma_tree<1>([&](int) { return fb.p[j]; }, [&](int) { return s_x[0][j][lane]; });
+        if (j <= r) y += mfma_tree<1>([&](int) { return fb.p[j]; }, [&](int) { return j < r ? s_x[0][j][lane] : own; });
       x += y;
       const int t = (c - first) * C + 16 * r + 4 * lg;
       float* o = out + (int64_t)(r0 + t) * ld_out + (int64_t)h * V + 16 * cb + lr;

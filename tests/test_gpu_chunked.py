@@ -159,3 +159,42 @@ def test_steps_longer_than_their_rows(delta, rows, tokens):
     for a, b in zip(*got):
         torch.testing.assert_close(b, a, rtol=1e-5, atol=1e-5 * a.abs().max().item())
     assert (got[1][0][sum(rows):] == 7.0).all()
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("at", [64 + 21, 64 + 15, 0, 130])
+@pytest.mark.parametrize("what", ["q", "k", "v", "gain", "decay", "state"])
+@pytest.mark.parametrize("delta,D,V", [(True, 128, 32), (False, 128, 16), (True, 64, 16), (False, 64, 16)])
+def test_a_bad_number_stays_with_what_follows_it(delta, D, V, what, at, bad):
+    """An infinity or NaN of one token: what the token-by-token kernel leaves finite is finite and the same in chunks, and what it
+    does not is not; the tokens before it, in its own block of 16 and chunk of 64 too, keep their numbers."""
+    from dinfer_amd.kernels import ops
+    G, H, T = 2, 2, 150
+    g = torch.Generator().manual_seed(at + D)
+    unit = torch.nn.functional.normalize
+    q, k = (unit(torch.randn(T, G, D, generator=g), dim=-1) for _ in range(2))
+    v, gain, decay = torch.randn(T, H, V, generator=g), 0.2 + 0.8 * torch.rand(T, H, generator=g), 1 - 0.1 * torch.rand(T, H, generator=g)
+    state0 = torch.randn(1, H, V, D, generator=g)
+    {"q": q[at, 1], "k": k[at, 1], "v": v[at, 1], "gain": gain[at], "decay": decay[at], "state": state0[0, 1, 3]}[what][1] = bad
+    cols = ops.delta_work_columns(G, H, D, V)
+    work = torch.cat([q.reshape(T, -1), k.reshape(T, -1), v.reshape(T, -1), gain, decay], dim=1)
+    work = torch.nn.functional.pad(work, (0, -(-cols // 4) * 4 - cols)).cuda()
+    i32 = dict(dtype=torch.int32, device="cuda")
+    common = dict(state_slots=torch.zeros(1, **i32), cu_seqlens=torch.tensor([0, T], **i32), seq_lens=torch.tensor([T + 5], **i32), num_reqs=1,
+                  heads=H, dim=D, vdim=V)
+    got = []
+    for more in (dict(), dict(tokens=T, scratch=torch.zeros(ops.chunk_scratch(delta, G, H, D, V, T, 1), device="cuda"))):
+        state, out = state0.cuda(), torch.full((T, H * V), 7.0, device="cuda")
+        if delta:
+            ops.delta_recurrence(work, state, out, qk_heads=G, **common, **more)
+        else:
+            qk, ve = G * D, 2 * G * D + H * V
+            ops.decay_recurrence(work[:, :qk], work[:, qk:2 * qk], work[:, 2 * qk:ve], work[:, ve + H:ve + 2 * H], work[:, ve:ve + H], state, out,
+                                 groups=G, **common, **more)
+        got.append((out, state))
+    for want, have in zip(*got):
+        fine = torch.isfinite(want)
+        assert torch.equal(fine, torch.isfinite(have))
+        torch.testing.assert_close(have[fine], want[fine], rtol=1e-5, atol=1e-5)     # (32 bits, two orders)
+    if what != "state":
+        assert torch.isfinite(got[1][0][:at]).all() and not torch.isfinite(got[1][0]).all()
