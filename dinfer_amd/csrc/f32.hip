@@ -458,7 +458,7 @@ extern "C" int dinfer_gemm_f32(const void* A, int64_t lda, const void* W, int64_
                                int64_t N, int64_t K, hipStream_t stream) {
   if (M <= 0 || N <= 0) return OK;
   if (K <= 0 || lda < K || ldw < K || ldc < N || M > 0x7fffffff - 64 || N > 0x7fffffff - 64 || K > 0x7fffffff - 64) return ERR_BAD_SHAPE;
-  if (!dinfer_gemm_f32_supports(A, lda, W, ldw, K) || (M + 31) / 32 > 65535) return ERR_UNSUPPORTED;
+  if (!dinfer_gemm_f32_supports(A, lda, W, ldw, K) || (M + 63) / 64 > 65535) return ERR_UNSUPPORTED;   // (as many rows as gemm_ref)
   const float *a = (const float*)A, *w = (const float*)W;
   float* c = (float*)C;
   const int m = (int)M, n = (int)N, k = (int)K;

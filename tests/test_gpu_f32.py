@@ -54,6 +54,14 @@ def test_gemm_f32_strides_and_what_it_leaves_to_the_plain_kernel():
     torch.testing.assert_close(gemm.matmul_nt(b, v, out, 9).double(), b.double() @ v.double().T, rtol=1e-5, atol=1e-4)
 
 
+@pytest.mark.parametrize("M", [32 * 65535 + 1, 64 * 65535])
+def test_gemm_f32_takes_as_many_rows_as_the_plain_kernel(M):
+    a, w = product(M, 5, 8, seed=9)
+    out = torch.empty(M, 5, device=DEV)
+    ops().gemm_f32(a, w, out, M)
+    torch.testing.assert_close(out.double(), a.double() @ w.double().T, rtol=1e-5, atol=1e-5)
+
+
 def test_gemm_f32_keeps_infinities_to_their_row():
     a, w = product(50, 70, 300, seed=8)
     clean = torch.empty(50, 70, device=DEV)
