@@ -104,9 +104,6 @@ __device__ __forceinline__ int first_chunk(const int32_t* __restrict__ cu, int n
   return __builtin_amdgcn_readfirstlane(sum);
 }
 
-// What other waves wrote to LDS, without waiting for this wave's loads from memory.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 // A B over 16 N entries: chains of 8 terms and the tree of their sums, which rounds about as often as lanes that add in pairs do
 // (one chain over 128 entries: 1.8 times the error, four: 1.3 times)

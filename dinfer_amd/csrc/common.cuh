@@ -88,6 +88,10 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   return t;
 }
 
+// A barrier for what waves hand each other through LDS: this wave's accesses of LDS are done, its loads from memory, those that
+// write LDS among them, stay in flight (__syncthreads would wait for all of them, a fence on LDS for the latter).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 static inline int launch_status() { return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH; }
 
 // One rotated pair (a, b) -> (a cos - b sin, b cos + a sin) and one step of a sum of squares, with their roundings

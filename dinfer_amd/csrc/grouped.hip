@@ -17,8 +17,11 @@
 //
 // Float operands run on the vector ALUs, every output element summed over k in ascending order by one thread (the
 // true 32-bit path; a row's result does not depend on which tile or group size it met). bf16 operands run on the
-// matrix cores, operands read straight from memory in the MFMA's own order (8 consecutive k a lane), in two forms:
-// tiles of 128 rows and tiles of 16 rows whose waves split k (see the kernels).
+// matrix cores, in three forms (see the kernels):
+//   heads, many rows      tiles of 128 rows: A through LDS, the weights straight into registers in the MFMA's order
+//   experts, many rows    tiles of 128 rows: A through LDS, the weights in whole lines into registers, brought into the MFMA's
+//                         order by exchanges between lanes
+//   few rows              tiles of 16 rows whose waves split k: both operands in whole lines, exchanged likewise
 //
 //   moe_route    two kernels: router logits in float (a wave an expert, a router row read once per 8 tokens), then per
 //                token the `top` largest (lowest index first among equals), the softmax over the chosen and the shared
@@ -183,8 +186,8 @@ __global__ void __launch_bounds__(256) grouped_valu_kernel(Groups p) {
 }
 
 // bf16 on the matrix cores. v_mfma_f32_16x16x32_bf16: lane l holds row (or column) l % 16 and the 8 consecutive k
-// starting at 8 (l / 16); of the result it holds column l % 16, rows 4 (l / 16) .. + 3. Operands are read straight from
-// memory in that order (16 bytes a lane).
+// starting at 8 (l / 16); of the result it holds column l % 16, rows 4 (l / 16) .. + 3. (The experts' kernels and the one for few
+// rows take the 32 x 32 x 16 form.)
 //
 // Many rows a head (tiles of 128): a workgroup's four waves stand side by side over the columns, a wave 128 rows x 64
 // columns; products of up to 128 columns have them 2 x 2, a wave 64 x 64. The rows of A are staged in LDS for all waves,
@@ -196,13 +199,6 @@ __global__ void __launch_bounds__(256) grouped_valu_kernel(Groups p) {
 constexpr int TM_BIG = 128, TM_SMALL = 16;
 
 constexpr int BIG_K = 64;            // k a step; a staged row is 128 bytes, its 16-byte pieces exchanged by the row's bits 1..3
-
-// LDS is written and read around this; loads from memory stay in flight across it (__syncthreads would wait for them)
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 // what becomes of a sum: an instance each (with all of them in one, the 128 results of a lane are 25,000 instructions)
 enum : int { END_PLAIN, END_SILU, END_GELU, END_RELU2, END_HEAD_GATE, END_ENTRY_GATE, END_GATED, END_GATED_CLAMPED };
@@ -475,7 +471,7 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_experts_kernel(Groups p) 
   if (threadIdx.x < TM_BIG) arow[threadIdx.x] = tl.a_row(threadIdx.x < tl.rows ? threadIdx.x : 0);   // rows beyond: computed, not stored
   __syncthreads();
 
-  // staging: 256 rows x 64 k = 2,048 pieces of 16 bytes, eight a thread; piece q of a thread is row (q * 256 + thread) / 8.
+  // staging: 128 rows x 64 k = 1,024 pieces of 16 bytes, four a thread; piece q of a thread is row (q * 256 + thread) / 8.
   // A staged row is 128 bytes, its pieces exchanged by bits 1..3 of the row's number: no bank is met twice
   const int sp = threadIdx.x & 7;
   const bf16* ag[PIECES];

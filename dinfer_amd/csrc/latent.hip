@@ -184,9 +184,6 @@ __global__ void __launch_bounds__(WAVES * 64) latent_attn_ref_kernel(
 
 
 // ---- attention over the latent pages on the matrix cores --------------------------------------------------------
-// LDS is written and read around this; loads from memory, those that write LDS among them, stay in flight across it (a fence
-// on LDS would wait for the latter)
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 constexpr float LOG2E = 1.4426950408889634f;
 
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
