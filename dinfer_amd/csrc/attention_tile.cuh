@@ -459,7 +459,7 @@ __global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu
   const int blk_first = all_lo >> 5, blk_end = (all_hi + 31) >> 5;
   const int blocks = blk_end - blk_first;
   const int per = HEADS ? max((blocks + PARTS) / WAVES, min(3, (blocks + 3) / 4)) : (blocks + PARTS) / WAVES;
-  const int parts = HEADS ? (blocks - 1) / per : PARTS;   // waves 1 .. parts have keys at all
+  int parts = HEADS ? (blocks - 1) / per : PARTS;   // waves 1 .. parts have keys at all
   const int blk0 = blk_first + wave * per;
   const int blk1 = blk0 + per < blk_end ? blk0 + per : blk_end;
   const int k_lo = blk0 * 32 > all_lo ? blk0 * 32 : all_lo;
@@ -480,7 +480,8 @@ __global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu
   if constexpr (EXT) {
     // the kept first keys that the window of the tile's first row has passed: one more run, every block masked
     const int kept = tl.keep_first < all_lo ? tl.keep_first : all_lo;
-    if (wave == 0 && kept > 0) {
+    if (HEADS && kept > 0) parts = PARTS;   // (the last wave's: it has the fewest keys of the window, mostly none)
+    if (wave == (HEADS ? PARTS : 0) && kept > 0) {
       tl.k_lo = 0;
       tl.k_hi = kept;
       tl.pages.init(bt, (int)max_blocks, ps, 0);
