@@ -1019,8 +1019,8 @@ extern "C" int dinfer_latent_attn_mfma(const void* qa, int64_t ld_qa, void* out,
   if (tiles > 0x7fffffff || splits > 65535) return ERR_UNSUPPORTED;
   const bool solo = tokens != num_reqs;      // some request brings more than one row
   // latents of 128, 256 or 512 with whole chunks of 32 in a key row, two blocks of which fit LDS: the kernel whose waves share
-  // their rows' weights
-  if (solo && (page_size & (page_size - 1)) == 0 && dr % 32 == 0 && (R == 128 || R == 256 || (R == 512 && dr <= 64))) {
+  // their rows' weights (which keeps offsets inside a page in 32 bits)
+  if (solo && (page_size & (page_size - 1)) == 0 && page_size <= 1 << 20 && dr % 32 == 0 && (R == 128 || R == 256 || (R == 512 && dr <= 64))) {
     const int64_t groups = (tokens * heads + 63) / 64 + num_reqs;
     if (groups > 0x7fffffff) return ERR_UNSUPPORTED;
     const int page_shift = __builtin_ctz(page_size);

@@ -69,3 +69,19 @@ def test_a_bad_key_stays_away_from_rows_before_it(n, hist, H, R, dr, page, at, b
     safe, sees = (at // 32 * 32 - hist) * H // 16 * 16 // H, at - hist      # tokens of the tiles before the block; the first that sees it
     assert safe > 0 and torch.equal(got[1][:safe], got[0][:safe])
     assert torch.isfinite(got[0]).all() and not torch.isfinite(got[1][sees:]).any()
+
+
+def test_pages_whose_offsets_pass_32_bits():
+    """A page of 2^22 tokens (4.3 GB, and as much again transposed): the kernel that keeps 32-bit offsets leaves it alone."""
+    from dinfer_amd.kernels import ops
+    n, H, R, page = 40, 2, 512, 1 << 22
+    g = torch.Generator().manual_seed(1)
+    keys, qa = torch.randn(n, R, generator=g).to(torch.bfloat16), (0.3 * torch.randn(n, H * R, generator=g)).to(torch.bfloat16)
+    cache, cache_t = torch.zeros(1, page, R, dtype=torch.bfloat16, device="cuda"), torch.zeros(1, R, page, dtype=torch.bfloat16, device="cuda")
+    cache[0, :n], cache_t[0, :, :n] = keys.cuda(), keys.T.cuda()
+    i32 = dict(dtype=torch.int32, device="cuda")
+    out = torch.zeros(n, H * R, dtype=torch.bfloat16, device="cuda")
+    ops.latent_attn_mfma(qa.cuda(), out, cache, cache_t, torch.zeros(1, 1, **i32), torch.tensor([0, n], **i32), torch.tensor([n], **i32), 1, n, 1,
+                         torch.zeros(n * H * (R + 4), device="cuda"), scale=0.1, window=0, heads=H, rank=R, rot_dim=0, page_size=page)
+    want = latent_plain(dict(qa=qa, cache=keys[None], bt=torch.zeros(1, 1, dtype=torch.int32)), [n], [n], H, R, 0, 0.1)
+    assert (out.double().cpu() - want).abs().max().item() < 0.015 * max(1.0, want.abs().max().item())
