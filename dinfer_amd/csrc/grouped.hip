@@ -17,11 +17,12 @@
 //
 // Float operands run on the vector ALUs, every output element summed over k in ascending order by one thread (the
 // true 32-bit path; a row's result does not depend on which tile or group size it met). bf16 operands run on the
-// matrix cores, in three forms (see the kernels):
+// matrix cores, in four forms (see the kernels):
 //   heads, many rows      tiles of 128 rows: A through LDS, the weights straight into registers in the MFMA's order
 //   experts, many rows    tiles of 128 rows: A through LDS, the weights in whole lines into registers, brought into the MFMA's
 //                         order by exchanges between lanes
-//   few rows              tiles of 16 rows whose waves split k: both operands in whole lines, exchanged likewise
+//   few rows              tiles of 16 rows whose waves split k: both operands in whole lines, exchanged likewise, or, where k is
+//                         short, straight from memory in the MFMA's order
 //
 //   moe_route    two kernels: router logits in float (a wave an expert, a router row read once per 8 tokens), then per
 //                token the `top` largest (lowest index first among equals), the softmax over the chosen and the shared
@@ -700,6 +701,67 @@ __global__ void __launch_bounds__(NW * 64) grouped_mfma_small_kernel(Groups p) {
   }
 }
 
+// Few rows, products that are over soon (takes_short below): 16 columns a workgroup (gated: of each half), both operands straight
+// from memory in the order of v_mfma_f32_16x16x32_bf16, no exchanges between lanes; its four waves take a quarter of k each, their
+// partial sums meet in LDS and are added in wave order. Bound by the latency of its one or two rounds of loads.
+template <class O, bool GATED>
+__global__ void __launch_bounds__(256) grouped_mfma_short_kernel(Groups p) {
+  __shared__ int64_t arow[TM_SMALL];
+  __shared__ float part[4][GATED ? 2 : 1][16][17];
+  Tile tl;
+  if (!tl.init(p)) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int n0 = blockIdx.x * 16;
+  const bool experts = p.tiles != nullptr;
+  const bf16* A = (const bf16*)p.A + (experts ? 0 : (int64_t)tl.z * p.a_zs);
+  const bf16* W = (const bf16*)p.W + (int64_t)tl.z * p.w_zs;
+  if (threadIdx.x < TM_SMALL) arow[threadIdx.x] = threadIdx.x < tl.rows ? tl.a_row(threadIdx.x) : -1;
+  __syncthreads();
+  const int lr = lane & 15, kq = lane >> 4;
+  const int64_t ar = arow[lr];
+  const int gn = n0 + lr;
+  const bf16* ap = ar >= 0 ? A + ar * p.lda + kq * 8 : nullptr;
+  const bf16* wp = gn < p.N ? W + (int64_t)gn * p.ldw + kq * 8 : nullptr;
+  const bf16* up = (GATED && gn < p.N) ? W + (int64_t)(gn + p.gate_n) * p.ldw + kq * 8 : nullptr;
+  bf16x8 zero;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) zero[i] = (bf16)0.f;
+  const int K = p.K;
+  const int steps = (K + 31) / 32, per = (steps + 3) / 4;
+  const int k_lo = wave * per * 32, k_hi = (wave + 1) * per * 32 < K ? (wave + 1) * per * 32 : K;
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f}, acu = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int k0 = k_lo; k0 < k_hi; k0 += 32) {
+    const bool in = k0 + kq * 8 < K;
+    const bf16x8 a = (ap && in) ? *(const bf16x8*)(ap + k0) : zero;
+    const bf16x8 w = (wp && in) ? __builtin_nontemporal_load((const bf16x8*)(wp + k0)) : zero;
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w, acc, 0, 0, 0);
+    if (GATED) {
+      const bf16x8 u = (up && in) ? __builtin_nontemporal_load((const bf16x8*)(up + k0)) : zero;
+      acu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, u, acu, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    part[wave][0][kq * 4 + r][lr] = acc[r];
+    if (GATED) part[wave][GATED ? 1 : 0][kq * 4 + r][lr] = acu[r];
+  }
+  __syncthreads();
+  const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
+  if (row >= tl.rows || n0 + col >= p.N) return;
+  float v = 0.f, u = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    v += part[w][0][row][col];
+    if (GATED) u += part[w][GATED ? 1 : 0][row][col];
+  }
+  const int64_t cr = tl.c_row(row);
+  const float g = head_gate<bf16>(p, cr, tl.z, n0 + col);
+  O* C = (O*)p.C + (experts ? 0 : (int64_t)tl.z * p.c_zs);
+  const float rs = tl.scale_of(p, row);
+  C[cr * p.ldc + n0 + col] = from_f32<O>((GATED ? gated_value(p, v * rs, u * rs) : plain_act(v * rs, p.act)) * g);
+}
+
 // ---- routing ---------------------------------------------------------------------------------------------------
 constexpr int MAX_EXPERTS = 1024;
 
@@ -1001,10 +1063,20 @@ void launch_big(const Groups& p, unsigned gy, unsigned gz, hipStream_t stream) {
     grouped_mfma_big_kernel<bf16, END, 2><<<dim3(1, gy, gz), 256, 0, stream>>>(p);
 }
 
+// Whether a product of few rows is over so soon that streaming the weights in whole lines does not pay. Measured with weights from
+// memory, 1 to 64 tokens on 8 to 64 experts and 16 to 128 heads, K of 128 to 4,096: up to a round of loads (K = 512) of each of four
+// waves the short form is as fast or faster (16 heads of 128 -> 512: 2.9 us against 3.6, 128 heads 6.0 against 10.3; 64 experts of 512 ->
+// 1,024 at 64 tokens equal; of 128 -> 2,048 14.0 against 21.3), gated, with twice the loads, up to half of that (256 -> 4,096 82.9 against
+// 96.8, 512 -> 1,024 42.2 against 32.6); beyond it loses (K = 1,024: 40.4 against 31.0).
+template <bool GATED>
+bool takes_short(const Groups& p) { return p.K <= (GATED ? 256 : 512); }
+
 template <bool GATED>
 int launch_groups(int dtype, Groups p, unsigned gy, unsigned gz, hipStream_t stream) {
   if (dtype != DT_F32 && dtype != DT_BF16) return ERR_BAD_DTYPE;
-  if (mfma_fits(dtype, p) && p.tm == TM_SMALL) {
+  if (mfma_fits(dtype, p) && p.tm == TM_SMALL && takes_short<GATED>(p)) {
+    grouped_mfma_short_kernel<bf16, GATED><<<dim3((unsigned)((p.N + 15) / 16), gy, gz), 256, 0, stream>>>(p);
+  } else if (mfma_fits(dtype, p) && p.tm == TM_SMALL) {
     const dim3 grid((unsigned)((p.N + 31) / 32), gy, gz);
     // fewer than two workgroups a CU: eight waves share a workgroup's k (one token, 6 experts: 14.8 -> 14.5, 12.5 -> 11.2 us)
     if (!GATED && p.tiles && p.entries * grid.x < 512) grouped_mfma_small_kernel<bf16, GATED, 8><<<grid, 512, 0, stream>>>(p);

@@ -205,3 +205,25 @@ def test_rows_too_wide_for_32_bit_offsets_take_tiles_of_16():
     wide = 2 ** 26
     assert ops.moe_tile_rows(torch.bfloat16, 1000, 2, wide - 8, 64) == 128
     assert ops.moe_tile_rows(torch.bfloat16, 1000, 2, wide, 64) == 16 and ops.moe_tile_rows(torch.bfloat16, 1000, 2, 64, wide) == 16
+
+
+# the last k of the form for products that are soon over, and the first of the other; columns in part of a workgroup's, odd widths
+@pytest.mark.parametrize("N,K,kind", [(33, 512, "silu"), (33, 520, None), (257, 584, "gelu"), (70, 256, "gated"), (70, 264, "gated"), (33, 328, "gated")])
+def test_experts_of_few_rows_in_both_forms(N, K, kind):
+    test_experts_of_few_rows(N, K, kind)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 33, 512), (1, 33, 520), (9, 72, 1032), (16, 130, 584)])
+def test_heads_of_few_rows_in_both_forms(M, N, K):
+    from dinfer_amd.kernels import ops
+    H = 3
+    g = torch.Generator(device=DEV).manual_seed(M)
+    a = torch.randn(M, H * K, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(H, N, K, generator=g, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    gates = torch.randn(M, H * N, generator=g, device=DEV).to(torch.bfloat16)
+    for gate in (None, gates):
+        out = torch.full((M, H * N + 1), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.heads_nt(a, 0, K, w, out, 0, N, M, **({} if gate is None else dict(gate=gate, gate_entries=True)))
+        want = torch.cat([a[:, h * K:(h + 1) * K].double() @ w[h].double().T for h in range(H)], dim=1)
+        close(out[:, :H * N], want if gate is None else want * torch.sigmoid(gate.double()))
+        assert (out[:, H * N] == 7.0).all()
