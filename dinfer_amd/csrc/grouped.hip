@@ -204,13 +204,18 @@ constexpr int BIG_K = 64;            // k a step; a staged row is 128 bytes, its
 // what becomes of a sum: an instance each (with all of them in one, the 128 results of a lane are 25,000 instructions)
 enum : int { END_PLAIN, END_SILU, END_GELU, END_RELU2, END_HEAD_GATE, END_ENTRY_GATE, END_GATED, END_GATED_CLAMPED };
 
+// 8 columns of a row in one store wherever the row begins (rows of an odd width begin at any even address, which such a store
+// takes; a store of 2 bytes costs as much for each of its lanes: 4,000 rows, 16 heads of 128 -> 511 99 us, 38 so, 82 by the kernel before).
+struct __attribute__((packed, aligned(2))) Packed8 { bf16x8 v; };
+template <class T>
+__device__ __forceinline__ void store8(T* c, const bf16x8& o) { ((Packed8*)c)->v = o; }
+
 // A wave's block of 64 rows (from row m0 of the tile on): lane l holds, of rows 16 i + l % 16, the 16 columns from
 // c0 + 16 (l / 16) on.
 template <class O, int END>
 __device__ __forceinline__ void store_block(const Groups& p, const Tile& tl, O* C, int m0, int c0, const f32x4 (&acc)[4][4]) {
   const int lane = threadIdx.x & 63, lr = lane & 15, kq = lane >> 4;
   const int n = c0 + kq * 16;   // a lane's first column
-  const bool pieces = sizeof(O) == 2 && p.ldc % 8 == 0 && ((uintptr_t)C & 15) == 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int row = m0 + i * 16 + lr;
@@ -227,15 +232,15 @@ __device__ __forceinline__ void store_block(const Groups& p, const Tile& tl, O* 
         v[x] = acc[i][2 * e + (x >> 2)][x & 3] * g1;
         if (END == END_ENTRY_GATE) v[x] *= n + 8 * e + x < p.N ? head_gate<bf16>(p, cr, tl.z, n + 8 * e + x) : 0.f;
       }
-      if (pieces && n + 8 * e + 8 <= p.N) {
-        bf16x8 o;
+      bf16x8 o;
 #pragma unroll
-        for (int x = 0; x < 8; ++x) o[x] = (bf16)v[x];
-        *(bf16x8*)(c + 8 * e) = o;
+      for (int x = 0; x < 8; ++x) o[x] = (bf16)v[x];
+      if (n + 8 * e + 8 <= p.N) {
+        store8(c + 8 * e, o);
       } else {
 #pragma unroll
         for (int x = 0; x < 8; ++x)
-          if (n + 8 * e + x < p.N) c[8 * e + x] = from_f32<O>(v[x]);
+          if (n + 8 * e + x < p.N) c[8 * e + x] = o[x];
       }
     }
   }
@@ -403,32 +408,29 @@ template <class O, int END>
 __device__ __forceinline__ void store_rows(const Groups& p, const Tile& tl, int m0, int c0, const f32x16 (&acc)[2]) {
   constexpr bool GATED = END >= END_GATED;
   const int lane = threadIdx.x & 63, row = m0 + (lane & 31);
-  if (row >= tl.rows) return;
-  const float rs = tl.scale_of(p, row);
-  O* c = (O*)p.C + tl.c_row(row) * p.ldc;
-  const bool pieces = sizeof(O) == 2 && p.ldc % 8 == 0 && ((uintptr_t)p.C & 15) == 0;
+  if (row < tl.rows) {
+    const float rs = tl.scale_of(p, row);
+    O* c = (O*)p.C + tl.c_row(row) * p.ldc;
 #pragma unroll
-  for (int j = 0; j < (GATED ? 1 : 2); ++j)
+    for (int j = 0; j < (GATED ? 1 : 2); ++j)
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {   // 8 columns at a time
-      const int n = c0 + 32 * j + 16 * (lane >> 5) + 8 * e;
-      if (n >= p.N) continue;
-      float v[8];
-#pragma unroll
-      for (int x = 0; x < 8; ++x)
-        v[x] = GATED ? gated_value<END == END_GATED_CLAMPED>(p, acc[0][8 * e + x] * rs, acc[1][8 * e + x] * rs)
-                     : plain_act(acc[j][8 * e + x] * rs, END);
-      if (pieces && n + 8 <= p.N) {
+      for (int e = 0; e < 2; ++e) {   // 8 columns at a time
+        const int n = c0 + 32 * j + 16 * (lane >> 5) + 8 * e;
+        if (n >= p.N) continue;
         bf16x8 o;
 #pragma unroll
-        for (int x = 0; x < 8; ++x) o[x] = (bf16)v[x];
-        *(bf16x8*)(c + n) = o;
-      } else {
-#pragma unroll
         for (int x = 0; x < 8; ++x)
-          if (n + x < p.N) c[n + x] = from_f32<O>(v[x]);
+          o[x] = (bf16)(GATED ? gated_value<END == END_GATED_CLAMPED>(p, acc[0][8 * e + x] * rs, acc[1][8 * e + x] * rs)
+                              : plain_act(acc[j][8 * e + x] * rs, END));
+        if (n + 8 <= p.N) {
+          store8(c + n, o);
+        } else {
+#pragma unroll
+          for (int x = 0; x < 8; ++x)
+            if (n + x < p.N) c[n + x] = o[x];
+        }
       }
-    }
+  }
 }
 
 // Tile j of the wave whose first column is c0 holds the expert's rows from weights_row on, weights_bytes of them: 32 rows, fewer

@@ -227,3 +227,15 @@ def test_heads_of_few_rows_in_both_forms(M, N, K):
         want = torch.cat([a[:, h * K:(h + 1) * K].double() @ w[h].double().T for h in range(H)], dim=1)
         close(out[:, :H * N], want if gate is None else want * torch.sigmoid(gate.double()))
         assert (out[:, H * N] == 7.0).all()
+
+
+# rows of the result that do not begin at 16 bytes: odd widths, halves of a wave's columns, blocks of rows in part
+@pytest.mark.parametrize("N,K,kind", [(257, 64, None), (65, 72, "silu"), (1001, 128, "relu2"), (33, 64, "gated"), (129, 72, "gated"), (508, 64, "gated")])
+def test_experts_of_many_rows_and_odd_widths(N, K, kind):
+    test_experts_of_many_rows(N, K, kind)
+
+
+@pytest.mark.parametrize("gate", [None, "head", "entry"])
+@pytest.mark.parametrize("M,N,K,extra", [(130, 257, 64, 0), (300, 127, 72, 0), (17, 511, 64, 3), (200, 130, 40, 0)])
+def test_heads_of_many_rows_and_odd_widths(M, N, K, extra, gate):
+    test_heads_of_many_rows(M, N, K, extra, gate)
