@@ -448,16 +448,17 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
 
-// Whether dinfer_gemm_f32 takes operands of these strides (in floats) and addresses: 16-byte pieces along k.
+// Whether dinfer_gemm_f32 takes operands of these strides (in floats) and addresses: 16-byte pieces along k, which ends so
+// early that two steps or a segment behind it are still 32-bit numbers.
 extern "C" int dinfer_gemm_f32_supports(const void* A, int64_t lda, const void* W, int64_t ldw, int64_t K) {
-  return K >= 4 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && aligned16(A) && aligned16(W);
+  return K >= 4 && K % 4 == 0 && K <= 0x7fffffff - 2 * SEG && lda % 4 == 0 && ldw % 4 == 0 && aligned16(A) && aligned16(W);
 }
 
 // C[M, N] = A[M, K] . W[N, K]^T, all float32.
 extern "C" int dinfer_gemm_f32(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, int64_t M,
                                int64_t N, int64_t K, hipStream_t stream) {
   if (M <= 0 || N <= 0) return OK;
-  if (K <= 0 || lda < K || ldw < K || ldc < N || M > 0x7fffffff - 64 || N > 0x7fffffff - 64 || K > 0x7fffffff - 64) return ERR_BAD_SHAPE;
+  if (K <= 0 || lda < K || ldw < K || ldc < N || M > 0x7fffffff - 64 || N > 0x7fffffff - 64) return ERR_BAD_SHAPE;
   if (!dinfer_gemm_f32_supports(A, lda, W, ldw, K) || (M + 63) / 64 > 65535) return ERR_UNSUPPORTED;   // (as many rows as gemm_ref)
   const float *a = (const float*)A, *w = (const float*)W;
   float* c = (float*)C;
