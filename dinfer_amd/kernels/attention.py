@@ -63,7 +63,8 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k_cache, v_cache, batc
     geo = dict(scale=scale, window=window, heads=heads, kv_heads=kv_heads, head_dim=head_dim, page_size=page_size)
     bt = batch.block_table[group]
     B, T = batch.num_reqs, batch.num_tokens
-    if ws.f32 and all(t.stride(0) % 4 == 0 and t.data_ptr() % 16 == 0 for t in (qkv, out)):
+    # (requests are the y of that kernel's grid)
+    if ws.f32 and B <= 65535 and all(t.stride(0) % 4 == 0 and t.data_ptr() % 16 == 0 for t in (qkv, out)):
         return ops.attn_f32(qkv, out, k_cache, v_cache, bt, batch.cu_seqlens, batch.seq_lens, B, T, batch.max_q_len, **geo)
     if not ws.mfma:
         return ops.attn_paged_ref(qkv, out, k_cache, v_cache, bt, batch.cu_seqlens, batch.seq_lens, B, T, **geo)
