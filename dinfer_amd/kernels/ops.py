@@ -398,17 +398,18 @@ def delta_conv_update(proj: torch.Tensor, *, qkv_off: int, conv_state: torch.Ten
 def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor, *, state_slots: torch.Tensor,
                      cu_seqlens: torch.Tensor, seq_lens: torch.Tensor, num_reqs: int, qk_heads: int, heads: int,
                      dim: int, vdim: int, tokens: int | None = None, scratch: torch.Tensor | None = None,
-                     one_row_each: bool | None = None) -> torch.Tensor:
+                     one_row_each: bool | None = None, max_rows: int | None = None) -> torch.Tensor:
     """The recurrence over each request's rows of the step. state [slots, heads, vdim, dim] float32 (a head's matrix
     transposed), updated in place; out [T, heads * vdim] float32. tokens, scratch: the step's rows (one a request at
     least) and a buffer of chunk_scratch's size; with them requests of CHUNKED_ROWS rows or more go chunk by chunk.
-    one_row_each: whether every request has one row, no more and no less (None: it has if tokens equals num_reqs)."""
+    one_row_each: whether every request has one row, no more and no less (None: it has if tokens equals num_reqs). max_rows: no
+    request has more rows than this (None: unknown)."""
     _need_gpu(work, state, out, state_slots, cu_seqlens, seq_lens)
     assert work.dtype == state.dtype == out.dtype == torch.float32 and state.is_contiguous()
     assert tuple(state.shape[1:]) == (heads, vdim, dim) and out.shape[1] >= heads * vdim
     assert work.shape[1] >= delta_work_columns(qk_heads, heads, dim, vdim)
     below = EVERY_ROW
-    if _may_be_long(tokens, num_reqs, scratch):
+    if _may_be_long(tokens, num_reqs, scratch, max_rows):
         qk, v_end = qk_heads * dim, 2 * qk_heads * dim + heads * vdim
         below = _chunked(True, work, work[:, qk:], work[:, 2 * qk:], work[:, v_end + heads:], work[:, v_end:], state, out,
                          state_slots, cu_seqlens, seq_lens, num_reqs, qk_heads, heads, dim, vdim, tokens, scratch)
@@ -439,9 +440,10 @@ def chunk_scratch(delta: bool, groups: int, heads: int, dim: int, vdim: int, max
     return min(most, CHUNKS_AT_ONCE), floats
 
 
-def _may_be_long(tokens: int | None, num_reqs: int, scratch: torch.Tensor | None) -> bool:
-    """Whether a request of the step may have CHUNKED_ROWS rows: every one has a row at least."""
-    return scratch is not None and tokens is not None and num_reqs > 0 and tokens - num_reqs + 1 >= CHUNKED_ROWS
+def _may_be_long(tokens: int | None, num_reqs: int, scratch: torch.Tensor | None, max_rows: int | None) -> bool:
+    """Whether a request of the step may have CHUNKED_ROWS rows: every one has a row at least, and max_rows at most."""
+    return (scratch is not None and tokens is not None and num_reqs > 0 and tokens - num_reqs + 1 >= CHUNKED_ROWS
+            and (max_rows is None or max_rows >= CHUNKED_ROWS))
 
 
 def _chunked(delta, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens, num_reqs, groups, heads, dim,
@@ -568,13 +570,13 @@ def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: t
                      state: torch.Tensor, out: torch.Tensor, *, state_slots: torch.Tensor, cu_seqlens: torch.Tensor,
                      seq_lens: torch.Tensor, num_reqs: int, groups: int, heads: int, dim: int, vdim: int,
                      tokens: int | None = None, scratch: torch.Tensor | None = None,
-                     one_row_each: bool | None = None) -> torch.Tensor:
+                     one_row_each: bool | None = None, max_rows: int | None = None) -> torch.Tensor:
     """Per request and head, token by token: S <- decay S + gain k v^T, out = S^T q. q, k: float32 views [T, groups dim]
     (head h reads group h // (heads / groups)); v [T, heads vdim]; decay [T, heads], or [heads] for one decay a head;
     gain [T, heads] or None. state [slots, heads, vdim, dim] float32, updated in place; out [T, >= heads vdim] float32.
     tokens, scratch: the step's rows (one a request at least) and a buffer of chunk_scratch's size; with them requests of
     CHUNKED_ROWS rows or more go chunk by chunk. one_row_each: whether every request has one row, no more and no less (None:
-    it has if tokens equals num_reqs)."""
+    it has if tokens equals num_reqs). max_rows: no request has more rows than this (None: unknown)."""
     _need_gpu(q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens)
     tensors = [q, k, v, decay, state, out] + ([gain] if gain is not None else [])
     assert all(t.dtype == torch.float32 for t in tensors) and state.is_contiguous()
@@ -588,7 +590,7 @@ def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: t
         ldd = _rows(decay)
     assert gain is None or gain.shape[1] >= heads
     below = EVERY_ROW
-    if _may_be_long(tokens, num_reqs, scratch):
+    if _may_be_long(tokens, num_reqs, scratch, max_rows):
         below = _chunked(False, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens, num_reqs, groups, heads,
                          dim, vdim, tokens, scratch)
     if below > 0:

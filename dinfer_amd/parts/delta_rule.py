@@ -132,6 +132,6 @@ class GatedDeltaRule(Mixer):
         if cache.owner:
             ops.delta_conv_update(proj_buf, qkv_off=col, conv_state=cache.conv, **common)
         ops.delta_recurrence(self.work, cache.state, self.o_buf, tokens=T, scratch=self.chunks,
-                             one_row_each=batch.all_decode, **common, **sizes)
+                             one_row_each=batch.all_decode, max_rows=batch.max_q_len, **common, **sizes)
         ops.delta_out(self.o_buf, proj_buf, col + self.g_off, self.norm_weight, gated_buf, T, heads=self.heads,
                       vdim=self.vdim, eps=self.norm_eps, col_off=out_col, out_scale=self.out_scale)

@@ -118,6 +118,6 @@ class Retention(Mixer):
         ops.decay_recurrence(w[:, :qk], w[:, qk:2 * qk], w[:, 2 * qk:], self.decay_vec, None, cache.state, self.o_buf,
                              state_slots=batch.state_slots, cu_seqlens=batch.cu_seqlens, seq_lens=batch.seq_lens,
                              num_reqs=batch.num_reqs, groups=self.heads, heads=self.heads, dim=self.dim, vdim=self.vdim,
-                             tokens=T, scratch=self.chunks, one_row_each=batch.all_decode)
+                             tokens=T, scratch=self.chunks, one_row_each=batch.all_decode, max_rows=batch.max_q_len)
         ops.gated_group_norm(self.o_buf, proj_buf, col + self.g_off, gated_buf, T, groups=self.heads, group=self.vdim,
                              eps=self.norm_eps, col_off=out_col, out_scale=self.out_scale, gate_first=False)

@@ -102,7 +102,7 @@ class StateSpace(Mixer):
         xs, bs, cs = w[:, :inner], w[:, inner:inner + gn], w[:, inner + gn:inner + 2 * gn]
         dt, decay = w[:, self.channels:self.channels + H], w[:, self.channels + H:self.channels + 2 * H]
         ops.decay_recurrence(cs, bs, xs, decay, dt, cache.state, self.y_buf, groups=self.groups, heads=H, dim=self.state,
-                             vdim=self.vdim, tokens=T, scratch=self.chunks, one_row_each=batch.all_decode, **common)
+                             vdim=self.vdim, tokens=T, scratch=self.chunks, one_row_each=batch.all_decode, max_rows=batch.max_q_len, **common)
         ops.gated_group_norm(self.y_buf, self.proj_buf, 0, self.gated_buf, T, groups=self.norm_groups,
                              group=inner // self.norm_groups, eps=self.norm_eps, weight=self.norm_weight, x=xs,
                              skip=self.skip, vdim=self.vdim)

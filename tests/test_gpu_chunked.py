@@ -198,3 +198,33 @@ def test_a_bad_number_stays_with_what_follows_it(delta, D, V, what, at, bad):
         torch.testing.assert_close(have[fine], want[fine], rtol=1e-5, atol=1e-5)     # (32 bits, two orders)
     if what != "state":
         assert torch.isfinite(got[1][0][:at]).all() and not torch.isfinite(got[1][0]).all()
+
+
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("rows,max_rows,calls_made", [([18] * 16, 18, 1), ([127, 3], 127, 1), ([127, 3], None, 2), ([128, 3], 128, 2)])
+def test_steps_of_short_portions_launch_nothing_for_long_ones(monkeypatch, delta, rows, max_rows, calls_made):
+    """Where the longest portion is known to be short, nothing of the chunked form is launched; the results are the same bits."""
+    from dinfer_amd.kernels import lib, ops
+    G, H, D, V, B, T = 1, 2, 64, 32, len(rows), sum(rows)
+    g = torch.Generator().manual_seed(T)
+    cols = -(-ops.delta_work_columns(G, H, D, V) // 4) * 4
+    work = (torch.rand(T, cols, generator=g) / 8).cuda()
+    state0 = torch.randn(B + 1, H, V, D, generator=g)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    common = dict(state_slots=torch.arange(B, **i32), cu_seqlens=torch.tensor([0] + rows).cumsum(0).to(**i32),
+                  seq_lens=torch.tensor([5 + n for n in rows], **i32), num_reqs=B, heads=H, dim=D, vdim=V, one_row_each=False, tokens=T,
+                  scratch=torch.zeros(ops.chunk_scratch(delta, G, H, D, V, T, B), device="cuda"))
+    calls, call, got = [], lib.call, []
+    monkeypatch.setattr(lib, "call", lambda name, *a: (calls.append(name), call(name, *a))[1])
+    for more in (dict(), dict(max_rows=max_rows)):
+        state, out = state0.cuda(), torch.zeros(T, H * V, device="cuda")
+        calls.clear()
+        if delta:
+            ops.delta_recurrence(work, state, out, qk_heads=G, **common, **more)
+        else:
+            qk, ve = G * D, 2 * G * D + H * V
+            ops.decay_recurrence(work[:, :qk], work[:, qk:2 * qk], work[:, 2 * qk:ve], work[:, ve + H:ve + 2 * H], work[:, ve:ve + H],
+                                 state, out, groups=G, **common, **more)
+        got.append((out, state))
+    assert len(calls) == calls_made
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
