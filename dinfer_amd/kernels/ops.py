@@ -410,9 +410,9 @@ def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor,
     assert work.shape[1] >= delta_work_columns(qk_heads, heads, dim, vdim)
     below = EVERY_ROW
     if _may_be_long(tokens, num_reqs, scratch, max_rows):
-        qk, v_end = qk_heads * dim, 2 * qk_heads * dim + heads * vdim
-        below = _chunked(True, work, work[:, qk:], work[:, 2 * qk:], work[:, v_end + heads:], work[:, v_end:], state, out,
-                         state_slots, cu_seqlens, seq_lens, num_reqs, qk_heads, heads, dim, vdim, tokens, scratch)
+        at, ld, qk, v_end = work.data_ptr(), _rows(work), qk_heads * dim, 2 * qk_heads * dim + heads * vdim
+        below = _chunked(True, at, ld, at + 4 * qk, ld, at + 8 * qk, ld, at + 4 * (v_end + heads), ld, at + 4 * v_end, ld, work.shape[0],
+                         state, out, state_slots, cu_seqlens, seq_lens, num_reqs, qk_heads, heads, dim, vdim, tokens, scratch)
     if below > 0:
         lib.call("dinfer_delta_recurrence", work.data_ptr(), _rows(work), state.data_ptr(), state_slots.data_ptr(),
                  cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), num_reqs, qk_heads, heads, dim,
@@ -446,21 +446,21 @@ def _may_be_long(tokens: int | None, num_reqs: int, scratch: torch.Tensor | None
             and (max_rows is None or max_rows >= CHUNKED_ROWS))
 
 
-def _chunked(delta, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens, num_reqs, groups, heads, dim,
-             vdim, tokens, scratch) -> int:
-    """Runs the chunked form of a recurrence for the requests it takes. Returns the rows below which a request is left to
-    the token-by-token kernel; 0: none is left."""
-    if q.stride(0) % 4 or k.stride(0) % 4 or (q.data_ptr() | k.data_ptr() | state.data_ptr()) % 16:
+def _chunked(delta, q, ldq, k, ldk, v, ldv, decay, ldd, gain, ldg, rows, state, out, state_slots, cu_seqlens, seq_lens, num_reqs,
+             groups, heads, dim, vdim, tokens, scratch) -> int:
+    """Runs the chunked form of a recurrence for the requests it takes. q to gain: addresses and row strides, `rows` rows of each
+    (views of one buffer cost a layer 10 us on the host, which is what a short prompt waits for). Returns the rows below which a request is
+    left to the token-by-token kernel; 0: none is left."""
+    if ldq % 4 or ldk % 4 or (q | k | state.data_ptr()) % 16:
         return EVERY_ROW
     floats = lib.get("dinfer_chunk_floats")(int(delta), groups, heads, dim, vdim)
     assert scratch.dtype == torch.float32 and scratch.is_contiguous() and floats > 0 and scratch.shape[1] >= floats
-    assert tokens <= q.shape[0] and tokens <= out.shape[0]
+    assert tokens <= rows and tokens <= out.shape[0]
     # (a lone request is taken however many rows it has: `tokens` may be more than those)
     shortest = 1 if num_reqs == 1 else CHUNKED_ROWS
-    lib.call("dinfer_chunked_recurrence", int(delta), q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v),
-             decay.data_ptr(), 0 if decay.dim() == 1 else _rows(decay), _ptr(gain), _rows(gain) if gain is not None else 0,
-             state.data_ptr(), state_slots.data_ptr(), cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out),
-             scratch.data_ptr(), scratch.shape[0], tokens, num_reqs, shortest, groups, heads, dim, vdim, _stream())
+    lib.call("dinfer_chunked_recurrence", int(delta), q, ldq, k, ldk, v, ldv, decay, ldd, gain, ldg, state.data_ptr(),
+             state_slots.data_ptr(), cu_seqlens.data_ptr(), seq_lens.data_ptr(), out.data_ptr(), _rows(out), scratch.data_ptr(),
+             scratch.shape[0], tokens, num_reqs, shortest, groups, heads, dim, vdim, _stream())
     return 0 if num_reqs == 1 else CHUNKED_ROWS
 
 
@@ -591,8 +591,9 @@ def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: t
     assert gain is None or gain.shape[1] >= heads
     below = EVERY_ROW
     if _may_be_long(tokens, num_reqs, scratch, max_rows):
-        below = _chunked(False, q, k, v, decay, gain, state, out, state_slots, cu_seqlens, seq_lens, num_reqs, groups, heads,
-                         dim, vdim, tokens, scratch)
+        below = _chunked(False, q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v), decay.data_ptr(), ldd, _ptr(gain),
+                         _rows(gain) if gain is not None else 0, q.shape[0], state, out, state_slots, cu_seqlens, seq_lens, num_reqs,
+                         groups, heads, dim, vdim, tokens, scratch)
     if below > 0:
         lib.call("dinfer_decay_recurrence", q.data_ptr(), _rows(q), k.data_ptr(), _rows(k), v.data_ptr(), _rows(v),
                  decay.data_ptr(), ldd, _ptr(gain), _rows(gain) if gain is not None else 0, state.data_ptr(),
