@@ -51,8 +51,10 @@ int launch_rows(const Args& p, hipStream_t stream) {
 // behind 1,000 in groups of 4: 40 -> 23); groups of one share nothing, so there only while the workgroups leave CUs empty (64 rows
 // behind 4,000: 37 -> 30 us, 256: 93 -> 94, 1,024 behind 40: 8 -> 12). Heads of 256 fill a CU's LDS: from 256 rows in groups of
 // 4 and more (25 -> 20 us; 64 rows behind 4,000: 46 -> 49), from 1,024 in smaller ones (403 -> 362; 256 rows: 105 -> 114).
-bool shares_heads(int group, int64_t rows, bool large) {
-  if (group > 16) return false;
+// Windows of up to 1,024 keys leave one or two requests nothing to gain, and inside a step the larger workgroups start later (16
+// heads over 4 of 128, two requests behind 300: 7.6 us by rows, 9.2 by heads; behind 1,100 14.6 and 14.9).
+bool shares_heads(int group, int64_t rows, bool large, int window) {
+  if (group > 16 || (window > 0 && window <= 1024 && rows <= 32)) return false;
   if (large) return group >= 4 ? rows >= 256 : group >= 2 && rows >= 1024;
   return group >= 2 || rows <= 128;
 }
@@ -62,7 +64,7 @@ bool shares_heads(int group, int64_t rows, bool large) {
 // the heads of a group instead of rows (shares_heads).
 template <int DT, int DV, int KIND>
 int launch(const Args& p, hipStream_t stream) {
-  if (p.max_q_len == 1 && shares_heads(p.H / p.Hkv, (int64_t)p.H * p.num_reqs, DT > 8)) return launch_rows<DT, DV, KIND, 1, true>(p, stream);
+  if (p.max_q_len == 1 && shares_heads(p.H / p.Hkv, (int64_t)p.H * p.num_reqs, DT > 8, p.window)) return launch_rows<DT, DV, KIND, 1, true>(p, stream);
   if constexpr (DT == 8 && DV == 8) {
     if (p.max_q_len > 32 && (int64_t)((p.max_q_len + 47) / 48) * p.H * p.num_reqs >= 2000) return launch_rows<DT, DV, KIND, 3>(p, stream);
   }

@@ -69,6 +69,8 @@ def test_heads_of_a_group_share_the_tile(case):
     (16, 4, 256, 256, 16, dict(softcap=5.0), [1, 900]),                 # ... and fewer: rows
     (16, 16, 32, 32, 16, {}, [5, 77, 130, 200, 64, 1, 300, 31]),        # groups of one: 128 rows,
     (16, 16, 32, 32, 16, {}, [5, 77, 130, 200, 64, 1, 300, 31, 9]),     # and more
+    (16, 4, 128, 128, 16, dict(window=1024, keep_first=4, sinks=True), [300, 1500]),   # 32 rows and a window: rows; one wider: heads
+    (16, 4, 128, 128, 16, dict(window=1025, keep_first=4), [300, 1500]),
 ])
 def test_runs_of_keys_and_the_choice_of_the_tile(case):
     test_heads_of_a_group_share_the_tile(case)
