@@ -422,8 +422,8 @@ def delta_recurrence(work: torch.Tensor, state: torch.Tensor, out: torch.Tensor,
 
 # A request of this many rows in a step goes chunk by chunk, the others token by token. One request, delta rule 16 x 128 x 128,
 # decays 16 x 128 x 128 and 64 x 128 x 64: at 96 rows 29, 17 and 20 us token by token against 27, 21 and 21 in chunks; at 128
-# 37, 21 and 26 against 27, 21 and 21; at 256 70, 43 and 50 against 33, 24 and 30; at 2,048 546, 323 and 362 against 128,
-# 117 and 125.
+# 37, 21 and 26 against 27, 21 and 21; at 256 70, 43 and 50 against 33, 24 and 30; at 2,048 546, 323 and 362 against 130,
+# 118 and 126.
 CHUNKED_ROWS = 128
 EVERY_ROW = 2 ** 31 - 1     # (no request has as many)
 CHUNK = 64              # tokens of a chunk (chunked.hip)
