@@ -247,10 +247,11 @@ __global__ void __launch_bounds__(WAVES * 64) qkv_post_neox_kernel(
   }
 }
 
-// V into its transposed pages for many tokens: one wave takes 8 consecutive tokens of one kv head.
-// When their slots are 8 consecutive slots starting at a multiple of 8 (a prompt portion that starts
-// on such a boundary), a lane gathers two dims of the 8 tokens and stores them as two 16-byte rows
-// of V^T; otherwise it falls back to one 2-byte store per element.
+// V into its transposed pages for many tokens: a wave looks after 8 consecutive tokens of one kv head. Eight tokens whose
+// slots are 8 consecutive ones from a multiple of 8 on (a run) are gathered by the wave that has the run's first token, wherever
+// among its 8 that lies: a lane takes two dims of the run and stores them as two 16-byte rows of V^T. Tokens in no such run
+// (a portion's ragged ends) are stored by 2 bytes. A step's portions begin anywhere among its tokens: with runs counted from
+// the step's first token only, all but the first portion's values went by 2 bytes.
 // (group: which run of 8 * WAVES tokens the workgroup takes.)
 __device__ __forceinline__ void v_write_transposed(const bf16* __restrict__ qkv, int64_t ld, int64_t v_off,
                                                    bf16* __restrict__ v_cache, const int64_t* __restrict__ slots, int T,
@@ -259,55 +260,57 @@ __device__ __forceinline__ void v_write_transposed(const bf16* __restrict__ qkv,
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int t0 = (group * WAVES + wave) * 8;
   if (t0 >= T) return;
-  const int n = T - t0 < 8 ? T - t0 : 8;
-  const int64_t s0 = slots[t0];
-  bool aligned = n == 8 && s0 >= 0 && (s0 & 7) == 0;
-  for (int j = 1; j < n && aligned; ++j) aligned = slots[t0 + j] == s0 + j;
+  // lane i looks at token t0 - 8 + i, i < 24: whether a run begins there (a bit of `runs`), and which tokens runs cover
+  const int ti = t0 - 8 + lane;
+  const int64_t slot = lane < 24 && ti >= 0 && ti < T ? slots[ti] : -1;
+  const uint64_t valid = __ballot(slot >= 0);
+  const int64_t prev = __shfl_up(slot, 1, 64);
+  const uint64_t follows = __ballot(lane > 0 && slot >= 0 && prev >= 0 && slot == prev + 1);
+  const uint64_t f1 = follows >> 1;                       // bit i: token i + 1 follows token i
+  const uint64_t f2 = f1 & (f1 >> 1), f4 = f2 & (f2 >> 2);
+  const uint64_t runs = __ballot(slot >= 0 && (slot & 7) == 0) & f4 & (f1 >> 4) & (f1 >> 5) & (f1 >> 6);
+  uint64_t covered = runs | (runs << 1);
+  covered |= covered << 2;
+  covered |= covered << 4;
+  const uint32_t mine = (uint32_t)(runs >> 8) & 255u, alone = (uint32_t)((valid & ~covered) >> 8) & 255u;
   const bf16* src = qkv + (int64_t)t0 * ld + v_off + (int64_t)hk * D;
-  for (int d2 = lane; d2 < D / 2; d2 += 64) {
-    bf16x2 v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j < n) v[j] = *(const bf16x2*)(src + (int64_t)j * ld + 2 * d2);
-    if (vb) {  // the head's bias (float), added as the kernels that take one value at a time add it
-      const float b0 = vb[2 * d2], b1 = vb[2 * d2 + 1];
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (j < n) {
-          v[j][0] = (bf16)((float)v[j][0] + b0);
-          v[j][1] = (bf16)((float)v[j][1] + b1);
-        }
+  auto value = [&](int j, int d2) {   // two dims of token t0 + j, as they are stored
+    bf16x2 v = *(const bf16x2*)(src + (int64_t)j * ld + 2 * d2);
+    if (vb || mix.first) {   // (the head's bias, float, then the other row's share, as the kernels for single tokens do it)
+      float a = (float)v[0] + (vb ? vb[2 * d2] : 0.f), b = (float)v[1] + (vb ? vb[2 * d2 + 1] : 0.f);
+      if (mix.first) {
+        a = mixed_value<bf16>(a, mix, t0 + j, hk * D + 2 * d2);
+        b = mixed_value<bf16>(b, mix, t0 + j, hk * D + 2 * d2 + 1);
+      }
+      v[0] = (bf16)a;
+      v[1] = (bf16)b;
     }
-    if (mix.first) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (j < n) {
-          v[j][0] = (bf16)mixed_value<bf16>((float)v[j][0], mix, t0 + j, hk * D + 2 * d2);
-          v[j][1] = (bf16)mixed_value<bf16>((float)v[j][1], mix, t0 + j, hk * D + 2 * d2 + 1);
-        }
-    }
-    if (aligned) {
-      const int64_t blk = s0 / page;
-      const int off = (int)(s0 % page);
-      bf16* vd = v_cache + ((blk * Hkv + hk) * (int64_t)D + 2 * d2) * page + off;
+    return v;
+  };
+  if (mine) {   // (two runs cannot begin within 8 tokens)
+    const int r = __builtin_ctz(mine);
+    const int64_t s0 = __shfl(slot, 8 + r, 64), blk = s0 / page;
+    bf16* vd = v_cache + (blk * Hkv + hk) * (int64_t)D * page + (int)(s0 - blk * page);
+    for (int d2 = lane; d2 < D / 2; d2 += 64) {
       bf16x8 a, b;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        a[j] = v[j][0];
-        b[j] = v[j][1];
+        const bf16x2 v = value(r + j, d2);
+        a[j] = v[0];
+        b[j] = v[1];
       }
-      *(bf16x8*)vd = a;
-      *(bf16x8*)(vd + page) = b;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (j >= n) break;
-        const int64_t sl = slots[t0 + j];
-        if (sl < 0) continue;
-        bf16* vd = v_cache + (((sl / page) * Hkv + hk) * (int64_t)D + 2 * d2) * page + sl % page;
-        vd[0] = v[j][0];
-        vd[page] = v[j][1];
-      }
+      *(bf16x8*)(vd + (int64_t)(2 * d2) * page) = a;
+      *(bf16x8*)(vd + (int64_t)(2 * d2 + 1) * page) = b;
+    }
+  }
+  for (uint32_t left = alone; left; left &= left - 1) {
+    const int j = __builtin_ctz(left);
+    const int64_t sl = __shfl(slot, 8 + j, 64), blk = sl / page;
+    bf16* vd = v_cache + (blk * Hkv + hk) * (int64_t)D * page + (int)(sl - blk * page);
+    for (int d2 = lane; d2 < D / 2; d2 += 64) {
+      const bf16x2 v = value(j, d2);
+      vd[(int64_t)(2 * d2) * page] = v[0];
+      vd[(int64_t)(2 * d2 + 1) * page] = v[1];
     }
   }
 }
@@ -316,25 +319,14 @@ __device__ __forceinline__ void v_write_transposed(const bf16* __restrict__ qkv,
 // consecutive dims in one 16-byte load; the partner of a pair (i, i + D / 2) sits LPH / 2 lanes away and comes by a
 // cross-lane read, pairs (2i, 2i + 1) (NEIGHBOURS) lie in the lane itself. A wave covers 64 / LPH heads of one token per instruction, an order of magnitude
 // fewer memory instructions than 2-byte accesses.
-// gather_v > 0: V is not written by the heads' lanes; the workgroups from blockIdx.x = `tokens` on (gather_v of them,
-// one per kv head and run of 8 * WAVES tokens) gather it into its transposed pages, in the same launch (a kernel of
-// its own for that cost a prefill layer 5.7 us, a step of prompt portions beside decoding requests 7.8).
 template <int LPH, bool NEIGHBOURS>
 __global__ void __launch_bounds__(WAVES * 64) qkv_post_vec_kernel(
     bf16* __restrict__ qkv, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, const void* __restrict__ wq,
     const void* __restrict__ wk, int wf32, float eps, float w_offset, const int32_t* __restrict__ pos,
     const float* __restrict__ cos_sin, bf16* __restrict__ k_cache, bf16* __restrict__ v_cache,
-    const int64_t* __restrict__ slots, int H, int Hkv, int page, int tokens, int gather_v,
-    const float* __restrict__ bias, float temp_coef, int temp_every, const float* __restrict__ head_scale, ValueMix mix) {
+    const int64_t* __restrict__ slots, int H, int Hkv, int page, const float* __restrict__ bias, float temp_coef,
+    int temp_every, const float* __restrict__ head_scale, ValueMix mix) {
   constexpr int D = LPH * 8, HALF = D / 2, HPW = 64 / LPH;  // heads per wave
-  if ((int)blockIdx.x >= tokens) {
-    const int j = (int)blockIdx.x - tokens;
-    if (blockIdx.y == 0)
-      v_write_transposed(qkv, ld, v_off, v_cache, slots, tokens, Hkv, D, page, j / Hkv, j % Hkv,
-                         bias ? bias + (int64_t)(H + Hkv + j % Hkv) * D : nullptr, mix);
-    return;
-  }
-  const bool skip_v = gather_v > 0;
   const int64_t t = blockIdx.x;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int sub = lane / LPH, l = lane % LPH;  // which head of the wave, which 8 dims of it
@@ -407,7 +399,7 @@ __global__ void __launch_bounds__(WAVES * 64) qkv_post_vec_kernel(
       for (int e = 0; e < 4; ++e) { x[e] += b0[e]; x[4 + e] += b1[e]; }
     }
     if (is_v) {
-      if (slot >= 0 && !skip_v) {
+      if (slot >= 0) {
         if (mix.first) {
           const bf16x8 f = *(const bf16x8*)((const bf16*)mix.first + t * mix.ld + (int64_t)(item - H - Hkv) * D + d0);
 #pragma unroll
@@ -469,6 +461,115 @@ __global__ void __launch_bounds__(WAVES * 64) qkv_post_vec_kernel(
       *(bf16x8*)(src + d0) = r;
     } else if (slot >= 0) {
       *(bf16x8*)(k_cache + (blk * Hkv + (item - H)) * (int64_t)page * D + k_page_offset((int)off, d0, page)) = r;
+    }
+  }
+}
+
+// The same for many tokens of prompt portions: a workgroup takes WAVES * 64 / LPH tokens and RH heads of one kind (q or
+// k), a wave 64 / LPH of the tokens, so that what goes into one line of a K page (the same 8 dims of consecutive keys) is
+// stored by one workgroup and meets in its L2, the angles of a lane's dims are fetched once, and a lane's values are all
+// asked for at the start. The workgroups behind `qk_groups` write V. With a workgroup a token (neighbouring tokens on
+// different XCDs, each with its own copy of the line) 2,048 tokens of 48 heads of 128 took 16.3 us, 11.0 here (4.6 TB/s); 1,033
+// tokens of 32 heads in 8 portions 13.0, 6.5; 543 of 56 heads, most in one portion, 9.2, 6.9; 100 of 48 4.0, 4.8.
+template <int LPH, bool NEIGHBOURS, int RH>
+__global__ void __launch_bounds__(WAVES * 64) qkv_post_runs_kernel(
+    bf16* __restrict__ qkv, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, const void* __restrict__ wq,
+    const void* __restrict__ wk, int wf32, float eps, float w_offset, const int32_t* __restrict__ pos,
+    const float* __restrict__ cos_sin, bf16* __restrict__ k_cache, bf16* __restrict__ v_cache,
+    const int64_t* __restrict__ slots, int H, int Hkv, int page, int tokens, int qk_groups,
+    const float* __restrict__ bias, float temp_coef, int temp_every, const float* __restrict__ head_scale, ValueMix mix) {
+  constexpr int D = LPH * 8, HALF = D / 2, TPW = 64 / LPH;
+  if ((int)blockIdx.x >= qk_groups) {
+    const int j = (int)blockIdx.x - qk_groups;
+    v_write_transposed(qkv, ld, v_off, v_cache, slots, tokens, Hkv, D, page, j / Hkv, j % Hkv,
+                       bias ? bias + (int64_t)(H + Hkv + j % Hkv) * D : nullptr, mix);
+    return;
+  }
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane / LPH, l = lane % LPH, d0 = 8 * l;
+  const int q_chunks = (H + RH - 1) / RH, chunks = q_chunks + (Hkv + RH - 1) / RH;
+  const int chunk = (int)blockIdx.x % chunks;
+  const int t_ = ((int)blockIdx.x / chunks * WAVES + wave) * TPW + sub;
+  const bool live = t_ < tokens;
+  const int64_t t = live ? t_ : tokens - 1;   // (lanes past the end repeat the last token and store nothing)
+  const bool is_q = chunk < q_chunks;
+  const int head0 = (is_q ? chunk : chunk - q_chunks) * RH, heads = is_q ? H : Hkv;
+  bf16* const src = qkv + t * ld + (is_q ? q_off : k_off) + d0;
+  const int p = cos_sin || temp_every > 0 ? pos[t] : 0;
+  const int64_t slot = is_q ? -1 : slots[t];
+  bf16x8 xv[RH];
+#pragma unroll
+  for (int u = 0; u < RH; ++u) xv[u] = *(const bf16x8*)(src + (int64_t)min(head0 + u, heads - 1) * D);
+  const void* const w = is_q ? wq : wk;
+  float g[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) g[e] = 1.f;
+  if (w && wf32) {
+    const f32x4 a = *(const f32x4*)((const float*)w + d0), b = *(const f32x4*)((const float*)w + d0 + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { g[e] = a[e] + w_offset; g[4 + e] = b[e] + w_offset; }
+  } else if (w) {
+    const bf16x8 gv = *(const bf16x8*)((const bf16*)w + d0);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] = (float)gv[e] + w_offset;
+  }
+  float c[8], sn[8];
+  const int pi = NEIGHBOURS ? d0 / 2 : d0 % HALF;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) { c[e] = 1.f; sn[e] = 0.f; }
+  if (cos_sin) {
+    const float* cs = cos_sin + (int64_t)p * D;
+#pragma unroll
+    for (int h = 0; h < (NEIGHBOURS ? 1 : 2); ++h) {
+      const f32x4 c0 = *(const f32x4*)(cs + pi + 4 * h), s0 = *(const f32x4*)(cs + HALF + pi + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { c[4 * h + e] = c0[e]; sn[4 * h + e] = s0[e]; }
+    }
+  }
+  const int64_t blk = slot >= 0 ? slot / page : 0;
+  const int off = slot >= 0 ? (int)(slot - blk * page) : 0;
+#pragma unroll
+  for (int u = 0; u < RH; ++u) {
+    const int head = head0 + u;
+    if (head >= heads) break;   // (the whole workgroup)
+    float x[8], ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = (float)xv[u][e];
+    if (bias) {
+      const float* hb = bias + (int64_t)((is_q ? 0 : H) + head) * D + d0;
+      const f32x4 b0 = *(const f32x4*)hb, b1 = *(const f32x4*)(hb + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { x[e] += b0[e]; x[4 + e] += b1[e]; }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss = add_square(ss, x[e]);
+#pragma unroll
+    for (int o = LPH / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    float inv = w ? 1.f / sqrtf(ss / (float)D + eps) : 1.f;
+    // a query grows with its position: 1 + coef ln(floor((p + 1) / every) + 1)
+    if (is_q && w && temp_every > 0) inv *= 1.f + temp_coef * logf((float)((p + 1) / temp_every) + 1.f);
+    if (is_q && w && head_scale) inv *= head_scale[head];
+    float y[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = w ? x[e] * inv * g[e] : x[e];
+    bf16x8 r;
+    if constexpr (NEIGHBOURS) {
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        r[e] = (bf16)rotated_first(y[e], y[e + 1], c[e / 2], sn[e / 2]);
+        r[e + 1] = (bf16)rotated_second(y[e], y[e + 1], c[e / 2], sn[e / 2]);
+      }
+    } else {
+      const bool first = l < LPH / 2;  // this lane holds the first elements of its pairs
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float other = __shfl_xor(y[e], LPH / 2, 64);
+        r[e] = (bf16)(first ? rotated_first(y[e], other, c[e], sn[e]) : rotated_second(other, y[e], c[e], sn[e]));
+      }
+    }
+    if (is_q) {
+      if (live) *(bf16x8*)(src + (int64_t)head * D) = r;
+    } else if (live && slot >= 0) {
+      *(bf16x8*)(k_cache + (blk * Hkv + head) * (int64_t)page * D + k_page_offset(off, d0, page)) = r;
     }
   }
 }
@@ -781,16 +882,33 @@ extern "C" int dinfer_qkv_post(int dtype, void* qkv, int64_t tokens, int64_t ld,
     // many tokens fill the chip with one workgroup each; few tokens spread their heads over several
     // many tokens: V goes to its transposed pages through workgroups that gather it (16-byte stores)
     const bool gather = slot_mapping && token_runs && tokens >= 64 && page_size % 8 == 0 && ((uintptr_t)v_cache % 16) == 0;
-    const int64_t gather_v = gather ? (tokens + 8 * WAVES - 1) / (8 * WAVES) * kv_heads : 0;
-    if (tokens + gather_v > 0x7fffffff) return ERR_BAD_SHAPE;
-    const dim3 vgrid((unsigned)(tokens + gather_v),
-                     tokens >= 512 ? 1u : (unsigned)((items + WAVES * hpw - 1) / (WAVES * hpw)));
     const bool pairs = style == 1 && cos_sin;
+    if (gather) {
+      // four heads a workgroup where the tokens fill the chip, one where they do not (100 tokens of 48 heads 4.8 us with four,
+      // 3.5 with one, 4.0 by a workgroup a token; 256 5.1 and 4.3, 5.2)
+      const int rh = tokens >= 512 ? 4 : 1;
+      const int64_t chunks = (heads + rh - 1) / rh + (kv_heads + rh - 1) / rh;
+      const int64_t qk_groups = (tokens + WAVES * hpw - 1) / (WAVES * hpw) * chunks;
+      const int64_t groups = qk_groups + (tokens + 8 * WAVES - 1) / (8 * WAVES) * kv_heads;
+      if (groups > 0x7fffffff) return ERR_BAD_SHAPE;
+#define DINFER_QKV_RUNS(LPH_)                                                                                          \
+  (rh == 4 ? pairs ? qkv_post_runs_kernel<LPH_, true, 4> : qkv_post_runs_kernel<LPH_, false, 4>                         \
+           : pairs ? qkv_post_runs_kernel<LPH_, true, 1> : qkv_post_runs_kernel<LPH_, false, 1>)                        \
+      <<<(unsigned)groups, WAVES * 64, 0, stream>>>(                                                                   \
+          (bf16*)qkv, ld, q_off, k_off, v_off, q_gain, k_gain, w_f32, eps, w_offset, positions, cos_sin, (bf16*)k_cache, \
+          (bf16*)v_cache, slot_mapping, heads, kv_heads, page_size, (int)tokens, (int)qk_groups, bias, temp_coef,      \
+          temp_every, head_scale, mix)
+      if (lph == 8) DINFER_QKV_RUNS(8);
+      else if (lph == 16) DINFER_QKV_RUNS(16);
+      else DINFER_QKV_RUNS(32);
+#undef DINFER_QKV_RUNS
+      return launch_status();
+    }
+    const dim3 vgrid((unsigned)tokens, tokens >= 512 ? 1u : (unsigned)((items + WAVES * hpw - 1) / (WAVES * hpw)));
 #define DINFER_QKV_VEC(LPH_)                                                                                          \
   (pairs ? qkv_post_vec_kernel<LPH_, true> : qkv_post_vec_kernel<LPH_, false>)<<<vgrid, WAVES * 64, 0, stream>>>(      \
       (bf16*)qkv, ld, q_off, k_off, v_off, q_gain, k_gain, w_f32, eps, w_offset, positions, cos_sin, (bf16*)k_cache, \
-      (bf16*)v_cache, slot_mapping, heads, kv_heads, page_size, (int)tokens, (int)gather_v, bias, temp_coef,       \
-      temp_every, head_scale, mix)
+      (bf16*)v_cache, slot_mapping, heads, kv_heads, page_size, bias, temp_coef, temp_every, head_scale, mix)
     if (lph == 8) DINFER_QKV_VEC(8);
     else if (lph == 16) DINFER_QKV_VEC(16);
     else DINFER_QKV_VEC(32);

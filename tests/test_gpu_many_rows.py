@@ -1,0 +1,51 @@
+"""Kernels for steps of many rows against the ones for few or for any rows, and against 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def ops():
+    from dinfer_amd.kernels import ops as o
+    return o
+
+
+def _slots(portions, page, blocks):
+    """Slots of portions (first position, tokens), each on pages of its own in shuffled order."""
+    order, out, g = torch.randperm(blocks, generator=torch.Generator().manual_seed(page)).tolist(), [], 0
+    for first, n in portions:
+        pages = [order[g + i] for i in range((first + n - 1) // page + 1)]
+        g += len(pages)
+        out += [pages[p // page] * page + p % page for p in range(first, first + n)]
+    return out
+
+
+@pytest.mark.parametrize("H,Hkv,D,style,extras", [(6, 3, 64, 0, True), (16, 8, 128, 0, False), (9, 1, 128, 1, True), (5, 5, 256, 0, True), (4, 2, 256, 1, False)])
+@pytest.mark.parametrize("portions", [[(0, 64)], [(5, 1), (0, 3), (3, 61), (8, 7), (16, 8), (1, 40)], [(i, 37 + i) for i in range(12)]])
+def test_qkv_post_of_portions(H, Hkv, D, style, extras, portions):
+    """The kernel for prompt portions leaves the bits of the kernel that takes single tokens, wherever portions begin."""
+    page, blocks = 16, sum((a + n - 1) // 16 + 1 for a, n in portions)
+    g = torch.Generator().manual_seed(D + style)
+    T, cols = sum(n for _, n in portions), (H + 2 * Hkv) * D
+    x = torch.randn(T, cols, generator=g).to(BF).cuda()
+    slots = _slots(portions, page, blocks)
+    slots[T // 2] = -1
+    slots = torch.tensor(slots).cuda()
+    ang = torch.rand(300, D // 2, generator=g) * 6
+    table = torch.cat([ang.cos(), ang.sin()], 1).cuda()
+    pos = torch.randint(0, 300, (T,), generator=g, dtype=torch.int32).cuda()
+    gains = [(1 + 0.2 * torch.randn(D, generator=g)).to(torch.float32 if extras else BF).cuda() for _ in range(2)]
+    more = dict(bias=torch.randn(cols, generator=g).cuda(), q_temp=(0.1, 16), q_head_scale=torch.rand(H, generator=g).cuda(),
+                v_first=torch.randn(T, Hkv * D, generator=g).to(BF).cuda(), v_share=0.3) if extras else {}
+    got = []
+    for runs in (False, True):
+        buf = x.clone()
+        kc = torch.full((blocks, Hkv, D // 8, page, 8), 9.0, dtype=BF, device="cuda")
+        vc = torch.full((blocks, Hkv, D, page), 9.0, dtype=BF, device="cuda")
+        ops().qkv_post(buf, T, heads=H, kv_heads=Hkv, head_dim=D, q_off=0, k_off=H * D, v_off=(H + Hkv) * D, q_gain=gains[0],
+                       k_gain=gains[1], eps=1e-6, gain_offset=0.5, positions=pos, cos_sin=table, rotary_dim=D, rope_style=style,
+                       k_cache=kc, v_cache=vc, slot_mapping=slots, page_size=page, token_runs=runs, **more)
+        got.append((buf, kc, vc))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
