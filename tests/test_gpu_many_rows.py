@@ -49,3 +49,22 @@ def test_qkv_post_of_portions(H, Hkv, D, style, extras, portions):
         got.append((buf, kc, vc))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("rows,width", [(1023, 2048), (1024, 8), (1025, 520), (1030, 2048), (1024, 2056), (1027, 4096), (1024, 4104)])
+@pytest.mark.parametrize("x_dtype,out_dtype,branch", [(BF, BF, True), (torch.float32, BF, False), (torch.float32, torch.float32, True)])
+def test_layernorm_of_many_rows(rows, width, x_dtype, out_dtype, branch):
+    g = torch.Generator().manual_seed(rows + width)
+    x = (torch.randn(rows, width, generator=g) + 0.5).to(x_dtype).cuda()
+    stream = torch.randn(rows, width, generator=g).cuda() if branch else None
+    w, b = torch.randn(width, generator=g).cuda(), torch.randn(width, generator=g).cuda()
+    out = torch.empty(rows, width, dtype=out_dtype, device="cuda")
+    y = x.double() + (stream.double() if branch else 0)
+    total = x.float() + stream if branch else None
+    ops().layernorm(x, w, b, out, 1e-5, rows, residual=stream)
+    want = torch.nn.functional.layer_norm(y, (width,), w.double(), b.double(), 1e-5)
+    if branch:
+        assert torch.equal(stream, total)
+    # sums of up to 4,104 floats, then one rounding: 2^-9 in bfloat16, some 2^-18 in float
+    tol = 2.0 ** -8 if out_dtype == BF else 2.0 ** -16
+    assert ((out.double() - want).abs() <= tol * (want.abs() + 1)).all()
