@@ -5,6 +5,8 @@
 // Reference behaviour: crates/kernels/cuda/activation.cu:8-16,80-99,121-129
 // (silu(x) = x / (1 + exp(-x)), an id outside [0, vocab) reads row 0) and
 // crates/kernels/cuda/elementwise.cu:42-46 (add in float, one rounding).
+#include <algorithm>
+
 #include "common.cuh"
 
 using namespace dinfer;
@@ -149,6 +151,43 @@ __global__ void __launch_bounds__(256) gate_kernel(S* __restrict__ x, int64_t ld
   const int64_t t = blockIdx.y;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     x[t * ld_x + i] = from_f32<S>(to_f32(x[t * ld_x + i]) * act1(to_f32(g[t * ld_g + (group > 1 ? i / group : i)]), act));
+}
+
+// act_kernel and gate_kernel (group 1, or whole pieces of 8 within a group) with 8 bf16 a thread and step: n % 8 == 0, rows of
+// 16-byte pieces. 4,096 rows x 8,192 43.4 us by 2-byte accesses, 27.0 here (5.0 TB/s); the gate of 2,023 rows x 2,048
+// 7.8, 6.5.
+// Fewer numbers than this go one by one, which puts more waves on them (64 x 2,816 3.0 us against 3.2).
+constexpr int64_t PIECES_FROM = 1 << 20;
+__global__ void __launch_bounds__(256) act_bf16x8_kernel(const bf16* in, int64_t ld_in, bf16* out, int64_t ld_out, int64_t n8,
+                                                         int act) {   // (in may be out)
+  const int64_t t = blockIdx.y;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += (int64_t)gridDim.x * blockDim.x) {
+    const bf16x8 v = *(const bf16x8*)(in + t * ld_in + 8 * i);
+    bf16x8 r;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) r[j] = (bf16)act1((float)v[j], act);
+    *(bf16x8*)(out + t * ld_out + 8 * i) = r;
+  }
+}
+
+__global__ void __launch_bounds__(256) gate_bf16x8_kernel(bf16* __restrict__ x, int64_t ld_x, const bf16* __restrict__ g,
+                                                          int64_t ld_g, int64_t n8, int act, int64_t group) {
+  const int64_t t = blockIdx.y;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += (int64_t)gridDim.x * blockDim.x) {
+    bf16* xp = x + t * ld_x + 8 * i;
+    const bf16x8 v = *(const bf16x8*)xp;
+    bf16x8 r;
+    if (group > 1) {   // one gate for the piece
+      const float gate = act1((float)g[t * ld_g + 8 * i / group], act);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) r[j] = (bf16)((float)v[j] * gate);
+    } else {
+      const bf16x8 gv = *(const bf16x8*)(g + t * ld_g + 8 * i);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) r[j] = (bf16)((float)v[j] * act1((float)gv[j], act));
+    }
+    *(bf16x8*)xp = r;
+  }
 }
 
 // out[t, i] = act(in[t, i]) * in[t, inter + i] for any activation of act1
@@ -325,6 +364,12 @@ extern "C" int dinfer_gate(int dtype, int act, void* x, int64_t ld_x, const void
   for (int64_t t0 = 0; t0 < tokens; t0 += 65535) {
     const int64_t nt = tokens - t0 < 65535 ? tokens - t0 : 65535;
     const dim3 grid((unsigned)((n + 1023) / 1024 < 64 ? (n + 1023) / 1024 : 64), (unsigned)nt);
+    if (dtype == DT_BF16 && tokens * n >= PIECES_FROM && n % 8 == 0 && ld_x % 8 == 0 && ((uintptr_t)x % 16) == 0 &&
+        (group > 1 ? group % 8 == 0 : ld_g % 8 == 0 && ((uintptr_t)g % 16) == 0)) {
+      const dim3 grid8((unsigned)std::min<int64_t>((n / 8 + 255) / 256, 64), (unsigned)nt);
+      gate_bf16x8_kernel<<<grid8, 256, 0, stream>>>((bf16*)x + t0 * ld_x, ld_x, (const bf16*)g + t0 * ld_g, ld_g, n / 8, act, group);
+      continue;
+    }
     DINFER_DISPATCH_DTYPE(dtype, {
       gate_kernel<S><<<grid, 256, 0, stream>>>((S*)x + t0 * ld_x, ld_x, (const S*)g + t0 * ld_g, ld_g, n, act, group);
     });
@@ -342,6 +387,11 @@ extern "C" int dinfer_act(int dtype, int act, const void* in, int64_t ld_in, voi
   for (int64_t t0 = 0; t0 < tokens; t0 += 65535) {
     const int64_t nt = tokens - t0 < 65535 ? tokens - t0 : 65535;
     const dim3 grid((unsigned)((n + 1023) / 1024 < 64 ? (n + 1023) / 1024 : 64), (unsigned)nt);
+    if (dtype == DT_BF16 && tokens * n >= PIECES_FROM && n % 8 == 0 && ld_in % 8 == 0 && ld_out % 8 == 0 && ((uintptr_t)in % 16) == 0 && ((uintptr_t)out % 16) == 0) {
+      const dim3 grid8((unsigned)std::min<int64_t>((n / 8 + 255) / 256, 64), (unsigned)nt);
+      act_bf16x8_kernel<<<grid8, 256, 0, stream>>>((const bf16*)in + t0 * ld_in, ld_in, (bf16*)out + t0 * ld_out, ld_out, n / 8, act);
+      continue;
+    }
     DINFER_DISPATCH_DTYPE(dtype, {
       act_kernel<S><<<grid, 256, 0, stream>>>((const S*)in + t0 * ld_in, ld_in, (S*)out + t0 * ld_out, ld_out, n, act);
     });

@@ -68,3 +68,27 @@ def test_layernorm_of_many_rows(rows, width, x_dtype, out_dtype, branch):
     # sums of up to 4,104 floats, then one rounding: 2^-9 in bfloat16, some 2^-18 in float
     tol = 2.0 ** -8 if out_dtype == BF else 2.0 ** -16
     assert ((out.double() - want).abs() <= tol * (want.abs() + 1)).all()
+
+
+@pytest.mark.parametrize("rows,n", [(1, 8), (3, 72), (70, 2816), (600, 2056), (9, 16392 * 8)])
+def test_activations_in_16_byte_pieces(rows, n):
+    """Rows that begin at a 16-byte piece against the same rows two entries further on, which are taken one by one."""
+    g = torch.Generator().manual_seed(n)
+    x, gates = torch.randn(rows, n, generator=g).to(BF) * 3, torch.randn(rows, n, generator=g).to(BF)
+    for kind in ("silu", "relu2", "gelu", "gelu_tanh", "sigmoid"):
+        got = []
+        for at in (0, 2):
+            a, b, o = (torch.zeros(rows, n + 8, dtype=BF, device="cuda") for _ in range(3))
+            a[:, at:at + n] = x.cuda()
+            b[:, at:at + n] = gates.cuda()
+            ops().act(a[:, at:at + n], o[:, at:at + n], rows, kind)
+            ys = [o[:, at:at + n]]
+            for group in (1, 8):
+                z = torch.zeros(rows, n + 8, dtype=BF, device="cuda")
+                z[:, at:at + n] = x.cuda()
+                ops().gate(z[:, at:at + n], b[:, at:at + n // group], rows, kind, group=group)
+                ys.append(z[:, at:at + n])
+                assert not z[:, :at].any() and not z[:, at + n:].any()
+            got.append(ys)
+        for a, b in zip(*got):
+            assert torch.equal(a, b)
