@@ -92,3 +92,26 @@ def test_activations_in_16_byte_pieces(rows, n):
             got.append(ys)
         for a, b in zip(*got):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("tokens,experts,width,gate", [(1024, 1, 32, False), (1030, 64, 2048, True), (1025, 47, 544, False), (1100, 130, 96, True), (1024, 64, 40, True)])
+def test_router_logits_of_many_tokens(tokens, experts, width, gate):
+    """The logits against 64 bits: as near as the kernel for few tokens (which a step of 1,000 of them gets), and the choice
+    made from them; an infinity of one token stays with that token."""
+    g = torch.Generator().manual_seed(tokens + experts)
+    x = torch.randn(tokens, width, generator=g).to(BF).cuda()
+    x[7, 3] = float("inf")
+    w, sg = torch.randn(experts, width, generator=g).cuda(), torch.randn(width, generator=g).cuda() if gate else None
+    top = min(2, experts)
+    want = x.double() @ torch.cat([w] + ([sg[None]] if gate else [])).double().t()
+    err = []
+    for n in (tokens, 1000):
+        idx, share = torch.zeros(n * top, dtype=torch.int32, device="cuda"), torch.zeros(n * top, device="cuda")
+        z = torch.zeros(n * (experts + 1), device="cuda")
+        ops().moe_route(x, w, sg, idx, share, torch.zeros(n, device="cuda"), n, top, z, all_scores=0, correction=None)
+        z = z.view(n, experts + 1)[:, :want.shape[1]]
+        keep = torch.arange(n, device="cuda") != 7
+        assert not torch.isfinite(z[7]).any()
+        err.append(((z.double() - want[:n])[keep].norm() / want[:n][keep].norm()).item())
+        assert torch.equal(idx.view(n, top)[keep, 0].long(), z[keep][:, :experts].argmax(1))
+    assert err[0] <= 1.1 * err[1] and err[0] < 2e-7
