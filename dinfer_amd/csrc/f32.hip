@@ -254,9 +254,15 @@ __global__ void __launch_bounds__(256, DT <= 8 ? 2 : 1) attn_f32_kernel(
   __shared__ float pm[WAVES][CT][16], pl[WAVES][CT][16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lg = lane >> 4;
-  const int b = blockIdx.y, hk = blockIdx.z;
+  // Workgroups in the order of their dispatch: kv heads fastest, then a request's row tiles, the later half from its end down
+  // (most keys), then the earlier half from its start up, so that the two or so workgroups that share a CU are a long and a
+  // short one (500 rows, 63 tiles x 8 heads: 30.0 us, 32.4 with the tiles of a head in ascending order).
+  const int tiles = (int)gridDim.x / Hkv;
+  const int hk = (int)blockIdx.x % Hkv, x = (int)blockIdx.x / Hkv, later = (tiles + 1) / 2;
+  const int tile = x < later ? tiles - 1 - x : x - later;
+  const int b = blockIdx.y;
   const int t0 = cu_seqlens[b], q_len = cu_seqlens[b + 1] - t0;
-  const int rows = q_len * G, r0 = blockIdx.x * 16 * CT;
+  const int rows = q_len * G, r0 = tile * 16 * CT;
   if (r0 >= rows) return;   // the whole workgroup
   const int hist = seq_lens[b] - q_len;
   const int32_t* bt = block_table + (int64_t)b * max_blocks;
@@ -440,7 +446,7 @@ template <int DT, int CT>
 void launch_attn(const float* q, int64_t ld_q, float* out, int64_t ld_out, const float* k, const float* v, const int32_t* bt,
                  int64_t max_blocks, const int32_t* cu, const int32_t* sl, int reqs, int max_q, float scale, int window, int G,
                  int Hkv, int page, hipStream_t stream) {
-  const dim3 grid((unsigned)(((int64_t)max_q * G + 16 * CT - 1) / (16 * CT)), (unsigned)reqs, (unsigned)Hkv);
+  const dim3 grid((unsigned)(((int64_t)max_q * G + 16 * CT - 1) / (16 * CT) * Hkv), (unsigned)reqs);
   attn_f32_kernel<DT, CT><<<grid, 256, 0, stream>>>(q, ld_q, out, ld_out, k, v, bt, max_blocks, cu, sl, scale, window, G, Hkv, page);
 }
 
@@ -495,7 +501,7 @@ extern "C" int dinfer_attn_f32(const void* q, int64_t ld_q, void* out, int64_t l
   if (heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || max_blocks <= 0 || window < 0) return ERR_BAD_SHAPE;
   if (!dinfer_attn_f32_supports(head_dim, page_size, heads, kv_heads) || num_reqs > 65535 || kv_heads > 65535 || ld_q % 4 != 0 ||
       ld_out % 4 != 0 || !aligned16(q) || !aligned16(out) || !aligned16(k_cache) || !aligned16(v_cache) ||
-      (int64_t)max_q * (heads / kv_heads) > 0x7fffffff - 64)
+      (int64_t)max_q * (heads / kv_heads) > 0x7fffffff - 64 || ((int64_t)max_q * (heads / kv_heads) + 15) / 16 * kv_heads > 0x7fffffff)
     return ERR_UNSUPPORTED;
   const int G = heads / kv_heads;
   const bool two = (int64_t)max_q * G > 16;   // two tiles of rows share the keys and values a wave loads (up to heads of 64: registers)
