@@ -526,7 +526,8 @@ int launch_decode(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, float*
     // Workgroups of `splits` waves are placed whole: where their number leaves the last round over the CUs thin
     // (320 workgroups on 256 CUs: some CUs get two, most one) single waves spread better and the merge kernel is the
     // lesser cost. Measured at 8 kv heads: 32, 56 and 64 requests gain 0.12 to 0.17 ms a step, 40 and 48 lose.
-    const double per_cu = (double)Hkv * num_reqs / compute_units();
+    // (beside single rows at least one request brings more: its workgroups leave at once)
+    const double per_cu = (double)Hkv * (cu && num_reqs > 1 ? num_reqs - 1 : num_reqs) / compute_units();
     if (splits <= JOIN_SPLITS && (per_cu <= 1. || ceil(per_cu) <= 1.15 * per_cu)) {
       auto kernel = p2 ? decode_kernel_for<DT, true, true, POST>(late) : decode_kernel_for<DT, false, true, POST>(late);
       kernel<<<dim3(1, (unsigned)Hkv, (unsigned)num_reqs), 64 * splits, 0, stream>>>(

@@ -65,6 +65,7 @@ typedef struct {
     int64_t* slot_mapping[DH_MAX_GROUPS];
     int32_t* block_table[DH_MAX_GROUPS];
     int32_t max_blocks[DH_MAX_GROUPS];
+    int32_t spare; /* made-up requests that the buffers hold beyond max_reqs */
 } dh_batch_buffers;
 
 typedef struct {

@@ -43,6 +43,7 @@ struct BatchBuffers {
     int64_t* slot_mapping[MAX_GROUPS];
     int32_t* block_table[MAX_GROUPS];
     int32_t max_blocks[MAX_GROUPS];
+    int32_t spare;  // made-up requests that the buffers hold beyond max_reqs
 };
 
 // What the host needs to know about the step it just described.
@@ -170,7 +171,7 @@ inline void fill_batch(const CacheManager& cache, const BatchBuffers& buf, const
 // logits rows point at the first made-up token (or at row 0). facts: the step's, brought up to date.
 inline void pad_batch(const BatchBuffers& buf, BatchFacts* facts, int reqs, int tokens, int rows) {
     const int B = facts->num_reqs, T = facts->num_tokens, R = facts->num_rows;
-    if (reqs < B || tokens < T || rows < R || reqs > buf.max_reqs || tokens > buf.max_tokens || rows > buf.max_rows)
+    if (reqs < B || tokens < T || rows < R || reqs > buf.max_reqs + buf.spare || tokens > buf.max_tokens || rows > buf.max_rows)
         throw Error(ERR_VALUE, "a step can be padded up to the engine's sizes only, never cut");
     const int more_reqs = reqs - B, more_tokens = tokens - T;
     if ((more_reqs == 0) != (more_tokens == 0) || more_tokens < more_reqs)

@@ -39,16 +39,17 @@ class Entry:
 
 
 class StepBatch:
-    def __init__(self, device, max_tokens: int, max_reqs: int, max_rows: int, max_blocks: list[int]):
+    def __init__(self, device, max_tokens: int, max_reqs: int, max_rows: int, max_blocks: list[int], spare: int = 0):
+        """spare: made-up requests of pad() that fit beside max_reqs real ones."""
         self.device = device
         self.max_tokens, self.max_reqs, self.max_rows = max_tokens, max_reqs, max_rows
         self.max_blocks = list(max_blocks)
         layout = [("slot_mapping%d" % g, np.int64, (max_tokens,)) for g in range(len(max_blocks))]
         layout += [("input_ids", np.int32, (max_tokens,)), ("positions", np.int32, (max_tokens,)),
-                   ("cu_seqlens", np.int32, (max_reqs + 1,)), ("seq_lens", np.int32, (max_reqs,)),
-                   ("state_slots", np.int32, (max_reqs,)), ("logits_rows", np.int32, (max(max_rows, 1),)),
+                   ("cu_seqlens", np.int32, (max_reqs + spare + 1,)), ("seq_lens", np.int32, (max_reqs + spare,)),
+                   ("state_slots", np.int32, (max_reqs + spare,)), ("logits_rows", np.int32, (max(max_rows, 1),)),
                    ("feedback_src", np.int32, (max_tokens,))]
-        layout += [("block_table%d" % g, np.int32, (max_reqs, mb)) for g, mb in enumerate(max_blocks)]
+        layout += [("block_table%d" % g, np.int32, (max_reqs + spare, mb)) for g, mb in enumerate(max_blocks)]
         off = 0
         spans = {}
         for name, dt, shape in layout:
@@ -77,6 +78,7 @@ class StepBatch:
         self._buffers = native.BatchBuffers()
         bb = self._buffers
         bb.n_groups, bb.max_tokens, bb.max_reqs, bb.max_rows = len(max_blocks), max_tokens, max_reqs, max_rows
+        bb.spare = spare
         for name in ("input_ids", "positions", "cu_seqlens", "seq_lens", "state_slots", "logits_rows", "feedback_src"):
             setattr(bb, name, self.h[name].ctypes.data)
         for g, mb in enumerate(max_blocks):

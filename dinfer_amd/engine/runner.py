@@ -76,15 +76,16 @@ class ModelRunner:
         self.max_rows = options.max_logits_rows or options.max_num_seqs
         # decode rows may ride on top of the prompt budget (service.rs:206-210)
         self.max_tokens = options.max_num_batched_tokens + (options.max_num_seqs if options.decode_exempt_from_budget else 0)
+        # (one request more than a step may bring: a full batch is padded by a made-up request too)
         self.ctx = BuildContext(device, self.dtype, self.max_tokens, self.max_rows, self.page_size,
-                                options.max_num_seqs, max_seq_len=options.max_model_len)
+                                options.max_num_seqs + 1, max_seq_len=options.max_model_len)
         blaslt.configure(tuning=options.gemm_tuning, plan_file=options.gemm_plan_file)
         if self.dtype == torch.bfloat16:
             blaslt.require()
         model.bind(self.ctx)
         self._build_caches()
         self.batch = StepBatch(device, self.max_tokens, options.max_num_seqs, self.max_rows,
-                               [self.max_blocks_per_seq] * len(self.group_specs))
+                               [self.max_blocks_per_seq] * len(self.group_specs), spare=1)
         # batch-size buckets of the decode graphs: powers of two; between 16 and 64 every multiple of 8 (the few-row
         # products load the activations row by row: at the 8B sizes a step of 24 rows takes 5.5 ms in a graph of 24
         # and 5.7 ms in one of 32); beyond, the step between two powers as well; and the largest batch
@@ -360,13 +361,13 @@ class ModelRunner:
 
         The counts: tokens up to the next row count the matrix products round to anyway (16 at most where the
         step has no more: the few-row products take other forms there), requests up to the next
-        bucket of the decode graphs, one logits row a request (none if the step wants none), the longest portion up
+        bucket of the decode graphs (or, where that is the most, one beyond), one logits row a request the engine admits (none if the step wants none), the longest portion up
         to the next power of two, and which of the three ways single rows are served (all of them are, some, none)."""
         b, opt = self.batch, self.options
         T, B, R = b.num_tokens, b.num_reqs, b.num_rows
         if R > B or B > self._buckets[-1]:
             return None
-        later = [x for x in self._buckets if x >= B]
+        later = [x for x in self._buckets if x >= B] + [self._buckets[-1] + 1]      # (a full batch: the spare request)
         Bp = Tp = None
         for cand in later:
             need = T + (cand - B)               # a made-up request brings a token at least
@@ -376,13 +377,13 @@ class ModelRunner:
                 continue                        # made-up tokens need a made-up request
             Bp, Tp = cand, tp
             break
-        if Bp is None or Tp > self.max_tokens or (R and Bp > self.max_rows):
+        if Bp is None or Tp > self.max_tokens:
             return None
         last = Tp - T - (Bp - B - 1) if Bp > B else 0         # tokens of the last made-up request
         if last > opt.max_model_len:
             return None
         real_rows = R
-        b.pad(Bp, Tp, Bp if R else 0)
+        b.pad(Bp, Tp, min(Bp, self._buckets[-1]) if R else 0)
         q = b.max_q_len
         qp = min(Tp, max(16, 1 << (q - 1).bit_length()))
         route = 2 if b.num_singles == Bp else 1 if b.num_singles >= 4 else 0

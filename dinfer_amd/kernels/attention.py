@@ -40,7 +40,8 @@ class Workspace:
         # a step of single rows: the split-K kernel can take the per-head norms, the rotation and the cache write along
         self.decode_takes_post = self.split_k and ops.attn_decode_post_supports(head_dim)
         if self.split_k:
-            max_units = max(self.splits(n) * n for n in range(1, ctx.max_reqs + 1)) * kv_heads
+            # (a step of n requests may be cut as one of n - 1)
+            max_units = max(self.splits(max(n - 1, 1)) * n for n in range(1, ctx.max_reqs + 1)) * kv_heads
             elems = max_units * (heads // kv_heads) * (head_dim + 4)
             self.part = ctx.workspace.buffer("attn_partials", elems, dtype=torch.float32, rows=1)
 
@@ -72,8 +73,9 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k_cache, v_cache, batc
     # a few single rows beside long portions are not worth two more launches
     use_decode = singles == B or singles >= 4
     if use_decode:
+        # (where not all bring one row, at least one request is the flash kernel's)
         ops.attn_decode(qkv, out, ws.part, k_cache, v_cache, bt, None if singles == B else batch.cu_seqlens,
-                        batch.seq_lens, B, ws.splits(B), **geo)
+                        batch.seq_lens, B, ws.splits(B if singles == B else B - 1), **geo)
         if singles == B:
             return out
     return ops.attn_flash(qkv, out, k_cache, v_cache, bt, batch.cu_seqlens, batch.seq_lens, B, T, batch.max_q_len,

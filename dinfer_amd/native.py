@@ -19,7 +19,7 @@ class BatchBuffers(Structure):
                 ("input_ids", _P), ("positions", _P), ("cu_seqlens", _P), ("seq_lens", _P),
                 ("state_slots", _P), ("logits_rows", _P), ("feedback_src", _P),
                 ("slot_mapping", _P * MAX_GROUPS), ("block_table", _P * MAX_GROUPS),
-                ("max_blocks", _I * MAX_GROUPS)]
+                ("max_blocks", _I * MAX_GROUPS), ("spare", _I)]
 
 
 class BatchFacts(Structure):

@@ -122,6 +122,35 @@ def test_padding_a_step_with_portions_up_to_given_counts():
     assert (b.num_tokens, b.num_reqs, b.num_rows) == (32, 2, 0) and b.q_lens == [13, 19]
 
 
+def test_a_full_batch_is_padded_by_the_spare_request():
+    """A batch with room for a made-up request beyond its largest takes it in pad(), with the state slot behind the real
+    ones; what real requests may bring stays bounded as without."""
+    import pytest
+    s, _ = setup(1000)
+    for k in "xy":
+        s.cache.admit(k)
+        s.cache.allocate(k, 0, 5)
+    b = StepBatch(torch.device("cpu"), 32, 2, 2, [4], spare=1)
+    entries = [Entry("x", [1, 2, 3], 0, [2]), Entry("y", [4, 5], 0, [1])]
+    b.fill(entries, s.cache)
+    before = {k: v.copy() for k, v in b.h.items()}
+    with pytest.raises(ValueError, match="never cut"):
+        b.pad(4, 16, 2)
+    with pytest.raises(ValueError, match="never cut"):
+        b.pad(3, 16, 3)
+    b.pad(3, 16, 2)
+    assert (b.num_tokens, b.num_reqs, b.num_rows, b.max_q_len) == (16, 3, 2, 11) and b.q_lens == [3, 2, 11]
+    assert b.h["state_slots"][2] == 2 and b.h["seq_lens"][2] == 11 and b.h["logits_rows"][:2].tolist() == [2, 4]
+    assert (b.h["slot_mapping0"][5:16] == -1).all() and not b.h["block_table0"][2].any()
+    assert (b.h["block_table0"][:2] == before["block_table0"][:2]).all() and (b.h["input_ids"][:5] == [1, 2, 3, 4, 5]).all()
+    with pytest.raises(ValueError, match="places, the engine was built for 2"):
+        b.fill([Entry("x", [1, 2, 3], 0, [0, 1]), entries[1]], s.cache)
+    s.cache.admit("z")
+    s.cache.allocate("z", 0, 1)
+    with pytest.raises(ValueError, match="requests in one step, the engine was built for 2"):
+        b.fill(entries + [Entry("z", [1], 0, [])], s.cache)
+
+
 def test_limits_are_refused():
     import pytest
     s, b = setup(1000)
