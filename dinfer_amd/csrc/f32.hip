@@ -15,6 +15,8 @@
 //
 // Reference behaviour: crates/layers/src/nn.rs:16-76 (y = x . W^T), crates/kernels/cuda/gqa.cu:1037-1118 (plain paged
 // attention: causal inclusive, query head h reads kv head h / G).
+#include <algorithm>
+
 #include "common.cuh"
 
 using namespace dinfer;
@@ -30,42 +32,53 @@ __device__ __forceinline__ f32x4 mfma4(const f32x4& a, const f32x4& b, f32x4 c) 
 }
 
 // ---- products of many rows --------------------------------------------------------------------------------------
-// A workgroup of 2 x 2 waves computes BM rows x BN columns; steps of 64 k go through two LDS buffers, the 16-byte loads
-// of the two steps after it in flight while one is multiplied (one step ahead, a workgroup a CU waits for memory most of
-// the time: 1,024 columns of K = 3,072 at 500 rows 70 us). Rows of LDS are 68 floats apart: the eight lanes that a
-// 16-byte read serves at a time lie in different banks. Bound by the matrix cores and, where the columns give a CU one
-// workgroup, by a step's latency: 500 rows x 6,144
-// x 1,024 in 73 us (86 TFLOP/s where a large library product reaches 153; the vector-ALU kernel 165), x 1,024 x 3,072 in
-// 43 (452).
-constexpr int KB = 64, LROW = KB + 4;
+// A workgroup of KG groups of WM x WN waves computes BM rows x BN columns, a wave a tile of 32 x 32; the groups deal the
+// segments of k among themselves and their sums are added in the segments' order. Steps of 32 k go through two LDS buffers: the
+// loads of a step go out three steps before it, it is written to LDS one step before, and of the two halves of a step the second is
+// read while the first is multiplied and the next step's first while the second is, so that a wave meets neither LDS nor
+// the barrier between its MFMAs. Loads are buffer loads (one addition an address; past the last row's k they give zero): 64-bit
+// addresses cost the vector ALUs a tenth of the MFMAs' time. v_mfma_f32_32x32x2_f32 with k in the order of the few-row kernel's
+// 16x16x4 rounds to the same bits. Rows of LDS are 36 floats apart: the lanes that a 16-byte read serves at a time lie in
+// different banks. Bound by the matrix cores and, where a CU gets one workgroup, by a step's latency (before: steps
+// of 64 k through 16x16x4 tiles, fetched two ahead, LDS read behind each barrier, accumulators moved between register files
+// every step): 500 rows x 6,144 x 1,024 74 -> 59 us (107 TFLOP/s where a large library product reaches 153), x 4,096 x 1,024
+// 49 -> 40, x 1,024 x 2,048 31 -> 26, x 1,024 x 3,072 44 -> 36; 2,000 x 6,144 x 1,024 256 -> 196.
+constexpr int KB = 32, LROW = KB + 4;
 
-template <int BM, int BN>
-__global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__ A, int64_t lda, const float* __restrict__ W,
-                                                       int64_t ldw, float* __restrict__ C, int64_t ldc, int M, int N, int K) {
-  constexpr int MT = BM / 32, NT = BN / 32;                       // tiles of 16 a wave
-  constexpr int LA = BM * KB / 4 / 256, LW = BN * KB / 4 / 256;   // 16-byte loads a thread and step
-  __shared__ float As[2][BM * LROW];
-  __shared__ float Ws[2][BN * LROW];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+template <int WM, int WN, int KG>
+__global__ void __launch_bounds__(64 * WM * WN * KG) gemm_f32_kernel(const float* __restrict__ A, int64_t lda,
+                                                                     const float* __restrict__ W, int64_t ldw,
+                                                                     float* __restrict__ C, int64_t ldc, int M, int N, int K) {
+  constexpr int BM = 32 * WM, BN = 32 * WN, GT = 64 * WM * WN;             // threads of a group
+  constexpr int PASS = GT / (KB / 4);                                      // rows a pass of 16-byte loads
+  constexpr int LA = BM / PASS, LW = BN / PASS;                            // passes a step
+  constexpr int STEPS = SEG / KB;                                          // of a segment
+  __shared__ float As[KG][2][BM * LROW];
+  __shared__ float Ws[KG][2][BN * LROW];
+  __shared__ f32x4 part[KG][KG > 1 ? 4 * GT : 1];
+  const int tid = threadIdx.x % GT, group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / GT) : 0;
+  const int lane = tid & 63, wave = tid >> 6;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
-  const int lr = lane & 15, lg = lane >> 4;
-  const int row = threadIdx.x >> 4, piece = (threadIdx.x & 15) * 4;   // 16 rows of 16 pieces a pass
+  const int wm = wave / WN * 32, wn = wave % WN * 32;
+  const int lr = lane & 31, lh = lane >> 5;
+  const int row = tid / (KB / 4), piece = tid % (KB / 4) * 4;
 
-  const float* pa[LA];
-  const float* pw[LW];
+  // rows past the last one are the last one; what lies behind its k reads as zero
+  const int a_last = min(BM, M - m0) - 1, w_last = min(BN, N - n0) - 1;
+  const auto ab = __builtin_amdgcn_make_buffer_rsrc((void*)(A + (int64_t)m0 * lda), 0, (int)(((int64_t)a_last * lda + K) * 4), 0x00020000);
+  const auto wb = __builtin_amdgcn_make_buffer_rsrc((void*)(W + (int64_t)n0 * ldw), 0, (int)(((int64_t)w_last * ldw + K) * 4), 0x00020000);
+  uint32_t oa[LA], ow[LW];
 #pragma unroll
-  for (int e = 0; e < LA; ++e) pa[e] = A + (int64_t)min(m0 + row + 16 * e, M - 1) * lda;
+  for (int e = 0; e < LA; ++e) oa[e] = ((uint32_t)min(row + PASS * e, a_last) * (uint32_t)lda + piece) * 4;
 #pragma unroll
-  for (int e = 0; e < LW; ++e) pw[e] = W + (int64_t)min(n0 + row + 16 * e, N - 1) * ldw;
+  for (int e = 0; e < LW; ++e) ow[e] = ((uint32_t)min(row + PASS * e, w_last) * (uint32_t)ldw + piece) * 4;
 
   f32x4 ra[2][LA], rw[2][LW];
-  auto fetch = [&](int k0, f32x4(&fa)[LA], f32x4(&fw)[LW]) {   // pieces past K are read at K - 4 (and cleared below)
-    const int kk = min(k0 + piece, K - 4);
+  auto fetch = [&](int k0, f32x4(&fa)[LA], f32x4(&fw)[LW]) {
 #pragma unroll
-    for (int e = 0; e < LA; ++e) fa[e] = *(const f32x4*)(pa[e] + kk);
+    for (int e = 0; e < LA; ++e) fa[e] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ab, oa[e] + k0 * 4, 0, 0));
 #pragma unroll
-    for (int e = 0; e < LW; ++e) fw[e] = *(const f32x4*)(pw[e] + kk);
+    for (int e = 0; e < LW; ++e) fw[e] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(wb, ow[e] + k0 * 4, 0, 0));
   };
   auto put = [&](int b, int k0, f32x4(&fa)[LA], f32x4(&fw)[LW]) {
     if (k0 + KB > K) {
@@ -79,70 +92,90 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__
       }
     }
 #pragma unroll
-    for (int e = 0; e < LA; ++e) *(f32x4*)&As[b][(row + 16 * e) * LROW + piece] = fa[e];
+    for (int e = 0; e < LA; ++e) *(f32x4*)&As[group][b][(row + PASS * e) * LROW + piece] = fa[e];
 #pragma unroll
-    for (int e = 0; e < LW; ++e) *(f32x4*)&Ws[b][(row + 16 * e) * LROW + piece] = fw[e];
+    for (int e = 0; e < LW; ++e) *(f32x4*)&Ws[group][b][(row + PASS * e) * LROW + piece] = fw[e];
+  };
+  struct Half { f32x4 a[2], w[2]; };   // of a step: 16 k
+  auto read = [&](int b, int c, Half& f) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f.a[h] = *(const f32x4*)&As[group][b][(wm + lr) * LROW + 16 * c + 8 * h + 4 * lh];
+      f.w[h] = *(const f32x4*)&Ws[group][b][(wn + lr) * LROW + 16 * c + 8 * h + 4 * lh];
+    }
+  };
+  constexpr int OWN = 4 / KG;   // with groups, a thread sums up the four columns of every KG-th of the four row pieces
+  f32x16 acc;
+  f32x4 tot[OWN];
+#pragma unroll
+  for (auto& t : tot) t = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](const Half& f) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(f.w[h][q], f.a[h][q], acc, 0, 0, 0);
   };
 
-  f32x4 acc[MT][NT], tot[MT][NT];
+  const int segs = (K + SEG - 1) / SEG;
+  const int rounds = (segs + KG - 1) / KG;
+  Half f0, f1;
+  {
+    const int k0 = group * SEG;
+    fetch(k0, ra[0], rw[0]);
+    fetch(k0 + KB, ra[1], rw[1]);
+    put(0, k0, ra[0], rw[0]);
+    fetch(k0 + 2 * KB, ra[0], rw[0]);
+    lds_barrier();
+    read(0, 0, f0);
+  }
+  for (int r0 = 0; r0 < rounds; ++r0) {
+    const int k0 = (r0 * KG + group) * SEG, next = k0 + KG * SEG;   // this segment, the group's next
+    const int steps = KG > 1 ? STEPS : (min(K - r0 * SEG, SEG) + 2 * KB - 1) / (2 * KB) * 2;
+    auto at = [&](int s) { return s < steps ? k0 + s * KB : next + (s - steps) * KB; };
+    acc = f32x16{};
+#pragma unroll 1
+    for (int s0 = 0; s0 < steps; s0 += 2) {
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = tot[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int steps = (K + KB - 1) / KB;
-  fetch(0, ra[0], rw[0]);
-  fetch(KB, ra[1], rw[1]);
-  put(0, 0, ra[0], rw[0]);
-  __syncthreads();
-  for (int s0 = 0; s0 < steps; s0 += 2) {
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int s = s0 + b;
-      if (s >= steps) break;
-      fetch((s + 2) * KB, ra[b], rw[b]);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int c = 0; c < KB / 16; ++c) {
-        f32x4 fa[MT], fw[NT];
-#pragma unroll
-        for (int i = 0; i < MT; ++i) fa[i] = *(const f32x4*)&As[b][(wm + 16 * i + lr) * LROW + 16 * c + 4 * lg];
-#pragma unroll
-        for (int j = 0; j < NT; ++j) fw[j] = *(const f32x4*)&Ws[b][(wn + 16 * j + lr) * LROW + 16 * c + 4 * lg];
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[j][q], fa[i][q], acc[i][j], 0, 0, 0);
+      for (int b = 0; b < 2; ++b) {
+        read(b, 1, f1);
+        put(b ^ 1, at(s0 + b + 1), ra[b ^ 1], rw[b ^ 1]);
+        fetch(at(s0 + b + 3), ra[b ^ 1], rw[b ^ 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(f0);
+        __builtin_amdgcn_sched_barrier(0);
+        lds_barrier();
+        read(b ^ 1, 0, f0);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(f1);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      if (s + 1 == steps || (s + 1) % (SEG / KB) == 0) {   // a segment is whole
+    }
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+    for (int r = 0; r < 4; ++r) {
+      const f32x4 x = {acc[4 * r], acc[4 * r + 1], acc[4 * r + 2], acc[4 * r + 3]};
+      if (KG > 1) part[group][r * GT + tid] = x;
+      else tot[r] += x;
+    }
+    if (KG > 1) {   // (the parts are written again behind the barriers of the next segment)
+      lds_barrier();
+      const int have = min(KG, segs - r0 * KG);
 #pragma unroll
-          for (int j = 0; j < NT; ++j) {
-            tot[i][j] += acc[i][j];
-            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-          }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      if (s + 1 < steps) put(b ^ 1, (s + 1) * KB, ra[b ^ 1], rw[b ^ 1]);
-      __syncthreads();
+      for (int o = 0; o < OWN; ++o)
+        for (int g = 0; g < have; ++g) tot[o] += part[g][o * KG * GT + threadIdx.x];
     }
   }
-  // a lane holds four consecutive columns of one row
+  // a lane holds four consecutive columns of one row at a time
+  const bool wide = ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const int m = m0 + wm + 16 * i + lr;
+  for (int o = 0; o < OWN; ++o) {
+    const int m = m0 + wm + lr, n = n0 + wn + 8 * (o * KG + group) + 4 * lh;
+    if (m >= M) continue;
+    float* c = C + (int64_t)m * ldc + n;
+    if (wide && n + 3 < N) *(f32x4*)c = tot[o];
+    else
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int n = n0 + wn + 16 * j + 4 * lg;
-      if (m >= M) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n + r < N) C[(int64_t)m * ldc + n + r] = tot[i][j][r];
-    }
+      for (int y = 0; y < 4; ++y)
+        if (n + y < N) c[y] = tot[o][y];
   }
 }
 
@@ -150,7 +183,7 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__
 // A workgroup takes 16 rows of the weight and 16 * MT rows of A and streams both straight into registers: its waves deal
 // the segments of k among themselves (no barrier inside one), GROUP pieces of 16 k in flight at a time, and after each
 // round the parts are added in segment order. Bound by the weight's bytes, and by latency where the weight is small:
-// 151,936 x 1,024 in 124 us at one row (5.0 TB/s; the vector-ALU kernel 401), 1,024 x 3,072 in 12 us (365), at 64 rows 32.
+// 151,936 x 1,024 in 124 us at one row (5.0 TB/s; the vector-ALU kernel 401), 1,024 x 3,072 in 12 us (365), at 32 rows 21.
 template <int NW, int MT>
 __global__ void __launch_bounds__(NW * 64) gemm_f32_few_kernel(const float* __restrict__ A, int64_t lda, const float* __restrict__ W,
                                                                int64_t ldw, float* __restrict__ C, int64_t ldc, int M, int N,
@@ -229,11 +262,15 @@ __global__ void __launch_bounds__(NW * 64) gemm_f32_few_kernel(const float* __re
 
 template <int MT>
 void launch_few(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int M, int N, int K, hipStream_t stream) {
-  const dim3 grid((unsigned)((N + 15) / 16), (unsigned)((M + 16 * MT - 1) / (16 * MT)));
-  if (K > 4 * SEG)
-    gemm_f32_few_kernel<8, MT><<<grid, 512, 0, stream>>>(a, lda, w, ldw, c, ldc, M, N, K);
-  else
-    gemm_f32_few_kernel<4, MT><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, M, N, K);
+  constexpr int MOST = 65535 * 16 * MT;   // rows that a grid's y holds
+  for (int m0 = 0; m0 < M; m0 += std::min(MOST, M - m0)) {
+    const int rows = std::min(MOST, M - m0);
+    const dim3 grid((unsigned)((N + 15) / 16), (unsigned)((rows + 16 * MT - 1) / (16 * MT)));
+    if (K > 4 * SEG)
+      gemm_f32_few_kernel<8, MT><<<grid, 512, 0, stream>>>(a + m0 * lda, lda, w, ldw, c + m0 * ldc, ldc, rows, N, K);
+    else
+      gemm_f32_few_kernel<4, MT><<<grid, 256, 0, stream>>>(a + m0 * lda, lda, w, ldw, c + m0 * ldc, ldc, rows, N, K);
+  }
 }
 
 // ---- attention --------------------------------------------------------------------------------------------------
@@ -469,17 +506,33 @@ extern "C" int dinfer_gemm_f32(const void* A, int64_t lda, const void* W, int64_
   const float *a = (const float*)A, *w = (const float*)W;
   float* c = (float*)C;
   const int m = (int)M, n = (int)N, k = (int)K;
-  auto groups = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  const dim3 blocks[] = {dim3((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64)), dim3((unsigned)((N + 63) / 64), (unsigned)((M + 31) / 32))};
-  // Up to 64 rows, and wherever tiles of 32 x 64 would leave CUs without one, the kernel whose waves split k (100 rows x
-  // 1,024 x 3,072: 30 us against 70 through LDS in steps of 32); from there the largest tile that gives every CU two
-  // workgroups (500 x 4,096 x 1,024: 51 us), or one of half the rows (500 x 1,024 x 3,072: 43 us, 128 tiles of 64 x 64
-  // being half the chip).
+  // Up to 32 rows the kernel whose waves split k (17 rows x 1,024 x 2,048: 12 us, 17 in tiles; from 33 rows on it would need two
+  // more tiles of 16: 64 rows 22 against 18, and x 151,936 x 1,024 373 against 207), and where a tile's rows
+  // reach past 2^31 bytes. Otherwise the tile whose workgroups take a CU the least time: x workgroups a CU and 1,024 k cost
+  // it these us, measured at 64 to 2,000 rows of six weights (workgroups of 32 x 128 share a CU three at a time; alone, a group
+  // of waves waits for its latencies, which is what groups over k are for).
+  auto spans = [&](int64_t rows, int64_t ld) { return ((rows - 1) * ld + K + 8 * SEG) * 4 < 0x7fffffff; };
   if (M <= 16) launch_few<1>(a, lda, w, ldw, c, ldc, m, n, k, stream);
-  else if (M <= 32) launch_few<2>(a, lda, w, ldw, c, ldc, m, n, k, stream);
-  else if (M <= 64 || groups(32, 64) < 256) launch_few<4>(a, lda, w, ldw, c, ldc, m, n, k, stream);
-  else if (groups(64, 64) >= 512) gemm_f32_kernel<64, 64><<<blocks[0], 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
-  else gemm_f32_kernel<32, 64><<<blocks[1], 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+  else if (M <= 32 || !spans(std::min<int64_t>(M, 64), lda) || !spans(std::min<int64_t>(N, 128), ldw)) launch_few<2>(a, lda, w, ldw, c, ldc, m, n, k, stream);
+  else {
+    auto a_cu = [&](int64_t bm, int64_t bn) { return (double)((((M + bm - 1) / bm) * ((N + bn - 1) / bn) + 255) / 256); };
+    const double t64x64 = a_cu(64, 64), t32x64 = a_cu(32, 64);
+    const double cost[] = {31 * a_cu(64, 128), 17 * a_cu(32, 128) + 4, 19 * t64x64, t32x64 < 2 ? 12 : 10 * t32x64,
+                           t32x64 < 2 ? 10 : 11.5 * t32x64, 7 * a_cu(32, 32)};
+    const int best = (int)(std::min_element(cost, cost + 6) - cost);
+#define DINFER_GEMM_F32(WM, WN, KG)                                                                                      \
+  gemm_f32_kernel<WM, WN, KG><<<dim3((unsigned)((N + 32 * WN - 1) / (32 * WN)), (unsigned)((M + 32 * WM - 1) / (32 * WM))), \
+                                64 * WM * WN * KG, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k)
+    switch ((M + 31) / 32 > 65535 ? 0 : best) {   // (the grid's y)
+      case 0: DINFER_GEMM_F32(2, 4, 1); break;
+      case 1: DINFER_GEMM_F32(1, 4, 1); break;
+      case 2: DINFER_GEMM_F32(2, 2, 2); break;
+      case 3: DINFER_GEMM_F32(1, 2, 2); break;
+      case 4: DINFER_GEMM_F32(1, 2, 4); break;
+      default: DINFER_GEMM_F32(1, 1, 4);
+    }
+#undef DINFER_GEMM_F32
+  }
   return launch_status();
 }
 

@@ -40,6 +40,21 @@ def test_gemm_f32(M, N, K):
             assert torch.equal(part, out[M - m:M]), f"{m} rows differ"
 
 
+# sizes that lead to each of the six tiles, none whole; K: less than a step, a segment and a piece, an odd number of segments
+@pytest.mark.parametrize("K", [20, 260, 1284])
+@pytest.mark.parametrize("M,N", [(250, 6150), (193, 9000), (130, 4090), (300, 4090), (1001, 331), (33, 1027)])
+def test_gemm_f32_tiles(M, N, K):
+    a, w = product(M, N, K, seed=M + N + K, lda=K + 8)
+    out = torch.full((M + 1, N + 2), 7.0, device=DEV)
+    ops().gemm_f32(a, w, out[:, :N], M)
+    bound = 16 * 2.0 ** -24 * K ** 0.5 * max(1.0, (min(K, 256) / 4 + K / 256) ** 0.5)   # as above
+    assert (out[:M, :N].double() - a.double() @ w.double().T).abs().max().item() <= bound
+    assert (out[M] == 7.0).all() and (out[:, N:] == 7.0).all()
+    part = torch.empty(16, N, device=DEV)
+    ops().gemm_f32(a[M - 16:].contiguous(), w, part, 16)
+    assert torch.equal(part, out[M - 16:M, :N])
+
+
 def test_gemm_f32_strides_and_what_it_leaves_to_the_plain_kernel():
     a, w = product(40, 48, 64, seed=5, lda=100)
     assert ops().gemm_f32_supports(a, w)
