@@ -162,12 +162,18 @@ constexpr int64_t STREAM_FROM_BYTES_FEW = 170 * 1000 * 1000;  // for one or two 
 // new key and stores it and the new value into their pages before it reads its last block.
 // (The pages are written through post.k_cache / v_cache and read through kc / vc: no __restrict__ on those.)
 // LATE (POST only): the new key is dealt with inside the walk instead of before it (see there).
+// OWN (JOIN, fewer requests than LATE is for): the row's own key and value are a part of their own, the last, of one more wave.
+// With POST that wave norms and rotates q and the new key in registers, scores the one with the other and stores key and value, while
+// the others walk the keys before it, so that nobody waits for a store to come back (one request of 250 keys, 16 heads on 8
+// of 128: 8.5 -> 7.7 us, in a step of 28 layers 1,019 -> 985; 8 requests 9.3 -> 8.5, 28 of 2,048 keys, 40 heads,
+// 45.1 -> 43.0; where the parts are workgroups of their own it loses 0.4 us and more from 2,048 keys on). Without POST, and for
+// a row that is written nowhere, the wave walks that key: the same parts, the same bits.
 // stream_from: from this many bytes of keys and values in a step on (the request's own visible keys times the number
 // of requests: a wave knows no more) they are read with non-temporal loads.
 template <int DT, bool P2, bool LATE, bool JOIN = false, bool POST = false>
 // (These launches aim at about one wave a SIMD, and JOIN runs where a CU holds 4 to 8 of its waves: registers are no
 // limit; POST holds a head, gains and angles at once in its prologue.)
-__global__ void __launch_bounds__(JOIN ? 64 * JOIN_SPLITS : 64)
+__global__ void __launch_bounds__(JOIN ? 64 * (JOIN_SPLITS + 1) : 64)
 __attribute__((amdgpu_waves_per_eu(2, 8)))
 attn_decode_kernel(
     const bf16* __restrict__ q, int64_t ld_q, float* __restrict__ part, const bf16* kc, const bf16* vc,
@@ -176,6 +182,7 @@ attn_decode_kernel(
     int64_t stream_from, bf16* __restrict__ out = nullptr, int64_t ld_out = 0, DecodePost post = DecodePost{}) {
   constexpr int D = DT * 16;
   constexpr int KS = (DT + 1) / 2;
+  constexpr bool OWN = JOIN && !LATE;
   static_assert(!POST || DT % 4 == 0, "the fused norm and rotation keep both elements of a pair in one lane");
   const int sp = JOIN ? (int)(threadIdx.x >> 6) : (int)blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
   const int G = H / Hkv;
@@ -194,7 +201,64 @@ attn_decode_kernel(
   bool writer = false;
   int w_pos = 0;
   int64_t w_slot = -1;
-  if constexpr (POST) {
+  const bool own = OWN && (int)blockDim.x > 64 * splits, own_part = own && sp == splits;   // (wave-uniform)
+  bool held = false;   // the own part needs no walk
+  float own_l = 0.f;
+  if constexpr (OWN && POST) {
+    if (own_part) {
+      const bf16* vn = post.v_new + (int64_t)row * ld_q + (int64_t)hk * D;
+      HeadPost<DT> qh, kh;
+      bf16x4 v4[DT];
+      bf16x8 vv, kr[KS];
+      qh.load(qp, i16 < G);
+      kh.load(post.k_new + (int64_t)row * ld_q + (int64_t)hk * D, i16 == 0);
+      if (post.wq) qh.load_gains(post.wq), kh.load_gains(post.wk);
+      const int pos_row = post.cos_sin ? post.pos[row] : 0;
+      const int64_t slot = post.slots ? post.slots[row] : -1;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) v4[d] = *(const bf16x4*)(vn + d * 16 + 4 * g4);
+      if (lane < D / 8) vv = *(const bf16x8*)(vn + lane * 8);
+      typename HeadPost<DT>::Angles ang;
+      if (post.cos_sin) ang.load(post.cos_sin + (int64_t)pos_row * D);
+      kh.finish(ang, post.wk != nullptr, post.eps, post.w_offset, post.cos_sin != nullptr, kr);
+      qh.finish(ang, post.wq != nullptr, post.eps, post.w_offset, post.cos_sin != nullptr, qf[0]);
+      held = slot >= 0;
+      if (!held) {   // nothing is written: the pages hold the key
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qf[0][ks] = i16 < G ? qf[0][ks] : zero8();
+        seq = seq_lens[b];
+        k_hi = max(seq, 0);
+        k_lo = max(seq - 1, 0);
+        tl.init(kc, vc, bt, (int)max_blocks, hk, Hkv, ps, k_lo, k_hi, scale_log2e);
+      } else {
+        const int64_t blk = slot / ps;
+        const int off = (int)(slot - blk * ps);
+        const int64_t head = (blk * Hkv + hk) * (int64_t)ps * D;
+        if (i16 == 0) {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks)
+            *(bf16x8*)(post.k_cache + head + k_page_offset(off, ks * 32 + g4 * 8, ps)) = kr[ks];
+        }
+        if (lane < D / 8) {  // V pages are transposed: the 8 dims of a piece go to 8 rows of keys
+          bf16* vd = post.v_cache + head + (int64_t)(lane * 8) * ps + off;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) vd[(int64_t)e * ps] = vv[e];
+        }
+        f32x4 x = {0.f, 0.f, 0.f, 0.f};   // row 0 is the key: lane group 0 gets its scores
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) x = mfma16(i16 == 0 ? kr[ks] : zero8(), i16 < G ? qf[0][ks] : zero8(), x);
+        // (as a walk of this one key leaves it)
+        tl.m[0] = __shfl(x[0], i16, 64);
+        own_l = exp2_raw(fmaf(tl.m[0], scale_log2e, -(tl.m[0] * scale_log2e)));
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) tl.o[0][d][e] = (float)v4[d][e] * (float)(bf16)own_l;
+      }
+    }
+  }
+  if (POST && own_part) {
+  } else if constexpr (POST) {
     // in the order of what is known when: the head, its gains, the row's position and slot at once; ...
     HeadPost<DT> qh;
     qh.load(qp, i16 < G);
@@ -204,12 +268,13 @@ attn_decode_kernel(
     seq = seq_lens[b];
     split_range(seq, window, splits, sp, &k_lo, &k_hi, &kps);
     if (!JOIN && k_lo >= k_hi) return;
+    if (own) k_hi = min(k_hi, seq - 1);
     // ... with the length the block table, with the position the angles; the part that ends with the row's own
     // position (wave-uniform) also takes the new key and value
     tl.init(kc, vc, bt, (int)max_blocks, hk, Hkv, ps, k_lo, k_hi, scale_log2e);
     typename HeadPost<DT>::Angles ang;
     if (post.cos_sin) ang.load(post.cos_sin + (int64_t)pos_row * D);
-    writer = slot >= 0 && k_lo < k_hi && k_hi == seq;
+    writer = !own && slot >= 0 && k_lo < k_hi && k_hi == seq;
     qh.finish(ang, post.wq != nullptr, post.eps, post.w_offset, post.cos_sin != nullptr, qf[0]);
     if (i16 >= G) {  // columns beyond the group stay zero whatever the norm made of nothing
 #pragma unroll
@@ -247,6 +312,12 @@ attn_decode_kernel(
     // an empty part writes nothing; the merge kernel skips it by the same rule. (JOIN: it walks no block and
     // leaves m = -inf, which weighs nothing; its wave must reach the barrier below.)
     if (!JOIN && k_lo >= k_hi) return;
+    if (own_part) {
+      k_hi = max(seq, 0);
+      k_lo = max(seq - 1, 0);
+    } else if (own) {
+      k_hi = min(k_hi, seq - 1);
+    }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int d = ks * 32 + g4 * 8;
@@ -270,7 +341,9 @@ attn_decode_kernel(
     else
       tl.template walk<false, false>(qf, col_lo, col_hi, partial, hook);
   };
-  if constexpr (POST && !LATE) {
+  if constexpr (OWN) {
+    if (!held) walk([](int, bool) {});
+  } else if constexpr (POST && !LATE) {
     // the key was stored in the prologue; the fence lets the wave's own loads of its last block see it
     walk([&](int, bool last) {
       if (writer && last) __threadfence_block();
@@ -325,13 +398,15 @@ attn_decode_kernel(
   } else {
     walk([](int, bool) {});
   }
-  const float lt = tl.sum_l(0);
+  const float lt = held ? own_l : tl.sum_l(0);
   if constexpr (JOIN) {
-    __shared__ __attribute__((aligned(16))) float joined[JOIN_SPLITS][16][D + 4];
+    const int parts = splits + (own ? 1 : 0);
+    __shared__ __attribute__((aligned(16))) float joined[JOIN_SPLITS + 1][16][D + 4];
     if (i16 < G) {
       float* pp = &joined[sp][i16][0];
       if (g4 == 0) {
-        pp[0] = tl.m[0] * scale_log2e;  // -inf for an empty part
+        // -inf for an empty part; a score of the own key that is no number may not pass for one
+        pp[0] = own_part && lt != lt && tl.m[0] != INFINITY ? 0.f : tl.m[0] * scale_log2e;
         pp[1] = lt;
       }
 #pragma unroll
@@ -342,9 +417,9 @@ attn_decode_kernel(
     for (int idx = threadIdx.x; idx < G * D; idx += blockDim.x) {
       const int i = idx / D, d = idx - i * D;
       float M = -INFINITY;
-      for (int s = 0; s < splits; ++s) M = fmaxf(M, joined[s][i][0]);
+      for (int s = 0; s < parts; ++s) M = fmaxf(M, joined[s][i][0]);
       float L = 0.f, acc = 0.f;
-      for (int s = 0; s < splits; ++s) {
+      for (int s = 0; s < parts; ++s) {
         const float m = joined[s][i][0];
         const float a = m == -INFINITY ? 0.f : exp2f(m - M);
         if (a > 0.f) {
@@ -530,7 +605,7 @@ int launch_decode(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, float*
     const double per_cu = (double)Hkv * (cu && num_reqs > 1 ? num_reqs - 1 : num_reqs) / compute_units();
     if (splits <= JOIN_SPLITS && (per_cu <= 1. || ceil(per_cu) <= 1.15 * per_cu)) {
       auto kernel = p2 ? decode_kernel_for<DT, true, true, POST>(late) : decode_kernel_for<DT, false, true, POST>(late);
-      kernel<<<dim3(1, (unsigned)Hkv, (unsigned)num_reqs), 64 * splits, 0, stream>>>(
+      kernel<<<dim3(1, (unsigned)Hkv, (unsigned)num_reqs), 64 * (splits + (late ? 0 : 1)), 0, stream>>>(
           q, ld_q, part, kc, vc, bt, max_blocks, cu, sl, splits, scale * LOG2E, window, H, Hkv, ps, stream_from, out, ld_out,
           post);
       return launch_status();

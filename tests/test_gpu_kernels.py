@@ -275,6 +275,29 @@ def test_attention_decode_takes_norm_rotation_and_cache_write_along(H, Hkv, D, p
         decode_post_case(H, Hkv, D, page, window, gains, hist, splits)
 
 
+@pytest.mark.parametrize("bad", ["key", "value"])
+@pytest.mark.parametrize("splits", [1, 4])
+def test_attention_decode_own_key_that_is_no_number(bad, splits):
+    """Where parts meet in a workgroup the row's own key is a part of its own: what is no number in it reaches the row's output and no
+    other's, and a row of one key is that key's value."""
+    H, Hkv, D, page, hist = 16, 8, 128, 16, [40, 0, 200]
+    _, kc, vc, m, _ = paged_case(torch.bfloat16, H, Hkv, D, page, hist, [1] * 3, seed=12)
+    raw = torch.randn(3, (H + 2 * Hkv) * D, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
+    raw[2, H * D if bad == "key" else (H + Hkv) * D] = float("nan")      # the first number of kv head 0
+    slots = torch.tensor([int(m["bt"][b, h // page]) * page + h % page for b, h in enumerate(hist)], device=DEV)
+    out = torch.zeros(3, H * D, device=DEV, dtype=torch.bfloat16)
+    part = torch.empty(3 * H * splits * (D + 4), device=DEV)
+    ops().attn_decode_post(raw.to(DEV), out, part, kc, vc, m["bt"], m["sl"], 3, splits, scale=D ** -0.5, window=0, heads=H,
+                           kv_heads=Hkv, head_dim=D, page_size=page, q_off=0, k_off=H * D, v_off=(H + Hkv) * D, q_gain=None,
+                           k_gain=None, eps=1e-5, gain_offset=0.0, positions=torch.tensor(hist, dtype=torch.int32, device=DEV),
+                           cos_sin=None, slot_mapping=slots)
+    out = out.cpu().view(3, H, D)
+    assert torch.equal(out[1], raw[1, (H + Hkv) * D:].view(Hkv, D).repeat_interleave(H // Hkv, 0))
+    assert out[0].isfinite().all() and out[2, H // Hkv:].isfinite().all()
+    group = out[2, :H // Hkv]
+    assert group.isnan().all() if bad == "key" else group[:, 0].isnan().all() and group[:, 1:].isfinite().all()
+
+
 def decode_post_case(H, Hkv, D, page, window, gains, hist, splits, device="cpu", spike=None, sharp=1.0):
     """One launch of the decode kernel that norms, rotates and writes the cache, against the plain functions and, bit
     for bit, against the two kernels it stands for. Request 1 writes nothing (slot -1)."""
