@@ -506,14 +506,15 @@ extern "C" int dinfer_gemm_f32(const void* A, int64_t lda, const void* W, int64_
   const float *a = (const float*)A, *w = (const float*)W;
   float* c = (float*)C;
   const int m = (int)M, n = (int)N, k = (int)K;
-  // Up to 32 rows the kernel whose waves split k (17 rows x 1,024 x 2,048: 12 us, 17 in tiles; from 33 rows on it would need two
-  // more tiles of 16: 64 rows 22 against 18, and x 151,936 x 1,024 373 against 207), and where a tile's rows
-  // reach past 2^31 bytes. Otherwise the tile whose workgroups take a CU the least time: x workgroups a CU and 1,024 k cost
-  // it these us, measured at 64 to 2,000 rows of six weights (workgroups of 32 x 128 share a CU three at a time; alone, a group
-  // of waves waits for its latencies, which is what groups over k are for).
+  // Up to 16 rows, and up to 32 of a weight that gives its workgroups of 16 columns no second round of the CUs, the kernel
+  // whose waves split k (17 and 32 rows x 1,024 x 2,048: 12 and 15 us, 17 and 18 in tiles; x 6,144 x 1,024 15 and 17 against 13
+  // and 14; from 33 rows on it would need two more tiles of 16: 64 rows x 1,024 x 2,048 22 against 18, x 151,936 x 1,024
+  // 373 against 207), and where a tile's rows reach past 2^31 bytes. Otherwise the tile whose workgroups take a CU the least
+  // time: x workgroups a CU and 1,024 k cost it these us, measured at 64 to 2,000 rows of six weights (workgroups of 32 x 128
+  // share a CU three at a time; alone, a group of waves waits for its latencies, which is what groups over k are for).
   auto spans = [&](int64_t rows, int64_t ld) { return ((rows - 1) * ld + K + 8 * SEG) * 4 < 0x7fffffff; };
   if (M <= 16) launch_few<1>(a, lda, w, ldw, c, ldc, m, n, k, stream);
-  else if (M <= 32 || !spans(std::min<int64_t>(M, 64), lda) || !spans(std::min<int64_t>(N, 128), ldw)) launch_few<2>(a, lda, w, ldw, c, ldc, m, n, k, stream);
+  else if ((M <= 32 && N <= 4096) || !spans(std::min<int64_t>(M, 64), lda) || !spans(std::min<int64_t>(N, 128), ldw)) launch_few<2>(a, lda, w, ldw, c, ldc, m, n, k, stream);
   else {
     auto a_cu = [&](int64_t bm, int64_t bn) { return (double)((((M + bm - 1) / bm) * ((N + bn - 1) / bn) + 255) / 256); };
     const double t64x64 = a_cu(64, 64), t32x64 = a_cu(32, 64);

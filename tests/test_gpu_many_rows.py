@@ -115,3 +115,30 @@ def test_router_logits_of_many_tokens(tokens, experts, width, gate):
         err.append(((z.double() - want[:n])[keep].norm() / want[:n][keep].norm()).item())
         assert torch.equal(idx.view(n, top)[keep, 0].long(), z[keep][:, :experts].argmax(1))
     assert err[0] <= 1.1 * err[1] and err[0] < 2e-7
+
+
+@pytest.mark.parametrize("width", [4, 1020, 1024, 1025, 1028, 4100, 5120, 5121])
+def test_float_rows(width):
+    """The norm of float rows at the edges of the widths that registers hold; their gated activation in 16-byte pieces beside
+    rows that do not begin at 16 bytes (the kernel of single numbers), bit for bit."""
+    g = torch.Generator().manual_seed(width)
+    T, eps = 5, 1e-6
+    x, res, w = torch.randn(T, width, generator=g).cuda(), torch.randn(T, width, generator=g).cuda(), torch.randn(width, generator=g).cuda()
+    x[3, width - 1] = float("inf")
+    gu = torch.randn(T, 2 * width, generator=g).cuda()
+    norms, acts = [], []
+    for at in (0, 1):
+        a, r, z = (torch.zeros(T, n + 4, device="cuda") for n in (width, width, 2 * width))
+        a[:, at:at + width], r[:, at:at + width], z[:, at:at + 2 * width] = x, res, gu
+        o, y = torch.full((T + 1, width), 7.0, device="cuda"), torch.full((T + 1, width), 7.0, device="cuda")
+        ops().rmsnorm(a[:, at:at + width], w, o, eps, T, residual=r[:, at:at + width], weight_offset=1.0)
+        ops().gated_act(z[:, at:at + 2 * width], y, T, "silu")
+        assert torch.equal(r[:, at:at + width], x + res) and not r[:, at + width:].any() and (o[T] == 7.0).all() and (y[T] == 7.0).all()
+        norms.append(o[:T]), acts.append(y[:T])
+    assert torch.equal(*acts)
+    keep = [0, 1, 2, 4]
+    s = (x + res).double()[keep]
+    want = s * torch.rsqrt((s * s).mean(-1, keepdim=True) + eps) * (w.double() + 1)
+    for o in norms:   # a sum of squares of up to 20 terms a thread, 8 levels of tree, a root, three products: 2^-24 each
+        assert ((o[keep].double() - want).abs() <= 32 * 2.0 ** -24 * want.abs()).all()
+        assert not torch.isfinite(o[3, -1])
