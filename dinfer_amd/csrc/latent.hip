@@ -24,6 +24,8 @@
 //                  between the two products, and a lane keeps the softmax state of one row. With `splits` > 1 the
 //                  keys of a request are cut into that many parts on the device (steps of single rows) and a merge
 //                  kernel joins them; the launch shape follows the step's counts alone.
+#include <algorithm>
+
 #include "common.cuh"
 
 #include <type_traits>
@@ -643,32 +645,41 @@ __global__ void __launch_bounds__(256) latent_attn_lds_kernel(
 // waves owns 64 rows (token, head) of a request and walks its keys in blocks of 32, each brought into LDS once for all of
 // them and one block ahead (global loads that write LDS: no register between; two buffers, objects of their own so that a
 // read of one does not wait for the loads into the other).
-//   scores  waves 2 r and 2 r + 1 take row tile r, half of the contraction each (their queries stay in registers, 40 a lane);
-//           the halves meet through LDS (16 KB a block), both waves then hold the tile's scores
+//   scores  waves r and r + 4 take row tile r, half of the contraction each (their queries stay in registers, 40 a lane);
+//           the halves meet through LDS (16 KB a block), and each of the two takes the softmax of eight of the rows (of
+//           all sixteen, both the same, 389 us where this takes 371)
 //   values  the weights pass through LDS (4 KB), and wave w takes an eighth of the latent entries for all 64 rows: a fragment
 //           of the values read from LDS feeds four MFMAs, where a wave that keeps to its rows reads all of them for one each
 // LDS rows are unpadded, their 16-byte pieces exchanged by the row's bits 1..3 (keys) or 2..3 (values), which the loads do by
 // asking for another piece: no bank is met twice. A block moves 310 KB through LDS, 2,400 cycles, beside 1,090 of MFMAs a
-// SIMD: LDS bounds it. 16 heads of 512 + 64: 16 portions of 256 tokens behind 1,000 each 1,099 -> 435 us (370
-// TFLOP/s), a prompt of 2,048 493 -> 185, 2,048 tokens behind 6,144 3,076 -> 1,070 (a wave that keeps its 16 rows, one workgroup
-// of four waves a CU, keys, values and queries in padded rows of LDS: 87 KB read a wave and block, and two more barriers).
+// SIMD and some 170 other instructions a wave; it takes 5,700, for its three parts wait for each other (the next block's scores
+// beside the values, with a barrier less, 371 us for 364; 128 rows a workgroup do not fit the registers). 16 heads of
+// 512 + 64: 16 portions of 256 tokens behind 1,000 each 403 -> 352 us (450 TFLOP/s), a prompt of 2,048 177 -> 155, 2,048 tokens
+// behind 6,144 1,060 -> 924 (a wave that keeps its 16 rows, one workgroup of four waves a CU, keys, values and queries in
+// padded rows of LDS: 1,099, 493 and 3,076).
 template <int DT, int KPS>   // R = 64 DT; pieces of a key row's place in LDS, at least (R + dr) / 8
 __global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
     const bf16* __restrict__ qa, int64_t ld_qa, bf16* __restrict__ out, int64_t ld_out, const bf16* __restrict__ cache,
     const bf16* __restrict__ cache_t, const int32_t* __restrict__ block_table, int64_t max_blocks,
     const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ seq_lens, int num_reqs, float scale_log2,
-    int window, int H, int dr, int page_shift) {
+    int window, int H, int dr, int page_shift, int groups, int run) {
   constexpr int R = 64 * DT, NC = KPS / 8, TW = DT / 2;   // a wave's chunks of the contraction, its tiles of the latent
   __shared__ __attribute__((aligned(16))) bf16 K0[32 * KPS * 8], K1[32 * KPS * 8];   // [32][8 KPS]
   __shared__ __attribute__((aligned(16))) bf16 V0[R * 32], V1[R * 32];               // [R][32]
   __shared__ __attribute__((aligned(16))) bf16x8 Ps[4][64];      // [row tile][lane]
   __shared__ __attribute__((aligned(16))) f32x4 Ss[8][2][64];    // [wave][key tile][lane]
   __shared__ float alphas[64];
-  __shared__ int moved[4];
+  __shared__ int moved[8];
   const int DK = R + dr, kp = DK >> 3, chunks = DK >> 5;
-  // which request and which of its groups of 64 rows; the last groups of a prompt walk the most keys and start first
-  int grp = (int)gridDim.x - 1 - (int)blockIdx.x, b = -1, q_len = 0;
+  // Which request and which of its groups of 64 rows; the last groups of a prompt walk the most keys and start first. An XCD (the
+  // workgroups of one id modulo 8) takes runs of four neighbours, which read the same keys at about the same time, from its
+  // own L2; every second round of runs goes the other way, so that no XCD has the longer ones throughout (one prompt of 2,048
+  // 161 -> 157 us; runs of 32 take 16 equal portions from 366 to 342, but two prompts of 1,500 from 192 to 248: too uneven).
+  int b = -1, q_len = 0, grp;
   {
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, round = slot / run;
+    grp = groups - 1 - ((round * 8 + (round & 1 ? 7 - xcd : xcd)) * run + slot % run);
+    if (grp < 0) return;
     const int ln = threadIdx.x & 63;
     for (int b0 = 0; b0 < num_reqs && b < 0; b0 += 64) {
       const int mine = b0 + ln < num_reqs ? cu_seqlens[b0 + ln + 1] - cu_seqlens[b0 + ln] : 0;
@@ -694,27 +705,28 @@ __global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
   grp = __builtin_amdgcn_readfirstlane(grp);
   q_len = __builtin_amdgcn_readfirstlane(q_len);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
-  const int rt = wave >> 1, half = wave & 1;     // this wave's row tile and half of the scores' contraction
+  // this wave's row tile, and which half of the contraction it scores (waves 4 apart share a SIMD)
+  const int rt = wave & 3, half = wave >> 2;
   const int t0 = cu_seqlens[b], start = seq_lens[b] - q_len, all_rows = q_len * H;
   const int row0 = grp * 64 + rt * 16;
   const int nrows = min(all_rows - row0, 16);    // <= 0: none
-  const bool rv = lr < nrows;
-  const int tok = rv ? (row0 + lr) / H : 0, head = rv ? (row0 + lr) % H : 0;
-  const int p = rv ? start + tok : -1;
+  // of the tile's softmax the wave has rows 8 half + lane % 8; a lane's four keys are 8 sg + 4 st + i of a block
+  const int srow = 8 * half + (lane & 7), sg = (lane >> 3) & 3, st = lane >> 5;
+  const int p = srow < nrows ? start + (row0 + srow) / H : -1;
   const int my_last = nrows > 0 ? start + (row0 + nrows - 1) / H : -1, my_first = start + row0 / H;
   const int lowest = window > 0 ? max(p - window + 1, 0) : 0;
   // the workgroup's keys
   const int p_first = start + grp * 64 / H, p_last = start + (min(all_rows, grp * 64 + 64) - 1) / H;
   const int first = window > 0 ? max(p_first - window + 1, 0) : 0;
-  int last[4];   // the last key that row tile r sees (tiles without rows: as the others)
-#pragma unroll
-  for (int r = 0; r < 4; ++r) last[r] = min(start + (grp * 64 + 16 * r + 15) / H, p_last);
+  // the last key that row tile r sees (tiles without rows: as the others)
+  auto last = [&](int r) { return min(start + (grp * 64 + 16 * r + 15) / H, p_last); };
   const int page = 1 << page_shift, pmask = page - 1, page_lo = first >> page_shift, page_hi = p_last >> page_shift;
   const int32_t* bt = block_table + (int64_t)b * max_blocks;
 
   bf16x8 qf[NC];
   {
-    const bf16* qrow = qa + (int64_t)(t0 + tok) * ld_qa + (int64_t)head * DK + 8 * g;
+    const int r = min(row0 + lr, all_rows - 1);   // (rows beyond: computed, not stored)
+    const bf16* qrow = qa + (int64_t)(t0 + r / H) * ld_qa + (int64_t)(r % H) * DK + 8 * g;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int ch = half * NC + c;   // (chunks past the row's end: zeros of the query meet the row's last chunk)
@@ -731,25 +743,22 @@ __global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
     for (int r = 0; r < 4; ++r) o[t][r] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
 
-  // A block's way into LDS: an instruction brings 64 pieces to 1 KB in a row. Where a lane's piece lies inside its page, and
-  // in which of the block's pages (blocks begin at multiples of 32: several where pages are shorter, else one and an offset
-  // that all lanes share), is the same for every block and worked out here: done a block at a time it was 400 instructions a
-  // wave, as long as all the rest.
+  // A block's way into LDS: an instruction brings 64 pieces to 1 KB in a row. Blocks begin at multiples of 32, so they hold several
+  // pages where those are shorter, else one and an offset that all lanes share. The rows of a page of keys end where an
+  // instruction ends (8 KPS is a multiple of 64), so their page is the instruction's; of the values a lane has the same eight
+  // keys in every instruction, so their page is the lane's. What depends on the lane inside a page is worked out here (all of it
+  // a block at a time was 400 instructions a wave, as long as all the rest; with a choice of page a lane and instruction 90).
+  static_assert(8 * KPS % 64 == 0);
   constexpr int KU = (KPS / 2 + 7) / 8, VU = R / 128;
-  int k_off[KU], v_off[VU], k_page = 0, v_page = 0;   // bytes inside the page; two bits an instruction: which page
   const int in_block = min(page, 32) - 1;
+  uint32_t k_off[KU];   // bytes inside the page
 #pragma unroll
   for (int u = 0; u < KU; ++u) {
     const int q = min(u * 8 + wave, KPS / 2 - 1) * 64 + lane, row = q / KPS, slot = q - row * KPS;
     k_off[u] = ((row & in_block) * DK + min((slot & ~7) | ((slot ^ (row >> 1)) & 7), kp - 1) * 8) * 2;
-    k_page |= (page < 32 ? row >> page_shift : 0) << (2 * u);
   }
-#pragma unroll
-  for (int u = 0; u < VU; ++u) {
-    const int q = (u * 8 + wave) * 64 + lane, d = q >> 2, key = 8 * ((q ^ (d >> 2)) & 3);
-    v_off[u] = ((d << page_shift) + (key & in_block)) * 2;
-    v_page |= (page < 32 ? key >> page_shift : 0) << (2 * u);
-  }
+  const int v_key = 8 * ((lane ^ (lane >> 4)) & 3), v_page = page < 32 ? v_key >> page_shift : 0;
+  const uint32_t v_off = (((wave * 16 + (lane >> 2)) << page_shift) + (v_key & in_block)) * 2;
   // (a page beyond the request's keys is replaced by its last one, whose rows exist: what they hold is masked)
   auto load = [&](int kb, bf16* Ks, bf16* Vs) {
     uint32_t pid[4];
@@ -762,15 +771,18 @@ __global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
     };
     const int kbm = kb & pmask;   // (0 where pages are no longer than a block)
     const char* kbase = (const char*)cache + (int64_t)kbm * DK * 2;
-    const char* vbase = (const char*)cache_t + kbm * 2;
+    const char* vrow = (const char*)cache_t + kbm * 2 + ((uint64_t)of(v_page) * (uint32_t)(R * 2 << page_shift) + v_off);
 #pragma unroll
     for (int u = 0; u < KU; ++u)
-      if (u * 8 + wave < KPS / 2)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kbase + ((uint64_t)of((k_page >> (2 * u)) & 3) * (uint32_t)(DK * 2 << page_shift) + (uint32_t)k_off[u])),
+      if (u * 8 + wave < KPS / 2) {
+        const int first_row = (u * 8 + wave) * 64 / KPS;   // (scalar)
+        const char* at = kbase + (uint64_t)of(page < 32 ? first_row >> page_shift : 0) * (uint32_t)(DK * 2 << page_shift);
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(at + k_off[u]),
                                          (__attribute__((address_space(3))) void*)(Ks + (u * 8 + wave) * 512), 16, 0, 0);
+      }
 #pragma unroll
     for (int u = 0; u < VU; ++u)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vbase + ((uint64_t)of((v_page >> (2 * u)) & 3) * (uint32_t)(R * 2 << page_shift) + (uint32_t)v_off[u])),
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vrow + ((uint64_t)u << (page_shift + 8))),
                                        (__attribute__((address_space(3))) void*)(Vs + (u * 8 + wave) * 512), 16, 0, 0);
   };
   // row lr of key tile t stands for key 8 (lr / 4) + 4 t + lr % 4 of the block, so that a lane's eight weights belong to the
@@ -781,76 +793,74 @@ __global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
     const bool busy = kb <= my_last;
     f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
     if (busy) {
+      // three chunks' keys are read while the three before them are multiplied (left to itself the compiler waits for each)
+      constexpr int AT = 3, PARTS = (NC + AT - 1) / AT;
+      bf16x8 f[2][AT][2];
+      auto read = [&](int x) {
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const int piece = 4 * min(half * NC + c, chunks - 1) + g;
+        for (int c = x * AT; c < min(x * AT + AT, NC); ++c) {
+          const int piece = 4 * min(half * NC + c, chunks - 1) + g;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int row = kofs + 4 * t;
-          s[t] = mfma16(*(const bf16x8*)(Ks + (row * KPS + (piece & ~7) + ((piece ^ (row >> 1)) & 7)) * 8), qf[c], s[t]);
+          for (int t = 0; t < 2; ++t) {
+            const int row = kofs + 4 * t;
+            f[x & 1][c % AT][t] = *(const bf16x8*)(Ks + (row * KPS + (piece & ~7) + ((piece ^ (row >> 1)) & 7)) * 8);
+          }
         }
+      };
+      read(0);
+#pragma unroll
+      for (int x = 0; x < PARTS; ++x) {
+        if (x + 1 < PARTS) read(x + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = x * AT; c < min(x * AT + AT, NC); ++c)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) s[t] = mfma16(f[x & 1][c % AT][t], qf[c], s[t]);
+        __builtin_amdgcn_sched_barrier(0);
       }
       Ss[wave][0][lane] = s[0];
       Ss[wave][1][lane] = s[1];
     }
     lds_barrier();
+    bf16x4 pb = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
+    float alpha = 1.f;
+    bool rescale = false;
     if (busy) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) s[t] += Ss[wave ^ 1][t][lane];
+      f32x4 x = (Ss[rt][st][16 * sg + srow] + Ss[rt + 4][st][16 * sg + srow]) * scale_log2;
       // a block that every row of the tile sees whole needs no mask (most blocks of a long prompt)
-      const bool whole = nrows == 16 && kb + 31 <= my_first && (window == 0 || kb >= my_last - window + 1);
-      float mx = -INFINITY;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
+      if (!(nrows == 16 && kb + 31 <= my_first && (window == 0 || kb >= my_last - window + 1))) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int key = kb + 8 * g + 4 * t + i;
-          const float v = s[t][i] * scale_log2;
-          s[t][i] = whole | ((key <= p) & (key >= lowest)) ? v : -INFINITY;
-          mx = fmaxf(mx, s[t][i]);
+          const int key = kb + 8 * sg + 4 * st + i;
+          x[i] = (key <= p) & (key >= lowest) ? x[i] : -INFINITY;
         }
+      }
+      float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+      mx = fmaxf(mx, __shfl_xor(mx, 8, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      // The running maximum follows the scores only when one of the tile's rows has outgrown it by more than 2^8 (or has
-      // none yet): the weights may then exceed 1, up to 256, which float sums and bf16 weights hold without loss. Both waves
-      // of a tile come to the same numbers.
-      const bool rescale = __any(mx > m + 8.f);
-      float alpha = 1.f;
+      // The running maximum follows the scores only when one of the wave's rows has outgrown it by more than 2^8 (or has
+      // none yet): the weights may then exceed 1, up to 256, which float sums and bf16 weights hold without loss.
+      rescale = __any(mx > m + 8.f);
       if (rescale) {
         const float m_new = fmaxf(m, mx);
         alpha = m == -INFINITY ? 0.f : exp2_of(m - m_new);
         l *= alpha;
         m = m_new;
       }
-      bf16x8 pb;
-      float psum = 0.f;
+      const float ref = m == -INFINITY ? 0.f : m;   // (nothing visible yet: all weights are 2^-inf)
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float pv = s[t][i] == -INFINITY ? 0.f : exp2_of(s[t][i] - m);
-          psum += pv;
-          pb[4 * t + i] = (bf16)pv;
-        }
-      l += psum;
-      if (half == 0) {
-        Ps[rt][lane] = pb;
-        if (g == 0) alphas[rt * 16 + lr] = alpha;
-        if (lane == 0) moved[rt] = rescale;
+      for (int i = 0; i < 4; ++i) {
+        const float pv = exp2_of(x[i] - ref);
+        l += pv;
+        pb[i] = (bf16)pv;
       }
-    } else if (half == 0) {
-      bf16x8 pb;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) pb[i] = (bf16)0.f;
-      Ps[rt][lane] = pb;
-      if (g == 0) alphas[rt * 16 + lr] = 1.f;
-      if (lane == 0) moved[rt] = 0;
     }
+    *((bf16x4*)&Ps[rt][16 * sg + srow] + st) = pb;
+    if (lane < 8) alphas[rt * 16 + srow] = alpha;
+    if (lane == 0) moved[wave] = rescale;
     lds_barrier();
-    bf16x8 pr[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) pr[r] = Ps[r][lane];
-    if (moved[0] | moved[1] | moved[2] | moved[3]) {
+    if (moved[0] | moved[1] | moved[2] | moved[3] | moved[4] | moved[5] | moved[6] | moved[7]) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float a = alphas[r * 16 + lr];
@@ -859,17 +869,19 @@ __global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
       }
     }
     auto values = [&](auto all) {
+      bf16x8 v[TW];
 #pragma unroll
-      for (int t = 0; t < TW; ++t) {
-        const int d = 16 * (TW * wave + t) + lr;
-        const bf16x8 v = *(const bf16x8*)(Vs + d * 32 + ((g ^ (lr >> 2)) & 3) * 8);
+      for (int t = 0; t < TW; ++t) v[t] = *(const bf16x8*)(Vs + (16 * (TW * wave + t) + lr) * 32 + ((g ^ (lr >> 2)) & 3) * 8);
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (decltype(all)::value || kb <= last[r]) o[t][r] = mfma16(v, pr[r], o[t][r]);
+      for (int r = 0; r < 4; ++r) {
+        const bf16x8 pr = Ps[r][lane];
+        if (decltype(all)::value || kb <= last(r))
+#pragma unroll
+          for (int t = 0; t < TW; ++t) o[t][r] = mfma16(v[t], pr, o[t][r]);
       }
     };
     // rows before the block take nothing of it, not 0 times what a later token left there (an infinity or NaN)
-    if (kb <= last[0]) values(std::true_type{});
+    if (kb <= last(0)) values(std::true_type{});
     else values(std::false_type{});
   };
   // this wave's loads into LDS have landed (a barrier alone does not wait for them), then everybody's; and everybody has read
@@ -888,10 +900,11 @@ __global__ void __launch_bounds__(512, 2) latent_attn_shared_kernel(
     if (blk + 2 < nblk) load(kb + 64, K0, V0);
     block(kb + 32, K1, V1);
   }
+  l += __shfl_xor(l, 8, 64);
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
   lds_barrier();
-  if (g == 0 && half == 0) alphas[rt * 16 + lr] = l > 0.f ? 1.f / l : 0.f;
+  if (lane < 8) alphas[rt * 16 + srow] = l > 0.f ? 1.f / l : 0.f;
   lds_barrier();
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -1022,12 +1035,14 @@ extern "C" int dinfer_latent_attn_mfma(const void* qa, int64_t ld_qa, void* out,
   // their rows' weights (which keeps offsets inside a page in 32 bits)
   if (solo && (page_size & (page_size - 1)) == 0 && page_size <= 1 << 20 && dr % 32 == 0 && (R == 128 || R == 256 || (R == 512 && dr <= 64))) {
     const int64_t groups = (tokens * heads + 63) / 64 + num_reqs;
-    if (groups > 0x7fffffff) return ERR_UNSUPPORTED;
+    if (groups > 0x7fffffff - 256) return ERR_UNSUPPORTED;
+    const int run = (int)std::min<int64_t>(4, (groups + 7) / 8);
+    const int64_t grid = (groups + 8 * run - 1) / (8 * run) * 8 * run;
     const int page_shift = __builtin_ctz(page_size);
 #define SHARED_LAUNCH(DT, KPS)                                                                                         \
-  latent_attn_shared_kernel<DT, KPS><<<(unsigned)groups, 512, 0, stream>>>(                                            \
+  latent_attn_shared_kernel<DT, KPS><<<(unsigned)grid, 512, 0, stream>>>(                                              \
       (const bf16*)qa, ld_qa, (bf16*)out, ld_out, (const bf16*)cache, (const bf16*)cache_t, block_table, max_blocks,   \
-      cu_seqlens, seq_lens, num_reqs, scale * LOG2E, window, heads, dr, page_shift)
+      cu_seqlens, seq_lens, num_reqs, scale * LOG2E, window, heads, dr, page_shift, (int)groups, run)
     if (R == 128) SHARED_LAUNCH(2, 32);
     else if (R == 256) SHARED_LAUNCH(4, 48);
     else SHARED_LAUNCH(8, 72);

@@ -19,6 +19,7 @@ CASES = [
     ([150, 70], [150, 3], 5, 512, 64, 16, 0, (0, 149, 1, 5)),           # the widest rows
     ([700], [130], 16, 512, 64, 16, 0, (0, 129, 15, 31)),               # several groups behind a history
     ([70] * 66, [2] * 66, 16, 128, 32, 16, 0, (65, 1, 3, 64)),          # more requests than a wave counts at once
+    ([200, 120, 75, 10], [150, 120, 40, 10], 16, 512, 64, 8, 0, (2, 39, 1, 70)),   # more row groups than two rounds over the XCDs take
 ]
 
 
