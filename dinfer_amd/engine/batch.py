@@ -11,6 +11,7 @@ whole prompts, portions of prompts and single decoded tokens side by side
   seq_lens     [B]   int32  request length after this step (start + n)
   block_table  [B, MB] int32 per cache group, -1 where no page is held
   state_slots  [B]   int32  the request's fixed-size state slot (padded rows: the spare slot max_reqs)
+  fresh_slots  [F]   int64  slots of requests admitted since the step before, whose state starts from nothing
   logits_rows  [R]   int32  rows of the flat batch whose logits are wanted
   feedback_src [T]   int32  -1, or: the token's id is not in input_ids but is the feedback_src-th of the tokens the
                             step before sampled (last_tokens, on the device): a step planned before that one ended
@@ -45,6 +46,7 @@ class StepBatch:
         self.max_tokens, self.max_reqs, self.max_rows = max_tokens, max_reqs, max_rows
         self.max_blocks = list(max_blocks)
         layout = [("slot_mapping%d" % g, np.int64, (max_tokens,)) for g in range(len(max_blocks))]
+        layout += [("fresh_slots", np.int64, (max_reqs + spare,))]
         layout += [("input_ids", np.int32, (max_tokens,)), ("positions", np.int32, (max_tokens,)),
                    ("cu_seqlens", np.int32, (max_reqs + spare + 1,)), ("seq_lens", np.int32, (max_reqs + spare,)),
                    ("state_slots", np.int32, (max_reqs + spare,)), ("logits_rows", np.int32, (max(max_rows, 1),)),
@@ -69,7 +71,7 @@ class StepBatch:
         self.input_ids, self.positions = d["input_ids"], d["positions"]
         self.cu_seqlens, self.seq_lens = d["cu_seqlens"], d["seq_lens"]
         self.state_slots, self.logits_rows = d["state_slots"], d["logits_rows"]
-        self.feedback_src = d["feedback_src"]
+        self.feedback_src, self.fresh_slots = d["feedback_src"], d["fresh_slots"]
         # the tokens the last step sampled, one per sampling request in the step's order: the sampler writes them here
         self.last_tokens = torch.zeros(max(max_rows, 1), dtype=torch.int32, device=device)
         self.slot_mapping = [d["slot_mapping%d" % g] for g in range(len(max_blocks))]

@@ -199,6 +199,7 @@ class ModelRunner:
         self.cache = CacheManager(self.group_specs, opt.max_num_seqs, prefix_caching=prefix)
         self.cache_views: list[CacheView] = []
         self._slotted: list[tuple] = []     # (spec, tensors) of the entries with per-request memory
+        self._fresh = 0                     # slots of the step that start from nothing (batch.fresh_slots)
         own: dict[int, CacheView] = {}
         for i, (e, need) in enumerate(zip(self.model.run, needs)):
             if e.cache != i:
@@ -221,9 +222,10 @@ class ModelRunner:
         return [t for _, tensors in self._slotted for t in tensors.values()]
 
     def _reset_fresh_slots(self) -> None:
-        fresh = self.cache.take_fresh_slots()
-        if fresh and self._slotted:
-            idx = torch.tensor(fresh, device=self.device, dtype=torch.long)
+        """Clears the state of the requests that _send() found admitted. Their slots came with the step: a copy of their own
+        made the host wait for everything the device still had to do (some 130 us a step that begins requests)."""
+        if self._fresh and self._slotted:
+            idx = self.batch.fresh_slots[:self._fresh]
             for need, tensors in self._slotted:
                 need.reset_slots(tensors, idx)
 
@@ -306,6 +308,9 @@ class ModelRunner:
         bracket the step on the device. shape: called between the two, may pad the step; its result is returned."""
         fill(pad)
         shaped = shape() if shape is not None else None
+        fresh = self.cache.take_fresh_slots()
+        self._fresh = len(fresh)
+        self.batch.h["fresh_slots"][:self._fresh] = fresh
         self.batch.upload()
         self._mark_sent()
         return shaped

@@ -274,3 +274,11 @@ def test_rows_of_prompt_positions_follow_the_sampling_rows():
     b.fill_planned(s)
     assert [(x.request.id, x.start, x.num_new) for x in out.scheduled] == [(1, 4, 1), (2, 7, 1), (3, 3, 6)]
     assert b.h["logits_rows"][:8].tolist() == [0, 1, 2, 3, 4, 5, 6, 7]
+
+
+def test_fresh_slots_travel_with_the_step():
+    """Slots whose state starts from nothing go to the device in the step's own copy, as many as requests fit."""
+    b = StepBatch(torch.device("cpu"), 64, 3, 3, [4], spare=1)
+    b.h["fresh_slots"][:4] = [2, 0, 1, 3]
+    b.upload()
+    assert b.fresh_slots.dtype == torch.int64 and b.fresh_slots.tolist() == [2, 0, 1, 3]
