@@ -40,6 +40,7 @@
 // gqa_decode_v3_core.cuh:72-242 and gqa.cu:1423-1461 (split-K decode, merge of
 // (m, l, o) partials).
 #include <cmath>
+#include <type_traits>
 
 #include "attention_tile.cuh"
 
@@ -522,7 +523,7 @@ inline bool aligned16(const void* p) { return ((uintptr_t)p % 16) == 0; }
 
 template <int DT>
 int launch_flash(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const bf16* kc, const bf16* vc,
-                 const int32_t* bt, int64_t max_blocks, const int32_t* cu, const int32_t* sl, int num_reqs,
+                 const int32_t* bt, int64_t max_blocks, const int32_t* cu, const int32_t* sl, int num_reqs, int64_t tokens,
                  int max_q_len, float scale, int window, int H, int Hkv, int ps, int skip_single, hipStream_t stream) {
   const float sl2 = scale * LOG2E;
   const bool p2 = (ps & (ps - 1)) == 0;
@@ -531,39 +532,37 @@ int launch_flash(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const b
   auto lds_of = [](int qt) { return (size_t)3 * qt * 64 * (sizeof(f32x4) * DT + 2 * sizeof(float)); };
   // 48 rows per workgroup at head size 128: every K and V fragment a wave loads serves three row tiles instead of two
   // (the path on which loads return is what this kernel fills first), at 256 registers, still two waves a SIMD.
-  // It pays where the rows still make several rounds of workgroups over the chip (measured, 32 heads: 3,072 rows
-  // 135 -> 121 us, 8,192 rows 783 -> 642 us = 34 % of the MFMA peak, 32,768 rows 37 %; 2,048 rows, 1,376 workgroups, level; a portion
-  // of 512 rows behind 30,000 keys, 352 workgroups instead of 512, loses 17 %). Head size 64 gains nothing.
-  constexpr bool WIDE_OK = DT == 8;
-  const int64_t wide_blocks = (int64_t)((max_q_len + 47) / 48) * H * num_reqs;
-  // (rows of at most two tiles a request never fill the third: many single rows of many heads are no case for it)
-  if (WIDE_OK && max_q_len > 32 && wide_blocks >= 2000) {
-    constexpr int QT = WIDE_OK ? 3 : 1;
+  // It pays where the step's rows still make several rounds of workgroups over the chip (measured, 32 heads: 3,072 rows
+  // 135 -> 121 us, 8,192 rows 783 -> 642 us = 34 % of the MFMA peak, 32,768 rows 37 %; 2,048 rows, 1,344 workgroups, level, behind 28,000
+  // keys 1,330 -> 1,302; a portion of 512 rows behind 30,000 keys, 352 workgroups instead of 512, loses 17 %). Head size
+  // 64 gains nothing. (Rows of at most two tiles a request never fill the third: many single rows of many heads are no case.)
+  const auto run = [&](auto qt) {
+    constexpr int QT = decltype(qt)::value;
     const int tiles = (max_q_len + 16 * QT - 1) / (16 * QT);
-    if (wide_blocks > 0x7fffffff) return ERR_UNSUPPORTED;
+    // A workgroup for every tile that a request might have: beside decoding requests nearly all of them find none (31 of them and
+    // a portion of 512 rows: 14,520 workgroups for 440), so there the tiles are counted up instead: that portion behind 1,024
+    // keys, 40 heads, 40 -> 36 us, 1,024 rows of 32 heads beside 48 requests 51 -> 29, 200 beside 16 17.7 -> 13.5. Where few are
+    // empty the count is a microsecond more for nothing.
+    const int64_t all = (int64_t)tiles * num_reqs, some = tokens / (16 * QT) + num_reqs;
+    const bool count = all >= 4 * some;
+    const int64_t blocks = (count ? some : all) * H;
+    if (blocks > 0x7fffffff) return (int)ERR_UNSUPPORTED;
     auto kernel = p2 ? attn_flash_kernel<DT, QT, true> : attn_flash_kernel<DT, QT, false>;
+    if (count) kernel = p2 ? attn_flash_kernel<DT, QT, true, PLAIN, DT, false, true> : attn_flash_kernel<DT, QT, false, PLAIN, DT, false, true>;
     // (more than the 64 KB of LDS a launch may ask for without saying so)
-    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_of(QT)) != hipSuccess)
-      return ERR_LAUNCH;
-    kernel<<<(unsigned)wide_blocks, 256, lds_of(QT), stream>>>(q, ld_q, out, ld_out, kc, vc, bt, max_blocks, cu, sl, tiles,
-                                                              sl2, window, H, Hkv, ps, skip_single, FlashExt{});
-  } else if (DT <= 8 && max_q_len > 16) {
-    constexpr int QT = DT <= 8 ? 2 : 1;
-    const int tiles = (max_q_len + 16 * QT - 1) / (16 * QT);
-    const int64_t blocks = (int64_t)tiles * H * num_reqs;
-    if (blocks > 0x7fffffff) return ERR_UNSUPPORTED;
-    auto kernel = p2 ? attn_flash_kernel<DT, QT, true> : attn_flash_kernel<DT, QT, false>;
-    kernel<<<(unsigned)blocks, 256, lds_of(QT), stream>>>(q, ld_q, out, ld_out, kc, vc, bt, max_blocks, cu, sl, tiles, sl2,
-                                                         window, H, Hkv, ps, skip_single, FlashExt{});
-  } else {
-    const int tiles = (max_q_len + 15) / 16;
-    const int64_t blocks = (int64_t)tiles * H * num_reqs;
-    if (blocks > 0x7fffffff) return ERR_UNSUPPORTED;
-    auto kernel = p2 ? attn_flash_kernel<DT, 1, true> : attn_flash_kernel<DT, 1, false>;
-    kernel<<<(unsigned)blocks, 256, lds_of(1), stream>>>(q, ld_q, out, ld_out, kc, vc, bt, max_blocks, cu, sl, tiles, sl2,
-                                                        window, H, Hkv, ps, skip_single, FlashExt{});
+    if (QT == 3 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_of(QT)) != hipSuccess)
+      return (int)ERR_LAUNCH;
+    kernel<<<(unsigned)blocks, 256, lds_of(QT), stream>>>(q, ld_q, out, ld_out, kc, vc, bt, max_blocks, cu, sl, count ? num_reqs : tiles,
+                                                         sl2, window, H, Hkv, ps, skip_single, FlashExt{});
+    return launch_status();
+  };
+  if constexpr (DT == 8) {
+    if (max_q_len > 32 && tokens / 48 * H >= 1300) return run(std::integral_constant<int, 3>{});
   }
-  return launch_status();
+  if constexpr (DT <= 8) {
+    if (max_q_len > 16) return run(std::integral_constant<int, 2>{});
+  }
+  return run(std::integral_constant<int, 1>{});
 }
 
 // CUs of the current device (asked once per device).
@@ -645,20 +644,20 @@ extern "C" int dinfer_attn_mfma_supports(int head_dim, int page_size, int heads,
   return (int64_t)kv_heads * page_size * head_dim < (int64_t)1 << 30 ? 1 : 0;
 }
 
-// skip_single: requests with one row are left to the split-K kernel.
+// tokens: rows of all requests together. skip_single: requests with one row are left to the split-K kernel.
 extern "C" int dinfer_attn_flash(const void* q, int64_t ld_q, void* out, int64_t ld_out, const void* k_cache,
                                  const void* v_cache, const int32_t* block_table, int64_t max_blocks,
-                                 const int32_t* cu_seqlens, const int32_t* seq_lens, int num_reqs, int max_q_len,
+                                 const int32_t* cu_seqlens, const int32_t* seq_lens, int num_reqs, int64_t tokens, int max_q_len,
                                  float scale, int window, int heads, int kv_heads, int head_dim, int page_size,
                                  int skip_single, hipStream_t stream) {
-  if (num_reqs <= 0 || max_q_len <= 0) return OK;
+  if (num_reqs <= 0 || max_q_len <= 0 || tokens <= 0) return OK;
   if (!dinfer_attn_mfma_supports(head_dim, page_size, heads, kv_heads)) return ERR_UNSUPPORTED;
   if (window < 0 || max_blocks <= 0 || ld_q % 8 || ld_out % 4 || !aligned16(q) || !aligned16(k_cache) ||
       !aligned16(v_cache) || ((uintptr_t)out % 8))
     return ERR_BAD_SHAPE;
   DINFER_DISPATCH_HEAD_DIM(head_dim, return launch_flash<DT>(
       (const bf16*)q, ld_q, (bf16*)out, ld_out, (const bf16*)k_cache, (const bf16*)v_cache, block_table, max_blocks,
-      cu_seqlens, seq_lens, num_reqs, max_q_len, scale, window, heads, kv_heads, page_size, skip_single, stream));
+      cu_seqlens, seq_lens, num_reqs, tokens, max_q_len, scale, window, heads, kv_heads, page_size, skip_single, stream));
 }
 
 // Single-row requests only. cu_seqlens null: every request brings exactly one row (row b belongs to

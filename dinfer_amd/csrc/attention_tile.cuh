@@ -386,7 +386,8 @@ struct FlashExt {
 // with all eight always joined, behind 40 5.3 -> 4.6 (tiles of rows 5.8 and 5.0).
 constexpr int flash_waves(bool heads) { return heads ? 8 : 4; }
 
-template <int DT, int QT, bool P2, int KIND = PLAIN, int DV = DT, bool HEADS = false>
+// COUNT: tiles_x is the number of requests, and the tiles that exist are counted up over them (a few long portions among many).
+template <int DT, int QT, bool P2, int KIND = PLAIN, int DV = DT, bool HEADS = false, bool COUNT = false>
 __global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu_waves_per_eu(2, 8))) attn_flash_kernel(
     const bf16* __restrict__ q, int64_t ld_q, bf16* __restrict__ out, int64_t ld_out, const bf16* __restrict__ kc,
     const bf16* __restrict__ vc, const int32_t* __restrict__ block_table, int64_t max_blocks,
@@ -413,7 +414,33 @@ __global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu
   // of K and V. Late query tiles (most keys) are issued first.
   const int L = blockIdx.x;
   const int e = HEADS ? L % Hkv : L % H, rest = HEADS ? L / Hkv : L / H;
-  const int tile = HEADS ? 0 : tiles_x - 1 - rest % tiles_x, b = HEADS ? rest : rest / tiles_x;
+  int tile = HEADS ? 0 : tiles_x - 1 - rest % tiles_x, b = HEADS ? rest : rest / tiles_x;
+  if constexpr (COUNT) {   // (64 requests at once)
+    const int ln = threadIdx.x & 63, reqs = tiles_x;
+    int at = rest;
+    b = -1;
+    for (int b0 = 0; b0 < reqs && b < 0; b0 += 64) {
+      const int len = b0 + ln < reqs ? cu_seqlens[b0 + ln + 1] - cu_seqlens[b0 + ln] : 0;
+      const int mine = skip_single && len == 1 ? 0 : (len + QW - 1) / QW;
+      int upto = mine;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(upto, o, 64);
+        if (ln >= o) upto += v;
+      }
+      const unsigned long long holds = __ballot(at < upto);
+      if (holds) {
+        const int l = __ffsll((long long)holds) - 1;
+        b = b0 + l;
+        tile = __shfl(upto, l, 64) - 1 - at;
+      } else {
+        at -= __shfl(upto, 63, 64);
+      }
+    }
+    if (b < 0) return;   // (the whole workgroup: every wave counts the same)
+    b = __builtin_amdgcn_readfirstlane(b);
+    tile = __builtin_amdgcn_readfirstlane(tile);
+  }
   const int G = H / Hkv;
   const int hk = e % Hkv;
   const int q_begin = cu_seqlens[b];

@@ -105,7 +105,7 @@ SIGNATURES = {
     "dinfer_attn_mfma_supports": ("attention", [_I, _I, _I, _I]),
     "dinfer_attn_flash": (
         "attention",
-        [_P, _L, _P, _L, _P, _P, _P, _L, _P, _P, _I, _I, _F, _I, _I, _I, _I, _I, _I, _P],
+        [_P, _L, _P, _L, _P, _P, _P, _L, _P, _P, _I, _L, _I, _F, _I, _I, _I, _I, _I, _I, _P],
     ),
     "dinfer_attn_flash_ext_supports": ("attention_ext", [_I, _I, _I, _I, _I, _I]),
     "dinfer_attn_flash_ext": (

@@ -1247,7 +1247,7 @@ def attn_flash(q, out, k_cache, v_cache, block_table, cu_seqlens, seq_lens, num_
     assert q.shape[0] >= tokens and out.shape[0] >= tokens
     lib.call("dinfer_attn_flash", q.data_ptr(), _rows(q), out.data_ptr(), _rows(out), k_cache.data_ptr(),
              v_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1], cu_seqlens.data_ptr(),
-             seq_lens.data_ptr(), num_reqs, max_q_len, float(scale), int(window), heads, kv_heads, head_dim,
+             seq_lens.data_ptr(), num_reqs, tokens, max_q_len, float(scale), int(window), heads, kv_heads, head_dim,
              page_size, 1 if skip_single else 0, _stream())
     return out
 
