@@ -69,23 +69,6 @@ __global__ void __launch_bounds__(256) swiglu_bf16x8_kernel(const bf16* __restri
   }
 }
 
-// 4 floats per thread and iteration: inter % 4 == 0 and 16-byte aligned rows. 500 rows x 3,072 4.2 -> 3.3 us.
-__global__ void __launch_bounds__(256) swiglu_f32x4_kernel(const float* __restrict__ in, float* __restrict__ out,
-                                                           int64_t inter, int64_t ld_in) {
-  const int64_t t = blockIdx.y;
-  const f32x4* g = (const f32x4*)(in + t * ld_in);
-  const f32x4* u = (const f32x4*)(in + t * ld_in + inter);
-  f32x4* o = (f32x4*)(out + t * inter);
-  const int64_t n4 = inter / 4;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
-    const f32x4 gv = g[i], uv = u[i];
-    f32x4 r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) r[j] = silu(gv[j]) * uv[j];
-    o[i] = r;
-  }
-}
-
 // dst[i] = round(float(dst[i]) + float(src[i]))
 template <class S>
 __global__ void __launch_bounds__(256) add_inplace_kernel(S* __restrict__ dst, const S* __restrict__ src, int64_t n) {
@@ -312,12 +295,8 @@ extern "C" int dinfer_gated_act(int dtype, int act, const void* in, void* out, i
       else
         swiglu_kernel<bf16><<<dim3(blocks_for(inter, 256, 64), (unsigned)nt), 256, 0, stream>>>(ip, op, inter, ld_in);
     } else if (dtype == DT_F32) {
-      const float* ip = (const float*)in + t0 * ld_in;
-      float* op = (float*)out + t0 * inter;
-      if (inter % 4 == 0 && ld_in % 4 == 0 && ((uintptr_t)ip % 16 == 0) && ((uintptr_t)op % 16 == 0))
-        swiglu_f32x4_kernel<<<dim3(blocks_for(inter / 4, 256, 64), (unsigned)nt), 256, 0, stream>>>(ip, op, inter, ld_in);
-      else
-        swiglu_kernel<float><<<dim3(blocks_for(inter, 256, 64), (unsigned)nt), 256, 0, stream>>>(ip, op, inter, ld_in);
+      swiglu_kernel<float><<<dim3(blocks_for(inter, 256, 64), (unsigned)nt), 256, 0, stream>>>(
+          (const float*)in + t0 * ld_in, (float*)out + t0 * inter, inter, ld_in);
     } else {
       return ERR_BAD_DTYPE;
     }
