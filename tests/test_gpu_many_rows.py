@@ -51,6 +51,35 @@ def test_qkv_post_of_portions(H, Hkv, D, style, extras, portions):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("H,Hkv,D", [(16, 8, 128), (3, 2, 64), (2, 1, 256), (2, 2, 320)])
+@pytest.mark.parametrize("portions", [[(0, 127)], [(0, 128)], [(5, 100), (16, 20), (3, 9)], [(7, 255)], [(i, 37 + i) for i in range(12)]])
+def test_qkv_post_of_portions_in_32_bits(H, Hkv, D, portions):
+    """From 128 tokens on neighbours share an XCD: the same bits, whatever the number of tokens leaves of the last 128."""
+    page, blocks = 16, sum((a + n - 1) // 16 + 1 for a, n in portions)
+    g = torch.Generator().manual_seed(D)
+    T, cols = sum(n for _, n in portions), (H + 2 * Hkv) * D
+    x = torch.randn(T, cols, generator=g).cuda()
+    slots = _slots(portions, page, blocks)
+    slots[T // 2] = -1
+    slots = torch.tensor(slots).cuda()
+    ang = torch.rand(300, D // 2, generator=g) * 6
+    table = torch.cat([ang.cos(), ang.sin()], 1).cuda()
+    pos = torch.randint(0, 300, (T,), generator=g, dtype=torch.int32).cuda()
+    gains = [(1 + 0.2 * torch.randn(D, generator=g)).cuda() for _ in range(2)]
+    got = []
+    for runs in (False, True):
+        buf = torch.cat([x, torch.full((3, cols), 9.0, device="cuda")])
+        kc = torch.full((blocks, Hkv, D // 8, page, 8), 9.0, device="cuda")
+        vc = torch.full((blocks, Hkv, D, page), 9.0, device="cuda")
+        ops().qkv_post(buf, T, heads=H, kv_heads=Hkv, head_dim=D, q_off=0, k_off=H * D, v_off=(H + Hkv) * D, q_gain=gains[0],
+                       k_gain=gains[1], eps=1e-6, gain_offset=0.0, positions=pos, cos_sin=table, rotary_dim=D, rope_style=0,
+                       k_cache=kc, v_cache=vc, slot_mapping=slots, page_size=page, token_runs=runs)
+        got.append((buf, kc, vc))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    assert bool((got[1][0][T:] == 9).all())
+
+
 @pytest.mark.parametrize("rows,width", [(1023, 2048), (1024, 8), (1025, 520), (1030, 2048), (1024, 2056), (1027, 4096), (1024, 4104)])
 @pytest.mark.parametrize("x_dtype,out_dtype,branch", [(BF, BF, True), (torch.float32, BF, False), (torch.float32, torch.float32, True)])
 def test_layernorm_of_many_rows(rows, width, x_dtype, out_dtype, branch):
@@ -119,8 +148,8 @@ def test_router_logits_of_many_tokens(tokens, experts, width, gate):
 
 @pytest.mark.parametrize("width", [4, 1020, 1024, 1025, 1028, 4100, 5120, 5121])
 def test_float_rows(width):
-    """The norm of float rows at the edges of the widths that registers hold; their gated activation in 16-byte pieces beside
-    rows that do not begin at 16 bytes (the kernel of single numbers), bit for bit."""
+    """The norm of float rows at the edges of the widths that registers hold; norms and gated
+    activations wherever the rows begin, the latter bit for bit."""
     g = torch.Generator().manual_seed(width)
     T, eps = 5, 1e-6
     x, res, w = torch.randn(T, width, generator=g).cuda(), torch.randn(T, width, generator=g).cuda(), torch.randn(width, generator=g).cuda()
