@@ -103,6 +103,7 @@ class ModelRunner:
         # steps with prompt portions: padded up to a few counts, and replayed from a graph of their own once the same
         # counts have come up PORTION_GRAPH_AFTER times (a capture costs about two eager steps)
         self._portion_graphs_allowed = self._graphs_allowed and model.capturable_portions()
+        self._layer_weights = model.layer_weights()
         self._portion_graphs: dict[tuple, torch.cuda.CUDAGraph] = {}
         self._portion_seen: dict[tuple, int] = {}
         self.portion_replays = 0            # steps with prompt portions served by a replay
@@ -384,10 +385,12 @@ class ModelRunner:
             break
         if Bp is None or Tp > self.max_tokens:
             return None
-        # A full batch has a made-up request only for the graph's sake. From some 128 tokens on the device, not the host, bounds
-        # most steps, and made-up rows cost it their share (195 tokens as 224: 1,559 -> 1,595 us), so there only few of them do
-        # (1,033 as 1,056, 28 layers of 1,024: 3,149 -> 2,975).
-        if Bp > self._buckets[-1] and T > 128 and (Tp - T) * 32 > T:
+        # A full batch has a made-up request only for the graph's sake, which is worth its rows where the host bounds the step: a
+        # layer's launches take it some 100 us, products of 2e10 multiplications about 60 us of the device beside its other
+        # kernels. Eager and padded, 28 layers of 16 million weights: 437 tokens 3,162 and 2,341 us, 1,000 3,157 and 3,009,
+        # 1,033 (as 1,152) 3,176 and 3,005, 2,023 4,616 and 4,719; wider layers: 437 tokens 1,697 and 1,734, 2,023 1,745 and
+        # 1,790, 3,343 and 3,428, 195 (as 224) 1,559 and 1,595. Up to 128 tokens the host bounds nearly all steps.
+        if Bp > self._buckets[-1] and T > 128 and T * self._layer_weights > 2e10:
             return None
         last = Tp - T - (Bp - B - 1) if Bp > B else 0         # tokens of the last made-up request
         if last > opt.max_model_len:

@@ -4,6 +4,8 @@ Knows no architecture by name.
 """
 from __future__ import annotations
 
+import math
+
 import torch
 
 from ..kernels import gemm, ops
@@ -80,6 +82,10 @@ class DecoderModel:
     # ---- weights -------------------------------------------------------------------------------
     def expected_tensors(self):
         return expected_tensors(self.spec, self.blocks)
+
+    def layer_weights(self) -> int:
+        """Weights of a layer, on the average over the layers."""
+        return sum(math.prod(t.shape) for b in self.blocks for t in b.tensors().values()) // max(len(self.blocks), 1)
 
     def load(self, loader) -> None:
         exp, optional = self.expected_tensors()

@@ -1,6 +1,7 @@
 """The flat batch a step is built into (no GPU), against the exact plans the reference's runner tests
 hold (crates/core/src/runner.rs:1058-1148), and the Engine loop with a stand-in runner."""
 import numpy as np
+import pytest
 import torch
 
 from dinfer_amd.cache import CacheManager, GroupSpec
@@ -282,3 +283,17 @@ def test_fresh_slots_travel_with_the_step():
     b.h["fresh_slots"][:4] = [2, 0, 1, 3]
     b.upload()
     assert b.fresh_slots.dtype == torch.int64 and b.fresh_slots.tolist() == [2, 0, 1, 3]
+
+
+@pytest.mark.parametrize("tokens,weights,padded", [(100, 10 ** 9, 128), (130, 10 ** 6, 160), (1033, 15 * 10 ** 6, 1152),
+                                                   (1033, 20 * 10 ** 6, None), (437, 4 * 10 ** 7, 448), (437, 5 * 10 ** 7, None)])
+def test_full_batches_are_padded_where_the_host_bounds_them(tokens, weights, padded):
+    """Up to 128 tokens always; beyond, where tokens times a layer's weights are few."""
+    from types import SimpleNamespace as N
+    from dinfer_amd.engine.runner import ModelRunner
+    pads = []
+    b = N(num_tokens=tokens, num_reqs=1, num_rows=1, max_q_len=tokens, num_singles=0, all_decode=False,
+          pad=lambda reqs, toks, rows: pads.append((reqs, toks)))
+    r = N(batch=b, options=N(max_model_len=4096), max_tokens=4096, _buckets=[1], _layer_weights=weights)
+    got = ModelRunner._portion_shape(r)
+    assert (got and got[0][0], pads) == (padded, [(2, padded)] if padded else [])
