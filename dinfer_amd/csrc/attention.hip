@@ -248,9 +248,9 @@ attn_decode_kernel(
         f32x4 x = {0.f, 0.f, 0.f, 0.f};   // row 0 is the key: lane group 0 gets its scores
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) x = mfma16(i16 == 0 ? kr[ks] : zero8(), i16 < G ? qf[0][ks] : zero8(), x);
-        // (as a walk of this one key leaves it)
+        // (as a walk of this one key leaves it: a score of -inf has the weight 0)
         tl.m[0] = __shfl(x[0], i16, 64);
-        own_l = exp2_raw(fmaf(tl.m[0], scale_log2e, -(tl.m[0] * scale_log2e)));
+        own_l = exp2_raw(fmaf(tl.m[0], scale_log2e, -((tl.m[0] == -INFINITY ? 0.f : tl.m[0]) * scale_log2e)));
 #pragma unroll
         for (int d = 0; d < DT; ++d)
 #pragma unroll

@@ -316,6 +316,72 @@ def test_attention_decode_own_key_that_is_no_number(bad, splits):
     assert group.isnan().all() if bad == "key" else group[:, 0].isnan().all() and group[:, 1:].isfinite().all()
 
 
+def decode_of_rows(raw, hist, kc, vc, m, H, Hkv, D, page, splits, written=True):
+    """Decode attention of raw q|k|v rows behind `hist` keys, by the kernel that writes the cache itself and by the two it stands
+    for. written False: the pages hold the rows' keys and values already."""
+    B, geo = len(hist), dict(heads=H, kv_heads=Hkv, head_dim=D, page_size=page)
+    slots = torch.tensor([int(m["bt"][b, h // page]) * page + h % page if written else -1 for b, h in enumerate(hist)], device=DEV)
+    post = dict(q_off=0, k_off=H * D, v_off=(H + Hkv) * D, q_gain=None, k_gain=None, eps=1e-5, gain_offset=0.0,
+                positions=torch.tensor(hist, dtype=torch.int32, device=DEV), cos_sin=None, slot_mapping=slots)
+    part, outs = torch.empty(B * H * splits * (D + 4), device=DEV), []
+    for fused in (True, False):
+        k, v, x, out = kc.clone(), vc.clone(), raw.to(DEV), torch.zeros(B, H * D, device=DEV, dtype=torch.bfloat16)
+        if fused:
+            ops().attn_decode_post(x, out, part, k, v, m["bt"], m["sl"], B, splits, scale=D ** -0.5, window=0, **geo, **post)
+        else:
+            ops().qkv_post(x, B, **geo, **post, rotary_dim=D, rope_style=0, k_cache=k, v_cache=v, token_runs=False)
+            ops().attn_decode(x, out, part, k, v, m["bt"], None, m["sl"], B, splits, scale=D ** -0.5, window=0, **geo)
+        outs.append(out.cpu().view(B, H, D))
+    return outs
+
+
+@pytest.mark.parametrize("written", [True, False])
+@pytest.mark.parametrize("splits", [1, 4, 5])
+def test_attention_decode_own_key_scored_minus_infinity(splits, written):
+    """The row's own key at a score of -inf weighs nothing beside finite ones: a product beyond 32 bits in the row, an infinity in
+    the pages (which a rotation would make no number)."""
+    H, Hkv, D, page, hist = 16, 8, 128, 16, [40, 7, 200, 64]
+    _, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, [1] * 4, seed=12)
+    raw = torch.randn(4, (H + 2 * Hkv) * D, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
+    x, want_outs = raw.view(4, H + 2 * Hkv, D), []
+    x[1:, :H, 0], x[1:, H:H + Hkv, 0] = -1e25 if written else 1.0, 1e25
+    for b, (_, k, v) in enumerate(outs):
+        k, v = k.clone(), v.clone()
+        if written:
+            k[-1], v[-1] = x[b, H:H + Hkv].double(), x[b, H + Hkv:].double()
+        k[:, :, 0] = 0          # (of the other keys: their scores stay where they are)
+        for i in range(hist[b] + 1):
+            kc[int(m["bt"][b, i // page]), :, 0, i % page, 0] = 0
+        if b:
+            k[-1, :, 0] = float("inf") if written else -float("inf")
+            kc[int(m["bt"][b, hist[b] // page]), :, 0, hist[b] % page, 0] = -float("inf")
+        elif written:
+            k[-1, :, 0] = x[b, H:H + Hkv, 0].double()
+        want_outs.append((x[b:b + 1, :H].double(), k, v))
+    fused, two = decode_of_rows(raw, hist, kc, vc, m, H, Hkv, D, page, splits, written)
+    torch.testing.assert_close(fused.double(), expected_attention(want_outs, hist, D ** -0.5, 0), rtol=2e-2, atol=2e-2)
+    assert torch.equal(fused, two)
+
+
+@pytest.mark.parametrize("bad", ["key", "value"])
+@pytest.mark.parametrize("splits", [1, 4])
+def test_attention_decode_own_key_that_is_no_number_beside_a_large_score(splits, bad):
+    """A score or value of the row's own key that is no number stays in the row's output though another key's score exceeds what
+    2^x holds beside it."""
+    H, Hkv, D, page, hist = 16, 8, 128, 16, [40, 0, 200]
+    _, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, [1] * 3, seed=12)
+    raw = torch.randn(3, (H + 2 * Hkv) * D, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
+    x = raw.view(3, H + 2 * Hkv, D)
+    x[2, :H] = x[2, :1]                                     # every head's query, and a cached key 40 times as long: 40 x 128 x 128 ** -0.5
+    blk, off = int(m["bt"][2, 3]), 50 % page
+    kc[blk, :, :, off, :] = (x[2, 0].float() * 40).to(torch.bfloat16).view(D // 8, 8).to(DEV)
+    x[2, H if bad == "key" else H + Hkv, 0] = float("nan")
+    for out in decode_of_rows(raw, hist, kc, vc, m, H, Hkv, D, page, splits):
+        assert out[:2].isfinite().all() and out[2, H // Hkv:].isfinite().all()
+        group = out[2, :H // Hkv]
+        assert group.isnan().all() if bad == "key" else group[:, 0].isnan().all() and group[:, 1:].isfinite().all()
+
+
 def decode_post_case(H, Hkv, D, page, window, gains, hist, splits, device="cpu", spike=None, sharp=1.0):
     """One launch of the decode kernel that norms, rotates and writes the cache, against the plain functions and, bit
     for bit, against the two kernels it stands for. Request 1 writes nothing (slot -1)."""
