@@ -406,7 +406,7 @@ attn_decode_kernel(
     if (i16 < G) {
       float* pp = &joined[sp][i16][0];
       if (g4 == 0) {
-        // -inf for an empty part; a score of the own key that is no number may not pass for one
+        // -inf for an empty part; a score of the own key that is no number may not pass for one (the sum then tells it)
         pp[0] = own_part && lt != lt && tl.m[0] != INFINITY ? 0.f : tl.m[0] * scale_log2e;
         pp[1] = lt;
       }
@@ -423,7 +423,9 @@ attn_decode_kernel(
       for (int s = 0; s < parts; ++s) {
         const float m = joined[s][i][0];
         const float a = m == -INFINITY ? 0.f : exp2f(m - M);
-        if (a > 0.f) {
+        // (the own part also at a weight of 0: what is no number in it stays so, as it does in a walk that meets the key
+        // beside others; that part holds written numbers whatever its weight)
+        if (a > 0.f || (own && s == splits && m != INFINITY)) {
           L += a * joined[s][i][1];
           acc += a * joined[s][i][4 + d];
         }
