@@ -195,10 +195,9 @@ attn_decode_kernel(
   const int lane = threadIdx.x & 63, i16 = lane & 15, g4 = lane >> 4;
   const int32_t* bt = block_table + (int64_t)b * max_blocks;
   const bf16* qp = q + (int64_t)row * ld_q + (int64_t)(hk * G + (i16 < G ? i16 : 0)) * D;
-  int k_lo, k_hi, kps;
+  int k_lo = 0, k_hi = 0, kps, seq = 0;   // (a wave that walks nothing asks for none of them)
   bf16x8 qf[1][KS];
   Tile<DT, 1, P2> tl;
-  int seq;
   bool writer = false;
   int w_pos = 0;
   int64_t w_slot = -1;
