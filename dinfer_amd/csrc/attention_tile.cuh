@@ -416,7 +416,11 @@ __global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu
   const int e = HEADS ? L % Hkv : L % H, rest = HEADS ? L / Hkv : L / H;
   int tile = HEADS ? 0 : tiles_x - 1 - rest % tiles_x, b = HEADS ? rest : rest / tiles_x;
   if constexpr (COUNT) {   // (64 requests at once)
-    const int ln = threadIdx.x & 63, reqs = tiles_x;
+    // (nothing of the count may outlive it: with the lane's number and the shuffles' own shared with the code below, 13 registers
+    // more, and eleven words more spilled at three row tiles, cost a portion behind 12,000 keys 4 %)
+    int ln = threadIdx.x & 63;
+    asm volatile("" : "+v"(ln));
+    const int reqs = tiles_x;
     int at = rest;
     b = -1;
     for (int b0 = 0; b0 < reqs && b < 0; b0 += 64) {
@@ -425,21 +429,19 @@ __global__ void __launch_bounds__(64 * flash_waves(HEADS)) __attribute__((amdgpu
       int upto = mine;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(upto, o, 64);
+        const int v = __builtin_amdgcn_ds_bpermute((ln - o) * 4, upto);   // (below lane 0: any lane, not taken)
         if (ln >= o) upto += v;
       }
       const unsigned long long holds = __ballot(at < upto);
       if (holds) {
         const int l = __ffsll((long long)holds) - 1;
         b = b0 + l;
-        tile = __shfl(upto, l, 64) - 1 - at;
+        tile = __builtin_amdgcn_readlane(upto, l) - 1 - at;
       } else {
-        at -= __shfl(upto, 63, 64);
+        at -= __builtin_amdgcn_readlane(upto, 63);
       }
     }
     if (b < 0) return;   // (the whole workgroup: every wave counts the same)
-    b = __builtin_amdgcn_readfirstlane(b);
-    tile = __builtin_amdgcn_readfirstlane(tile);
   }
   const int G = H / Hkv;
   const int hk = e % Hkv;

@@ -240,17 +240,21 @@ def test_attention_flash(H, Hkv, D, page, window):
 
 
 @pytest.mark.parametrize("skip", [False, True])
-@pytest.mark.parametrize("H,Hkv,D,new", [(4, 2, 64, [1] * 20 + [90, 1, 33] + [1] * 20), (4, 1, 128, [1] * 80 + [130, 1, 65]),
-                                         (64, 8, 128, [1] * 30 + [1000] + [1] * 8), (2, 2, 48, [40] + [1] * 66 + [17])])
-def test_attention_flash_counts_the_tiles_of_few_portions(H, Hkv, D, new, skip):
+@pytest.mark.parametrize("H,Hkv,D,page,window,tile,new", [
+    (4, 2, 64, 16, 0, 32, [1] * 20 + [290, 1, 33] + [1] * 20), (4, 1, 128, 16, 0, 32, [1] * 80 + [130, 1, 65]),
+    (2, 1, 32, 8, 0, 32, [1] * 20 + [161, 1, 160] + [1] * 40), (2, 2, 96, 24, 50, 32, [1] * 40 + [257, 31]),
+    (64, 8, 128, 16, 0, 48, [1] * 30 + [1000] + [1] * 8), (32, 8, 128, 24, 100, 48, [1] * 50 + [1500, 500] + [1] * 20),
+    (2, 2, 48, 16, 0, 32, [300] + [1] * 66 + [17]), (3, 1, 256, 16, 0, 16, [1] * 66 + [150, 1, 15, 17])])
+def test_attention_flash_counts_the_tiles_of_few_portions(H, Hkv, D, page, window, tile, new, skip):
     """A few portions among many single rows: workgroups for the tiles that exist only, over more requests than a wave counts at
     once, at 16, 32 and 48 rows a tile; single rows are served or left as they are."""
-    hist, page = [(7 * i + 3) % 90 for i in range(len(new))], 16
+    assert -(-max(new) // tile) * len(new) >= 4 * (sum(new) // tile + len(new))     # where the tiles are counted
+    hist = [(7 * i + 3) % 90 for i in range(len(new))]
     q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=13)
     out = torch.full((sum(new) + 1, H * D), 7.0, device=DEV, dtype=torch.bfloat16)
-    ops().attn_flash(q, out, kc, vc, m["bt"], m["cu"], m["sl"], len(new), sum(new), max(new), scale=D ** -0.5, window=0,
+    ops().attn_flash(q, out, kc, vc, m["bt"], m["cu"], m["sl"], len(new), sum(new), max(new), scale=D ** -0.5, window=window,
                      heads=H, kv_heads=Hkv, head_dim=D, page_size=page, skip_single=skip)
-    want = expected_attention(outs, hist, D ** -0.5, 0)
+    want = expected_attention(outs, hist, D ** -0.5, window)
     rows = torch.tensor([not (skip and n == 1) for n in new for _ in range(n)])
     got = out[:-1].double().cpu().view(-1, H, D)
     torch.testing.assert_close(got[rows], want[rows], rtol=2e-2, atol=2e-2)
