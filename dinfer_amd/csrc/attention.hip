@@ -522,6 +522,18 @@ __global__ void __launch_bounds__(64) attn_decode_merge_kernel(const float* __re
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p % 16) == 0; }
 
+// CUs of the current device (asked once per device).
+inline int compute_units() {
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!cached[dev]) {
+    int n = 0;
+    cached[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+  }
+  return cached[dev];
+}
+
 template <int DT>
 int launch_flash(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const bf16* kc, const bf16* vc,
                  const int32_t* bt, int64_t max_blocks, const int32_t* cu, const int32_t* sl, int num_reqs, int64_t tokens,
@@ -533,10 +545,9 @@ int launch_flash(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const b
   auto lds_of = [](int qt) { return (size_t)3 * qt * 64 * (sizeof(f32x4) * DT + 2 * sizeof(float)); };
   // 48 rows per workgroup at head size 128: every K and V fragment a wave loads serves three row tiles instead of two
   // (the path on which loads return is what this kernel fills first), at 256 registers, still two waves a SIMD.
-  // It pays where the step's rows still make several rounds of workgroups over the chip (measured, 32 heads: 3,072 rows
-  // 135 -> 121 us, 8,192 rows 783 -> 642 us = 34 % of the MFMA peak, 32,768 rows 37 %; 2,048 rows, 1,344 workgroups, level, behind 28,000
-  // keys 1,330 -> 1,302; a portion of 512 rows behind 30,000 keys, 352 workgroups instead of 512, loses 17 %). Head size
-  // 64 gains nothing. (Rows of at most two tiles a request never fill the third: many single rows of many heads are no case.)
+  // It pays where the rows still make several rounds of workgroups over the chip (measured, 32 heads: 3,072 rows
+  // 135 -> 121 us, 8,192 rows 783 -> 642 us = 34 % of the MFMA peak, 32,768 rows 37 %). Head size 64 gains nothing. (Rows of
+  // at most two tiles a request never fill the third: many single rows of many heads are no case.)
   const auto run = [&](auto qt) {
     constexpr int QT = decltype(qt)::value;
     const int tiles = (max_q_len + 16 * QT - 1) / (16 * QT);
@@ -558,24 +569,21 @@ int launch_flash(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const b
     return launch_status();
   };
   if constexpr (DT == 8) {
-    if (max_q_len > 32 && tokens / 48 * H >= 1300) return run(std::integral_constant<int, 3>{});
+    // One request, us at 32 and at 48 rows a tile (32 heads), from nothing and behind 8,000 keys: 992 workgroups of 48 rows 40 and
+    // 42, 285 and 254; 1,120 50 and 53, 340 and 326; 1,312 61 and 61, 380 and 363; 1,472 75 and 70, 449 and 384. Several begin
+    // later, taken for as long as the longest: 8 x 256 rows (1,536) 30 and 36, 4 x 500 (1,408) 35 and 40, behind 1,000 76 and
+    // 76. Where one is long and the others are not, fewer exist than that, and 48 rows have to save a round of the places,
+    // two a CU: behind 8,000 keys beside 12 rows 440 rows (360 workgroups, one round for two) 150 and 113 at 40 heads, 89 and
+    // 112 at 32 (288, one each); 1,000 rows of 32 heads (two each) 184 and 206, 1,500 (two for three) 274 and 245.
+    const int64_t longest = (int64_t)((max_q_len + 47) / 48) * num_reqs * H, places = 2 * compute_units();
+    auto rounds = [&](int64_t rows) { return (tokens / rows * H + places - 1) / places; };
+    const bool wide = num_reqs == 1 ? tokens / 48 * H >= 1300 : longest >= 2000 && rounds(48) < rounds(32);
+    if (max_q_len > 32 && wide) return run(std::integral_constant<int, 3>{});
   }
   if constexpr (DT <= 8) {
     if (max_q_len > 16) return run(std::integral_constant<int, 2>{});
   }
   return run(std::integral_constant<int, 1>{});
-}
-
-// CUs of the current device (asked once per device).
-inline int compute_units() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cached[dev]) {
-    int n = 0;
-    cached[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
-  }
-  return cached[dev];
 }
 
 // The form of the decode kernel for a launch. LATE exists where the new key is the kernel's business and its

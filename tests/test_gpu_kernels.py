@@ -249,6 +249,9 @@ def test_attention_flash_counts_the_tiles_of_few_portions(H, Hkv, D, page, windo
     """A few portions among many single rows: workgroups for the tiles that exist only, over more requests than a wave counts at
     once, at 16, 32 and 48 rows a tile; single rows are served or left as they are."""
     assert -(-max(new) // tile) * len(new) >= 4 * (sum(new) // tile + len(new))     # where the tiles are counted
+    if D == 128:    # 48 rows a tile where that saves a round of two workgroups a CU
+        places = 2 * torch.cuda.get_device_properties(0).multi_processor_count
+        assert (tile == 48) == (-(-(sum(new) // 48 * H) // places) < -(-(sum(new) // 32 * H) // places))
     hist = [(7 * i + 3) % 90 for i in range(len(new))]
     q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=13)
     out = torch.full((sum(new) + 1, H * D), 7.0, device=DEV, dtype=torch.bfloat16)
