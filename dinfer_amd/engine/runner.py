@@ -63,6 +63,23 @@ def _first_graph(device) -> None:
         torch.cuda.synchronize(device)
 
 
+def padded_full_batches(dtype: torch.dtype, layer_weights: int, has_state: bool) -> int:
+    """The most tokens of a full batch with portions that is padded by a made-up request, for a graph's sake. The made-up rows
+    are worth that where the host bounds the step, which takes some 110 us to launch a layer: in bfloat16, where a layer's
+    weights (all experts' among them, for a few dozen tokens choose nearly all) take the device far less to read, and the tokens'
+    products with them too. Launched one by one against padded and replayed, us a step:
+      28 layers of 16 million weights: 20 tokens 2,164 and 1,270, 100 3,072 and 1,583, 437 3,075 and 2,259, 1,000 3,072 and
+        2,930; beyond 1,024, where row counts are 128 apart, 1,030 (as 1,152) 3,109 and 3,172
+      4 of 66, with state of their own (the device also runs its recurrence): 20 511 and 380, 100 624 and 527, 195 639 and 645,
+        300 685 and 710
+      8 of 193: 20 970 and 994, 100 1,497 and 1,476, 437 2,203 and 2,196, 1,040 3,891 and 3,922; 8 of 330: 20 1,537 and 1,639
+      4 of 316 and 415, with 64 experts: 100 964 and 1,010, 1,225 and 1,307; 1,040 1,657 and 1,710, 2,540 and 2,629
+      in 32 bits, 28 of 16: 20 2,255 and 2,326, 195 3,664 and 3,797, 437 5,676 and 5,688"""
+    if dtype != torch.bfloat16 or layer_weights > 100_000_000:
+        return 0
+    return 128 if has_state else min(1023, max(128, 17_000_000_000 // max(layer_weights, 1)))
+
+
 class ModelRunner:
     def __init__(self, model: DecoderModel, options: EngineOptions, device: torch.device):
         options.check()
@@ -103,7 +120,7 @@ class ModelRunner:
         # steps with prompt portions: padded up to a few counts, and replayed from a graph of their own once the same
         # counts have come up PORTION_GRAPH_AFTER times (a capture costs about two eager steps)
         self._portion_graphs_allowed = self._graphs_allowed and model.capturable_portions()
-        self._layer_weights = model.layer_weights()
+        self._pad_full_up_to = padded_full_batches(self.dtype, model.layer_weights(), bool(self._slotted))
         self._portion_graphs: dict[tuple, torch.cuda.CUDAGraph] = {}
         self._portion_seen: dict[tuple, int] = {}
         self.portion_replays = 0            # steps with prompt portions served by a replay
@@ -367,8 +384,12 @@ class ModelRunner:
 
         The counts: tokens up to the next row count the matrix products round to anyway (16 at most where the
         step has no more: the few-row products take other forms there), requests up to the next
-        bucket of the decode graphs (or, where that is the most, one beyond), one logits row a request the engine admits (none if the step wants none), the longest portion up
-        to the next power of two, and which of the three ways single rows are served (all of them are, some, none)."""
+        bucket of the decode graphs (or, where that is the most, one beyond), one logits row a request the engine admits
+        (none if the step wants none), the longest portion up to the next power of two, and which of the three ways
+        single rows are served (all of them are, some, none).
+
+        A full batch, which needs a request more than the engine admits, stays as it is beyond _pad_full_up_to tokens, and
+        until its counts have come up often enough for a graph."""
         b, opt = self.batch, self.options
         T, B, R = b.num_tokens, b.num_reqs, b.num_rows
         if R > B or B > self._buckets[-1]:
@@ -385,24 +406,28 @@ class ModelRunner:
             break
         if Bp is None or Tp > self.max_tokens:
             return None
-        # A full batch has a made-up request only for the graph's sake, which is worth its rows where the host bounds the step: a
-        # layer's launches take it some 100 us, products of 2e10 multiplications about 60 us of the device beside its other
-        # kernels. Eager and padded, 28 layers of 16 million weights: 437 tokens 3,162 and 2,341 us, 1,000 3,157 and 3,009,
-        # 1,033 (as 1,152) 3,176 and 3,005, 2,023 4,616 and 4,719; wider layers: 437 tokens 1,697 and 1,734, 2,023 1,745 and
-        # 1,790, 3,343 and 3,428, 195 (as 224) 1,559 and 1,595. Up to 128 tokens the host bounds nearly all steps.
-        if Bp > self._buckets[-1] and T > 128 and T * self._layer_weights > 2e10:
+        full = Bp > self._buckets[-1]
+        if full and T > self._pad_full_up_to:
             return None
-        last = Tp - T - (Bp - B - 1) if Bp > B else 0         # tokens of the last made-up request
+        made_up = Bp - B
+        last = Tp - T - (made_up - 1) if made_up else 0       # tokens of the last made-up request
         if last > opt.max_model_len:
             return None
-        real_rows = R
-        b.pad(Bp, Tp, min(Bp, self._buckets[-1]) if R else 0)
-        q = b.max_q_len
-        qp = min(Tp, max(16, 1 << (q - 1).bit_length()))
-        route = 2 if b.num_singles == Bp else 1 if b.num_singles >= 4 else 0
+        rows = min(Bp, self._buckets[-1]) if R else 0
+        qp = min(Tp, max(16, 1 << (max(b.max_q_len, last) - 1).bit_length()))
+        singles = b.num_singles + max(made_up - 1, 0) + (last == 1)
+        route = 2 if singles == Bp else 1 if singles >= 4 else 0
+        key = (Tp, Bp, rows, qp, route)
+        if full and key not in self._portion_graphs:
+            # no graph, or none to come: nothing that the made-up rows would be worth
+            seen = self._portion_seen.get(key, 0) + 1
+            if seen < self.PORTION_GRAPH_AFTER or len(self._portion_graphs) >= self.MAX_PORTION_GRAPHS:
+                self._portion_seen[key] = seen
+                return None
+        b.pad(Bp, Tp, rows)
         b.max_q_len, b.all_decode = qp, route == 2
         b.num_singles = Bp if route == 2 else 4 if route == 1 else 0
-        return (Tp, Bp, b.num_rows, qp, route), real_rows
+        return key, R
 
     def _portion_step(self, fill) -> torch.Tensor:
         """A step with prompt portions: eager the first times its counts come up, then captured, then replayed."""

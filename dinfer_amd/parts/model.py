@@ -84,7 +84,7 @@ class DecoderModel:
         return expected_tensors(self.spec, self.blocks)
 
     def layer_weights(self) -> int:
-        """Weights of a layer, on the average over the layers."""
+        """Weights of a layer, all of its experts' among them, on the average over the layers."""
         return sum(math.prod(t.shape) for b in self.blocks for t in b.tensors().values()) // max(len(self.blocks), 1)
 
     def load(self, loader) -> None:

@@ -285,15 +285,23 @@ def test_fresh_slots_travel_with_the_step():
     assert b.fresh_slots.dtype == torch.int64 and b.fresh_slots.tolist() == [2, 0, 1, 3]
 
 
-@pytest.mark.parametrize("tokens,weights,padded", [(100, 10 ** 9, 128), (130, 10 ** 6, 160), (1033, 15 * 10 ** 6, 1152),
-                                                   (1033, 20 * 10 ** 6, None), (437, 4 * 10 ** 7, 448), (437, 5 * 10 ** 7, None)])
-def test_full_batches_are_padded_where_the_host_bounds_them(tokens, weights, padded):
-    """Up to 128 tokens always; beyond, where tokens times a layer's weights are few."""
-    from types import SimpleNamespace as N
-    from dinfer_amd.engine.runner import ModelRunner
-    pads = []
-    b = N(num_tokens=tokens, num_reqs=1, num_rows=1, max_q_len=tokens, num_singles=0, all_decode=False,
-          pad=lambda reqs, toks, rows: pads.append((reqs, toks)))
-    r = N(batch=b, options=N(max_model_len=4096), max_tokens=4096, _buckets=[1], _layer_weights=weights)
-    got = ModelRunner._portion_shape(r)
-    assert (got and got[0][0], pads) == (padded, [(2, padded)] if padded else [])
+def test_full_batches_are_padded_where_the_host_bounds_them():
+    """Layers that the device reads and multiplies faster than the host launches them; never wide ones, routed ones of 64 experts, or
+    32 bits."""
+    from dinfer_amd.config import get_architecture
+    from dinfer_amd.engine.runner import padded_full_batches
+    from dinfer_amd.parts import DecoderModel
+
+    def model(hidden, inter, heads):
+        arch = get_architecture("Qwen3ForCausalLM")
+        return DecoderModel(arch.build_spec(arch.config_class.from_dict(dict(
+            architectures=["Qwen3ForCausalLM"], model_type="qwen3", hidden_act="silu", attention_bias=False, vocab_size=1000,
+            hidden_size=hidden, intermediate_size=inter, num_hidden_layers=2, num_attention_heads=heads, num_key_value_heads=8,
+            head_dim=128, rms_norm_eps=1e-6, rope_theta=1e6, max_position_embeddings=40960, tie_word_embeddings=True))))
+
+    small, wide = model(1024, 3072, 16).layer_weights(), model(4096, 12288, 32).layer_weights()
+    assert small == 1024 * 128 * 48 + 3 * 1024 * 3072 + 2 * 1024 + 2 * 128
+    bf = torch.bfloat16
+    assert padded_full_batches(bf, small, False) == 1023 and padded_full_batches(bf, small, True) == 128
+    assert padded_full_batches(bf, wide, False) == padded_full_batches(torch.float32, small, False) == 0
+    assert padded_full_batches(bf, 64 * 3 * 2048 * 1408, True) == 0

@@ -394,3 +394,47 @@ def test_steps_with_portions_replayed_from_graphs(model_dirs, name, dtype):
         else:
             spread = got[False][k].std()
             assert float((got[True][k] - got[False][k]).abs().max() / spread) < 0.08, k
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_full_batches_with_portions_replayed(model_dirs, dtype):
+    """Steps that fill the engine's batch, of 100 and of 400 rows and beside a decoded row: in bfloat16 the first of its counts
+    runs as it is, the second padded, the others from a graph; every one against the same step run eagerly, with decode
+    steps between them. In 32 bits none is padded."""
+    name, ids, steps = "B", {}, []
+    for i in range(6):
+        for n, m in ((60, 40), (220, 180), (1, 97)):
+            pair = [f"r{len(ids) + j}" for j in range(2)]
+            for k, count in zip(pair, (n, m)):
+                ids[k] = tokens_for(name, max(count, 30) + 2, len(ids))
+            a, b = pair
+            if n == 1:
+                steps.append(([(a, ids[a][:30], [29])], []))
+                steps.append(([(a, ids[a][30:31], [0]), (b, ids[b][:m], [m - 1])], []))
+                steps.append(([(a, ids[a][31:], [0]), (b, ids[b][m:m + 1], [0])], [a, b]))
+            else:
+                steps.append(([(k, ids[k][:c], [c - 1]) for k, c in ((a, n), (b, m))], []))
+                steps.append(([(k, ids[k][c:c + 1], [0]) for k, c in ((a, n), (b, m))], [a, b]))
+    got, seen = {}, []
+    for graph in (False, True):
+        r = make_runner(model_dirs[name], name, dtype, max_tokens=512, max_len=256, max_seqs=2, graph=graph)
+        send = r._send
+        def counted(fill, pad, shape=None):
+            out = send(fill, pad, shape)
+            if shape is not None:
+                seen.append(r.batch.num_tokens)
+            return out
+        if graph:
+            r._send = counted
+        got[graph] = replay(r, steps)
+        if graph:
+            assert r.portion_replays == (4 if dtype == "float32" else 4 * 4)     # (prompts of 30 leave a request free)
+    per = [seen.count(n) for n in (100, 128, 400, 416, 98)]
+    assert per == ([6, 0, 6, 0, 6] if dtype == "float32" else [1, 10, 1, 5, 1])
+    assert got[True].keys() == got[False].keys()
+    for k in got[True]:
+        if dtype == "float32":
+            assert torch.equal(got[True][k], got[False][k]), k
+        else:
+            spread = got[False][k].std()
+            assert float((got[True][k] - got[False][k]).abs().max() / spread) < 0.08, k
