@@ -69,7 +69,8 @@ def padded_full_batches(dtype: torch.dtype, layer_weights: int, has_state: bool)
     weights (all experts' among them, for a few dozen tokens choose nearly all) take the device far less to read, and the tokens'
     products with them too. Launched one by one against padded and replayed, us a step:
       28 layers of 16 million weights: 20 tokens 2,164 and 1,270, 100 3,072 and 1,583, 437 3,075 and 2,259, 1,000 3,072 and
-        2,930; beyond 1,024, where row counts are 128 apart, 1,030 (as 1,152) 3,109 and 3,172
+        2,930; beyond 1,024, where row counts are 128 apart and the made-up rows up to an eighth, in short requests alone: 8 of
+        some 130 (as 1,152) 3,129 to 3,200 and 3,000 to 3,013 (beside a quicker host 2,961 and 3,066), one of 1,030 3,109 and 3,172
       4 of 66, with state of their own (the device also runs its recurrence): 20 511 and 380, 100 624 and 527, 195 639 and 645,
         300 685 and 710
       8 of 193: 20 970 and 994, 100 1,497 and 1,476, 437 2,203 and 2,196, 1,040 3,891 and 3,922; 8 of 330: 20 1,537 and 1,639
@@ -77,7 +78,7 @@ def padded_full_batches(dtype: torch.dtype, layer_weights: int, has_state: bool)
       in 32 bits, 28 of 16: 20 2,255 and 2,326, 195 3,664 and 3,797, 437 5,676 and 5,688"""
     if dtype != torch.bfloat16 or layer_weights > 100_000_000:
         return 0
-    return 128 if has_state else min(1023, max(128, 17_000_000_000 // max(layer_weights, 1)))
+    return 128 if has_state else max(128, 17_000_000_000 // max(layer_weights, 1))
 
 
 class ModelRunner:
@@ -407,7 +408,7 @@ class ModelRunner:
         if Bp is None or Tp > self.max_tokens:
             return None
         full = Bp > self._buckets[-1]
-        if full and T > self._pad_full_up_to:
+        if full and (T > self._pad_full_up_to or (Tp > 1024 and b.max_seq_len > 256)):
             return None
         made_up = Bp - B
         last = Tp - T - (made_up - 1) if made_up else 0       # tokens of the last made-up request

@@ -302,6 +302,6 @@ def test_full_batches_are_padded_where_the_host_bounds_them():
     small, wide = model(1024, 3072, 16).layer_weights(), model(4096, 12288, 32).layer_weights()
     assert small == 1024 * 128 * 48 + 3 * 1024 * 3072 + 2 * 1024 + 2 * 128
     bf = torch.bfloat16
-    assert padded_full_batches(bf, small, False) == 1023 and padded_full_batches(bf, small, True) == 128
+    assert 1040 <= padded_full_batches(bf, small, False) < 1100 and padded_full_batches(bf, small, True) == 128
     assert padded_full_batches(bf, wide, False) == padded_full_batches(torch.float32, small, False) == 0
     assert padded_full_batches(bf, 64 * 3 * 2048 * 1408, True) == 0
