@@ -22,7 +22,8 @@ def _slots(portions, page, blocks):
 
 
 @pytest.mark.parametrize("H,Hkv,D,style,extras", [(6, 3, 64, 0, True), (16, 8, 128, 0, False), (9, 1, 128, 1, True), (5, 5, 256, 0, True), (4, 2, 256, 1, False)])
-@pytest.mark.parametrize("portions", [[(0, 64)], [(5, 1), (0, 3), (3, 61), (8, 7), (16, 8), (1, 40)], [(i, 37 + i) for i in range(12)]])
+@pytest.mark.parametrize("portions", [[(0, 64)], [(5, 1), (0, 3), (3, 61), (8, 7), (16, 8), (1, 40)], [(i, 37 + i) for i in range(12)],
+                                      [(0, 512)], [(i, 43 + i) for i in range(12)]])     # from 512 tokens on four heads a workgroup
 def test_qkv_post_of_portions(H, Hkv, D, style, extras, portions):
     """The kernel for prompt portions leaves the bits of the kernel that takes single tokens, wherever portions begin."""
     page, blocks = 16, sum((a + n - 1) // 16 + 1 for a, n in portions)
@@ -99,9 +100,11 @@ def test_layernorm_of_many_rows(rows, width, x_dtype, out_dtype, branch):
     assert ((out.double() - want).abs() <= tol * (want.abs() + 1)).all()
 
 
-@pytest.mark.parametrize("rows,n", [(1, 8), (3, 72), (70, 2816), (600, 2056), (9, 16392 * 8)])
+@pytest.mark.parametrize("rows,n", [(131073, 8), (14564, 72), (400, 2816), (600, 2056), (9, 16392 * 8)])
 def test_activations_in_16_byte_pieces(rows, n):
-    """Rows that begin at a 16-byte piece against the same rows two entries further on, which are taken one by one."""
+    """Rows that begin at a 16-byte piece against the same rows two entries further on, which are taken one by one: rows of one
+    piece, more than a launch takes, and rows of more pieces than its workgroups of a row."""
+    assert rows * n >= 1 << 20      # fewer numbers are taken one by one wherever they begin
     g = torch.Generator().manual_seed(n)
     x, gates = torch.randn(rows, n, generator=g).to(BF) * 3, torch.randn(rows, n, generator=g).to(BF)
     for kind in ("silu", "relu2", "gelu", "gelu_tanh", "sigmoid"):
