@@ -167,7 +167,8 @@ constexpr int64_t STREAM_FROM_BYTES_FEW = 170 * 1000 * 1000;  // for one or two 
 // With POST that wave norms and rotates q and the new key in registers, scores the one with the other and stores key and value, while
 // the others walk the keys before it, so that nobody waits for a store to come back (one request of 250 keys, 16 heads on 8
 // of 128: 8.5 -> 7.7 us, in a step of 28 layers 1,019 -> 985; 8 requests 9.3 -> 8.5, 28 of 2,048 keys, 40 heads,
-// 45.1 -> 43.0; where the parts are workgroups of their own it loses 0.4 us and more from 2,048 keys on). Without POST, and for
+// 45.1 -> 43.0; where the parts are workgroups of their own it loses 0.4 us and more from 2,048 keys on). Where its at most
+// four parts meet, at 8 kv heads: engines of at most 256 positions, or 26 to 31 requests at any length. Without POST, and for
 // a row that is written nowhere, the wave walks that key: the same parts, the same bits.
 // stream_from: from this many bytes of keys and values in a step on (the request's own visible keys times the number
 // of requests: a wave knows no more) they are read with non-temporal loads.

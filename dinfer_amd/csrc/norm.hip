@@ -46,8 +46,9 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const S* __restrict__ x, S
 }
 
 // Float rows of at most 256 ITERS, kept in registers between the two phases, the gains asked for with the row; a thread has the
-// numbers it has in rmsnorm_kernel, so the bits are the same. Bound by the trips to memory: rows of 1,024 with a
-// residual, 1 to 32 of them 3.4 to 3.7 -> 2.5 to 2.8 us, 500 4.3 -> 3.3; 500 of 5,120 13.8 -> 7.0.
+// numbers it has in rmsnorm_kernel, so the bits are the same. Bound by the trips to memory: with a residual, over rows that
+// lie in the caches, 1 to 32 of 1,024 3.4 to 3.7 -> 2.5 to 2.8 us, 500 4.3 -> 3.3, 500 of 5,120 13.8 -> 7.0; behind the product that
+// writes them, as a layer runs it, 500 of 1,024 5.8 -> 5.5.
 template <int ITERS>
 __global__ void __launch_bounds__(256) rmsnorm_f32_regs_kernel(const float* __restrict__ x, float* __restrict__ residual,
                                                                const int32_t* __restrict__ rows, const float* __restrict__ w,

@@ -639,8 +639,8 @@ __global__ void __launch_bounds__(256) qkv_row_post_kernel(
 // bf16 rows of whole 16-byte pieces that no boundary of a head, of its rotated part or (style 0) of that part's halves cuts:
 // a thread owns one piece of 8 entries (ITERS of them) of q | k and keeps its bias and gains in registers for the per_block
 // tokens its workgroup goes through, one after the other with the next one's piece on its way. Pairs (2i, 2i + 1) lie in a
-// piece; for pairs (i, i + rot/2) the row passes through LDS. gather_v as in qkv_post_vec_kernel: then the workgroups from
-// blockIdx.x = `blocks` on write V (8 * WAVES tokens of a kv head each, by their first WAVES waves).
+// piece; for pairs (i, i + rot/2) the row passes through LDS. gather_v > 0: V is not written token by token, but by so many
+// workgroups from blockIdx.x = `blocks` on (8 * WAVES tokens of a kv head each, by their first WAVES waves).
 template <int ITERS>
 __global__ void __launch_bounds__(1024) qkv_row_post_vec_kernel(
     bf16* __restrict__ qkv, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, const float* __restrict__ wq,
@@ -882,8 +882,7 @@ extern "C" int dinfer_qkv_post(int dtype, void* qkv, int64_t tokens, int64_t ld,
                                      : (!cos_sin || rotary_dim == head_dim) && v_dim == head_dim && (v_cache || !slot_mapping);
   if (whole_head && vec_ok) {
     const int lph = head_dim / 8, hpw = 64 / lph;
-    // many tokens fill the chip with one workgroup each; few tokens spread their heads over several
-    // many tokens: V goes to its transposed pages through workgroups that gather it (16-byte stores)
+    // portions of many tokens: V goes to its transposed pages through workgroups that gather it (16-byte stores)
     const bool gather = slot_mapping && token_runs && tokens >= 64 && page_size % 8 == 0 && ((uintptr_t)v_cache % 16) == 0;
     const bool pairs = style == 1 && cos_sin;
     if (gather) {
@@ -907,6 +906,7 @@ extern "C" int dinfer_qkv_post(int dtype, void* qkv, int64_t tokens, int64_t ld,
 #undef DINFER_QKV_RUNS
       return launch_status();
     }
+    // many tokens fill the chip with one workgroup each; few tokens spread their heads over several
     const dim3 vgrid((unsigned)tokens, tokens >= 512 ? 1u : (unsigned)((items + WAVES * hpw - 1) / (WAVES * hpw)));
 #define DINFER_QKV_VEC(LPH_)                                                                                          \
   (pairs ? qkv_post_vec_kernel<LPH_, true> : qkv_post_vec_kernel<LPH_, false>)<<<vgrid, WAVES * 64, 0, stream>>>(      \
