@@ -305,3 +305,14 @@ def test_full_batches_are_padded_where_the_host_bounds_them():
     assert 1040 <= padded_full_batches(bf, small, False) < 1100 and padded_full_batches(bf, small, True) == 128
     assert padded_full_batches(bf, wide, False) == padded_full_batches(torch.float32, small, False) == 0
     assert padded_full_batches(bf, 64 * 3 * 2048 * 1408, True) == 0
+
+
+def test_parts_of_single_rows_beside_longer_ones():
+    """As many parts as a step of those rows alone would have where these come to 1,024 waves exactly, else as the whole step's."""
+    from dinfer_amd.kernels.attention import Workspace
+    ws = object.__new__(Workspace)
+    ws.max_splits, ws.kv_heads = 32, 8
+    assert [ws.splits_beside(n) for n in (5, 9, 17, 33, 65)] == [32, 16, 8, 4, 2] == [ws.splits(n - 1) for n in (5, 9, 17, 33, 65)]
+    assert all(ws.splits_beside(n) == ws.splits(n) for n in (1, 6, 7, 8, 11, 12, 30, 32, 64, 200))
+    ws.max_splits, ws.kv_heads = 4, 3       # 1,024 waves are no whole number of parts of 3 kv heads
+    assert all(ws.splits_beside(n) == ws.splits(n) for n in range(1, 100))
