@@ -163,7 +163,7 @@ ERRORS = {
 
 _libs: dict[str, ctypes.CDLL] = {}
 _funcs: dict[str, ctypes._CFuncPtr] = {}
-_lock = threading.Lock()
+_lock = threading.RLock()   # (taken again by a collected object's own call while this thread loads another library)
 
 
 class KernelError(RuntimeError):
@@ -171,6 +171,9 @@ class KernelError(RuntimeError):
 
 
 def load_library(name: str) -> ctypes.CDLL:
+    lib = _libs.get(name)
+    if lib is not None:     # a loaded one needs no lock
+        return lib
     with _lock:
         lib = _libs.get(name)
         if lib is not None:

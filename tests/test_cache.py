@@ -245,3 +245,24 @@ def test_random_prefix_traffic_keeps_the_invariants():
 def test_prefix_cache_refuses_window_groups():
     with pytest.raises(ValueError, match="every key"):
         CacheManager([GroupSpec(4, 8, 6)], 2, prefix_caching=True)
+
+
+def test_a_collected_manager_does_not_wait_for_a_library_that_is_being_loaded(monkeypatch):
+    """The collector may run while load_library holds its lock, in the same thread, and destroy a manager for the first time in the
+    process."""
+    import threading
+    from dinfer_amd import native
+    from dinfer_amd.kernels import lib
+    done = []
+
+    def load_and_collect():
+        m = CacheManager([GroupSpec(4, 8)], 2, prefix_caching=False)
+        monkeypatch.delitem(native._fns, "dh_cache_destroy", raising=False)
+        with lib._lock:
+            m.__del__()
+        done.append(True)
+
+    t = threading.Thread(target=load_and_collect, daemon=True)
+    t.start()
+    t.join(20)
+    assert done
