@@ -554,7 +554,7 @@ int launch_flash(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const b
     const int tiles = (max_q_len + 16 * QT - 1) / (16 * QT);
     // A workgroup for every tile that a request might have: beside decoding requests nearly all of them find none (31 of them and
     // a portion of 512 rows: 14,520 workgroups for 440), so there the tiles are counted up instead: that portion behind 1,024
-    // keys, 40 heads, 40 -> 36 us, 1,024 rows of 32 heads beside 48 requests 51 -> 29, 200 beside 16 17.7 -> 13.5. Where few are
+    // keys, 40 heads, 37 -> 29 us, 1,024 rows of 32 heads beside 48 requests 51 -> 29, 200 beside 16 17.7 -> 13.5. Where few are
     // empty the count is a microsecond more for nothing.
     const int64_t all = (int64_t)tiles * num_reqs, some = tokens / (16 * QT) + num_reqs;
     const bool count = all >= 4 * some;
