@@ -196,7 +196,7 @@ attn_decode_kernel(
   const int lane = threadIdx.x & 63, i16 = lane & 15, g4 = lane >> 4;
   const int32_t* bt = block_table + (int64_t)b * max_blocks;
   const bf16* qp = q + (int64_t)row * ld_q + (int64_t)(hk * G + (i16 < G ? i16 : 0)) * D;
-  int k_lo = 0, k_hi = 0, kps, seq = 0;   // (a wave that walks nothing asks for none of them)
+  int k_lo, k_hi, kps, seq;   // (not set, and not read, where the wave holds its part without a walk)
   bf16x8 qf[1][KS];
   Tile<DT, 1, P2> tl;
   bool writer = false;
@@ -326,7 +326,6 @@ attn_decode_kernel(
     }
     tl.init(kc, vc, bt, (int)max_blocks, hk, Hkv, ps, k_lo, k_hi, scale_log2e);
   }
-  const int col_lo[1] = {k_lo}, col_hi[1] = {k_hi};
   // (reading the first block before q is normed, or two blocks ahead, was measured at 1 and 8 requests: no gain)
   const auto partial = [&](int kb) { return kb < k_lo || kb + 32 > k_hi; };
   // Where a step's keys and values exceed the caches they are read past them (every layer has keys of its own, so
@@ -334,8 +333,8 @@ attn_decode_kernel(
   // 8 of 4k 33.6 -> 31.7; below about 100 MB a step the plain loads are faster (one request of 8k keys 19.0 against
   // 21.6 us, 4 of 2k 16.1 against 17.6; one or two requests up to 170 MB: one of 32k 39.7 against 42.1, of 48k 51.5
   // against 48.9). Both walks are in the kernel, the choice is uniform over the wave.
-  const int seen = window > 0 && window < seq ? window : seq;
   const auto walk = [&](auto hook) {
+    const int col_lo[1] = {k_lo}, col_hi[1] = {k_hi}, seen = window > 0 && window < seq ? window : seq;
     // (LATE is for many requests, whose keys exceed the caches at any length worth a thought)
     if (LATE || (int64_t)gridDim.z * seen * (Hkv * D * 4) >= stream_from)
       tl.template walk<false, true>(qf, col_lo, col_hi, partial, hook);
@@ -419,13 +418,14 @@ attn_decode_kernel(
       const int i = idx / D, d = idx - i * D;
       float M = -INFINITY;
       for (int s = 0; s < parts; ++s) M = fmaxf(M, joined[s][i][0]);
+      const int keep = own && M != INFINITY ? splits : -1;
       float L = 0.f, acc = 0.f;
       for (int s = 0; s < parts; ++s) {
         const float m = joined[s][i][0];
         const float a = m == -INFINITY ? 0.f : exp2f(m - M);
         // (the own part also at a weight of 0: what is no number in it stays so, as it does in a walk that meets the key
-        // beside others; that part holds written numbers whatever its weight)
-        if (a > 0.f || (own && s == splits && m != INFINITY)) {
+        // beside others; beside an infinite score it goes like the other parts)
+        if (a > 0.f || s == keep) {
           L += a * joined[s][i][1];
           acc += a * joined[s][i][4 + d];
         }
