@@ -19,7 +19,8 @@
 // A query (a column, l % 16) keeps its running maximum, sum and output column in
 // the same lanes through both products.
 //
-//   flash:  query rows with or without history, causal, optional window; a
+//   flash:  query rows with or without history, causal, optional window; many
+//           rows of head size 128 in attention_pair.cuh, all others here: a
 //           workgroup owns QT x 16 query rows of one head, its four waves walk a
 //           quarter of the keys each in blocks of 32 (online softmax in base 2)
 //           and combine their results in LDS.
@@ -39,9 +40,11 @@
 // paged: 64-key tiles, base-2 online softmax, P rounded to bf16 before P.V),
 // gqa_decode_v3_core.cuh:72-242 and gqa.cu:1423-1461 (split-K decode, merge of
 // (m, l, o) partials).
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
+#include "attention_pair.cuh"
 #include "attention_tile.cuh"
 
 using namespace dinfer;
@@ -535,6 +538,49 @@ inline int compute_units() {
   return cached[dev];
 }
 
+// The kernel of paired waves over all tiles of a step (see its header).
+template <bool HALVES>
+int launch_pair(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const bf16* kc, const bf16* vc, const int32_t* bt,
+                int64_t max_blocks, const int32_t* cu, const int32_t* sl, int num_reqs, int64_t tokens, int max_q_len, float scale,
+                int H, int Hkv, int ps, int skip_single, hipStream_t stream) {
+  constexpr int COLS = pair_columns(HALVES);
+  const int64_t G = H / Hkv, tiles = (max_q_len * G + COLS - 1) / COLS;
+  // (counted where most of the tiles that requests might have do not exist, as below)
+  const int64_t all = tiles * num_reqs, some = tokens * G / COLS + num_reqs;
+  const bool count = all >= 4 * some;
+  const int64_t blocks = (count ? some : all) * Hkv;
+  if (blocks > 0x7fffffff) return ERR_UNSUPPORTED;
+  auto kernel = attn_pair_kernel<HALVES>;
+  if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, pair_lds(HALVES)) != hipSuccess) return ERR_LAUNCH;
+  kernel<<<(unsigned)blocks, 512, pair_lds(HALVES), stream>>>(q, ld_q, out, ld_out, kc, vc, bt, max_blocks, cu, sl, num_reqs, (int)tiles,
+                                                              count, scale * LOG2E, H, Hkv, ps, skip_single);
+  return launch_status();
+}
+
+// (16 keys of a block lie in one page, and every row sees all keys before it)
+inline bool takes_pair(int ps, int window) { return window == 0 && ps >= 16 && (ps & (ps - 1)) == 0; }
+
+// Whether a step's rows are many enough for the kernel of paired waves: 0 no, 1 with 256 columns a workgroup, 2 with 128 and
+// two halves of the keys. One workgroup fills a CU, so what counts is how many there are for the CUs, w1 and w2, and whether they
+// end together: the tiles of a long request grow with the causal mask. us with the tile of rows, 1 and 2 (H heads over 8):
+//   one request from nothing     H 32: 1,000 rows (w2 256) 21.5, 30.6, 23.5; 1,300 (328) 31.8, 37.2, 31.7; 2,001 (w1 256)
+//                                57, 53, 48; 2,500 (320) 81, 68, 76; 4,000 165, 128, 150. H 16: 2,500 (w2 320) 44, 60, 42
+//   one behind 6,000             H 32: 1,300 200, 156, 176; 2,001 274, 213, 216; 4,000 583, 444, 477
+//   requests of few tiles        8 x 130 rows, H 16 (w2 192) 10.8, 13.7, 11.3; H 32 (w1 192) 16.3, 14.0, 20.7; H 40 20.3,
+//                                15.4, 21.1. 16 x 100 behind 500, H 16 (w2 256) 23.4, 26.9, 22.2; H 32 (w1 256) 41.8, 29.5, 40.6.
+//                                16 x 256, H 32 59, 49, 61; 4 x 500 behind 1,500, H 16 (w2 256) 49, 56, 40; H 32 90, 65, 71
+//   two of 1,000, H 16 (w2 256)  23.3, 32.8, 23.8
+inline int pair_form(int64_t tokens, int num_reqs, int max_q_len, int H, int Hkv) {
+  const int64_t G = H / Hkv, cus = compute_units();
+  const int64_t requests = std::max<int64_t>(1, std::min<int64_t>(num_reqs, (tokens + max_q_len / 2) / max_q_len));   // as long as the longest
+  auto tiles = [&](bool halves) { return (max_q_len * G + pair_columns(halves) - 1) / pair_columns(halves); };
+  const int64_t w1 = requests * tiles(false) * Hkv, w2 = requests * tiles(true) * Hkv;
+  if (w1 >= cus + cus / 4) return 1;
+  if (tiles(false) <= 10 && w1 >= cus - cus / 4) return 1;
+  if (w2 >= (num_reqs == 1 || tiles(false) > 6 ? cus + cus / 4 : cus)) return 2;
+  return 0;
+}
+
 template <int DT>
 int launch_flash(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const bf16* kc, const bf16* vc,
                  const int32_t* bt, int64_t max_blocks, const int32_t* cu, const int32_t* sl, int num_reqs, int64_t tokens,
@@ -570,6 +616,12 @@ int launch_flash(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const b
     return launch_status();
   };
   if constexpr (DT == 8) {
+    if (takes_pair(ps, window)) {
+      const int form = pair_form(tokens, num_reqs, max_q_len, H, Hkv);
+      if (form)
+        return (form == 1 ? launch_pair<false> : launch_pair<true>)(q, ld_q, out, ld_out, kc, vc, bt, max_blocks, cu, sl, num_reqs,
+                                                                    tokens, max_q_len, scale, H, Hkv, ps, skip_single, stream);
+    }
     // One request, us at 32 and at 48 rows a tile (32 heads), from nothing and behind 8,000 keys: 992 workgroups of 48 rows 40 and
     // 42, 285 and 254; 1,120 50 and 53, 340 and 326; 1,312 61 and 61, 380 and 363; 1,472 75 and 70, 449 and 384. Several begin
     // later, taken for as long as the longest: 8 x 256 rows (1,536) 30 and 36, 4 x 500 (1,408) 35 and 40, behind 1,000 76 and
@@ -652,6 +704,11 @@ extern "C" int dinfer_attn_mfma_supports(int head_dim, int page_size, int heads,
   if (!(page_size > 0 && page_size % 8 == 0 && kv_heads > 0 && heads % kv_heads == 0)) return 0;
   // the kernels keep the elements of one page (all kv heads) in 32-bit arithmetic
   return (int64_t)kv_heads * page_size * head_dim < (int64_t)1 << 30 ? 1 : 0;
+}
+
+// Which kernel dinfer_attn_flash takes at head size 128 without a window: 0 the tile of rows, 1 and 2 the paired waves' (see pair_form).
+extern "C" int dinfer_attn_flash_form(int64_t tokens, int num_reqs, int max_q_len, int heads, int kv_heads, int page_size) {
+  return takes_pair(page_size, 0) ? pair_form(tokens, num_reqs, max_q_len, heads, kv_heads) : 0;
 }
 
 // tokens: rows of all requests together. skip_single: requests with one row are left to the split-K kernel.

@@ -1237,6 +1237,11 @@ def _check_paged(q, out, k_cache, v_cache, block_table, seq_lens, num_reqs, head
     assert q.shape[1] >= heads * head_dim and out.shape[1] >= heads * (v_dim or head_dim)
 
 
+def attn_flash_form(tokens: int, num_reqs: int, max_q_len: int, heads: int, kv_heads: int, page_size: int) -> int:
+    """Which kernel attn_flash takes at head size 128 without a window (see dinfer_attn_flash_form)."""
+    return lib.get("dinfer_attn_flash_form")(tokens, num_reqs, max_q_len, heads, kv_heads, page_size)
+
+
 def attn_flash(q, out, k_cache, v_cache, block_table, cu_seqlens, seq_lens, num_reqs: int, tokens: int,
                max_q_len: int, *, scale: float, window: int, heads: int, kv_heads: int, head_dim: int,
                page_size: int, skip_single: bool = False):

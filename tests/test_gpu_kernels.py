@@ -485,6 +485,39 @@ def test_attention_flash_three_row_tiles_a_workgroup(window, page):
     torch.testing.assert_close(out.double().cpu().view(-1, H, D), want, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("H,Hkv,page,hist,new,skip,form", [
+    # all columns against every block: heads in groups of 1, 3 and 5, whole and ragged tiles, one to many blocks of 64 keys, ends on
+    # and beside a block's and a page's edge
+    (64, 64, 16, [0, 63, 130, 0, 70], [256, 65, 256, 1, 256], False, 1), (32, 32, 32, [0, 64, 500, 1, 31, 200], [257, 256, 255, 64, 63, 129], False, 1),
+    (40, 8, 16, [0] * 12, [128, 64, 63, 65, 1, 127, 129, 130, 100, 130, 130, 130], False, 1), (24, 8, 16, [3000], [3700], False, 1),
+    # halves of the keys: one block and none for the second group, an odd number of blocks, an even one
+    (64, 64, 16, [0, 0, 64], [200, 62, 130], False, 2), (16, 16, 64, [0, 40, 64, 128, 65, 63], [300, 24, 400, 399, 400, 64], False, 2),
+    (32, 8, 128, [700], [1310], False, 2), (8, 8, 16, [1000, 5, 0, 63], [1280, 1200, 1000, 1025], False, 2),
+    # few portions among many single rows: tiles are counted
+    (64, 8, 16, [9] * 30 + [100] + [70] * 8, [1] * 30 + [1290] + [1] * 8, True, 1), (32, 8, 16, [5] * 70 + [333], [1] * 70 + [1300], True, 2),
+    (32, 8, 16, [5] * 70 + [333, 80], [1] * 70 + [1300, 1], False, 2)])
+def test_attention_flash_paired_waves(H, Hkv, page, hist, new, skip, form):
+    """The kernel for long runs of rows at head size 128 in both forms, and which sizes take it. What the pages hold past a request's
+    keys is no number."""
+    D, T = 128, sum(new)
+    assert ops().attn_flash_form(T, len(new), max(new), H, Hkv, page) == form
+    assert ops().attn_flash_form(T, len(new), max(new), H, Hkv, 8) == 0 and ops().attn_flash_form(T, len(new), max(new), H, Hkv, 24) == 0
+    q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=17, sharp=4.0)
+    for b, (h, n) in enumerate(zip(hist, new)):
+        last = int(m["bt"][b, (h + n - 1) // page])
+        vc[last, :, :, (h + n - 1) % page + 1:] = float("nan")
+        kc.view(kc.shape[0], Hkv, D // 8, page, 8)[last, :, :, (h + n - 1) % page + 1:] = float("nan")
+    out = torch.full((T + 1, H * D), 7.0, device=DEV, dtype=torch.bfloat16)
+    ops().attn_flash(q, out, kc, vc, m["bt"], m["cu"], m["sl"], len(new), T, max(new), scale=D ** -0.5, window=0,
+                     heads=H, kv_heads=Hkv, head_dim=D, page_size=page, skip_single=skip)
+    want = expected_attention(outs, hist, D ** -0.5, 0, device=DEV)
+    rows = torch.tensor([not (skip and n == 1) for n in new for _ in range(n)])
+    got = out[:-1].double().cpu().view(-1, H, D)
+    # weights and results are rounded to 8 bits: half a unit of a weight, at most, on every value of size up to 5, and of the result
+    torch.testing.assert_close(got[rows], want[rows], rtol=2e-2, atol=2e-2)
+    assert (got[~rows] == 7.0).all() and (out[-1] == 7.0).all()
+
+
 @pytest.mark.parametrize("splits", [5, 3])   # parts merged by a kernel of their own, and inside the workgroup
 def test_attention_mixed_routes_single_rows_to_split_k(splits):
     H, Hkv, D, page = 16, 4, 128, 16
