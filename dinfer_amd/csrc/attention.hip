@@ -553,7 +553,7 @@ int launch_pair(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const bf
   auto kernel = attn_pair_kernel<HALVES>;
   if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, pair_lds(HALVES)) != hipSuccess) return ERR_LAUNCH;
   kernel<<<(unsigned)blocks, 512, pair_lds(HALVES), stream>>>(q, ld_q, out, ld_out, kc, vc, bt, max_blocks, cu, sl, num_reqs, (int)tiles,
-                                                              count, scale * LOG2E, H, Hkv, ps, skip_single);
+                                                              count, scale * LOG2E, H, Hkv, ps, skip_single, PairExpanded{});
   return launch_status();
 }
 

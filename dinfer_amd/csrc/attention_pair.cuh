@@ -56,18 +56,37 @@ constexpr int pair_ahead(bool halves) { return halves ? 2 : 3; }    // turns fro
 constexpr int pair_behind(bool halves) { return halves ? 2 : 1; }   // turns from a block of keys' loads to its values'
 constexpr int pair_keys(bool halves) { return pair_ahead(halves) + 1; }
 constexpr int pair_values(bool halves) { return pair_ahead(halves) - pair_behind(halves) + 2; }
-constexpr int pair_lds(bool halves) { return (pair_keys(halves) + pair_values(halves)) * PAIR_BLOCK * (halves ? 2 : 1); }
+constexpr int PAIR_ROT = 8192;      // bytes of 64 keys' rotated parts of 64 (EXPANDED)
+constexpr int pair_lds(bool halves, bool expanded = false) {
+  return (pair_keys(halves) * (PAIR_BLOCK + (expanded ? PAIR_ROT : 0)) + pair_values(halves) * PAIR_BLOCK) * (halves ? 2 : 1);
+}
+
+// EXPANDED: keys and values of every head made from a latent cache for this step (H of 16 keys' pages each, request after request
+// without a table), a key's last 64 entries shared by the heads: `rot`, a page of 16 keys [8 pieces][16][8] each. q holds the first 128
+// entries of a head's query, qr the others. gate (may be null): a row's outputs are multiplied by the sigmoid of entry h, or
+// (gate_entries) by that of entry 128 h + d.
+struct PairExpanded {
+  const bf16* rot;
+  const bf16* qr;
+  int64_t ld_qr;
+  int q_stride, qr_stride;   // from head to head
+  const bf16* gate;
+  int64_t ld_gate;
+  int gate_entries;
+};
 
 // ps: a power of two, 16 or more. count: `tiles_x` is not a request's tiles; those that exist are counted up over the requests.
-template <bool HALVES>
+template <bool HALVES, bool EXPANDED = false>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_pair_kernel(
     const bf16* __restrict__ q, int64_t ld_q, bf16* __restrict__ out, int64_t ld_out, const bf16* __restrict__ kc,
     const bf16* __restrict__ vc, const int32_t* __restrict__ block_table, int64_t max_blocks,
     const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ seq_lens, int num_reqs, int tiles_x, int count,
-    float scale_log2e, int H, int Hkv, int ps, int skip_single) {
+    float scale_log2e, int H, int Hkv, int ps, int skip_single, PairExpanded ex = PairExpanded{}) {
   constexpr int D = 128, COLS = pair_columns(HALVES);
   constexpr int AK = pair_ahead(HALVES), LAG = pair_behind(HALVES), AV = AK - LAG, NK = pair_keys(HALVES), NV = pair_values(HALVES);
   constexpr int LOADS = HALVES ? 4 : 2;   // instructions a wave brings of a block's 16 of keys, and of its values
+  constexpr int PIECES = EXPANDED ? 12 : 8, KEY_FRAGS = 2 * PIECES, KEY_BLOCK = PAIR_BLOCK + (EXPANDED ? PAIR_ROT : 0);
+  static_assert(!(HALVES && EXPANDED), "does not fit LDS");
   // (the reference the weights are taken against follows the maximum once that has risen by this much, in base-2 units: with 6
   // instead of 2 1 % faster, but the largest weights, 1 exactly where the reference is their own score, are rounded more often)
   constexpr float LAZY = 2.f;
@@ -120,6 +139,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   auto first_key = [&](int j) __attribute__((always_inline)) { return (HALVES ? 2 * j + grp : j) * 64; };
 
   // ---- loads: chunk c (16 keys) and quarter t of its pieces, or of its value rows, an instruction --------------------------
+  constexpr int VALUES = NK * KEY_BLOCK;   // where the ring of values begins
   char* const ring = pair_smem + (HALVES ? grp * (NK + NV) * PAIR_BLOCK : 0);
   const uint32_t ring_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
   const int n0 = member * LOADS;
@@ -131,12 +151,25 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int ps_shift = __builtin_ctz(ps), last_chunk = (all_hi - 1) >> 4;
   int chunk = (HALVES ? grp * 4 : 0) + (n0 >> 2), page;
   uint64_t k_at, v_at[LAG + 1];
-  const char *k_src, *v_src;
+  const char *k_src, *v_src, *r_src = nullptr;
+  int first_page = 0;                    // EXPANDED: the request's
+  if constexpr (EXPANDED) {
+    int ln = threadIdx.x & 63, pages = 0;
+    asm volatile("" : "+v"(ln));
+    for (int b0 = ln; b0 < b; b0 += 64) pages += (seq_lens[b0] + 15) >> 4;
+#pragma unroll
+    for (int x = 32; x > 0; x >>= 1) pages += __shfl_xor(pages, x, 64);
+    first_page = __builtin_amdgcn_readfirstlane(pages);
+  }
+  const char* const rh = (const char*)ex.rot + (uint32_t)((4 * (member & 1) + (lane >> 4)) * 16 + (lane & 15)) * 16;
   // The entry of the next block's chunk (past the last: that one again, its keys are masked), and a turn later what follows from it.
-  auto look = [&]() __attribute__((always_inline)) { page = bt[(min(chunk, last_chunk) << 4) >> ps_shift]; };
+  auto look = [&]() __attribute__((always_inline)) {
+    page = EXPANDED ? first_page + min(chunk, last_chunk) : bt[(min(chunk, last_chunk) << 4) >> ps_shift];
+  };
   auto aim = [&]() __attribute__((always_inline)) {
     const uint64_t at = (uint64_t)(uint32_t)page * page_bytes;
-    const int off = (min(chunk, last_chunk) << 4) & (ps - 1);
+    const int off = EXPANDED ? 0 : (min(chunk, last_chunk) << 4) & (ps - 1);
+    if constexpr (EXPANDED) r_src = rh + (uint64_t)(uint32_t)page * 2048;
     k_at = at + (uint32_t)(off * 16);
 #pragma unroll
     for (int i = 0; i < LAG; ++i) v_at[i] = v_at[i + 1];
@@ -144,19 +177,27 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     chunk += HALVES ? 8 : 4;
   };
   auto send_k = [&](int j, int x) __attribute__((always_inline)) {
-    load_to_lds(ring_at + (uint32_t)(j % NK * PAIR_BLOCK + (n0 + x) * 1024), k_src + (uint32_t)(x * 64 * ps));
+    load_to_lds(ring_at + (uint32_t)(j % NK * KEY_BLOCK + (n0 + x) * 1024), k_src + (uint32_t)(x * 64 * ps));
   };
   auto send_v = [&](int j, int x) __attribute__((always_inline)) {
-    load_to_lds(ring_at + (uint32_t)((NK + j % NV) * PAIR_BLOCK + (n0 + x) * 1024), v_src + (uint32_t)(x * 64 * ps));
+    load_to_lds(ring_at + (uint32_t)(VALUES + j % NV * PAIR_BLOCK + (n0 + x) * 1024), v_src + (uint32_t)(x * 64 * ps));
+  };
+  auto send_r = [&](int j) __attribute__((always_inline)) {   // (chunk member / 2: the one this wave brings keys of)
+    load_to_lds(ring_at + (uint32_t)(j % NK * KEY_BLOCK + PAIR_BLOCK + member * 1024), r_src);
   };
 
-  bf16x8 qf[8];
+  bf16x8 qf[PIECES];
   {
-    const bf16* qp = q + (int64_t)(q_begin + row) * ld_q + (int64_t)head * D + half * 8;
+    const bf16* qp = q + (int64_t)(q_begin + row) * ld_q + (int64_t)head * (EXPANDED ? ex.q_stride : D) + half * 8;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) qf[ks] = *(const bf16x8*)(qp + ks * 16);
+    if constexpr (EXPANDED) {
+      const bf16* rp = ex.qr + (int64_t)(q_begin + row) * ex.ld_qr + (int64_t)head * ex.qr_stride + half * 8;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]));   // here before the first counted wait
+      for (int ks = 8; ks < PIECES; ++ks) qf[ks] = *(const bf16x8*)(rp + (ks - 8) * 16);
+    }
+#pragma unroll
+    for (int ks = 0; ks < PIECES; ++ks) asm volatile("" : "+v"(qf[ks]));   // here before the first counted wait
   }
   f32x16 o[4], s[2];
 #pragma unroll
@@ -166,13 +207,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   float m = -INFINITY, l = 0.f;
   bf16x8 pf[4], fr[8];   // weights; fragments of keys and values, eight ahead
 
-  // fragment x of a turn's 32: keys (piece x / 2 of the tile x % 2), then values (chunk (x - 16) / 4, rows 32 (x % 4) ..)
-  const uint32_t k_frag = (uint32_t)((l32 >> 4) * 4096 + half * 256 + (8 * ((l32 >> 2) & 1) + 4 * ((l32 >> 3) & 1) + (l32 & 3)) * 16);
+  // a turn's fragments: keys (piece x / 2 of the tile x % 2), then values (chunk x / 4, rows 32 (x % 4) ..)
+  const uint32_t k_frag = (uint32_t)(half * 256 + (8 * ((l32 >> 2) & 1) + 4 * ((l32 >> 3) & 1) + (l32 & 3)) * 16), k_page = l32 >> 4;
   auto key_frag = [&](int j, int x) __attribute__((always_inline)) {
-    return *(const bf16x8*)(ring + j % NK * PAIR_BLOCK + k_frag + (x & 1) * 8192 + (x >> 1) * 512);
+    const char* at = ring + j % NK * KEY_BLOCK + k_frag;
+    return EXPANDED && x >= 16 ? *(const bf16x8*)(at + k_page * 2048 + PAIR_BLOCK + (x & 1) * 4096 + ((x >> 1) - 8) * 512)
+                               : *(const bf16x8*)(at + k_page * 4096 + (x & 1) * 8192 + (x >> 1) * 512);
   };
   auto value_frag = [&](int j, int x) __attribute__((always_inline)) {
-    return *(const bf16x8*)(ring + (NK + j % NV) * PAIR_BLOCK + lane * 16 + x * 1024);
+    return *(const bf16x8*)(ring + VALUES + j % NV * PAIR_BLOCK + lane * 16 + x * 1024);
   };
   auto first_frags = [&](int j) __attribute__((always_inline)) {
 #pragma unroll
@@ -188,7 +231,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   // the loads of the blocks ahead need (beside the softmax, which has no issue slots to spare, they cost 5 %).
   auto products = [&](int j, auto first, auto masked) __attribute__((always_inline)) {
     constexpr bool FIRST = decltype(first)::value, MASK = decltype(masked)::value;
-    constexpr int LAST = FIRST ? 16 : 32;
+    constexpr int LAST = KEY_FRAGS + (FIRST ? 0 : 16);
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -196,13 +239,13 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int x = 0; x < LAST; ++x) {
-      if (x < 16) {
+      if (x < KEY_FRAGS) {
         s[x & 1] = mfma32(fr[x & 7], qf[x >> 1], s[x & 1]);
       } else {
-        if constexpr (MASK) clean(fr[x & 7], first_key(j - 1) + 16 * ((x - 16) >> 2) + 8 * half);
-        o[x & 3] = mfma32(fr[x & 7], pf[(x - 16) >> 2], o[x & 3]);
+        if constexpr (MASK) clean(fr[x & 7], first_key(j - 1) + 16 * ((x - KEY_FRAGS) >> 2) + 8 * half);
+        o[x & 3] = mfma32(fr[x & 7], pf[(x - KEY_FRAGS) >> 2], o[x & 3]);
       }
-      if (x + 8 < LAST) fr[x & 7] = x + 8 < 16 ? key_frag(j, x + 8) : value_frag(j - 1, x - 8);
+      if (x + 8 < LAST) fr[x & 7] = x + 8 < KEY_FRAGS ? key_frag(j, x + 8) : value_frag(j - 1, x + 8 - KEY_FRAGS);
       if (x == 1) { aim(); k_src = kh + k_at; }
       if (x == 3) v_src = vh + v_at[0];
       if constexpr (HALVES) {
@@ -210,6 +253,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         if (x >= 9 && x < 13) send_k(j + AK, x - 9);
       } else {
         if (x == 4 || x == 6) send_k(j + AK, (x - 4) / 2);
+        if (EXPANDED && x == 8) send_r(j + AK);
         if (x == 9 || x == 12) send_v(j + AV, (x - 9) / 3);
       }
       if (x == LAST - 1) look();
@@ -260,8 +304,9 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   // way round. Behind barrier 2 j values j - 1 and keys j must have landed, behind 2 j + 1 keys j + 1 (the fragments that the first
   // group reads beside its softmax) and values j - 1; HALVES, where a group waits for its own loads only: keys j + 1 behind the
   // products of block j, values j - 1 before them. What may then still be on its way, in instructions of a wave:
-  constexpr int TOP_1 = HALVES ? 4 : least(4 * AV, 4 * AK - 2), END_1 = HALVES ? 8 : least(4 * AK - 2, 4 * AV + 4);
-  constexpr int TOP_2 = HALVES ? 4 : least(4 * AK - 6, 4 * AV), END_2 = HALVES ? 8 : least(4 * AV, 4 * AK - 2);
+  constexpr int TURN = EXPANDED ? 5 : 4;   // keys, then 2 of values
+  constexpr int TOP_1 = HALVES ? 4 : least(TURN * AV, TURN * (AK - 1) + 2), END_1 = HALVES ? 8 : least(TURN * (AK - 1) + 2, TURN * (AV + 1));
+  constexpr int TOP_2 = HALVES ? 4 : least(TURN * (AK - 2) + 2, TURN * AV), END_2 = HALVES ? 8 : TOP_1;
   static_assert(HALVES ? AK == 2 && AV == 0 : AV == AK - 1, "the counts above");
   auto turn = [&](int j, auto first, auto masked) __attribute__((always_inline)) {
     if (grp) loads_barrier<TOP_2>(); else loads_barrier<TOP_1>();
@@ -283,6 +328,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     k_src = kh + k_at;
 #pragma unroll
     for (int x = 0; x < LOADS; ++x) send_k(i, x);
+    if (EXPANDED) send_r(i);
     if (i >= LAG) {
       v_src = vh + v_at[0];
 #pragma unroll
@@ -290,7 +336,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
   }
   look();
-  loads_barrier<LOADS*(AK + AV - 1)>();   // keys 0
+  loads_barrier<HALVES ? 4 : TURN * (AK - 1)>();   // keys 0
   first_frags(0);
   if (grp) loads_barrier<END_2>();
   if (plain > 0) turn(0, Yes{}, No{}); else turn(0, Yes{}, Yes{});
@@ -337,8 +383,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       }
   }
   l += __shfl_xor(l, 32, 64);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  float inv = l > 0.f ? 1.f / l : 0.f;
   if (col >= q_len * G) return;
+  const bf16* gate = nullptr;
+  if constexpr (EXPANDED) {
+    if (ex.gate) {
+      gate = ex.gate + (int64_t)(q_begin + row) * ex.ld_gate + (ex.gate_entries ? head * D + 4 * half : head);
+      if (!ex.gate_entries) inv *= 1.f / (1.f + expf(-(float)*gate));
+    }
+  }
   bf16* op = out + (int64_t)(q_begin + row) * ld_out + (int64_t)head * D + 4 * half;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
@@ -347,6 +400,13 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       bf16x4 r;
 #pragma unroll
       for (int k = 0; k < 4; ++k) r[k] = (bf16)(o[t][4 * i + k] * inv);
+      if constexpr (EXPANDED) {
+        if (gate && ex.gate_entries) {
+          const bf16x4 g = *(const bf16x4*)(gate + 32 * t + 8 * i);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) r[k] = (bf16)(o[t][4 * i + k] * inv * (1.f / (1.f + expf(-(float)g[k]))));
+        }
+      }
       *(bf16x4*)(op + 32 * t + 8 * i) = r;
     }
 }

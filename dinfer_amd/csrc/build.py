@@ -37,6 +37,7 @@ SOURCES = {
     "gemm_mid": "gemm_mid.hip",
     "gemm_wide": "gemm_wide.hip",
     "latent": "latent.hip",
+    "latent_expand": "latent_expand.hip",
     "grouped": "grouped.hip",
     "delta": "delta.hip",
     "decay": "decay.hip",
@@ -50,7 +51,8 @@ SOURCES = {
 }
 HEADERS = ["common.cuh"]
 # headers of single libraries (their C interface, or device code two of them share), hashed with them
-OWN_HEADERS = {"gemm_mid": ["gemm_mid.h"], "attention": ["attention_tile.cuh", "attention_pair.cuh"], "attention_ext": ["attention_tile.cuh"]}
+OWN_HEADERS = {"gemm_mid": ["gemm_mid.h"], "attention": ["attention_tile.cuh", "attention_pair.cuh"], "attention_ext": ["attention_tile.cuh"],
+               "latent_expand": ["attention_tile.cuh", "attention_pair.cuh"]}
 # libraries without device code, and the headers each is made of
 HOST_ONLY = {"host": ["host/dinfer_host.h", "host/errors.hpp", "host/block_pool.hpp", "host/cache_manager.hpp",
                       "host/step_batch.hpp", "host/scheduler.hpp"]}

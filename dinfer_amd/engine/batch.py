@@ -93,6 +93,9 @@ class StepBatch:
         self.max_q_len = self.max_seq_len = self.num_singles = 0
         self.all_decode = False
         self.req_ids: list = []
+        # whether the host's lengths (h["seq_lens"]) are those of the step that runs (a graph captured now may be replayed for
+        # others), and what parts have worked out from them, for this step only
+        self.lengths_known, self.notes = False, {}
         self._copied = torch.cuda.Event() if pin else None
 
     @property
@@ -152,6 +155,7 @@ class StepBatch:
         self.num_tokens, self.num_reqs, self.num_rows = f.num_tokens, f.num_reqs, f.num_rows
         self.max_q_len, self.max_seq_len, self.num_singles = f.max_q_len, f.max_seq_len, f.num_singles
         self.all_decode = f.num_singles == f.num_reqs
+        self.lengths_known, self.notes = True, {}
 
     def pad(self, reqs: int, tokens: int, rows: int) -> None:
         """After fill(): made-up requests that write nothing bring the step to these counts (csrc/host/step_batch.hpp,

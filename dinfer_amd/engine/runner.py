@@ -390,10 +390,10 @@ class ModelRunner:
         single rows are served (all of them are, some, none).
 
         A full batch, which needs a request more than the engine admits, stays as it is beyond _pad_full_up_to tokens, and
-        until its counts have come up often enough for a graph."""
+        until its counts have come up often enough for a graph. So does a step whose requests' lengths a part wants to know."""
         b, opt = self.batch, self.options
         T, B, R = b.num_tokens, b.num_reqs, b.num_rows
-        if R > B or B > self._buckets[-1]:
+        if R > B or B > self._buckets[-1] or self.model.wants_lengths(T, B):
             return None
         later = [x for x in self._buckets if x >= B] + [self._buckets[-1] + 1]      # (a full batch: the spare request)
         Bp = Tp = None
@@ -427,6 +427,7 @@ class ModelRunner:
                 return None
         b.pad(Bp, Tp, rows)
         b.max_q_len, b.all_decode = qp, route == 2
+        b.lengths_known = False
         b.num_singles = Bp if route == 2 else 4 if route == 1 else 0
         return key, R
 

@@ -3,9 +3,13 @@
 float32 storage: always the plain kernel (fixed key order, any sizes). bfloat16 storage: the MFMA kernel where the
 sizes fit it (latent a multiple of 16 up to 512, rotated part a multiple of 8 up to 128, pages of a multiple of 8), with the keys of single rows cut into parts on the
 device; the plain kernel otherwise.
+
+Steps with many rows a request make the heads' keys and values again (Expanded) where the lengths of the requests are known and
+that is the lesser work.
 """
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from . import ops
@@ -44,3 +48,79 @@ def paged_attention(qa: torch.Tensor, out: torch.Tensor, cache: torch.Tensor, ca
         return ops.latent_attn_ref(qa, out, cache, bt, batch.cu_seqlens, batch.seq_lens, B, T, **geo)
     splits = ws.splits(B) if batch.all_decode else 1
     return ops.latent_attn_mfma(qa, out, cache, cache_t, bt, batch.cu_seqlens, batch.seq_lens, B, T, splits, ws.part, **geo)
+
+
+EXPANDED_BYTES = 512 << 20     # scratch for expanded keys and values, at most: 32 or 64 thousand keys of 32 or 16 heads
+CUS = 256
+
+
+class Expanded:
+    """Attention over keys and values made again from the latents (csrc/latent_expand.hip): scratch, sized once and shared by the
+    layers of one geometry, and the choice for a step."""
+
+    def __init__(self, ctx, heads: int, rank: int):
+        self.heads, self.rank = heads, rank
+        per_chunk = 2 * heads * 4096 + 2048
+        longest = ctx.max_seq_len or 4096
+        self.chunks = min(ctx.max_reqs * (-(-longest // 16) + 1), EXPANDED_BYTES // per_chunk)
+        buf = ctx.workspace.buffer
+        self.keys, self.values = (buf(f"latent_expanded_{n}", heads * 2048, rows=self.chunks) for n in ("keys", "values"))
+        self.rot = buf("latent_expanded_rot", 1024, rows=self.chunks)
+
+    @staticmethod
+    def supports(ctx, dim: int, rot_dim: int, vdim: int, rank: int) -> bool:
+        return ctx.dtype == torch.bfloat16 and ops.latent_expanded_supports(dim, rot_dim, vdim, rank, ctx.page_size)
+
+    def wants(self, tokens: int, num_reqs: int) -> bool:
+        """Whether a step of these counts may gain: then its requests' lengths are worth knowing (a replayed step's are not)."""
+        return tokens >= 128 * num_reqs
+
+    def plan(self, starts, counts):
+        """[(first request, requests, their keys, longest portion)] of the launches for requests of `counts` rows behind `starts`
+        keys, or None where the queries' side is the better one.
+
+        Both sides' times in us as measured with 16 heads of 128 + 64 over latents of 512. Queries' side: 77 ns a key of a round of
+        256 workgroups of 64 (row, head) pairs and 15.5 ns a row for the products around them; keys' side: 6.5 ns a key (1.3
+        PFLOP/s) and 2.3 us for 64 keys of 256 workgroups of 256 rows of a head, 1.7 where few run. 16 x 256 rows behind 1,000: 438
+        and 178; 16 x 130 87 and 45, behind 500 179 and 104; 16 x 128 behind 2,000 321 and 299; 16 x 64 behind 6,000 453 and 826;
+        2,048 rows from nothing 200 and 85; 512 behind 4,000 318 and 151."""
+        starts, counts = np.asarray(starts, dtype=np.float64), np.asarray(counts, dtype=np.float64)
+        scale = self.heads * self.rank / (16 * 512)
+        ends, middle = starts + counts, starts + counts / 2
+        groups = counts * self.heads / 64
+        queries = 0.077 * self.rank / 512 * max((groups * middle).sum() / CUS, ends.max()) + 0.0155 * scale * counts.sum()
+        tiles = np.ceil(counts / 256) * self.heads
+        keys = 0.0065 * scale * ends.sum() + max((tiles * middle).sum() / CUS * 2.3, ends.max() * 1.7) / 64
+        if keys > 0.9 * queries:
+            return None
+        lengths, rows = ends.astype(np.int64), counts.astype(np.int64)
+        launches, first, total = [], 0, 0
+        for i, n in enumerate(lengths.tolist()):
+            if n // 16 + 1 > self.chunks:
+                return None
+            if i > first and (total + n) // 16 + i - first + 1 > self.chunks:
+                launches.append((first, i - first, total, int(rows[first:i].max())))
+                first, total = i, 0
+            total += n
+        launches.append((first, len(lengths) - first, total, int(rows[first:].max())))
+        return launches
+
+    def launches(self, batch):
+        """plan() of the step in `batch`, worked out once a step; None for a step whose lengths are not known."""
+        if not batch.lengths_known or not self.wants(batch.num_tokens, batch.num_reqs):
+            return None
+        key = ("latent", self.heads, self.rank)
+        if key not in batch.notes:
+            B = batch.num_reqs
+            counts = np.diff(batch.h["cu_seqlens"][:B + 1])
+            batch.notes[key] = self.plan(batch.h["seq_lens"][:B] - counts, counts)
+        return batch.notes[key]
+
+    def attention(self, launches, q, q_off: int, qa, uk, uv, out, cache, batch, group: int, *, scale: float, page_size: int, gate,
+                  gate_off: int, gate_entries: bool):
+        """out [T, heads * 128]: the gated outputs of the heads."""
+        for first, reqs, total, longest in launches:
+            ops.latent_attn_expanded(q, qa, uk, uv, out, cache, batch.block_table[group], batch.cu_seqlens, batch.seq_lens, reqs, total,
+                                     longest, self.keys, self.values, self.rot, scale=scale, q_off=q_off, rank=self.rank,
+                                     page_size=page_size, gate=gate, gate_off=gate_off, gate_entries=gate_entries, first=first)
+        return out

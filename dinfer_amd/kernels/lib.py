@@ -30,6 +30,9 @@ SIGNATURES = {
     "dinfer_latent_post": ("latent", [_I, _P, _L, _L, _I, _I, _I, _I, _I, _I, _P, _I, _F, _P, _P, _I, _P, _L, _P, _P, _I, _P, _I,
                                       _P, _L, _P]),
     "dinfer_latent_mfma_supports": ("latent", [_I, _I, _I]),
+    "dinfer_latent_expanded_supports": ("latent_expand", [_I, _I, _I, _I, _I]),
+    "dinfer_latent_attn_expanded": ("latent_expand", [
+        _P, _L, _I, _P, _L, _I, _P, _P, _P, _L, _P, _L, _I, _P, _P, _L, _P, _P, _I, _L, _I, _F, _I, _I, _I, _P, _P, _P, _L, _P]),
     "dinfer_latent_attn_mfma": ("latent", [_P, _L, _P, _L, _P, _L, _P, _P, _P, _L, _P, _P, _I, _L, _F, _I, _I, _I, _I, _I, _I, _P]),
     "dinfer_latent_attn_ref": ("latent", [_I, _P, _L, _P, _L, _P, _P, _L, _P, _P, _I, _L, _F, _I, _I, _I, _I, _I, _P]),
     "dinfer_heads_nt": ("grouped", [_I, _P, _L, _L, _P, _L, _L, _P, _L, _L, _L, _L, _L, _L, _P, _L, _I, _P]),

@@ -908,6 +908,44 @@ def latent_attn_mfma(qa: torch.Tensor, out: torch.Tensor, cache: torch.Tensor, c
     return out
 
 
+def latent_expanded_supports(dim: int, rot_dim: int, vdim: int, rank: int, page_size: int) -> bool:
+    return bool(lib.get("dinfer_latent_expanded_supports")(dim, rot_dim, vdim, rank, page_size))
+
+
+def latent_attn_expanded(q: torch.Tensor, qa: torch.Tensor, uk: torch.Tensor, uv: torch.Tensor, out: torch.Tensor, cache: torch.Tensor,
+                         block_table: torch.Tensor, cu_seqlens: torch.Tensor, seq_lens: torch.Tensor, num_reqs: int, total_keys: int,
+                         max_q_len: int, keys: torch.Tensor, values: torch.Tensor, rot: torch.Tensor, *, scale: float, q_off: int,
+                         rank: int, page_size: int, gate: torch.Tensor | None = None, gate_off: int = 0, gate_entries: bool = False,
+                         first: int = 0) -> torch.Tensor:
+    """Latent attention with the heads' keys and values made again (bfloat16, sizes latent_expanded_supports names): requests
+    first .. first + num_reqs - 1 of the batch. q: the queries, head h's unrotated entries at q_off + h (dim + 64); qa: their rotated
+    parts where latent_post left them; uk, uv [heads, 128, rank]; out [T, heads * 128], the gated outputs of the heads. keys, values
+    [chunks, heads * 2048] and rot [chunks, 1024]: scratch for `chunks` pieces of 16 keys, total_keys / 16 + num_reqs at least;
+    total_keys: the requests' lengths summed up, or more."""
+    _need_gpu(q, qa, uk, uv, out, cache, block_table, cu_seqlens, seq_lens, keys, values, rot, gate)
+    heads, dim, _ = uk.shape
+    rot_dim = cache.shape[2] - rank
+    for t in (q, qa, uk, uv, out, cache, keys, values, rot):
+        assert t.dtype == torch.bfloat16
+    assert tuple(uk.shape) == tuple(uv.shape) == (heads, dim, rank) and uk.is_contiguous() and uv.is_contiguous()
+    assert cache.is_contiguous() and cache.shape[1] == page_size
+    assert block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.is_contiguous() and block_table.shape[0] >= first + num_reqs
+    assert cu_seqlens.dtype == seq_lens.dtype == torch.int32
+    assert cu_seqlens.numel() > first + num_reqs and seq_lens.numel() >= first + num_reqs
+    assert q_off + heads * (dim + rot_dim) <= q.shape[1] and qa.shape[1] >= heads * (rank + rot_dim) and out.shape[1] >= heads * dim
+    assert keys.is_contiguous() and values.is_contiguous() and rot.is_contiguous()
+    chunks = min(keys.numel() // (heads * 2048), values.numel() // (heads * 2048), rot.numel() // 1024)
+    if gate is not None:
+        assert gate.dtype == torch.bfloat16 and gate_off + heads * (dim if gate_entries else 1) <= gate.shape[1]
+    lib.call("dinfer_latent_attn_expanded", q.data_ptr() + q_off * 2, _rows(q), dim + rot_dim, qa.data_ptr() + rank * 2, _rows(qa),
+             rank + rot_dim, uk.data_ptr(), uv.data_ptr(), out.data_ptr(), _rows(out),
+             gate.data_ptr() + gate_off * 2 if gate is not None else 0, _rows(gate) if gate is not None else 0, int(gate_entries),
+             cache.data_ptr(), block_table.data_ptr() + first * block_table.shape[1] * 4, block_table.shape[1],
+             cu_seqlens.data_ptr() + first * 4, seq_lens.data_ptr() + first * 4, num_reqs, total_keys, max_q_len, float(scale), heads,
+             rank, page_size, keys.data_ptr(), values.data_ptr(), rot.data_ptr(), chunks, _stream())
+    return out
+
+
 # ---- many small products in one launch ---------------------------------------------------------------
 def heads_nt(a: torch.Tensor, a_off: int, a_stride: int, w: torch.Tensor, out: torch.Tensor, c_off: int, c_stride: int,
              m: int, *, gate: torch.Tensor | None = None, gate_off: int = 0, gate_entries: bool = False) -> torch.Tensor:

@@ -72,6 +72,11 @@ class Part:
     # the same promise for steps with prompt portions (see Mixer.capturable_portions)
     capturable_portions = True
 
+    def wants_lengths(self, tokens: int, num_reqs: int) -> bool:
+        """Whether forward may take a better way through a step of these counts where batch.lengths_known: such a step stays out
+        of the graphs."""
+        return False
+
     def tensors(self) -> dict[str, TensorSpec]:
         """Local tensor name -> what the weight file must hold for it."""
         return {}

@@ -58,6 +58,9 @@ class PreNormBlock(Block):
     def capturable_portions(self):
         return all(part.capturable and part.capturable_portions for _, part in self._parts())
 
+    def wants_lengths(self, tokens, num_reqs):
+        return any(part.wants_lengths(tokens, num_reqs) for _, part in self._parts())
+
     def tensors(self):
         return {p + n: s for p, part in self._parts() for n, s in part.tensors().items()}
 
@@ -147,6 +150,9 @@ class SandwichBlock(Block):
     @property
     def capturable_portions(self):
         return all(part.capturable and part.capturable_portions for _, part in self._parts())
+
+    def wants_lengths(self, tokens, num_reqs):
+        return any(part.wants_lengths(tokens, num_reqs) for _, part in self._parts())
 
     def tensors(self):
         t = {p + n: s for p, part in self._parts() for n, s in part.tensors().items()}
@@ -270,6 +276,9 @@ class OutNormBlock(Block):
     @property
     def capturable_portions(self):
         return all(part.capturable and part.capturable_portions for _, part in self._parts())
+
+    def wants_lengths(self, tokens, num_reqs):
+        return any(part.wants_lengths(tokens, num_reqs) for _, part in self._parts())
 
     def tensors(self):
         return {p + n: s for p, part in self._parts() for n, s in part.tensors().items()}

@@ -66,6 +66,9 @@ class JoinedMixers(Mixer):
     def capturable_portions(self):
         return all(m.capturable_portions for _, m, _, _ in self.members)
 
+    def wants_lengths(self, tokens, num_reqs):
+        return any(m.wants_lengths(tokens, num_reqs) for _, m, _, _ in self.members)
+
     def cache_spec(self):
         return JoinedSpec({name: m.cache_spec() for name, m, _, _ in self.members})
 

@@ -13,8 +13,9 @@ latent size:
 
 The cache holds [c | kr] per token (LatentSpec). The products with Wuk and Wuv are done on the query side:
 qa_h = Wuk_h^T qn_h, s = scale * <[qa_h | qr_h], [c | kr]>, and the attention's output in latent space is multiplied
-by Wuv_h afterwards, so no key or value is ever expanded and prompt portions and single decoded tokens run through
-the same kernels. A layer with `shares_cache` has no down projection: it reads the cache of the run entry it is
+by Wuv_h afterwards, so no key or value is expanded and prompt portions and single decoded tokens run through
+the same kernels; only where a step brings many rows a request, and the sizes have the kernels, are its keys and values made
+again for it (kernels/latent.py, Expanded). A layer with `shares_cache` has no down projection: it reads the cache of the run entry it is
 given (written by a layer whose latent sizes and rotation equal its own) with heads, Wuk and Wuv of its own.
 
 With `q_rank` the queries go through a latent of their own: cq = rmsnorm(Wdq h) * wq (the latent norm's kind and eps),
@@ -36,7 +37,7 @@ from .spec import LatentSpec, PartSpec, TensorSpec
 @MIXERS.register("latent_attention")
 class LatentAttention(Mixer):
     capturable = True            # every kernel reads tokens, positions, slots, tables and lengths from the batch's device buffers
-    capturable_portions = True   # the choice of kernels follows the step's counts alone
+    capturable_portions = True   # the choice of kernels follows the step's counts alone where lengths are not known
 
     def __init__(self, hidden: int, heads: int, dim: int, rot_dim: int, vdim: int, rank: int, scale: float,
                  position: PartSpec, latent_norm: PartSpec, gated: bool | str = True, shares_cache: bool = False,
@@ -63,6 +64,7 @@ class LatentAttention(Mixer):
         self.proj = Linear(hidden, -(-used // 8) * 8)      # q | down projection | gate in one product (rows padded to 8)
         self.used = used
         self.o = Linear(heads * vdim, hidden)
+        self.may_expand = self.dim == 128 and vdim == 128 and rot_dim == 64 and not window
         self.position = POSITION_ENCODINGS.get(position.kind)(head_dim=rot_dim, **position.params)
         if not self.position.fused:
             raise ValueError("latent attention rotates by a table: a position encoding of another kind has no kernel here")
@@ -122,6 +124,8 @@ class LatentAttention(Mixer):
         # Wuk_h^T [R, dn] per head: the query side of the key expansion; Wuv_h [dv, R] as stored
         self.uk_t = get(n["uk"], compute=True).view(H, self.dim, self.rank).transpose(1, 2).contiguous()
         self.uv = get(n["uv"], compute=True).view(H, self.vdim, self.rank).contiguous()
+        # (as stored once more, for the keys' side)
+        self.uk = get(n["uk"], compute=True).view(H, self.dim, self.rank).contiguous() if self.may_expand else None
         self.o.set_weight(get(n["o"], compute=True))
 
     def bind(self, ctx):
@@ -138,6 +142,12 @@ class LatentAttention(Mixer):
         self.attn_buf = ws.buffer("latent_heads", H * self.vdim)
         self.out_buf = ws.buffer("mixer_out", self.hidden)
         self.attn_ws = latent_kernels.Workspace(ctx, H, self.rank, self.rot_dim)
+        self.expanded = None
+        if self.may_expand and latent_kernels.Expanded.supports(ctx, self.dim, self.rot_dim, self.vdim, self.rank):
+            self.expanded = latent_kernels.Expanded(ctx, H, self.rank)
+
+    def wants_lengths(self, tokens, num_reqs):
+        return self.expanded is not None and self.expanded.wants(tokens, num_reqs)
 
     def forward(self, x, batch, cache: CacheView):
         T, g = batch.num_tokens, cache.group
@@ -154,6 +164,12 @@ class LatentAttention(Mixer):
                         cos_sin=self.position.table(), rotary_dim=self.position.rotary_dim, qa=self.qa_buf,
                         cache=cache.latent if write else None, slot_mapping=batch.slot_mapping[g] if write else None,
                         cache_t=cache.tensors.get("latent_t") if write else None, style=self.position.style, q_src=q_src)
+        launches = self.expanded.launches(batch) if self.expanded is not None else None
+        if launches:
+            self.expanded.attention(launches, self.proj_buf if q_src is None else q_src, 0, self.qa_buf, self.uk, self.uv, self.attn_buf,
+                                    cache.latent, batch, g, scale=self.scale, page_size=self.page_size,
+                                    gate=self.proj_buf if self.gated else None, gate_off=self.g_off, gate_entries=self.gate_entries)
+            return self.o.forward(self.attn_buf, self.out_buf, T, scratch=True)
         ops.heads_nt(self.proj_buf if q_src is None else q_src, 0, dn + dr, self.uk_t, self.qa_buf, 0, R + dr, T)
         latent_kernels.paged_attention(self.qa_buf, self.ol_buf, cache.latent, cache.tensors.get("latent_t"), batch, g,
                                        self.attn_ws, scale=self.scale,

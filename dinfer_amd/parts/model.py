@@ -142,6 +142,9 @@ class DecoderModel:
         return (self.capturable() and all(self.blocks[e.layer].capturable_portions for e in self.run)
                 and self.final_norm.capturable_portions)
 
+    def wants_lengths(self, tokens: int, num_reqs: int) -> bool:
+        return any(self.blocks[e.layer].wants_lengths(tokens, num_reqs) for e in self.run)
+
     # ---- execution -----------------------------------------------------------------------------
     def bind(self, ctx: BuildContext) -> None:
         self.ctx = ctx
