@@ -13,9 +13,9 @@
 // The same sums in another order as in latent.hip, with keys and values rounded where that form rounds queries and outputs.
 //
 // 16 heads over latents of 512, us with the products of the queries' side (which this form has not) and here: 16 x 256 rows behind
-// 1,000 keys 438 and 178 (some 130 for 20,096 keys, 1.3 PFLOP/s, and 48), 2,048 rows from nothing 200 and 85, 4,000 595 and 136,
+// 1,000 keys 438 and 178 (some 125 for 20,096 keys, 670 TFLOP/s, 165 MB written, and 48), 2,048 rows from nothing 200 and 85, 4,000 595 and 136,
 // 512 behind 4,000 318 and 151. Its error against 64 bits is no larger: 2.7e-3 for 3.1e-3 at the first of these. Bound by the matrix
-// cores: 4.2 million multiply-adds a key, 192 + 128 a head and score.
+// cores: 2.1 million multiply-adds a key, 192 + 128 a head and score.
 #include <algorithm>
 
 #include "attention_pair.cuh"
@@ -30,7 +30,8 @@ constexpr int ROWS = 256, KEYS = 256, STAGE = 32768, STAGES = 4;   // a tile; by
 // straight into LDS, 32 k a stage, three stages ahead, 16 rows x 64 bytes an instruction; a row's four pieces are exchanged by bits
 // 2 and 3 of its number, so that the fragments' reads meet no bank twice. Fragments are read one set of eight MFMAs ahead in program
 // order. Key tiles compute [weight rows][keys], value tiles [keys][weight rows]: a lane ends up with four consecutive entries of a
-// key's piece, or four consecutive keys of a value row, either way 8 bytes of what lies together.
+// key's piece, or four consecutive keys of a value row, either way 8 bytes of what lies together. (Two workgroups of 128 weight rows x 256
+// keys a CU, one's beginning and end beside the other's products: 20,096 keys 158 us for 125, more bytes of both operands a product.)
 template <bool VALUES>
 __device__ __forceinline__ void expand_tile(const char* const (&src)[4], int steps, char* lds, f32x16 (&acc)[2][4]) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;

@@ -80,8 +80,8 @@ class Expanded:
         keys, or None where the queries' side is the better one.
 
         Both sides' times in us as measured with 16 heads of 128 + 64 over latents of 512. Queries' side: 77 ns a key of a round of
-        256 workgroups of 64 (row, head) pairs and 15.5 ns a row for the products around them; keys' side: 6.5 ns a key (1.3
-        PFLOP/s) and 2.3 us for 64 keys of 256 workgroups of 256 rows of a head, 1.7 where few run. 16 x 256 rows behind 1,000: 438
+        256 workgroups of 64 (row, head) pairs and 15.5 ns a row for the products around them; keys' side: 6.5 ns a key
+        and 2.3 us for 64 keys of 256 workgroups of 256 rows of a head, 1.7 where few run. 16 x 256 rows behind 1,000: 438
         and 178; 16 x 130 87 and 45, behind 500 179 and 104; 16 x 128 behind 2,000 321 and 299; 16 x 64 behind 6,000 453 and 826;
         2,048 rows from nothing 200 and 85; 512 behind 4,000 318 and 151."""
         starts, counts = np.asarray(starts, dtype=np.float64), np.asarray(counts, dtype=np.float64)
