@@ -109,7 +109,7 @@ class Expanded:
         """plan() of the step in `batch`, worked out once a step; None for a step whose lengths are not known."""
         if not batch.lengths_known or not self.wants(batch.num_tokens, batch.num_reqs):
             return None
-        key = ("latent", self.heads, self.rank)
+        key = ("latent", self.heads, self.rank, self.chunks)
         if key not in batch.notes:
             B = batch.num_reqs
             counts = np.diff(batch.h["cu_seqlens"][:B + 1])

@@ -64,7 +64,9 @@ class LatentAttention(Mixer):
         self.proj = Linear(hidden, -(-used // 8) * 8)      # q | down projection | gate in one product (rows padded to 8)
         self.used = used
         self.o = Linear(heads * vdim, hidden)
-        self.may_expand = self.dim == 128 and vdim == 128 and rot_dim == 64 and not window
+        # (the keys' side reads an entry gate in fours: one that begins elsewhere, behind a query latent of such a rank, stays
+        # with the queries' side)
+        self.may_expand = self.dim == 128 and vdim == 128 and rot_dim == 64 and not window and not (self.gate_entries and self.g_off % 4)
         self.position = POSITION_ENCODINGS.get(position.kind)(head_dim=rot_dim, **position.params)
         if not self.position.fused:
             raise ValueError("latent attention rotates by a table: a position encoding of another kind has no kernel here")

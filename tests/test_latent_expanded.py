@@ -6,6 +6,8 @@ import pytest
 import torch
 
 from dinfer_amd.kernels import latent, ops
+from dinfer_amd.parts.latent_attention import LatentAttention
+from dinfer_amd.parts.spec import part
 
 DEV = "cuda"
 
@@ -45,6 +47,15 @@ def test_lengths_that_are_not_known_are_not_used():
     ex = made(16, 512, 4096)
     step = SimpleNamespace(lengths_known=False, num_tokens=4096, num_reqs=16, notes={})
     assert ex.launches(step) is None and not step.notes
+
+
+@pytest.mark.parametrize("q_rank,gated,window,taken", [(96, "entries", None, True), (98, "entries", None, False), (98, True, None, True),
+                                                       (None, "entries", None, True), (96, "entries", 64, False)])
+def test_an_entry_gate_that_begins_anywhere_keeps_its_way(q_rank, gated, window, taken):
+    position = part("rotary", theta=10000.0, max_positions=64, rotary_dim=64)
+    mixer = LatentAttention(256, 4, 128, 64, 128, 128, 0.1, position, part("rmsnorm", eps=1e-6, weight_name=""), gated=gated, q_rank=q_rank,
+                            window=window)
+    assert mixer.may_expand == taken
 
 
 @pytest.mark.gpu
