@@ -80,17 +80,17 @@ class Expanded:
         keys, or None where the queries' side is the better one.
 
         Both sides' times in us as measured with 16 heads of 128 + 64 over latents of 512. Queries' side: 77 ns a key of a round of
-        256 workgroups of 64 (row, head) pairs and 15.5 ns a row for the products around them; keys' side: 6.5 ns a key
-        and 2.3 us for 64 keys of 256 workgroups of 256 rows of a head, 1.7 where few run. 16 x 256 rows behind 1,000: 438
-        and 178; 16 x 130 87 and 45, behind 500 179 and 104; 16 x 128 behind 2,000 321 and 299; 16 x 64 behind 6,000 453 and 826;
-        2,048 rows from nothing 200 and 85; 512 behind 4,000 318 and 151."""
+        256 workgroups of 64 (row, head) pairs and 15.5 ns a row for the products around them; keys' side: 5.5 ns a key
+        and 2.3 us for 64 keys of 256 workgroups of 256 rows of a head, 1.7 where few run. 16 x 256 rows behind 1,000: 437
+        and 164; 16 x 130 87 and 45, behind 500 179 and 96; 16 x 128 behind 2,000 321 and 268; 16 x 64 behind 6,000 457 and 735;
+        2,048 rows from nothing 200 and 84; 512 behind 4,000 317 and 150."""
         starts, counts = np.asarray(starts, dtype=np.float64), np.asarray(counts, dtype=np.float64)
         scale = self.heads * self.rank / (16 * 512)
         ends, middle = starts + counts, starts + counts / 2
         groups = counts * self.heads / 64
         queries = 0.077 * self.rank / 512 * max((groups * middle).sum() / CUS, ends.max()) + 0.0155 * scale * counts.sum()
         tiles = np.ceil(counts / 256) * self.heads
-        keys = 0.0065 * scale * ends.sum() + max((tiles * middle).sum() / CUS * 2.3, ends.max() * 1.7) / 64
+        keys = 0.0055 * scale * ends.sum() + max((tiles * middle).sum() / CUS * 2.3, ends.max() * 1.7) / 64
         if keys > 0.9 * queries:
             return None
         lengths, rows = ends.astype(np.int64), counts.astype(np.int64)

@@ -62,7 +62,9 @@ def test_an_entry_gate_that_begins_anywhere_keeps_its_way(q_rank, gated, window,
 @pytest.mark.parametrize("H,R,page,hist,new,gate", [
     (16, 512, 16, [1000, 0, 17, 255, 256, 5], [256, 300, 5, 257, 1, 250], "heads"),   # edges of tiles of 256 keys and rows, of pieces of 16
     (3, 128, 32, [33, 0], [200, 64], None), (4, 384, 8, [0, 700, 9], [15, 513, 7], "entries"), (5, 160, 64, [100], [300], "heads"),
-    (2, 256, 16, [4000], [140], None)])
+    (2, 256, 16, [4000], [140], None),
+    (4, 128, 1, [i % 3 for i in range(4000)], [1 + i % 2 for i in range(4000)], "heads"),   # more tiles a workgroup than it looks up at once
+    (33, 128, 16, [700, 0, 31], [40, 1500, 2], None)])                                      # several tiles a workgroup, of keys and of values
 def test_expanded_attention(H, R, page, hist, new, gate):
     g = torch.Generator().manual_seed(H + R)
     rn = lambda *s: torch.randn(*s, generator=g)
