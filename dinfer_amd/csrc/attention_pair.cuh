@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "attention_tile.cuh"
+#include "lds_loads.cuh"
 
 namespace dinfer {
 namespace {
@@ -41,12 +42,6 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
 template <int N>
 __device__ __forceinline__ void loads_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-// 16 bytes a lane from `at` to LDS, lane after lane from byte `lds` on. (Not the builtin: behind it the compiler waits for all loads
-// on their way before every read of LDS.)
-__device__ __forceinline__ void load_to_lds(uint32_t lds, const char* at) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(at) : "m0");
 }
 
 constexpr int least(int a, int b) { return a < b ? a : b; }

@@ -51,8 +51,8 @@ SOURCES = {
 }
 HEADERS = ["common.cuh"]
 # headers of single libraries (their C interface, or device code two of them share), hashed with them
-OWN_HEADERS = {"gemm_mid": ["gemm_mid.h"], "attention": ["attention_tile.cuh", "attention_pair.cuh"], "attention_ext": ["attention_tile.cuh"],
-               "latent_expand": ["attention_tile.cuh", "attention_pair.cuh"]}
+OWN_HEADERS = {"gemm_mid": ["gemm_mid.h"], "attention": ["attention_tile.cuh", "attention_pair.cuh", "lds_loads.cuh"], "attention_ext": ["attention_tile.cuh"],
+               "latent_expand": ["attention_tile.cuh", "attention_pair.cuh", "lds_loads.cuh"], "grouped": ["lds_loads.cuh"]}
 # libraries without device code, and the headers each is made of
 HOST_ONLY = {"host": ["host/dinfer_host.h", "host/errors.hpp", "host/block_pool.hpp", "host/cache_manager.hpp",
                       "host/step_batch.hpp", "host/scheduler.hpp"]}

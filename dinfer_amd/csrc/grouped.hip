@@ -30,7 +30,9 @@
 //   moe_scatter  counts, offsets, the sorted list and the work list, one workgroup (LDS counters)
 //   moe_combine  out[t] = sum_c share[t, c] * y[t * top + c] + shared_gate[t] * shared[t]   (no gate: + shared[t]; no
 //                shares: every row of y counts as it is)
-#include "common.cuh"
+#include <type_traits>
+
+#include "lds_loads.cuh"
 
 using namespace dinfer;
 
@@ -404,8 +406,8 @@ __device__ __forceinline__ void swap_in_quads(u32x4& x0, u32x4& x1) {
 
 // 32 rows of a wave (from row m0 of the tile on): a lane holds, of row m0 + lane % 32, 16 columns from n0 + 16 (lane / 32)
 // on of the wave's two tiles of columns (gated: of the same columns of both halves).
-template <class O, int END>
-__device__ __forceinline__ void store_rows(const Groups& p, const Tile& tl, int m0, int c0, const f32x16 (&acc)[2]) {
+template <class O, int END, class Rows>
+__device__ __forceinline__ void store_rows(const Groups& p, const Rows& tl, int m0, int c0, const f32x16 (&acc)[2]) {
   constexpr bool GATED = END >= END_GATED;
   const int lane = threadIdx.x & 63, row = m0 + (lane & 31);
   if (row < tl.rows) {
@@ -587,6 +589,179 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_experts_kernel(Groups p) 
 #pragma unroll
   for (int h = 0; h < BLOCKS; ++h)
     if (h < live) store_rows<O, END>(p, tl, h * 32, c0, acc[h]);
+}
+
+// The same products where there are many tiles and K is a multiple of 64: one workgroup of eight waves a CU walks its tiles of 128
+// rows x 256 columns (gated: 128 of each half), a wave four blocks of 32 x 32: rows 32 (2 a + wave % 2), columns 64 (wave / 2) on.
+// Both operands go from memory straight into LDS, 64 k a stage, eight rows x 128 bytes an instruction, into three stages; where the
+// tiles lie is looked up for WALK_TILES of them before the first, the last three steps of a tile send the first stages of the next, and
+// its results leave beside the next one's products. A step reads the second half of its own stage beside the first eight MFMAs of a
+// wave and the first half of the next one's beside the other eight; in between all meet, and the step's own place is sent anew.
+// A row's eight pieces are exchanged so that 16 lanes, which LDS serves at once, find their own banks: by bits 1..3 of a row of A, by
+// bits 1, 2 and 4 of one of the weights, whose rows are read in the order of store_rows.
+//
+// Bound by the loads' way into a CU (64 bytes a cycle: 768 cycles a step of 1,024 of MFMAs) and the MFMAs, which do not overlap
+// wholly (1,650 a step), and by the ends of tiles, where nothing else runs (gelu by the error function 18,000 cycles of 72,000). Loads in
+// pieces of 64 bytes a row take the way into a CU twice as long (72 GB/s for 137, from L2): with stages of 32 k these products
+// were no faster than those of the kernel above. 64 experts of 1,408 in a width of 2,048, us there and here: 190 rows each gelu 168 and 133,
+// down 116 and 114, gated 230 and 221; 60 to 320 rows 161 and 134, 118 and 113, 240 and 238; 512 each 269 and 252, 232 and 217,
+// 445 and 415. Few tiles end unevenly (the kernel above has two workgroups a CU): 96 rows each 109 and 115, 82 and 87, 175 and 172.
+constexpr int WALK_K = 64, WALK_STAGES = 3, WALK_A = TM_BIG * WALK_K * 2, WALK_STAGE = WALK_A + 256 * WALK_K * 2, WALK_TILES = 28;
+struct WalkTile {
+  int z, base, rows, bx;
+};
+constexpr int WALK_LDS = WALK_STAGES * WALK_STAGE + WALK_TILES * (TM_BIG * 4 + (int)sizeof(WalkTile)) + 16;
+
+// the rows of a tile as store_rows asks for them, from the list in LDS
+struct ListedRows {
+  int rows, base, c_to_perm;
+  const int* list;
+  __device__ __forceinline__ int64_t c_row(int r) const { return c_to_perm ? list[r] : base + r; }
+  __device__ __forceinline__ float scale_of(const Groups& p, int r) const { return p.row_scale ? p.row_scale[list[r]] : 1.f; }
+};
+
+template <class O, int END>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) grouped_mfma_walk_kernel(Groups p) {
+  constexpr bool GATED = END >= END_GATED;
+  constexpr int COLS = GATED ? 32 : 64, NS = WALK_STAGES;
+  extern __shared__ __attribute__((aligned(1024))) char walk_smem[];
+  WalkTile* const tiles = (WalkTile*)(walk_smem + NS * WALK_STAGE);
+  int* const count = (int*)(tiles + WALK_TILES);
+  int* const lists = count + 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
+  const int wm = wave & 1, wn = wave >> 1;   // this wave's 64 rows, and 64 columns (gated: 32 of each half)
+  const int nx = (p.N + 4 * COLS - 1) / (4 * COLS), steps = p.K / WALK_K;
+  const int xcd = blockIdx.x & 7, stride = gridDim.x >> 3;
+  const int64_t slots = (p.max_tiles + 31) / 32 * (int64_t)(4 * nx);   // of an XCD
+  const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)walk_smem;
+  // what this wave sends of a stage: 16 rows of A, 32 of the weights; a row's four pieces are exchanged (see the fragments)
+  const char* src[6];
+  uint32_t to = 0;   // the stage of the step, bytes
+  const uint32_t fa_at = (uint32_t)((wm * 32 + l32) * 128 + ((half ^ ((l32 >> 1) & 7)) * 16));
+  const int wr = 16 * ((l32 >> 2) & 1) + 4 * (l32 >> 3) + (l32 & 3);
+  const uint32_t fw_at = (uint32_t)(WALK_A + (wn * 64 + wr) * 128 + ((half ^ (((wr >> 1) & 3) | ((wr >> 4) & 1) << 2)) * 16));
+  bf16x8 fa[2][2][2], fw[2][2][2];   // [step's parity][16 k][rows, columns]
+
+  for (int64_t t0 = blockIdx.x >> 3; t0 < slots; t0 += (int64_t)stride * WALK_TILES) {
+    if (wave == 0) {
+      const int64_t slot = t0 + (int64_t)lane * stride, group = slot / (4 * nx);
+      const int r = (int)(slot % (4 * nx));
+      const int64_t by = (group * 4 + (r & 3)) * 8 + xcd;
+      const int z = lane < WALK_TILES && by < p.max_tiles ? p.tiles[2 * by] : -1;
+      const int base = z >= 0 ? p.tiles[2 * by + 1] : 0, rows = z >= 0 ? min(p.offsets[z + 1] - base, TM_BIG) : 0;
+      const unsigned long long there = __ballot(rows > 0);
+      if (rows > 0) tiles[__popcll(there & ((1ull << lane) - 1))] = WalkTile{z, base, rows, r >> 2};
+      if (lane == 0) *count = __popcll(there);
+    }
+    __syncthreads();
+    const int n = __builtin_amdgcn_readfirstlane(*count);
+    for (int e = threadIdx.x; e < n * TM_BIG; e += 512) {   // (rows beyond a tile's: its first again, computed and not stored)
+      const WalkTile t = tiles[e / TM_BIG];
+      const int r = e % TM_BIG;
+      lists[e] = p.perm[t.base + (r < t.rows ? r : 0)];
+    }
+    __syncthreads();
+    auto sources = [&](int i) __attribute__((always_inline)) {
+      int lane = threadIdx.x & 63;
+      asm volatile("" : "+v"(lane));   // (nothing of this lives on in registers)
+      const WalkTile t = tiles[i];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int r = wave * 16 + x * 8 + (lane >> 3);
+        const int64_t row = p.a_div > 0 ? lists[i * TM_BIG + r] / p.a_div : t.base + (r < t.rows ? r : 0);
+        src[x] = (const char*)p.A + row * p.lda * 2 + ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int q = wave * 32 + x * 8 + (lane >> 3), c0 = (t.bx * 4 + (q >> 6)) * COLS, r = q & 31;
+        const int64_t w = GATED ? (int64_t)((q >> 5) & 1) * p.N + min(c0 + r, p.N - 1) : min(c0 + (q & 63), p.N - 1);
+        src[2 + x] = (const char*)p.W + (t.z * p.w_zs + w * p.ldw) * 2 + ((lane & 7) ^ (((q >> 1) & 3) | ((q >> 4) & 1) << 2)) * 16;
+      }
+    };
+    auto send = [&](uint32_t stage, int x) __attribute__((always_inline)) {
+      load_to_lds(lds + stage + (x < 2 ? wave * 2048 + x * 1024 : WALK_A + wave * 4096 + (x - 2) * 1024), src[x]);
+      src[x] += WALK_K * 2;
+    };
+    auto frag = [&](uint32_t stage, int b, int x) __attribute__((always_inline)) {   // x: 4 u + (columns 0, 1, rows 0, 1)
+      const char* at = walk_smem + stage;
+      const int u = x >> 2;
+      if ((x & 3) < 2) fw[b][u][x & 1] = *(const bf16x8*)(at + (fw_at ^ ((2 * b + u) * 32)) + (x & 1) * 4096);
+      else fa[b][u][x & 1] = *(const bf16x8*)(at + (fa_at ^ ((2 * b + u) * 32)) + (x & 1) * 8192);
+    };
+    if (n == 0) { __syncthreads(); continue; }
+    sources(0);
+#pragma unroll
+    for (int x = 0; x < 6; ++x) asm volatile("" : "+v"(src[x]));
+    to = 0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int x = 0; x < 6; ++x) send(s * WALK_STAGE, x);
+    asm volatile("s_waitcnt vmcnt(6)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int x = 0; x < 8; ++x) frag(0, 0, x);
+
+    for (int i = 0; i < n; ++i) {
+      const int rows = __builtin_amdgcn_readfirstlane(tiles[i].rows), bx = __builtin_amdgcn_readfirstlane(tiles[i].bx);
+      const int c0 = (bx * 4 + wn) * COLS;
+      const int live = c0 < p.N ? ((rows + 31) / 32 + 1 - wm) / 2 : 0;   // blocks of 32 rows that hold any
+      f32x16 acc[2][2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[a][j][e] = 0.f;
+      auto step = [&](int s, auto blocks) __attribute__((always_inline)) {
+        constexpr int LIVE = decltype(blocks)::value;
+        if (s == steps - NS) sources(min(i + 1, n - 1));   // (past the last tile: its own first stages again, which nobody reads)
+        const uint32_t ahead = to + WALK_STAGE == NS * WALK_STAGE ? 0 : to + WALK_STAGE;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+#pragma unroll
+          for (int x = 0; x < 8; ++x) {
+            const int u = x >> 2, a = (x >> 1) & 1, j = x & 1;
+            if (a < LIVE) acc[a][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[b][u][j], fa[b][u][a], acc[a][j], 0, 0, 0);
+            if (LIVE > 0 && x < 4) {
+              frag(b ? ahead : to, b ^ 1, 2 * x);
+              frag(b ? ahead : to, b ^ 1, 2 * x + 1);
+            }
+            if (b == 1 && x >= 1 && x < 7) send(to, x - 1);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          // Stage s + 1 is here (the first two of a tile were waited for at the end of the one before), and every wave has all of
+          // stage s in registers: its place is free for stage s + 3.
+          if (b == 0) {
+            if (s < 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        to = ahead;
+      };
+      auto tile = [&](auto blocks) __attribute__((always_inline)) {
+#pragma nounroll
+        for (int s = 0; s < steps; ++s) step(s, blocks);
+      };
+      if (live == 2) tile(std::integral_constant<int, 2>{});
+      else if (live == 1) tile(std::integral_constant<int, 1>{});
+      else {
+        tile(std::integral_constant<int, 0>{});
+        if (i + 1 < n) {   // (the next tile's first fragments all the same: its stage 0 is here since the last step)
+#pragma unroll
+          for (int x = 0; x < 8; ++x) frag(to, 0, x);
+        }
+      }
+      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");   // the next tile's first four stages (its products do not wait for the stores)
+      const ListedRows tl{rows, __builtin_amdgcn_readfirstlane(tiles[i].base), p.c_to_perm, lists + i * TM_BIG};
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+        if (a < live) store_rows<O, END>(p, tl, (2 * a + wm) * 32, c0, acc[a]);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing on its way into LDS
+    __syncthreads();
+  }
 }
 
 // Few rows (tiles of 16: steps of single tokens): time is the time to stream the weights, so a workgroup takes only 32
@@ -1123,11 +1298,31 @@ __global__ void __launch_bounds__(256) moe_combine_bf16x8_kernel(const bf16* __r
 
 // grid.y arrives from the caller (tiles or blocks of rows), grid.z too (groups); grid.x is set here from the kernel's
 // columns a workgroup.
+// Whether the tiles are many enough to be walked, by the full ones that the entries would fill (the experts' number is not known
+// here). us at 64 experts of 1,408 in a width of 2,048, by the kernel above and walked, full tiles in brackets: gelu 96 rows each
+// (288) 109 and 115; 128 (384) 118 and 119; 60 to 320 (440) 161 and 134; 190 (570) 168 and 133; 256 (768) 176 and 148. Gated 40 each
+// (220) 170 and 158; 128 of half the experts (352) 109 and 113; 96 (528) 175 and 172; 128 (704) 184 and 180; 256 (1,408) 259 and 255.
+// Down 128 (512) 88 and 92; 60 to 320 (584) 118 and 113; 190 (760) 116 and 114; 256 (1,024) 130 and 128; 512 232 and 217.
+constexpr int WALK_PLACES = 256;
+bool takes_walk(const Groups& p, int end) {
+  if (p.K % WALK_K != 0 || p.K < WALK_STAGES * WALK_K) return false;
+  const int cols = end >= END_GATED ? 128 : 256;
+  const int64_t full = p.entries / TM_BIG * ((p.N + cols - 1) / cols);
+  return full >= (end == END_PLAIN ? 704 : 400);
+}
+
 template <int END>
-void launch_experts(const Groups& p, unsigned gy, hipStream_t stream) {
+int launch_experts(const Groups& p, unsigned gy, hipStream_t stream) {
   const int cols = END >= END_GATED ? 128 : 256;
+  if (takes_walk(p, END)) {
+    auto kernel = grouped_mfma_walk_kernel<bf16, END>;
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, WALK_LDS) != hipSuccess) return ERR_LAUNCH;
+    kernel<<<WALK_PLACES, 512, WALK_LDS, stream>>>(p);
+    return OK;
+  }
   // eight XCDs, four tiles at a time (y and z together: the places rounded up may be more than y takes)
   grouped_mfma_experts_kernel<bf16, END><<<dim3((unsigned)((p.N + cols - 1) / cols), (gy + 31) / 32, 32), 256, 0, stream>>>(p);
+  return OK;
 }
 template <int END>
 void launch_big(const Groups& p, unsigned gy, unsigned gz, hipStream_t stream) {
@@ -1157,14 +1352,16 @@ int launch_groups(int dtype, Groups p, unsigned gy, unsigned gz, hipStream_t str
     if (!GATED && p.tiles && p.entries * grid.x < 512) grouped_mfma_small_kernel<bf16, GATED, 8><<<grid, 512, 0, stream>>>(p);
     else grouped_mfma_small_kernel<bf16, GATED, 4><<<grid, 256, 0, stream>>>(p);
   } else if (mfma_fits(dtype, p) && p.tiles && p.tm == TM_BIG) {
+    int launched;
     switch (GATED ? (p.clamped ? END_GATED_CLAMPED : END_GATED) : p.act) {
-      case END_PLAIN: launch_experts<END_PLAIN>(p, gy, stream); break;
-      case END_SILU: launch_experts<END_SILU>(p, gy, stream); break;
-      case END_GELU: launch_experts<END_GELU>(p, gy, stream); break;
-      case END_RELU2: launch_experts<END_RELU2>(p, gy, stream); break;
-      case END_GATED: launch_experts<END_GATED>(p, gy, stream); break;
-      default: launch_experts<END_GATED_CLAMPED>(p, gy, stream); break;
+      case END_PLAIN: launched = launch_experts<END_PLAIN>(p, gy, stream); break;
+      case END_SILU: launched = launch_experts<END_SILU>(p, gy, stream); break;
+      case END_GELU: launched = launch_experts<END_GELU>(p, gy, stream); break;
+      case END_RELU2: launched = launch_experts<END_RELU2>(p, gy, stream); break;
+      case END_GATED: launched = launch_experts<END_GATED>(p, gy, stream); break;
+      default: launched = launch_experts<END_GATED_CLAMPED>(p, gy, stream); break;
     }
+    if (launched != OK) return launched;
   } else if (mfma_fits(dtype, p) && !p.tiles && p.tm == TM_BIG) {
     if (!p.gate) launch_big<END_PLAIN>(p, gy, gz, stream);
     else if (!p.gate_entries) launch_big<END_HEAD_GATE>(p, gy, gz, stream);

@@ -239,3 +239,67 @@ def test_experts_of_many_rows_and_odd_widths(N, K, kind):
 @pytest.mark.parametrize("M,N,K,extra", [(130, 257, 64, 0), (300, 127, 72, 0), (17, 511, 64, 3), (200, 130, 40, 0)])
 def test_heads_of_many_rows_and_odd_widths(M, N, K, extra, gate):
     test_heads_of_many_rows(M, N, K, extra, gate)
+
+
+# many tiles (the bound of the entries says so, not the rows that are there): workgroups walk them; columns in part of a workgroup's
+# 256 and of a wave's, k in the fewest steps and in odd and even numbers
+@pytest.mark.parametrize("N,K,kind,top,to_perm,factor", [
+    (200, 192, None, 0, True, False), (256, 256, "gelu", 3, False, False), (33, 448, "silu", 3, True, True),
+    (300, 192, "relu2", 0, False, False), (130, 320, "gated", 3, True, False), (72, 192, "clamped", 3, False, True), (600, 1408, None, 0, True, False)])
+def test_experts_that_walk_their_tiles(N, K, kind, top, to_perm, factor):
+    from dinfer_amd.kernels import ops
+    E, n, gated = len(COUNTS), sum(COUNTS), kind in ("gated", "clamped")
+    idx = sorted_entries(COUNTS, top, n, N).to(DEV)
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    a = torch.randn(-(-n // top) if top else n, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(E, 2 * N if gated else N, K, generator=g, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    scale = torch.rand(n, generator=g, device=DEV) if factor else None
+    limit, slope = (0.7, 1.3) if kind == "clamped" else (0.0, 0.0)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    perm, offsets, tiles = torch.zeros(n, **i32), torch.zeros(E + 1, **i32), torch.full((ops.moe_max_tiles(n, E, 16), 2), -1, **i32)
+    ops.moe_scatter(idx, n, E, offsets, perm, tiles, 128)
+    out = torch.full((n + 1, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    form = 1 if gated else {None: 0, "silu": 2, "gelu": 3, "relu2": 4}[kind]
+    ops.lib.call("dinfer_experts_nt", ops.dtype_code(a.dtype), form, a.data_ptr(), K, w.data_ptr(), K, w.shape[1] * K, out.data_ptr(), N, N, K,
+                 tiles.data_ptr(), tiles.shape[0], 128, offsets.data_ptr(), perm.data_ptr(), top, int(to_perm),
+                 0 if scale is None else scale.data_ptr(), limit, slope, 704 * 128, ops._stream())
+    assert (out[n] == 7.0).all()
+    for e in range(E):
+        lo, hi = int(offsets[e]), int(offsets[e + 1])
+        entry = perm[lo:hi].long()
+        rows = (a[entry // top] if top else a[lo:hi]).double()
+        z = rows @ w[e].double().T
+        if scale is not None:
+            z = z * scale[entry].double()[:, None]
+        if kind == "clamped":
+            gate, up = z[:, :N].clamp(max=limit), z[:, N:].clamp(-limit, limit)
+            want = gate * torch.sigmoid(slope * gate) * (up + 1)
+        else:
+            want = act(z[:, :N], "silu") * z[:, N:] if gated else act(z, kind)
+        close(out[entry] if to_perm else out[lo:hi], want)
+
+
+def test_a_walk_past_what_is_looked_up_at_once():
+    """A work list with places left empty, and more tiles a workgroup than it keeps in mind (tiles named twice write the same)."""
+    from dinfer_amd.kernels import ops
+    E, N, K, n, places = 3, 40, 192, 700, 9000
+    g = torch.Generator(device=DEV).manual_seed(9)
+    a = torch.randn(n, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(E, N, K, generator=g, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    out = torch.full((n, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    ends = [0, 400, 400, n]
+    perm = torch.randperm(n, generator=torch.Generator().manual_seed(1)).to(torch.int32).to(DEV)
+    offsets = torch.tensor(ends, dtype=torch.int32, device=DEV)
+    there = [(e, at) for e in range(E) for at in range(ends[e], ends[e + 1], 128)]
+    tiles = torch.full((places, 2), -1, dtype=torch.int32)
+    for at in range(places):
+        if at % 5 and at not in (places - 1, places - 2):
+            tiles[at] = torch.tensor(there[at % (len(there) - 1)], dtype=torch.int32)
+    tiles[places - 1] = torch.tensor(there[-1], dtype=torch.int32)
+    tiles = tiles.to(DEV)
+    ops.lib.call("dinfer_experts_nt", ops.dtype_code(a.dtype), 0, a.data_ptr(), K, w.data_ptr(), K, N * K, out.data_ptr(), N, N, K,
+                 tiles.data_ptr(), places, 128, offsets.data_ptr(), perm.data_ptr(), 0, 1, 0, 0.0, 0.0, 704 * 128, ops._stream())
+    want = torch.empty(n, N, dtype=torch.double, device=DEV)
+    for e in range(E):
+        want[perm[ends[e]:ends[e + 1]].long()] = a[ends[e]:ends[e + 1]].double() @ w[e].double().T
+    close(out, want)
