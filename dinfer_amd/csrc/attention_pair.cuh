@@ -19,11 +19,14 @@
 //   HALVES = true   128 columns; the first four waves take the even blocks, the others the odd ones, each with a ring of
 //                   their own, and the two results meet in LDS at the end: twice the tiles, half as long each
 //
-// Bound by the matrix cores and LDS, whose reads (256 KB a block of 64 keys and 256 columns, 128 bytes a cycle) take as many
-// cycles as the MFMAs. 2,001 rows behind 28,000, 32 heads over 8: 1,272 us with the tile of rows (747 TFLOP/s; keys and values
-// through registers, a wave's softmax and its MFMAs after each other) and 818 here (1,160). Of that: fragments read eight ahead
-// of their MFMA in program order 1,111 -> 880; table entries looked up a turn ahead, behind the MFMAs, and keys and values of one
-// page an instruction 862 -> 818; blocks further ahead or the loads beside the softmax nothing, or slower (846, 906).
+// Bound by the two phases, a group's 1,180 cycles of MFMAs (1,024 at least) beside the other's 1,250 of softmax, and by power:
+// behind a long history the MFMAs fill 61 to 63 % of the cycles and the chip lowers its clock to 1.4 to 1.7 GHz (a prompt of 4,096:
+// 46 %, 2.0 GHz). LDS is read in 31 % of the cycles, at 256 bytes each.
+//
+// 2,001 rows behind 28,000, 32 heads over 8: 1,272 us with the tile of rows (747 TFLOP/s; keys and values through registers, a
+// wave's softmax and its MFMAs after each other) and 818 here (1,160). Of that: fragments read eight ahead of their MFMA in program
+// order 1,111 -> 880; table entries looked up a turn ahead, behind the MFMAs, and keys and values of one page an instruction 862 ->
+// 818; blocks further ahead or the loads beside the softmax nothing, or slower (846, 906).
 #pragma once
 #include <type_traits>
 

@@ -1,6 +1,6 @@
 // Latent attention: every token keeps one vector of R + dr numbers that all heads share (the RMS-normed latent c
 // [R] and one rotated key part kr [dr]); a head's unrotated key is Wuk_h c and its value Wuv_h c. The products
-// with Wuk and Wuv are moved to the query side (the "absorbed" form), so the kernels here never expand a key:
+// with Wuk and Wuv are moved to the query side (the "absorbed" form), so the kernels here never expand a key (latent_expand.hip does):
 //
 //   qa_h = [ Wuk_h^T qn_h | rot(qr_h) ]          (R + dr numbers a head, made before these kernels run)
 //   s_j  = scale * < qa_h , [c_j | kr_j] >       j <= p  (and j > p - window, where a window is given)
