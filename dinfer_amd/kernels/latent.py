@@ -58,6 +58,8 @@ class Expanded:
     """Attention over keys and values made again from the latents (csrc/latent_expand.hip): scratch, sized once and shared by the
     layers of one geometry, and the choice for a step."""
 
+    ROWS = 128      # a request, from which on a step may gain: then its requests' lengths are worth knowing (a replayed step's are not)
+
     def __init__(self, ctx, heads: int, rank: int):
         self.heads, self.rank = heads, rank
         per_chunk = 2 * heads * 4096 + 2048
@@ -70,10 +72,6 @@ class Expanded:
     @staticmethod
     def supports(ctx, dim: int, rot_dim: int, vdim: int, rank: int) -> bool:
         return ctx.dtype == torch.bfloat16 and ops.latent_expanded_supports(dim, rot_dim, vdim, rank, ctx.page_size)
-
-    def wants(self, tokens: int, num_reqs: int) -> bool:
-        """Whether a step of these counts may gain: then its requests' lengths are worth knowing (a replayed step's are not)."""
-        return tokens >= 128 * num_reqs
 
     def plan(self, starts, counts):
         """[(first request, requests, their keys, longest portion)] of the launches for requests of `counts` rows behind `starts`
@@ -107,7 +105,7 @@ class Expanded:
 
     def launches(self, batch):
         """plan() of the step in `batch`, worked out once a step; None for a step whose lengths are not known."""
-        if not batch.lengths_known or not self.wants(batch.num_tokens, batch.num_reqs):
+        if not batch.lengths_known or batch.num_tokens < self.ROWS * batch.num_reqs:
             return None
         key = ("latent", self.heads, self.rank, self.chunks)
         if key not in batch.notes:

@@ -66,16 +66,20 @@ class BuildContext:
         return self._shared[key]
 
 
+def least_rows(parts) -> int | None:
+    """lengths_from of several parts together (see Part)."""
+    return min((p.lengths_from for p in parts if p.lengths_from is not None), default=None)
+
+
 class Part:
     # True: forward reads what changes from step to step from the batch's device tensors only (see Mixer.capturable)
     capturable = True
     # the same promise for steps with prompt portions (see Mixer.capturable_portions)
     capturable_portions = True
 
-    def wants_lengths(self, tokens: int, num_reqs: int) -> bool:
-        """Whether forward may take a better way through a step of these counts where batch.lengths_known: such a step stays out
-        of the graphs."""
-        return False
+    # after bind: from so many rows a request on forward may take a better way through a step where batch.lengths_known (such a step
+    # stays out of the graphs); None: never
+    lengths_from: int | None = None
 
     def tensors(self) -> dict[str, TensorSpec]:
         """Local tensor name -> what the weight file must hold for it."""

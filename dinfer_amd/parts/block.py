@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 
 from ..kernels import gemm, ops
-from .base import Block, CacheView, Carried, Into
+from .base import Block, CacheView, Carried, Into, least_rows
 from .registry import BLOCKS, FEED_FORWARDS, MIXERS, NORMS
 from .spec import LayerSpec
 
@@ -58,8 +58,9 @@ class PreNormBlock(Block):
     def capturable_portions(self):
         return all(part.capturable and part.capturable_portions for _, part in self._parts())
 
-    def wants_lengths(self, tokens, num_reqs):
-        return any(part.wants_lengths(tokens, num_reqs) for _, part in self._parts())
+    @property
+    def lengths_from(self):
+        return least_rows(part for _, part in self._parts())
 
     def tensors(self):
         return {p + n: s for p, part in self._parts() for n, s in part.tensors().items()}
@@ -151,8 +152,9 @@ class SandwichBlock(Block):
     def capturable_portions(self):
         return all(part.capturable and part.capturable_portions for _, part in self._parts())
 
-    def wants_lengths(self, tokens, num_reqs):
-        return any(part.wants_lengths(tokens, num_reqs) for _, part in self._parts())
+    @property
+    def lengths_from(self):
+        return least_rows(part for _, part in self._parts())
 
     def tensors(self):
         t = {p + n: s for p, part in self._parts() for n, s in part.tensors().items()}
@@ -277,8 +279,9 @@ class OutNormBlock(Block):
     def capturable_portions(self):
         return all(part.capturable and part.capturable_portions for _, part in self._parts())
 
-    def wants_lengths(self, tokens, num_reqs):
-        return any(part.wants_lengths(tokens, num_reqs) for _, part in self._parts())
+    @property
+    def lengths_from(self):
+        return least_rows(part for _, part in self._parts())
 
     def tensors(self):
         return {p + n: s for p, part in self._parts() for n, s in part.tensors().items()}

@@ -18,7 +18,7 @@ from __future__ import annotations
 import torch
 
 from ..kernels import gemm, ops
-from .base import CacheView, Carried, Mixer
+from .base import CacheView, Carried, Mixer, least_rows
 from .linear import Linear
 from .norm import GroupRMSNorm
 from .registry import MIXERS
@@ -66,8 +66,9 @@ class JoinedMixers(Mixer):
     def capturable_portions(self):
         return all(m.capturable_portions for _, m, _, _ in self.members)
 
-    def wants_lengths(self, tokens, num_reqs):
-        return any(m.wants_lengths(tokens, num_reqs) for _, m, _, _ in self.members)
+    @property
+    def lengths_from(self):
+        return least_rows(m for _, m, _, _ in self.members)
 
     def cache_spec(self):
         return JoinedSpec({name: m.cache_spec() for name, m, _, _ in self.members})

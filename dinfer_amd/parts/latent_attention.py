@@ -148,8 +148,9 @@ class LatentAttention(Mixer):
         if self.may_expand and latent_kernels.Expanded.supports(ctx, self.dim, self.rot_dim, self.vdim, self.rank):
             self.expanded = latent_kernels.Expanded(ctx, H, self.rank)
 
-    def wants_lengths(self, tokens, num_reqs):
-        return self.expanded is not None and self.expanded.wants(tokens, num_reqs)
+    @property
+    def lengths_from(self):
+        return None if self.expanded is None else self.expanded.ROWS
 
     def forward(self, x, batch, cache: CacheView):
         T, g = batch.num_tokens, cache.group

@@ -9,7 +9,7 @@ import math
 import torch
 
 from ..kernels import gemm, ops
-from .base import BuildContext, Carried
+from .base import BuildContext, Carried, least_rows
 from .linear import Linear
 from .registry import BLOCKS, NORMS, STREAM_OPS
 from .spec import ModelSpec, RunEntry, TensorSpec
@@ -143,13 +143,14 @@ class DecoderModel:
                 and self.final_norm.capturable_portions)
 
     def wants_lengths(self, tokens: int, num_reqs: int) -> bool:
-        return any(self.blocks[e.layer].wants_lengths(tokens, num_reqs) for e in self.run)
+        return self._lengths_from is not None and tokens >= self._lengths_from * num_reqs
 
     # ---- execution -----------------------------------------------------------------------------
     def bind(self, ctx: BuildContext) -> None:
         self.ctx = ctx
         for b in self.blocks:
             b.bind(ctx)
+        self._lengths_from = least_rows(self.blocks[e.layer] for e in self.run)   # (asked once: steps are launched against the clock)
         for op in (self.embed_post, self.logits_post):
             if op is not None:
                 op[1].bind(ctx)
