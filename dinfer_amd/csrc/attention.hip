@@ -711,6 +711,20 @@ extern "C" int dinfer_attn_flash_form(int64_t tokens, int num_reqs, int max_q_le
   return takes_pair(page_size, 0) ? pair_form(tokens, num_reqs, max_q_len, heads, kv_heads) : 0;
 }
 
+// dinfer_attn_flash at head size 128 without a window by the kernel of paired waves in one of its forms, whatever the counts.
+extern "C" int dinfer_attn_flash_pair(int form, const void* q, int64_t ld_q, void* out, int64_t ld_out, const void* k_cache,
+                                      const void* v_cache, const int32_t* block_table, int64_t max_blocks,
+                                      const int32_t* cu_seqlens, const int32_t* seq_lens, int num_reqs, int64_t tokens, int max_q_len,
+                                      float scale, int heads, int kv_heads, int page_size, int skip_single, hipStream_t stream) {
+  if (num_reqs <= 0 || max_q_len <= 0 || tokens <= 0) return OK;
+  if (!dinfer_attn_mfma_supports(128, page_size, heads, kv_heads) || !takes_pair(page_size, 0) || form < 1 || form > 2) return ERR_UNSUPPORTED;
+  if (max_blocks <= 0 || ld_q % 8 || ld_out % 4 || !aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache) || ((uintptr_t)out % 8))
+    return ERR_BAD_SHAPE;
+  return (form == 1 ? launch_pair<false> : launch_pair<true>)((const bf16*)q, ld_q, (bf16*)out, ld_out, (const bf16*)k_cache,
+                                                              (const bf16*)v_cache, block_table, max_blocks, cu_seqlens, seq_lens, num_reqs,
+                                                              tokens, max_q_len, scale, heads, kv_heads, page_size, skip_single, stream);
+}
+
 // tokens: rows of all requests together. skip_single: requests with one row are left to the split-K kernel.
 extern "C" int dinfer_attn_flash(const void* q, int64_t ld_q, void* out, int64_t ld_out, const void* k_cache,
                                  const void* v_cache, const int32_t* block_table, int64_t max_blocks,

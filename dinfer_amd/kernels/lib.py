@@ -107,6 +107,7 @@ SIGNATURES = {
     "dinfer_streams_step": ("streams", [_I, _P, _L, _I, _I, _P, _P, _L, _P, _P, _P, _P, _P, _F, _P, _L, _P, _L, _L, _P]),
     "dinfer_attn_mfma_supports": ("attention", [_I, _I, _I, _I]),
     "dinfer_attn_flash_form": ("attention", [_L, _I, _I, _I, _I, _I]),
+    "dinfer_attn_flash_pair": ("attention", [_I, _P, _L, _P, _L, _P, _P, _P, _L, _P, _P, _I, _L, _I, _F, _I, _I, _I, _I, _P]),
     "dinfer_attn_flash": (
         "attention",
         [_P, _L, _P, _L, _P, _P, _P, _L, _P, _P, _I, _L, _I, _F, _I, _I, _I, _I, _I, _I, _P],

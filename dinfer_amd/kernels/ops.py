@@ -1282,12 +1282,19 @@ def attn_flash_form(tokens: int, num_reqs: int, max_q_len: int, heads: int, kv_h
 
 def attn_flash(q, out, k_cache, v_cache, block_table, cu_seqlens, seq_lens, num_reqs: int, tokens: int,
                max_q_len: int, *, scale: float, window: int, heads: int, kv_heads: int, head_dim: int,
-               page_size: int, skip_single: bool = False):
-    """MFMA flash attention over the pages: rows with or without history, causal, optional window."""
+               page_size: int, skip_single: bool = False, form: int | None = None):
+    """MFMA flash attention over the pages: rows with or without history, causal, optional window. form (head size 128, no window): the
+    kernel of paired waves in that form, 1 or 2, whatever attn_flash_form says."""
     _need_gpu(q, out, k_cache, v_cache, block_table, cu_seqlens, seq_lens)
     _check_paged(q, out, k_cache, v_cache, block_table, seq_lens, num_reqs, heads, kv_heads, head_dim, page_size)
     assert cu_seqlens.dtype == torch.int32 and cu_seqlens.numel() >= num_reqs + 1
     assert q.shape[0] >= tokens and out.shape[0] >= tokens
+    if form is not None:
+        assert head_dim == 128 and window == 0
+        lib.call("dinfer_attn_flash_pair", form, q.data_ptr(), _rows(q), out.data_ptr(), _rows(out), k_cache.data_ptr(),
+                 v_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1], cu_seqlens.data_ptr(), seq_lens.data_ptr(), num_reqs,
+                 tokens, max_q_len, float(scale), heads, kv_heads, page_size, 1 if skip_single else 0, _stream())
+        return out
     lib.call("dinfer_attn_flash", q.data_ptr(), _rows(q), out.data_ptr(), _rows(out), k_cache.data_ptr(),
              v_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1], cu_seqlens.data_ptr(),
              seq_lens.data_ptr(), num_reqs, tokens, max_q_len, float(scale), int(window), heads, kv_heads, head_dim,
