@@ -545,9 +545,11 @@ int launch_pair(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const bf
                 int H, int Hkv, int ps, int skip_single, hipStream_t stream) {
   constexpr int COLS = pair_columns(HALVES);
   const int64_t G = H / Hkv, tiles = (max_q_len * G + COLS - 1) / COLS;
-  // (counted where most of the tiles that requests might have do not exist, as below)
+  // Counted where that takes a tenth fewer workgroups: a whole CU each, they cost more than the count where they find nothing, but
+  // otherwise the longest tiles of all requests come first. 2,300 steps of several requests where it does take 0.93 of the time
+  // (geometric mean), 6,100 others would 1.03.
   const int64_t all = tiles * num_reqs, some = tokens * G / COLS + num_reqs;
-  const bool count = all >= 4 * some;
+  const bool count = all * 10 >= some * 11;
   const int64_t blocks = (count ? some : all) * Hkv;
   if (blocks > 0x7fffffff) return ERR_UNSUPPORTED;
   auto kernel = attn_pair_kernel<HALVES>;
@@ -561,24 +563,37 @@ int launch_pair(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const bf
 inline bool takes_pair(int ps, int window) { return window == 0 && ps >= 16 && (ps & (ps - 1)) == 0; }
 
 // Whether a step's rows are many enough for the kernel of paired waves: 0 no, 1 with 256 columns a workgroup, 2 with 128 and
-// two halves of the keys. One workgroup fills a CU, so what counts is how many there are for the CUs, w1 and w2, and whether they
-// end together: the tiles of a long request grow with the causal mask. us with the tile of rows, 1 and 2 (H heads over 8):
-//   one request from nothing     H 32: 1,000 rows (w2 256) 21.5, 30.6, 23.5; 1,300 (328) 31.8, 37.2, 31.7; 2,001 (w1 256)
-//                                57, 53, 48; 2,500 (320) 81, 68, 76; 4,000 165, 128, 150. H 16: 2,500 (w2 320) 44, 60, 42
-//   one behind 6,000             H 32: 1,300 200, 156, 176; 2,001 274, 213, 216; 4,000 583, 444, 477
-//   requests of few tiles        8 x 130 rows, H 16 (w2 192) 10.8, 13.7, 11.3; H 32 (w1 192) 16.3, 14.0, 20.7; H 40 20.3,
-//                                15.4, 21.1. 16 x 100 behind 500, H 16 (w2 256) 23.4, 26.9, 22.2; H 32 (w1 256) 41.8, 29.5, 40.6.
-//                                16 x 256, H 32 59, 49, 61; 4 x 500 behind 1,500, H 16 (w2 256) 49, 56, 40; H 32 90, 65, 71
-//   two of 1,000, H 16 (w2 256)  23.3, 32.8, 23.8
+// two halves of the keys. One workgroup fills a CU, the tiles of rows are two a CU. The histories are not known here.
+//
+// One request: what counts is how many workgroups there are for the CUs, w1 and w2, and that the tiles are full (w2 by the rows there
+// are); the tiles grow with the causal mask and end apart. us with the tile of rows, 1 and 2 (H heads over 8):
+//   from nothing     H 32: 1,000 rows (w2 256) 21.5, 30.6, 23.5; 1,300 (328) 31.8, 37.2, 31.7; 2,001 (w1 256) 57, 53, 48; 2,500 (320)
+//                    81, 68, 76; 4,000 165, 128, 150. H 16: 2,500 (w2 320) 44, 60, 42. 64 over 64: 531 (w1 192, w2 265 of rows) 25, 33, 31
+//   behind 6,000     H 32: 1,300 200, 156, 176; 2,001 274, 213, 216; 4,000 583, 444, 477
+// Several: form 1 or none, by the rounds that the tiles of each make over its places, taken half for requests as long as the longest and
+// half for any lengths, a last round that is not full by a quarter as a whole one. A round of form 1 costs 2.9 of the tile of rows, and
+// where lengths differ its last long tiles run alone, three more at most; 3 where one request has nearly all rows. Fitted over 27,900
+// steps of 2 to 48 requests with 4 to 64 heads and 24,700 of 16 to 40 heads over 4 or 8 whose lengths differ by a quarter at most or
+// are one portion beside single rows: 0.969 and 0.974 of the time with the tile of rows alone (geometric means), 2.7 % and 0.3 % more
+// than 3 % slower; with form 2 as well no better. us with the tile of rows, 1 and 2:
+//   equal            16 x 256, H 32 62, 46, 62; 4 x 500 behind 1,500 91, 68, 75; two of 1,000, H 16 24, 34, 26; 8 x 130, H 16 13, 16, 14;
+//                    H 32 18.5, 16.5, 23.5; 21 x 20, 64 over 64 18, 37, 46
+//   unequal          22 of 19 to 134 behind up to 2,955, H 16 50, 69, 51; 19 of 8 to 77 behind up to 3,598, 32 over 32 74, 85, 62
 inline int pair_form(int64_t tokens, int num_reqs, int max_q_len, int H, int Hkv) {
-  const int64_t G = H / Hkv, cus = compute_units();
-  const int64_t requests = std::max<int64_t>(1, std::min<int64_t>(num_reqs, (tokens + max_q_len / 2) / max_q_len));   // as long as the longest
-  auto tiles = [&](bool halves) { return (max_q_len * G + pair_columns(halves) - 1) / pair_columns(halves); };
-  const int64_t w1 = requests * tiles(false) * Hkv, w2 = requests * tiles(true) * Hkv;
-  if (w1 >= cus + cus / 4) return 1;
-  if (tiles(false) <= 10 && w1 >= cus - cus / 4) return 1;
-  if (w2 >= (num_reqs == 1 || tiles(false) > 6 ? cus + cus / 4 : cus)) return 2;
-  return 0;
+  const int cus = compute_units();
+  if (num_reqs == 1) {
+    const int64_t w1 = ((int64_t)max_q_len * (H / Hkv) + 255) / 256 * Hkv, full = std::min<int64_t>(tokens, max_q_len) * H;
+    return w1 >= cus + cus / 4 ? 1 : full >= (int64_t)128 * (cus + cus / 4) ? 2 : 0;
+  }
+  const double T = (double)tokens, long_ones = (double)std::max<int64_t>(1, std::min<int64_t>(num_reqs, (tokens + max_q_len / 2) / max_q_len));
+  const double apart = std::max(0., 1. - T / ((double)num_reqs * max_q_len));
+  auto rounds = [&](int cols, int group, int heads, int places) {   // of tiles of `cols` columns
+    const double equal = long_ones * std::ceil(T / long_ones * group / cols), any = T * group / cols + .5 * num_reqs;
+    const double x = (equal + any) / 2 * heads / places;
+    return x < 1. ? 1. : .75 * x + .25 * std::ceil(x);
+  };
+  const double r1 = rounds(256, H / Hkv, Hkv, cus);
+  return (long_ones == 1. ? 3. * r1 : 2.9 * r1 + 3. * apart) < rounds(32, 1, H, 2 * cus) ? 1 : 0;
 }
 
 template <int DT>

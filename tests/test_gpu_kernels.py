@@ -519,225 +519,6 @@ def test_attention_flash_paired_waves(H, Hkv, page, hist, new, skip, form):
     assert (got[~rows] == 7.0).all() and (out[-1] == 7.0).all()
 
 
-@pytest.mark.parametrize("bad", ["key", "value"])
-@pytest.mark.parametrize("splits", [1, 4])
-def test_attention_decode_own_key_that_is_no_number(bad, splits):
-    """Where parts meet in a workgroup the row's own key is a part of its own: what is no number in it reaches the row's output and no
-    other's, and a row of one key is that key's value."""
-    H, Hkv, D, page, hist = 16, 8, 128, 16, [40, 0, 200]
-    _, kc, vc, m, _ = paged_case(torch.bfloat16, H, Hkv, D, page, hist, [1] * 3, seed=12)
-    raw = torch.randn(3, (H + 2 * Hkv) * D, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
-    raw[2, H * D if bad == "key" else (H + Hkv) * D] = float("nan")      # the first number of kv head 0
-    slots = torch.tensor([int(m["bt"][b, h // page]) * page + h % page for b, h in enumerate(hist)], device=DEV)
-    out = torch.zeros(3, H * D, device=DEV, dtype=torch.bfloat16)
-    part = torch.empty(3 * H * splits * (D + 4), device=DEV)
-    ops().attn_decode_post(raw.to(DEV), out, part, kc, vc, m["bt"], m["sl"], 3, splits, scale=D ** -0.5, window=0, heads=H,
-                           kv_heads=Hkv, head_dim=D, page_size=page, q_off=0, k_off=H * D, v_off=(H + Hkv) * D, q_gain=None,
-                           k_gain=None, eps=1e-5, gain_offset=0.0, positions=torch.tensor(hist, dtype=torch.int32, device=DEV),
-                           cos_sin=None, slot_mapping=slots)
-    out = out.cpu().view(3, H, D)
-    assert torch.equal(out[1], raw[1, (H + Hkv) * D:].view(Hkv, D).repeat_interleave(H // Hkv, 0))
-    assert out[0].isfinite().all() and out[2, H // Hkv:].isfinite().all()
-    group = out[2, :H // Hkv]
-    assert group.isnan().all() if bad == "key" else group[:, 0].isnan().all() and group[:, 1:].isfinite().all()
-
-
-def decode_of_rows(raw, hist, kc, vc, m, H, Hkv, D, page, splits, written=True):
-    """Decode attention of raw q|k|v rows behind `hist` keys, by the kernel that writes the cache itself and by the two it stands
-    for. written False: the pages hold the rows' keys and values already."""
-    B, geo = len(hist), dict(heads=H, kv_heads=Hkv, head_dim=D, page_size=page)
-    slots = torch.tensor([int(m["bt"][b, h // page]) * page + h % page if written else -1 for b, h in enumerate(hist)], device=DEV)
-    post = dict(q_off=0, k_off=H * D, v_off=(H + Hkv) * D, q_gain=None, k_gain=None, eps=1e-5, gain_offset=0.0,
-                positions=torch.tensor(hist, dtype=torch.int32, device=DEV), cos_sin=None, slot_mapping=slots)
-    part, outs = torch.empty(B * H * splits * (D + 4), device=DEV), []
-    for fused in (True, False):
-        k, v, x, out = kc.clone(), vc.clone(), raw.to(DEV), torch.zeros(B, H * D, device=DEV, dtype=torch.bfloat16)
-        if fused:
-            ops().attn_decode_post(x, out, part, k, v, m["bt"], m["sl"], B, splits, scale=D ** -0.5, window=0, **geo, **post)
-        else:
-            ops().qkv_post(x, B, **geo, **post, rotary_dim=D, rope_style=0, k_cache=k, v_cache=v, token_runs=False)
-            ops().attn_decode(x, out, part, k, v, m["bt"], None, m["sl"], B, splits, scale=D ** -0.5, window=0, **geo)
-        outs.append(out.cpu().view(B, H, D))
-    return outs
-
-
-@pytest.mark.parametrize("written", [True, False])
-@pytest.mark.parametrize("splits", [1, 4, 5])
-def test_attention_decode_own_key_scored_minus_infinity(splits, written):
-    """The row's own key at a score of -inf weighs nothing beside finite ones: a product beyond 32 bits in the row, an infinity in
-    the pages (which a rotation would make no number)."""
-    H, Hkv, D, page, hist = 16, 8, 128, 16, [40, 7, 200, 64]
-    _, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, [1] * 4, seed=12)
-    raw = torch.randn(4, (H + 2 * Hkv) * D, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
-    x, want_outs = raw.view(4, H + 2 * Hkv, D), []
-    x[1:, :H, 0], x[1:, H:H + Hkv, 0] = -1e25 if written else 1.0, 1e25
-    for b, (_, k, v) in enumerate(outs):
-        k, v = k.clone(), v.clone()
-        if written:
-            k[-1], v[-1] = x[b, H:H + Hkv].double(), x[b, H + Hkv:].double()
-        k[:, :, 0] = 0          # (of the other keys: their scores stay where they are)
-        for i in range(hist[b] + 1):
-            kc[int(m["bt"][b, i // page]), :, 0, i % page, 0] = 0
-        if b:
-            k[-1, :, 0] = float("inf") if written else -float("inf")
-            kc[int(m["bt"][b, hist[b] // page]), :, 0, hist[b] % page, 0] = -float("inf")
-        elif written:
-            k[-1, :, 0] = x[b, H:H + Hkv, 0].double()
-        want_outs.append((x[b:b + 1, :H].double(), k, v))
-    fused, two = decode_of_rows(raw, hist, kc, vc, m, H, Hkv, D, page, splits, written)
-    torch.testing.assert_close(fused.double(), expected_attention(want_outs, hist, D ** -0.5, 0), rtol=2e-2, atol=2e-2)
-    assert torch.equal(fused, two)
-
-
-@pytest.mark.parametrize("bad", ["key", "value"])
-@pytest.mark.parametrize("splits", [1, 4])
-def test_attention_decode_own_key_that_is_no_number_beside_a_large_score(splits, bad):
-    """A score or value of the row's own key that is no number stays in the row's output though another key's score exceeds what
-    2^x holds beside it."""
-    H, Hkv, D, page, hist = 16, 8, 128, 16, [40, 0, 200]
-    _, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, [1] * 3, seed=12)
-    raw = torch.randn(3, (H + 2 * Hkv) * D, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
-    x = raw.view(3, H + 2 * Hkv, D)
-    x[2, :H] = x[2, :1]                                     # every head's query, and a cached key 40 times as long: 40 x 128 x 128 ** -0.5
-    blk, off = int(m["bt"][2, 3]), 50 % page
-    kc[blk, :, :, off, :] = (x[2, 0].float() * 40).to(torch.bfloat16).view(D // 8, 8).to(DEV)
-    x[2, H if bad == "key" else H + Hkv, 0] = float("nan")
-    for out in decode_of_rows(raw, hist, kc, vc, m, H, Hkv, D, page, splits):
-        assert out[:2].isfinite().all() and out[2, H // Hkv:].isfinite().all()
-        group = out[2, :H // Hkv]
-        assert group.isnan().all() if bad == "key" else group[:, 0].isnan().all() and group[:, 1:].isfinite().all()
-
-
-def decode_post_case(H, Hkv, D, page, window, gains, hist, splits, device="cpu", spike=None, sharp=1.0):
-    """One launch of the decode kernel that norms, rotates and writes the cache, against the plain functions and, bit
-    for bit, against the two kernels it stands for. Request 1 writes nothing (slot -1)."""
-    theta, eps, scale = 1e4, 1e-5, D ** -0.5
-    B = len(hist)
-    _, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, [1] * B, seed=11)
-    g = torch.Generator().manual_seed(B)
-    raw = torch.randn(B, (H + 2 * Hkv) * D, generator=g).to(torch.bfloat16)
-    wq = wk = None
-    if gains != "none":
-        wq = ((torch.rand(D, generator=g) + 0.5) * sharp).to(torch.bfloat16)   # (a norm undoes any scale of q itself)
-        wk = (torch.rand(D, generator=g) + 0.5).to(torch.bfloat16)
-    else:
-        raw[:, :H * D] = (raw[:, :H * D].float() * sharp).to(torch.bfloat16)
-    pos = [h for h in hist]
-    table = rope_table(max(hist) + 25, D, theta).to(DEV)
-    slots = []
-    for b in range(B):
-        blk = int(m["bt"][b, hist[b] // page])
-        slots.append(blk * page + hist[b] % page)
-    slots[1] = -1
-    # what the plain functions make of the rows
-    x = raw.double()
-    ang = plain.rope_angles(pos, D, theta)
-    norm = (lambda t, w: plain.rms_norm(t, w.double(), eps)) if wq is not None else (lambda t, w: t)
-    q = plain.rope_neox(norm(x[:, :H * D].view(B, H, D), wq), ang).to(torch.bfloat16).double()
-    k = plain.rope_neox(norm(x[:, H * D:(H + Hkv) * D].view(B, Hkv, D), wk), ang).to(torch.bfloat16).double()
-    v = x[:, (H + Hkv) * D:].view(B, Hkv, D)
-    want_outs = []
-    for b, (_, kk, vv) in enumerate(outs):
-        kk, vv = kk.clone(), vv.clone()
-        if slots[b] >= 0:
-            kk[-1], vv[-1] = k[b], v[b]
-        sp = spike.get(b) if isinstance(spike, dict) else spike
-        if sp is not None:   # a cached key along the row's first query head of each group, as it is after norm and rotation
-            key, amp = sp
-            kk[key] = (q[b, ::H // Hkv] * amp).to(torch.bfloat16).double()
-            blk, off = int(m["bt"][b, key // page]), key % page
-            kc[blk, :, :, off, :] = kk[key].to(torch.bfloat16).view(Hkv, D // 8, 8).to(DEV)
-        want_outs.append((q[b:b + 1], kk, vv))
-    want = expected_attention(want_outs, hist, scale, window, device)
-    dev = lambda t: None if t is None else t.to(DEV)
-    args = dict(heads=H, kv_heads=Hkv, head_dim=D, page_size=page)
-    post = dict(q_off=0, k_off=H * D, v_off=(H + Hkv) * D, q_gain=dev(wq), k_gain=dev(wk), eps=eps, gain_offset=0.0,
-                positions=torch.tensor(pos, dtype=torch.int32, device=DEV))
-    slot_t = torch.tensor(slots, dtype=torch.int64, device=DEV)
-    part = torch.full((B * H * splits * (D + 4),), float("nan"), device=DEV)
-    # the two kernels
-    kc2, vc2, qkv2 = kc.clone(), vc.clone(), raw.to(DEV)
-    out2 = torch.zeros(B, H * D, device=DEV, dtype=torch.bfloat16)
-    ops().qkv_post(qkv2, B, **args, **post, cos_sin=table, rotary_dim=D, rope_style=0, k_cache=kc2, v_cache=vc2,
-                   slot_mapping=slot_t, token_runs=False)
-    ops().attn_decode(qkv2, out2, part, kc2, vc2, m["bt"], None, m["sl"], B, splits, scale=scale, window=window,
-                      **args)
-    # the one
-    kc1, vc1, qkv1 = kc.clone(), vc.clone(), raw.to(DEV)
-    out1 = torch.zeros(B, H * D, device=DEV, dtype=torch.bfloat16)
-    part.fill_(float("nan"))
-    ops().attn_decode_post(qkv1, out1, part, kc1, vc1, m["bt"], m["sl"], B, splits, scale=scale, window=window,
-                           **args, **post, cos_sin=table, slot_mapping=slot_t)
-    assert torch.equal(qkv1.cpu(), raw), "the product's rows are left as they were"
-    assert torch.equal(vc1, vc2) and torch.equal(kc1, kc2), "the pages hold the same bits as after the two kernels"
-    torch.testing.assert_close(out1.double().cpu().view(-1, H, D), want, rtol=2e-2, atol=2e-2)
-    assert torch.equal(out1, out2), f"differs from the two kernels by {float((out1.float() - out2.float()).abs().max())}"
-
-
-@pytest.mark.parametrize("window", [0, 200])
-@pytest.mark.parametrize("H,Hkv,D,page", [(8, 2, 128, 16), (5, 5, 64, 8), (6, 1, 128, 24), (4, 2, 256, 16)])
-def test_attention_flash_long_portions(H, Hkv, D, page, window):
-    """Long portions: a whole prompt of 700, a portion of 300 on top of a history of 333, short requests in
-    the same launch (idle waves), and a single row behind 1000 keys."""
-    hist, new = [0, 333, 0, 77, 1000], [700, 300, 5, 130, 1]
-    q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=13)
-    out = torch.zeros(sum(new), H * D, device=DEV, dtype=torch.bfloat16)
-    ops().attn_flash(q, out, kc, vc, m["bt"], m["cu"], m["sl"], len(hist), sum(new), max(new), scale=D ** -0.5,
-                     window=window, heads=H, kv_heads=Hkv, head_dim=D, page_size=page)
-    want = expected_attention(outs, hist, D ** -0.5, window)
-    torch.testing.assert_close(out.double().cpu().view(-1, H, D), want, rtol=2e-2, atol=2e-2)
-
-
-@pytest.mark.parametrize("page", [16, 24])
-@pytest.mark.parametrize("window", [0, 300])
-def test_attention_flash_three_row_tiles_a_workgroup(window, page):
-    """Head size 128 with enough rows for several rounds of workgroups: 48 rows a workgroup (three row tiles share every
-    key and value fragment). Rows with and without history, a request that ends inside a tile, one shorter than a tile;
-    pages of a power of two and not."""
-    H, Hkv, D = 16, 4, 128
-    hist, new = [0, 100, 555, 31, 7, 0], [1000, 700, 300, 49, 120, 33]     # ceil(1000 / 48) x 16 heads x 6 requests = 2,016 workgroups
-    q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=9)
-    out = torch.zeros(sum(new), H * D, device=DEV, dtype=torch.bfloat16)
-    ops().attn_flash(q, out, kc, vc, m["bt"], m["cu"], m["sl"], len(hist), sum(new), max(new), scale=D ** -0.5,
-                     window=window, heads=H, kv_heads=Hkv, head_dim=D, page_size=page)
-    want = expected_attention(outs, hist, D ** -0.5, window)
-    torch.testing.assert_close(out.double().cpu().view(-1, H, D), want, rtol=2e-2, atol=2e-2)
-
-
-@pytest.mark.parametrize("H,Hkv,page,hist,new,skip,form", [
-    # all columns against every block: heads in groups of 1, 3 and 5, whole and ragged tiles, one to many blocks of 64 keys, ends on
-    # and beside a block's and a page's edge
-    (64, 64, 16, [0, 63, 130, 0, 70], [256, 65, 256, 1, 256], False, 1), (32, 32, 32, [0, 64, 500, 1, 31, 200], [257, 256, 255, 64, 63, 129], False, 1),
-    (40, 8, 16, [0] * 12, [128, 64, 63, 65, 1, 127, 129, 130, 100, 130, 130, 130], False, 1), (24, 8, 16, [3000], [3700], False, 1),
-    # halves of the keys: one block and none for the second group, an odd number of blocks, an even one
-    (64, 64, 16, [0, 0, 64], [200, 62, 130], False, 2), (16, 16, 64, [0, 40, 64, 128, 65, 63], [300, 24, 400, 399, 400, 64], False, 2),
-    (32, 8, 128, [700], [1310], False, 2), (8, 8, 16, [1000, 5, 0, 63], [1280, 1200, 1000, 1025], False, 2),
-    # few portions among many single rows: tiles are counted
-    (64, 8, 16, [9] * 30 + [100] + [70] * 8, [1] * 30 + [1290] + [1] * 8, True, 1), (32, 8, 16, [5] * 70 + [333], [1] * 70 + [1300], True, 2),
-    (32, 8, 16, [5] * 70 + [333, 80], [1] * 70 + [1300, 1], False, 2),
-    # requests that move on by one from tile to tile: an even number, few kv heads, one long one among them
-    (16, 4, 16, [0, 0, 100, 9, 0, 70, 0, 283], [2, 588, 14, 23, 4, 275, 301, 901], False, 1), (8, 1, 32, [0, 200], [400, 380], False, 1),
-    (16, 4, 16, [0, 0, 100, 9, 0, 70, 0, 283], [2, 588, 14, 23, 4, 275, 301, 901], False, 2), (16, 2, 16, [90] * 6, [150] * 6, False, 2)])
-def test_attention_flash_paired_waves(H, Hkv, page, hist, new, skip, form):
-    """The kernel for long runs of rows at head size 128 in both forms, at sizes that take it and others. What the pages hold past a
-    request's keys is no number."""
-    D, T = 128, sum(new)
-    q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=17, sharp=4.0)
-    for b, (h, n) in enumerate(zip(hist, new)):
-        last = int(m["bt"][b, (h + n - 1) // page])
-        vc[last, :, :, (h + n - 1) % page + 1:] = float("nan")
-        kc.view(kc.shape[0], Hkv, D // 8, page, 8)[last, :, :, (h + n - 1) % page + 1:] = float("nan")
-    out = torch.full((T + 1, H * D), 7.0, device=DEV, dtype=torch.bfloat16)
-    ops().attn_flash(q, out, kc, vc, m["bt"], m["cu"], m["sl"], len(new), T, max(new), scale=D ** -0.5, window=0,
-                     heads=H, kv_heads=Hkv, head_dim=D, page_size=page, skip_single=skip, form=form)
-    want = expected_attention(outs, hist, D ** -0.5, 0, device=DEV)
-    rows = torch.tensor([not (skip and n == 1) for n in new for _ in range(n)])
-    got = out[:-1].double().cpu().view(-1, H, D)
-    # weights and results are rounded to 8 bits: half a unit of a weight, at most, on every value of size up to 5, and of the result
-    torch.testing.assert_close(got[rows], want[rows], rtol=2e-2, atol=2e-2)
-    assert (got[~rows] == 7.0).all() and (out[-1] == 7.0).all()
-
-
 @pytest.mark.parametrize("H,Hkv,hist,new", [(32, 8, [500], [2100]), (32, 8, [1500] * 4, [500] * 4), (32, 32, [0], [1500])])
 def test_attention_flash_takes_paired_waves_by_itself(H, Hkv, hist, new):
     form = ops().attn_flash_form(sum(new), len(new), max(new), H, Hkv, 16)
