@@ -390,10 +390,11 @@ class ModelRunner:
         single rows are served (all of them are, some, none).
 
         A full batch, which needs a request more than the engine admits, stays as it is beyond _pad_full_up_to tokens, and
-        until its counts have come up often enough for a graph. So does a step whose requests' lengths a part wants to know."""
+        until its counts have come up often enough for a graph. So does a step that gains by its requests' lengths
+        (DecoderModel.wants_lengths)."""
         b, opt = self.batch, self.options
         T, B, R = b.num_tokens, b.num_reqs, b.num_rows
-        if R > B or B > self._buckets[-1] or self.model.wants_lengths(T, B):
+        if R > B or B > self._buckets[-1] or self.model.wants_lengths(b):
             return None
         later = [x for x in self._buckets if x >= B] + [self._buckets[-1] + 1]      # (a full batch: the spare request)
         Bp = Tp = None

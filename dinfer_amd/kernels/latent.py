@@ -58,7 +58,7 @@ class Expanded:
     """Attention over keys and values made again from the latents (csrc/latent_expand.hip): scratch, sized once and shared by the
     layers of one geometry, and the choice for a step."""
 
-    ROWS = 128      # a request, from which on a step may gain: then its requests' lengths are worth knowing (a replayed step's are not)
+    ROWS = 128      # a request, from which on a step may gain
 
     def __init__(self, ctx, heads: int, rank: int):
         self.heads, self.rank = heads, rank
@@ -75,7 +75,12 @@ class Expanded:
 
     def plan(self, starts, counts):
         """[(first request, requests, their keys, longest portion)] of the launches for requests of `counts` rows behind `starts`
-        keys, or None where the queries' side is the better one.
+        keys, or None where the queries' side is the better one (see weigh)."""
+        planned = self.weigh(starts, counts)
+        return planned and planned[0]
+
+    def weigh(self, starts, counts):
+        """(launches as plan() has them, us of the queries' side), or None.
 
         Both sides' times in us as measured with 16 heads of 128 + 64 over latents of 512. Queries' side: 77 ns a key of a round of
         256 workgroups of 64 (row, head) pairs and 15.5 ns a row for the products around them; keys' side: 5.5 ns a key
@@ -101,18 +106,28 @@ class Expanded:
                 first, total = i, 0
             total += n
         launches.append((first, len(lengths) - first, total, int(rows[first:].max())))
-        return launches
+        return launches, float(queries)
 
-    def launches(self, batch):
-        """plan() of the step in `batch`, worked out once a step; None for a step whose lengths are not known."""
+    def _weighed(self, batch):
+        """weigh() of the step in `batch`, worked out once a step; None for a step whose lengths are not known."""
         if not batch.lengths_known or batch.num_tokens < self.ROWS * batch.num_reqs:
             return None
         key = ("latent", self.heads, self.rank, self.chunks)
         if key not in batch.notes:
             B = batch.num_reqs
             counts = np.diff(batch.h["cu_seqlens"][:B + 1])
-            batch.notes[key] = self.plan(batch.h["seq_lens"][:B] - counts, counts)
+            batch.notes[key] = self.weigh(batch.h["seq_lens"][:B] - counts, counts)
         return batch.notes[key]
+
+    def launches(self, batch):
+        """plan() of the step in `batch`."""
+        weighed = self._weighed(batch)
+        return weighed and weighed[0]
+
+    def usual_way(self, batch):
+        """us of the queries' side where the keys' side is better, else None (see Part.choices)."""
+        weighed = self._weighed(batch)
+        return weighed and weighed[1]
 
     def attention(self, launches, q, q_off: int, qa, uk, uv, out, cache, batch, group: int, *, scale: float, page_size: int, gate,
                   gate_off: int, gate_entries: bool):

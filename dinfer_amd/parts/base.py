@@ -66,20 +66,11 @@ class BuildContext:
         return self._shared[key]
 
 
-def least_rows(parts) -> int | None:
-    """lengths_from of several parts together (see Part)."""
-    return min((p.lengths_from for p in parts if p.lengths_from is not None), default=None)
-
-
 class Part:
     # True: forward reads what changes from step to step from the batch's device tensors only (see Mixer.capturable)
     capturable = True
     # the same promise for steps with prompt portions (see Mixer.capturable_portions)
     capturable_portions = True
-
-    # after bind: from so many rows a request on forward may take a better way through a step where batch.lengths_known (such a step
-    # stays out of the graphs); None: never
-    lengths_from: int | None = None
 
     def tensors(self) -> dict[str, TensorSpec]:
         """Local tensor name -> what the weight file must hold for it."""
@@ -91,6 +82,12 @@ class Part:
 
     def bind(self, ctx: BuildContext) -> None:
         """Reserves buffers; called once before the first forward."""
+
+    def choices(self) -> list:
+        """After bind: what chooses between two ways through a step by its requests' lengths, an entry for every time a step meets it
+        (usual_way(batch): the time of the usual way, us, where the other is better; kernels/latent.py, Expanded). Only a step where
+        batch.lengths_known can take the other way, and it stays out of the graphs where that pays (DecoderModel.wants_lengths)."""
+        return []
 
 
 class Norm(Part):

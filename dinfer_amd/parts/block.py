@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 
 from ..kernels import gemm, ops
-from .base import Block, CacheView, Carried, Into, least_rows
+from .base import Block, CacheView, Carried, Into
 from .registry import BLOCKS, FEED_FORWARDS, MIXERS, NORMS
 from .spec import LayerSpec
 
@@ -58,9 +58,8 @@ class PreNormBlock(Block):
     def capturable_portions(self):
         return all(part.capturable and part.capturable_portions for _, part in self._parts())
 
-    @property
-    def lengths_from(self):
-        return least_rows(part for _, part in self._parts())
+    def choices(self):
+        return [c for _, part in self._parts() for c in part.choices()]
 
     def tensors(self):
         return {p + n: s for p, part in self._parts() for n, s in part.tensors().items()}
@@ -152,9 +151,8 @@ class SandwichBlock(Block):
     def capturable_portions(self):
         return all(part.capturable and part.capturable_portions for _, part in self._parts())
 
-    @property
-    def lengths_from(self):
-        return least_rows(part for _, part in self._parts())
+    def choices(self):
+        return [c for _, part in self._parts() for c in part.choices()]
 
     def tensors(self):
         t = {p + n: s for p, part in self._parts() for n, s in part.tensors().items()}
@@ -279,9 +277,8 @@ class OutNormBlock(Block):
     def capturable_portions(self):
         return all(part.capturable and part.capturable_portions for _, part in self._parts())
 
-    @property
-    def lengths_from(self):
-        return least_rows(part for _, part in self._parts())
+    def choices(self):
+        return [c for _, part in self._parts() for c in part.choices()]
 
     def tensors(self):
         return {p + n: s for p, part in self._parts() for n, s in part.tensors().items()}

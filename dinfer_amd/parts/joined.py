@@ -18,7 +18,7 @@ from __future__ import annotations
 import torch
 
 from ..kernels import gemm, ops
-from .base import CacheView, Carried, Mixer, least_rows
+from .base import CacheView, Carried, Mixer
 from .linear import Linear
 from .norm import GroupRMSNorm
 from .registry import MIXERS
@@ -66,9 +66,8 @@ class JoinedMixers(Mixer):
     def capturable_portions(self):
         return all(m.capturable_portions for _, m, _, _ in self.members)
 
-    @property
-    def lengths_from(self):
-        return least_rows(m for _, m, _, _ in self.members)
+    def choices(self):
+        return [c for _, m, _, _ in self.members for c in m.choices()]
 
     def cache_spec(self):
         return JoinedSpec({name: m.cache_spec() for name, m, _, _ in self.members})

@@ -146,11 +146,10 @@ class LatentAttention(Mixer):
         self.attn_ws = latent_kernels.Workspace(ctx, H, self.rank, self.rot_dim)
         self.expanded = None
         if self.may_expand and latent_kernels.Expanded.supports(ctx, self.dim, self.rot_dim, self.vdim, self.rank):
-            self.expanded = latent_kernels.Expanded(ctx, H, self.rank)
+            self.expanded = ctx.share(("latent_expanded", H, self.rank), lambda: latent_kernels.Expanded(ctx, H, self.rank))
 
-    @property
-    def lengths_from(self):
-        return None if self.expanded is None else self.expanded.ROWS
+    def choices(self):
+        return [] if self.expanded is None else [self.expanded]
 
     def forward(self, x, batch, cache: CacheView):
         T, g = batch.num_tokens, cache.group

@@ -9,7 +9,7 @@ import math
 import torch
 
 from ..kernels import gemm, ops
-from .base import BuildContext, Carried, least_rows
+from .base import BuildContext, Carried
 from .linear import Linear
 from .registry import BLOCKS, NORMS, STREAM_OPS
 from .spec import ModelSpec, RunEntry, TensorSpec
@@ -142,15 +142,34 @@ class DecoderModel:
         return (self.capturable() and all(self.blocks[e.layer].capturable_portions for e in self.run)
                 and self.final_norm.capturable_portions)
 
-    def wants_lengths(self, tokens: int, num_reqs: int) -> bool:
-        return self._lengths_from is not None and tokens >= self._lengths_from * num_reqs
+    def wants_lengths(self, batch) -> bool:
+        """Whether the step in `batch` is better launched one by one than padded and replayed, because parts then know its requests'
+        lengths: where one finds a better way by them, and the device has as much to do in the usual way as the host to launch.
+
+        That is some 110 us a layer; what of it the usual way (Part.choices) and the weights (read at 4.7 TB/s, or multiplied at 1
+        PFLOP/s) leave to its other kernels is 65. Replayed the usual way, and launched one by one the other, us a step (us of these 45):
+          6 layers of 3 million weights, 4 heads: one request of 128 (12) 504 and 761, three of 200 behind 300 (45) 729 and 762, one of
+            128 behind 1,000 (89) 893 and 757
+          8 of 10, 8 heads: 128 (15) 718 and 983, 384 (40) 957 and 996, 512 (54) 1,042 and 1,005, 8 of 130 (39) 1,006 and 1,007, three of
+            200 behind 300 (55) 1,102 and 987
+          8 of 30, 16 heads: 128 (24) 915 and 982, 256 (39) 1,057 and 1,002, 4 of 128 (48) 1,153 and 1,071
+          4 of 316 with 64 experts: 128 (146) 1,006 and 978"""
+        usual, better = 0.0, False
+        for choice, times in self._choices:
+            us = choice.usual_way(batch)
+            if us is not None:
+                usual, better = usual + us * times, True
+        return better and usual / len(self.run) + self._weights * max(2 / 4.7e6, 2e-9 * batch.num_tokens) >= 45.0
 
     # ---- execution -----------------------------------------------------------------------------
     def bind(self, ctx: BuildContext) -> None:
         self.ctx = ctx
         for b in self.blocks:
             b.bind(ctx)
-        self._lengths_from = least_rows(self.blocks[e.layer] for e in self.run)   # (asked once: steps are launched against the clock)
+        # (asked once: steps are launched against the clock)
+        met = [c for e in self.run for c in self.blocks[e.layer].choices()]
+        self._choices = [(c, sum(x is c for x in met)) for i, c in enumerate(met) if not any(x is c for x in met[:i])]
+        self._weights = self.layer_weights()
         for op in (self.embed_post, self.logits_post):
             if op is not None:
                 op[1].bind(ctx)

@@ -2,10 +2,12 @@
 import random
 from types import SimpleNamespace
 
+import numpy as np
 import pytest
 import torch
 
 from dinfer_amd.kernels import latent, ops
+from dinfer_amd.parts import DecoderModel
 from dinfer_amd.parts.latent_attention import LatentAttention
 from dinfer_amd.parts.spec import part
 
@@ -115,3 +117,24 @@ def test_expanded_attention(H, R, page, hist, new, gate):
     # rounded to 8 bits on the way: keys (a score of size 4 is off by 0.01 or so), weights, values, the result
     torch.testing.assert_close(out[:-1].double().cpu().view(T, H, 128), want, rtol=2e-2, atol=2e-2)
     assert (out[-1] == 7.0).all()
+
+
+def step_of(starts, counts, known=True):
+    cu, lens = np.concatenate([[0], np.cumsum(counts)]), np.add(starts, counts)
+    return SimpleNamespace(lengths_known=known, num_tokens=sum(counts), num_reqs=len(counts), notes={}, h=dict(cu_seqlens=cu, seq_lens=lens))
+
+
+def test_a_step_leaves_the_graphs_only_where_that_pays():
+    """Eight heads over 512: a layer of 10 million weights is launched slower than it runs, unless the attention is long; one of 316 million
+    never; and where the queries' side is the better one nothing is gained by launching."""
+    ex = made(8, 512, 65536 // 16)
+    wants = lambda step, weights: DecoderModel.wants_lengths(SimpleNamespace(_choices=[(ex, 8)], run=[None] * 8, _weights=weights), step)
+    for starts, counts in (([0], [128]), ([0], [384]), ([0] * 8, [130] * 8), ([0, 0], [256, 256])):
+        assert ex.plan(starts, counts) and not wants(step_of(starts, counts), 10e6) and wants(step_of(starts, counts), 316e6)
+        assert not wants(step_of(starts, counts, known=False), 316e6)
+    for starts, counts in (([0], [512]), ([1000], [128]), ([300] * 3, [200] * 3)):
+        assert wants(step_of(starts, counts), 10e6)
+    ex = made(16, 512, 65536 // 16)
+    for starts, counts in (([3000] * 31 + [1024], [1] * 31 + [512]), ([100] * 4, [20] * 4), ([70000], [512])):   # few rows a request; no room
+        assert ex.launches(step_of(starts, counts)) is None and not wants(step_of(starts, counts), 316e6)
+    assert not DecoderModel.wants_lengths(SimpleNamespace(_choices=[], run=[None], _weights=10**9), step_of([0], [2048]))
