@@ -93,8 +93,8 @@ class StepBatch:
         self.max_q_len = self.max_seq_len = self.num_singles = 0
         self.all_decode = False
         self.req_ids: list = []
-        # whether the host's lengths (h["seq_lens"]) are those of the step that runs (a graph captured now may be replayed for
-        # others), and what parts have worked out from them, for this step only
+        # whether the host's lengths (h["seq_lens"]) are those of the step that runs (a padded step may be captured and replayed for
+        # others: False), and what parts have worked out from them, for this step only
         self.lengths_known, self.notes = False, {}
         self._copied = torch.cuda.Event() if pin else None
 
@@ -128,7 +128,7 @@ class StepBatch:
         if rc < 0:
             raise self._named(native.error(rc), [e.req_id for e in entries])
         self.req_ids = [e.req_id for e in entries]
-        self._take_facts()
+        self._take_facts(lengths_known=pad_to is None)
 
     def fill_planned(self, scheduler, pad_to: int | None = None) -> None:
         """The same for the step a scheduler has just planned, straight from the tokens it holds."""
@@ -137,7 +137,7 @@ class StepBatch:
         if rc < 0:
             raise self._named(native.error(rc), scheduler.planned_ids())
         self.req_ids = scheduler.planned_ids()
-        self._take_facts()
+        self._take_facts(lengths_known=pad_to is None)
 
     @staticmethod
     def _named(exc: Exception, ids: list) -> Exception:
@@ -150,12 +150,12 @@ class StepBatch:
         if self._copied is not None:
             self._copied.synchronize()  # the last upload has read the pinned buffer
 
-    def _take_facts(self) -> None:
+    def _take_facts(self, lengths_known: bool) -> None:
         f = self._facts
         self.num_tokens, self.num_reqs, self.num_rows = f.num_tokens, f.num_reqs, f.num_rows
         self.max_q_len, self.max_seq_len, self.num_singles = f.max_q_len, f.max_seq_len, f.num_singles
         self.all_decode = f.num_singles == f.num_reqs
-        self.lengths_known, self.notes = True, {}
+        self.lengths_known, self.notes = lengths_known, {}
 
     def pad(self, reqs: int, tokens: int, rows: int) -> None:
         """After fill(): made-up requests that write nothing bring the step to these counts (csrc/host/step_batch.hpp,
@@ -163,7 +163,7 @@ class StepBatch:
         rc = native.fn("dh_batch_pad")(self._buffers, self._facts, reqs, tokens, rows)
         if rc < 0:
             raise native.error(rc)
-        self._take_facts()
+        self._take_facts(lengths_known=False)
 
     def upload(self) -> None:
         self._dev.copy_(self._host, non_blocking=True)

@@ -428,7 +428,6 @@ class ModelRunner:
                 return None
         b.pad(Bp, Tp, rows)
         b.max_q_len, b.all_decode = qp, route == 2
-        b.lengths_known = False
         b.num_singles = Bp if route == 2 else 4 if route == 1 else 0
         return key, R
 
@@ -453,6 +452,7 @@ class ModelRunner:
 
     def _capture(self, forward) -> torch.cuda.CUDAGraph:
         """Records forward()'s launches into a graph without running them (the step has run eagerly just before)."""
+        assert not self.batch.lengths_known, "a graph must not hold what follows from one step's lengths"
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
         if self._capture_stream is None:

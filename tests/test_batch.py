@@ -223,6 +223,29 @@ def test_engine_loop_with_a_stand_in_runner():
     assert eng.stats()["request_abort"] == 1
 
 
+def test_lengths_are_known_only_of_a_step_that_nothing_was_added_for():
+    """A padded step may be captured and replayed for requests of other lengths; what was worked out for a step before is gone."""
+    s, b = setup(1000)
+    assert not b.lengths_known
+    for i, n in ((1, 20), (2, 5)):
+        s.add_request(Request(i, list(range(n)), SamplingParams(max_tokens=5)))
+    run(s, b)
+    assert b.lengths_known and b.notes == {}
+    b.notes["a part"] = 1
+    out = s.schedule()
+    entries = [Entry(x.request.id, x.request.tokens(x.start, 1), x.start, [0]) for x in out.scheduled]
+    for pad in (2, 4):      # of a bucket's own size too
+        b.fill(entries, s.cache, pad_to=pad)
+        assert not b.lengths_known and b.notes == {}
+        b.fill_planned(s, pad_to=pad)
+        assert not b.lengths_known
+    b.fill_planned(s)
+    assert b.lengths_known
+    b.notes["a part"] = 1
+    b.pad(2, 2, 2)          # to the counts it has
+    assert not b.lengths_known and b.notes == {}
+
+
 def test_planned_fill_writes_what_the_entries_would():
     """The scheduler's plan written straight from the core's tokens equals the same step given as entries."""
     import numpy as np
