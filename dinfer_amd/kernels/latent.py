@@ -51,6 +51,7 @@ def paged_attention(qa: torch.Tensor, out: torch.Tensor, cache: torch.Tensor, ca
 
 
 EXPANDED_BYTES = 512 << 20     # scratch for expanded keys and values, at most: 32 or 64 thousand keys of 32 or 16 heads
+EXPANDED_SHARE = 32            # and of the device's free memory: what is left is the cache's
 CUS = 256
 
 
@@ -63,15 +64,19 @@ class Expanded:
     def __init__(self, ctx, heads: int, rank: int):
         self.heads, self.rank = heads, rank
         per_chunk = 2 * heads * 4096 + 2048
-        longest = ctx.max_seq_len or 4096
-        self.chunks = min(ctx.max_reqs * (-(-longest // 16) + 1), EXPANDED_BYTES // per_chunk)
+        longest, room = ctx.max_seq_len or 4096, EXPANDED_BYTES
+        if ctx.device.type == "cuda":
+            room = min(room, torch.cuda.mem_get_info(ctx.device)[0] // EXPANDED_SHARE)
+        # (no more requests than can bring ROWS rows each; a chunk at least, whose step then finds no room)
+        self.chunks = max(1, min(min(ctx.max_reqs, ctx.max_tokens // self.ROWS) * (-(-longest // 16) + 1), room // per_chunk))
         buf = ctx.workspace.buffer
         self.keys, self.values = (buf(f"latent_expanded_{n}", heads * 2048, rows=self.chunks) for n in ("keys", "values"))
         self.rot = buf("latent_expanded_rot", 1024, rows=self.chunks)
 
     @staticmethod
     def supports(ctx, dim: int, rot_dim: int, vdim: int, rank: int) -> bool:
-        return ctx.dtype == torch.bfloat16 and ops.latent_expanded_supports(dim, rot_dim, vdim, rank, ctx.page_size)
+        return (ctx.dtype == torch.bfloat16 and ctx.max_tokens >= Expanded.ROWS
+                and ops.latent_expanded_supports(dim, rot_dim, vdim, rank, ctx.page_size))
 
     def plan(self, starts, counts):
         """[(first request, requests, their keys, longest portion)] of the launches for requests of `counts` rows behind `starts`

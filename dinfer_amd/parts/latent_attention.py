@@ -147,6 +147,8 @@ class LatentAttention(Mixer):
         self.expanded = None
         if self.may_expand and latent_kernels.Expanded.supports(ctx, self.dim, self.rot_dim, self.vdim, self.rank):
             self.expanded = ctx.share(("latent_expanded", H, self.rank), lambda: latent_kernels.Expanded(ctx, H, self.rank))
+        else:
+            self.uk = None     # (the copy is the keys' side's alone)
 
     def choices(self):
         return [] if self.expanded is None else [self.expanded]

@@ -51,6 +51,21 @@ def test_lengths_that_are_not_known_are_not_used():
     assert ex.launches(step) is None and not step.notes
 
 
+def test_scratch_holds_what_a_step_can_bring_and_no_more():
+    sizes = {}
+    def ctx(**kw):
+        buffer = lambda name, cols, rows: sizes.__setitem__(name, (rows, cols))
+        return SimpleNamespace(**{**dict(device=torch.device("cpu"), dtype=torch.bfloat16, max_tokens=2048, max_reqs=257, max_seq_len=1000,
+                                         page_size=16, workspace=SimpleNamespace(buffer=buffer)), **kw})
+    assert latent.Expanded(ctx(), 2, 512).chunks == 16 * 64          # of 257 requests 16 can bring 128 rows
+    assert latent.Expanded(ctx(max_reqs=3), 2, 512).chunks == 3 * 64
+    ex = latent.Expanded(ctx(max_seq_len=40960), 16, 512)
+    assert 500 << 20 < sum(r * c * 2 for r, c in sizes.values()) <= 512 << 20 and sizes["latent_expanded_rot"] == (ex.chunks, 1024)
+    assert latent.Expanded.supports(ctx(), 128, 64, 128, 512)
+    for other in (dict(max_tokens=127), dict(dtype=torch.float32), dict(page_size=24)):
+        assert not latent.Expanded.supports(ctx(**other), 128, 64, 128, 512)
+
+
 @pytest.mark.parametrize("q_rank,gated,window,taken", [(96, "entries", None, True), (98, "entries", None, False), (98, True, None, True),
                                                        (None, "entries", None, True), (96, "entries", 64, False)])
 def test_an_entry_gate_that_begins_anywhere_keeps_its_way(q_rank, gated, window, taken):
