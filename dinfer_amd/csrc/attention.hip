@@ -526,18 +526,6 @@ __global__ void __launch_bounds__(64) attn_decode_merge_kernel(const float* __re
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p % 16) == 0; }
 
-// CUs of the current device (asked once per device).
-inline int compute_units() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cached[dev]) {
-    int n = 0;
-    cached[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
-  }
-  return cached[dev];
-}
-
 // The kernel of paired waves over all tiles of a step (see its header).
 template <bool HALVES>
 int launch_pair(const bf16* q, int64_t ld_q, bf16* out, int64_t ld_out, const bf16* kc, const bf16* vc, const int32_t* bt,

@@ -30,6 +30,7 @@
 //   moe_scatter  counts, offsets, the sorted list and the work list, one workgroup (LDS counters)
 //   moe_combine  out[t] = sum_c share[t, c] * y[t * top + c] + shared_gate[t] * shared[t]   (no gate: + shared[t]; no
 //                shares: every row of y counts as it is)
+#include <algorithm>
 #include <type_traits>
 
 #include "lds_loads.cuh"
@@ -595,8 +596,9 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_experts_kernel(Groups p) 
 // rows x 256 columns (gated: 128 of each half), a wave four blocks of 32 x 32: rows 32 (2 a + wave % 2), columns 64 (wave / 2) on.
 // Both operands go from memory straight into LDS, 64 k a stage, eight rows x 128 bytes an instruction, into three stages; where the
 // tiles lie is looked up for WALK_TILES of them before the first, the last three steps of a tile send the first stages of the next, and
-// its results leave beside the next one's products. A step reads the second half of its own stage beside the first eight MFMAs of a
-// wave and the first half of the next one's beside the other eight; in between all meet, and the step's own place is sent anew.
+// its results leave beside the next one's first step (the second waits for them too: it counts what was sent since). A step reads
+// the second half of its own stage beside the first eight MFMAs of a wave and the first half of the next one's beside the other
+// eight; in between all meet, and the step's own place is sent anew.
 // A row's eight pieces are exchanged so that 16 lanes, which LDS serves at once, find their own banks: by bits 1..3 of a row of A, by
 // bits 1, 2 and 4 of one of the weights, whose rows are read in the order of store_rows.
 //
@@ -753,7 +755,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
           for (int x = 0; x < 8; ++x) frag(to, 0, x);
         }
       }
-      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");   // the next tile's first four stages (its products do not wait for the stores)
+      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");   // the next tile's first two stages (not the stores below)
       const ListedRows tl{rows, __builtin_amdgcn_readfirstlane(tiles[i].base), p.c_to_perm, lists + i * TM_BIG};
 #pragma unroll
       for (int a = 0; a < 2; ++a)
@@ -1296,14 +1298,15 @@ __global__ void __launch_bounds__(256) moe_combine_bf16x8_kernel(const bf16* __r
   }
 }
 
-// grid.y arrives from the caller (tiles or blocks of rows), grid.z too (groups); grid.x is set here from the kernel's
-// columns a workgroup.
 // Whether the tiles are many enough to be walked, by the full ones that the entries would fill (the experts' number is not known
 // here). us at 64 experts of 1,408 in a width of 2,048, by the kernel above and walked, full tiles in brackets: gelu 96 rows each
 // (288) 109 and 115; 128 (384) 118 and 119; 60 to 320 (440) 161 and 134; 190 (570) 168 and 133; 256 (768) 176 and 148. Gated 40 each
 // (220) 170 and 158; 128 of half the experts (352) 109 and 113; 96 (528) 175 and 172; 128 (704) 184 and 180; 256 (1,408) 259 and 255.
 // Down 128 (512) 88 and 92; 60 to 320 (584) 118 and 113; 190 (760) 116 and 114; 256 (1,024) 130 and 128; 512 232 and 217.
-constexpr int WALK_PLACES = 256;
+//
+// The same line over ten geometries (8 to 256 experts of 512 to 14,336 in widths of 1,024 to 4,096, 256 to 4,096 tokens, even and uneven
+// choices): of 144 products that are walked the time is 0.92 (gelu 0.88, down 0.92, gated 0.95; geometric means), the worst 1.05
+// (gated, 32 of 2,880, 128 rows each, 326 and 343).
 bool takes_walk(const Groups& p, int end) {
   if (p.K % WALK_K != 0 || p.K < WALK_STAGES * WALK_K) return false;
   const int cols = end >= END_GATED ? 128 : 256;
@@ -1311,13 +1314,15 @@ bool takes_walk(const Groups& p, int end) {
   return full >= (end == END_PLAIN ? 704 : 400);
 }
 
+// grid.y arrives from the caller (tiles or blocks of rows), grid.z too (groups); grid.x is set here from the kernel's
+// columns a workgroup.
 template <int END>
 int launch_experts(const Groups& p, unsigned gy, hipStream_t stream) {
   const int cols = END >= END_GATED ? 128 : 256;
   if (takes_walk(p, END)) {
     auto kernel = grouped_mfma_walk_kernel<bf16, END>;
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, WALK_LDS) != hipSuccess) return ERR_LAUNCH;
-    kernel<<<WALK_PLACES, 512, WALK_LDS, stream>>>(p);
+    kernel<<<std::max(1, compute_units() / 8) * 8, 512, WALK_LDS, stream>>>(p);   // (as many on every XCD)
     return OK;
   }
   // eight XCDs, four tiles at a time (y and z together: the places rounded up may be more than y takes)

@@ -42,7 +42,8 @@ constexpr int EXPAND_LDS = STAGE * STAGES + TILES * (int)sizeof(Tile) + 16 + PAG
 //
 // A tile is 16 stages of 32 k for latents of 512, not much longer than its beginning (lengths, table, first loads) and its 128 KB of
 // stores. So workgroups stay, one a CU, and walk tiles: where the tiles lie is worked out for all of them before the first, the last
-// four steps of a tile send the first stages of the next, and its stores leave while the next one's products run. 20,096 keys, 16
+// four steps of a tile send the first stages of the next, and its stores leave beside the next one's first two steps (the third waits
+// for them too: it counts what was sent since). 20,096 keys, 16
 // heads, 5 tiles a workgroup: 111 us with a workgroup a tile, 97 with this one's walk, 93 with a stage sent as soon as the middle of the
 // step that read its place is behind all waves (three steps before its use instead of one to two); one tile each 22 and 23. A step
 // is 0.85 us, 1.26 PFLOP/s, and what is left is the beginning, the ends of tiles and the caches' writing back at the end. (Two
@@ -195,7 +196,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       f32x16 acc[2][4];
       if (is_value) expand_tile<true>(src, steps, stage, expand_smem, fw, fk, acc, next);
       else expand_tile<false>(src, steps, stage, expand_smem, fw, fk, acc, next);
-      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");   // the next tile's first three stages (its products do not wait for the stores)
+      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");   // the next tile's first three stages (not the stores below)
       bf16* const out = is_value ? values : keys;
       const int first = __builtin_amdgcn_readfirstlane(t.chunk0 + (t.key0 >> 4));
       const int chunks = __builtin_amdgcn_readfirstlane(((t.len + 15) >> 4) - (t.key0 >> 4));   // from this tile's first on
@@ -228,14 +229,6 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing on its way into LDS
     __syncthreads();   // before the next batch is looked up
   }
-}
-
-// CUs of the current device.
-inline int compute_units() {
-  int dev = 0, n = 0;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-  return n > 0 ? n : 256;
 }
 
 }  // namespace

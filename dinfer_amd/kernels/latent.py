@@ -52,7 +52,6 @@ def paged_attention(qa: torch.Tensor, out: torch.Tensor, cache: torch.Tensor, ca
 
 EXPANDED_BYTES = 512 << 20     # scratch for expanded keys and values, at most: 32 or 64 thousand keys of 32 or 16 heads
 EXPANDED_SHARE = 32            # and of the device's free memory: what is left is the cache's
-CUS = 256
 
 
 class Expanded:
@@ -60,6 +59,7 @@ class Expanded:
     layers of one geometry, and the choice for a step."""
 
     ROWS = 128      # a request, from which on a step may gain
+    cus = 256       # of the device
 
     def __init__(self, ctx, heads: int, rank: int):
         self.heads, self.rank = heads, rank
@@ -67,6 +67,7 @@ class Expanded:
         longest, room = ctx.max_seq_len or 4096, EXPANDED_BYTES
         if ctx.device.type == "cuda":
             room = min(room, torch.cuda.mem_get_info(ctx.device)[0] // EXPANDED_SHARE)
+            self.cus = torch.cuda.get_device_properties(ctx.device).multi_processor_count
         # (no more requests than can bring ROWS rows each; a chunk at least, whose step then finds no room)
         self.chunks = max(1, min(min(ctx.max_reqs, ctx.max_tokens // self.ROWS) * (-(-longest // 16) + 1), room // per_chunk))
         buf = ctx.workspace.buffer
@@ -96,9 +97,9 @@ class Expanded:
         scale = self.heads * self.rank / (16 * 512)
         ends, middle = starts + counts, starts + counts / 2
         groups = counts * self.heads / 64
-        queries = 0.077 * self.rank / 512 * max((groups * middle).sum() / CUS, ends.max()) + 0.0155 * scale * counts.sum()
+        queries = 0.077 * self.rank / 512 * max((groups * middle).sum() / self.cus, ends.max()) + 0.0155 * scale * counts.sum()
         tiles = np.ceil(counts / 256) * self.heads
-        keys = 0.0055 * scale * ends.sum() + max((tiles * middle).sum() / CUS * 2.3, ends.max() * 1.7) / 64
+        keys = 0.0055 * scale * ends.sum() + max((tiles * middle).sum() / self.cus * 2.3, ends.max() * 1.7) / 64
         if keys > 0.9 * queries:
             return None
         lengths, rows = ends.astype(np.int64), counts.astype(np.int64)
