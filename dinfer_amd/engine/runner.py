@@ -8,6 +8,8 @@ a loader of its own (models/qwen3/src/executor.rs:977-1031, model.rs:684-832).
 """
 from __future__ import annotations
 
+import gc
+import threading
 from pathlib import Path
 
 import torch
@@ -32,6 +34,29 @@ def _require_gpu(device_index: int) -> torch.device:
     return dev
 
 
+class _Uncollected:
+    """While any thread is inside, the process collects no garbage: a runner that some cycle of references has outlived would take its
+    graphs with it, and to destroy a graph waits for the device, which a capture forbids: the error leaves a destructor and ends the
+    process."""
+
+    def __init__(self):
+        self._lock, self._inside, self._was = threading.Lock(), 0, False
+
+    def __enter__(self):
+        with self._lock:
+            if self._inside == 0:
+                self._was = gc.isenabled()
+                gc.disable()
+            self._inside += 1
+
+    def __exit__(self, *exc):
+        with self._lock:
+            self._inside -= 1
+            if self._inside == 0 and self._was:
+                gc.enable()
+
+
+_uncollected = _Uncollected()
 _first_graph_done: set = set()
 
 
@@ -52,7 +77,7 @@ def _first_graph(device) -> None:
         side = torch.cuda.Stream(device=device)
         graph = torch.cuda.CUDAGraph()
         side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
+        with torch.cuda.stream(side), _uncollected:
             graph.capture_begin()
             try:
                 ops.fill_zero(cell)
@@ -459,7 +484,7 @@ class ModelRunner:
             self._capture_stream = torch.cuda.Stream(device=self.device)
         side = self._capture_stream
         side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
+        with torch.cuda.stream(side), _uncollected:
             # by hand: torch's capture context would collect garbage and empty the allocator's cache first
             g.capture_begin(pool=self._graph_pool)
             try:

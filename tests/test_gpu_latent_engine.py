@@ -53,17 +53,25 @@ def models(tmp_path_factory):
     return out
 
 
+@pytest.fixture
+def launched(monkeypatch):
+    """The keys' side's launches of the last step, call by call."""
+    from dinfer_amd.kernels.latent import Expanded
+    seen, inner = [], Expanded.attention
+
+    def attention(self, launches, *a, **kw):
+        seen.append(launches)
+        return inner(self, launches, *a, **kw)
+    monkeypatch.setattr(Expanded, "attention", attention)
+    return seen
+
+
 def make_runner(models, name, graph=False, rows=1024, page=16):
     from dinfer_amd.config import EngineOptions
     from dinfer_amd.engine.runner import ModelRunner
     opt = EngineOptions(dtype="bfloat16", max_model_len=1024, max_num_seqs=4, max_num_batched_tokens=1024, block_size=page,
                         num_blocks=2048 // page, max_logits_rows=rows, decode_exempt_from_budget=False, hip_graph=graph)
-    r = ModelRunner.from_dir(models[name][0], opt)
-    r.expanded = []      # launches of the keys' side, call by call
-    for c, _ in r.model._choices:
-        inner = c.attention
-        c.attention = lambda launches, *a, _inner=inner, **kw: (r.expanded.append(launches), _inner(launches, *a, **kw))[1]
-    return r
+    return ModelRunner.from_dir(models[name][0], opt)
 
 
 # (request, tokens) a step: from nothing, behind histories, single rows beside, requests that end and whose pages are taken again
@@ -72,7 +80,7 @@ STEPS = [[("a", 300)], [("a", 1), ("b", 400)], [("b", 200), ("a", 1), ("c", 290)
 TAKEN = [True, True, True, False, False, False, False]      # ([("d", 140), ("b", 3)]: fewer than 128 rows a request)
 
 
-def run(r, ids, steps, want_all=True):
+def run(r, launched, ids, steps, want_all=True):
     """{(request, position): logits} and per step whether the keys' side ran."""
     from dinfer_amd.engine.batch import Entry
     at, rows, taken = {}, {}, []
@@ -83,9 +91,9 @@ def run(r, ids, steps, want_all=True):
             assert r.reserve(k, start, n)
             entries.append(Entry(k, ids[k][start:start + n], start, list(range(n)) if want_all else [n - 1]))
             at[k] = start + n
-        del r.expanded[:]
+        del launched[:]
         logits = r.step(entries).double().cpu()
-        taken.append(len(r.expanded))
+        taken.append(len(launched))
         i = 0
         for e in entries:
             for x in e.want:
@@ -109,15 +117,15 @@ def error(rows, wants):
 
 @pytest.mark.parametrize("page", [16, 8])
 @pytest.mark.parametrize("name", list(CONFIGS))
-def test_steps_that_take_the_keys_side(models, name, page):
+def test_steps_that_take_the_keys_side(models, launched, name, page):
     _, _, ids, want = models[name]
     r = make_runner(models, name, page=page)
-    rows, taken = run(r, ids, STEPS)
+    rows, taken = run(r, launched, ids, STEPS)
     layers = len(CONFIGS[name]["layers"])
     assert taken == [layers if t else 0 for t in TAKEN]
     for c, _ in r.model._choices:
         c.weigh = lambda starts, counts: None
-    other, none = run(r, ids, STEPS)
+    other, none = run(r, launched, ids, STEPS)
     assert not any(none) and other.keys() == rows.keys()
     (most, rms), (most_q, rms_q) = error(rows, want), error(other, want)
     # roundings to 8 bits add up to 0.01 or so of the logits; a wrong operand, head or gate is off by several tenths and more
@@ -125,22 +133,22 @@ def test_steps_that_take_the_keys_side(models, name, page):
 
 
 @pytest.mark.parametrize("name", list(CONFIGS))
-def test_requests_dealt_to_several_launches(models, name):
+def test_requests_dealt_to_several_launches(models, launched, name):
     """Scratch that holds one long request or two short ones: the same bits."""
     _, _, ids, _ = models[name]
     steps = [[("a", 200), ("b", 300), ("c", 250)], [("c", 80), ("a", 140), ("b", 340)]]
     r = make_runner(models, name)
-    once, _ = run(r, ids, steps)
-    assert all(len(l) == 1 for l in r.expanded)
+    once, _ = run(r, launched, ids, steps)
+    assert all(len(l) == 1 for l in launched)
     for c, _ in r.model._choices:
         c.chunks = 45
-    parts, taken = run(r, ids, steps)
-    assert all(taken) and [l[:2] for l in r.expanded[0]] == [(0, 2), (2, 1)]
+    parts, taken = run(r, launched, ids, steps)
+    assert all(taken) and [l[:2] for l in launched[0]] == [(0, 2), (2, 1)]
     assert all(torch.equal(once[k], parts[k]) for k in once)
 
 
 @pytest.mark.parametrize("name", list(CONFIGS))
-def test_long_steps_between_replays(models, name):
+def test_long_steps_between_replays(models, launched, name):
     """Steps of the same counts replay a captured graph; those that gain by their lengths are launched one by one between the replays, at
     other lengths each time, and the replays after them are as exact as before."""
     _, _, ids, want = models[name]
@@ -151,7 +159,7 @@ def test_long_steps_between_replays(models, name):
         steps += [[("b", long_one)], [("b", 20), ("c", 12)], [("c", 12), ("b", 20)], [("b", 1), ("c", 1)], [("b", 20), ("c", 12)]]
     replays = []
     for i in range(3):
-        rows, taken = run(r, ids, steps[5 * i:5 * i + 5], want_all=False)
+        rows, taken = run(r, launched, ids, steps[5 * i:5 * i + 5], want_all=False)
         assert [t > 0 for t in taken] == [True, False, False, False, False]
         most, rms = error(rows, want)
         assert most < 0.2 and rms < 0.03, (i, most, rms)
@@ -159,11 +167,11 @@ def test_long_steps_between_replays(models, name):
     assert replays[0] < replays[1] < replays[2]
 
 
-def test_a_small_models_prompts_stay_in_the_graphs(models):
+def test_a_small_models_prompts_stay_in_the_graphs(models, launched):
     _, _, ids, want = models["kudurax"]
     r = make_runner(models, "kudurax", graph=True, rows=4)
     for _ in range(4):
-        rows, taken = run(r, ids, [[("a", 130)], [("a", 128)]], want_all=False)
+        rows, taken = run(r, launched, ids, [[("a", 130)], [("a", 128)]], want_all=False)
         most, rms = error(rows, want)
         assert most < 0.2 and rms < 0.03 and not any(taken)
     assert r.portion_replays >= 2
