@@ -98,6 +98,9 @@ def configure(tuning: str | None = None, plan_file=..., log: bool | None = None)
         _save_stored()
         _settings["plan_file"] = plan_file
         _stored = _stored_path = None
+        for plan in (*_plans.values(), *_ends.values()):
+            if plan:
+                plan.asked = False      # shapes without a choice are looked up in the new file
 
 
 @contextlib.contextmanager
@@ -403,11 +406,12 @@ def _choose(handle, plan, key, a, w, out, workspace, beta) -> None:
         return
     dev = key[0]
     skey = _shape_key(*key[1:])
-    stored = None if plan.asked else _load_stored(dev).get(skey)
+    stored = _load_stored(dev)
+    known = None if plan.asked else stored.get(skey)
     plan.asked = True
-    if isinstance(stored, dict):
-        i, tile = stored.get("index", -1), stored.get("tile")
-        if 0 <= i < len(plan.candidates) and bytes(plan.candidates[i].data).hex() == stored.get("algo"):
+    if isinstance(known, dict):
+        i, tile = known.get("index", -1), known.get("tile")
+        if 0 <= i < len(plan.candidates) and bytes(plan.candidates[i].data).hex() == known.get("algo"):
             own = next((t for t in plan.tiles if t.name() == tile), None)
             if tile is None or own is not None:
                 plan.algo, plan.tile, plan.index, plan.tuned = plan.candidates[i], own, i, True
@@ -415,9 +419,9 @@ def _choose(handle, plan, key, a, w, out, workspace, beta) -> None:
     if not _measuring or torch.cuda.is_current_stream_capturing():
         return
     _tune(handle, plan, key[1], a, w, out, workspace, beta)
-    _stored[skey] = {"index": plan.index, "algo": bytes(plan.algo.data).hex()}
+    stored[skey] = {"index": plan.index, "algo": bytes(plan.algo.data).hex()}
     if plan.tile is not None:
-        _stored[skey]["tile"] = plan.tile.name()
+        stored[skey]["tile"] = plan.tile.name()
     _stored_dirty = True
 
 
@@ -462,10 +466,11 @@ def _choose_end(plan, shape, a, w, out, separate, gated) -> None:
     if plan.asked and not _measuring:
         return
     skey = ",".join(map(str, shape))
-    known = {} if plan.asked else _load_stored(a.device)
+    stored = _load_stored(a.device)
+    known = None if plan.asked else stored.get(skey)
     plan.asked = True
-    if skey in known and isinstance(known[skey], dict) and "tile" in known[skey]:
-        name = known[skey]["tile"]
+    if isinstance(known, dict) and "tile" in known:
+        name = known["tile"]
         plan.tile = _tile_named(name, shape[2], gated) if name is not None else None
         plan.tuned = name is None or plan.tile is not None
         if plan.tuned:
@@ -484,5 +489,5 @@ def _choose_end(plan, shape, a, w, out, separate, gated) -> None:
     if _settings["log"]:
         print(f"[dinfer_amd] product {m} x {n} x {k} and {end}: {plan.tile.name() if plan.tile else 'a pass of its own'} of {plan.times} (us)",
               file=sys.stderr, flush=True)
-    _stored[skey] = {"tile": plan.tile.name() if plan.tile else None}
+    stored[skey] = {"tile": plan.tile.name() if plan.tile else None}
     _stored_dirty = True

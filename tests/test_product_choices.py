@@ -1,0 +1,73 @@
+"""How a product's kernel is chosen and remembered (kernels/blaslt.py), with the library, the kernels and their times stood in for."""
+import json
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from dinfer_amd.kernels import blaslt, tiles
+
+ALGORITHMS = [SimpleNamespace(data=bytes([i] * 16)) for i in range(3)]
+
+
+@pytest.fixture
+def choices(monkeypatch, tmp_path):
+    """blaslt with nothing chosen, a plan file of its own, and all candidates equally fast."""
+    for name in ("_plans", "_ends", "_settings"):
+        monkeypatch.setattr(blaslt, name, dict(getattr(blaslt, name)))
+    blaslt._plans.clear()
+    blaslt._ends.clear()
+    for name in ("_stored", "_stored_path"):
+        monkeypatch.setattr(blaslt, name, None)
+    monkeypatch.setattr(blaslt, "_stored_dirty", False)
+    monkeypatch.setattr(tiles, "shapes", lambda: [(96, 64, 384, False), (128, 128, 256, True), (256, 256, 192, True)])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    ran = []
+    monkeypatch.setattr(blaslt.ops, "gemm_tile", lambda a, w, out, m, shape, **_: ran.append(shape))
+
+    def tune(handle, plan, *rest):
+        plan.index, plan.tuned, plan.algo = 1, True, plan.candidates[1]
+
+    monkeypatch.setattr(blaslt, "_tune", tune)
+    monkeypatch.setattr(blaslt, "_least_of_three", lambda a, run: 10.0)
+    blaslt.configure(tuning="measured", plan_file=str(tmp_path / "first.json"))
+    return SimpleNamespace(ran=ran, folder=tmp_path)
+
+
+A, W, OUT = (torch.zeros(s, dtype=torch.bfloat16) for s in ((320, 512), (1024, 512), (320, 512)))
+
+
+def _end():
+    return blaslt.with_end(A, W, OUT, 320, "gated", 300, lambda: None)
+
+
+def _product():
+    plan = blaslt._plans.setdefault("p", SimpleNamespace(asked=False, tuned=False, candidates=ALGORITHMS, algo=ALGORITHMS[0], index=0,
+                                                         tile=None, tiles=[]))
+    key = (torch.device("cpu"), 320, 512, 512, 512, 512, 512, torch.bfloat16, True, False)
+    if not plan.tuned:
+        blaslt._choose(None, plan, key, A, W, OUT, None, blaslt._zero)
+    return plan
+
+
+def test_a_plan_file_named_later_is_asked_and_written(choices):
+    """Shapes that were met before anything was measured, under one plan file, are looked up in the next one, and what is measured then is
+    written there."""
+    assert not _end() and not _product().tuned
+    second = choices.folder / "second.json"
+    blaslt.configure(plan_file=str(second))
+    with blaslt.measuring():
+        _end()
+        _product()
+    assert len(json.loads(second.read_text())) == 2
+    assert not (choices.folder / "first.json").exists()
+
+
+def test_a_plan_file_named_later_is_read(choices):
+    assert not _end() and not _product().tuned
+    second = choices.folder / "second.json"
+    skey = ",".join(map(str, (320, 1024, 512, 512, 512, 512, "gated")))
+    second.write_text(json.dumps({skey: {"tile": [256, 256]}, "320,512,512,512,512,512,bf16,0": {"index": 2, "algo": ALGORITHMS[2].data.hex()}}))
+    blaslt.configure(plan_file=str(second))
+    assert _end() and choices.ran == [2]
+    assert _product().index == 2
