@@ -484,8 +484,11 @@ def _choose_end(plan, shape, a, w, out, separate, gated) -> None:
     times += [_least_of_three(a, lambda: ops.gemm_tile(a, w, out, m, t.shape, gated=gated, act=None if gated else end)) for t in found]
     best = _first_near(times[1:]) if found else 0
     allowed = next(f for least, f in END_ALLOWANCE if times[0] >= least)
+    plan.tuned = True
+    if min(times) == float("inf"):
+        return      # nothing could be timed: a pass of its own, and no choice in the file
     plan.tile = found[best] if found and times[1 + best] <= times[0] * allowed else None
-    plan.tuned, plan.times = True, [round(t * 1e3, 1) if t < float("inf") else None for t in times]
+    plan.times = [round(t * 1e3, 1) if t < float("inf") else None for t in times]
     if _settings["log"]:
         print(f"[dinfer_amd] product {m} x {n} x {k} and {end}: {plan.tile.name() if plan.tile else 'a pass of its own'} of {plan.times} (us)",
               file=sys.stderr, flush=True)

@@ -71,3 +71,11 @@ def test_a_plan_file_named_later_is_read(choices):
     blaslt.configure(plan_file=str(second))
     assert _end() and choices.ran == [2]
     assert _product().index == 2
+
+
+def test_no_tile_where_nothing_could_be_timed(choices, monkeypatch):
+    """Launches that all fail while they are timed leave the pass of its own, and no choice in the file."""
+    monkeypatch.setattr(blaslt, "_least_of_three", lambda a, run: float("inf"))
+    with blaslt.measuring():
+        assert not _end()
+    assert not choices.ran and not (choices.folder / "first.json").exists()
