@@ -296,8 +296,8 @@ def flush_caches(dev) -> None:
     flush.sum()
 
 
-def _least_of_three(a, run) -> float:
-    """Milliseconds of run(), each time behind a read that empties the caches and one of the activations a, which in a model were
+def _least_of_three(a, m, run) -> float:
+    """Milliseconds of run(), each time behind a read that empties the caches and one of the activations a[:m], which in a model were
     written just before (without it 4,096 x 8,192 x 2,048 takes the library 87 and the tile kernel 125 us, in a step both 100); inf where it
     raises."""
     t = float("inf")
@@ -306,7 +306,7 @@ def _least_of_three(a, run) -> float:
         run()   # first use of a kernel loads it
         for _ in range(3):   # the least of three: a single timing wanders by a few per cent, as much as the candidates differ
             flush_caches(a.device)
-            a.sum()
+            a[:m].sum()     # (the rows of this product alone: a is a buffer of the engine's largest step)
             start.record()
             run()
             end.record()
@@ -331,7 +331,7 @@ def _tune(handle, plan, m, a, w, out, workspace, beta=_zero) -> None:
     if beta is not _zero:
         out = out.clone()
     found = [*plan.candidates, *plan.tiles]
-    times = [_least_of_three(a, lambda: _run(handle, plan, algo, a, w, out, workspace, beta, m)) for algo in found]
+    times = [_least_of_three(a, m, lambda: _run(handle, plan, algo, a, w, out, workspace, beta, m)) for algo in found]
     library = len(plan.candidates)
     plan.index, plan.tuned = _first_near(times[:library]), True
     plan.algo, first = plan.candidates[plan.index], _first_near(times)
@@ -480,8 +480,8 @@ def _choose_end(plan, shape, a, w, out, separate, gated) -> None:
     m, n, k = shape[:3]
     found = [_Tile(i) for i in tiles.candidates(m, n, k, gated)]
     end = shape[-1]
-    times = [_least_of_three(a, separate)]
-    times += [_least_of_three(a, lambda: ops.gemm_tile(a, w, out, m, t.shape, gated=gated, act=None if gated else end)) for t in found]
+    times = [_least_of_three(a, m, separate)]
+    times += [_least_of_three(a, m, lambda: ops.gemm_tile(a, w, out, m, t.shape, gated=gated, act=None if gated else end)) for t in found]
     best = _first_near(times[1:]) if found else 0
     allowed = next(f for least, f in END_ALLOWANCE if times[0] >= least)
     plan.tuned = True

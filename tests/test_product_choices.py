@@ -29,7 +29,7 @@ def choices(monkeypatch, tmp_path):
         plan.index, plan.tuned, plan.algo = 1, True, plan.candidates[1]
 
     monkeypatch.setattr(blaslt, "_tune", tune)
-    monkeypatch.setattr(blaslt, "_least_of_three", lambda a, run: 10.0)
+    monkeypatch.setattr(blaslt, "_least_of_three", lambda a, m, run: 10.0)
     blaslt.configure(tuning="measured", plan_file=str(tmp_path / "first.json"))
     return SimpleNamespace(ran=ran, folder=tmp_path)
 
@@ -75,7 +75,26 @@ def test_a_plan_file_named_later_is_read(choices):
 
 def test_no_tile_where_nothing_could_be_timed(choices, monkeypatch):
     """Launches that all fail while they are timed leave the pass of its own, and no choice in the file."""
-    monkeypatch.setattr(blaslt, "_least_of_three", lambda a, run: float("inf"))
+    monkeypatch.setattr(blaslt, "_least_of_three", lambda a, m, run: float("inf"))
     with blaslt.measuring():
         assert not _end()
     assert not choices.ran and not (choices.folder / "first.json").exists()
+
+
+def test_a_timed_run_finds_its_own_rows_in_the_caches(monkeypatch):
+    """Of an activation buffer as long as the engine's budget only the product's rows are read before a timed run."""
+    read = []
+
+    class Buffer:
+        device = "cpu"
+
+        def __getitem__(self, rows):
+            return SimpleNamespace(sum=lambda: read.append(rows))
+
+        def sum(self):
+            read.append(slice(None))
+
+    monkeypatch.setattr(torch.cuda, "Event", lambda **_: SimpleNamespace(record=lambda: None, synchronize=lambda: None, elapsed_time=lambda _: 1.0))
+    monkeypatch.setattr(blaslt, "flush_caches", lambda dev: None)
+    assert blaslt._least_of_three(Buffer(), 64, lambda: None) == 1.0
+    assert read == [slice(None, 64)] * 3
