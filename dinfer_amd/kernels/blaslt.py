@@ -6,7 +6,7 @@ far off (N 5,120, K 17,408 at 520 rows: 167 us against 102 us for the best of th
 so here the library is called directly and its candidate list for a shape is timed.
 
 Beside the library's list stand a few shapes of the tile kernel (csrc/gemm_tile.hip; tiles.py names those worth timing), which
-also takes what follows a product into its end (`with_end`): timed against the library's product and the pass of its own together.
+also takes what follows a product into its end (`with_end`): timed against the library's product and the pass of its own together, in trains.
 
 When it is timed, and what a product runs with otherwise, is settled so that results repeat:
   * a product outside `measuring()` never times anything: it runs the algorithm its shape was given earlier,
@@ -43,12 +43,17 @@ FLUSH_BYTES = 512 << 20       # read before each timed run: twice the memory-sid
 TUNE_FROM_ROWS = 33           # every size that comes here (up to 32 rows the weight-streaming kernel runs)
 TUNE_FROM_WORK = 1 << 24      # rows x columns x depth below which no choice of kernel repays its measurement
 TIE = 0.03                    # candidates within this fraction of the fastest count as equal: the lowest index wins
-# A product with its end in one kernel is taken up to this much above the product and its pass timed alone (milliseconds of the latter:
-# factor). In a step, where products follow each other, the chip lowers its clock and the library's, bound by the matrix cores, take
-# longer than timed alone, the tile kernel, bound by its loads, does not: alone and in a step, us, 2,048 x 24,576 x 4,096 257 and 303
-# against 289 and 286; 2,048 x 16,384 x 2,048 111 and 119, 108 and 104; 544 x 34,816 x 5,120 186 and 194, 184 and 182;
-# 4,096 x 8,192 x 2,048 and relu2 113 and 120, 129 and 117.
-END_ALLOWANCE = ((0.1, 1.13), (0.0, 1.03))
+# A product with its end in one kernel is timed against the product and its pass in trains: launches of one form back to back, each with another
+# copy of the weight. Behind emptied caches a single launch runs at a clock that a step does not have: the library's, bound by the matrix
+# cores, take longer in a step than timed alone, the tile kernel, bound by its loads, does not. us, the product and its pass and the tile, alone,
+# in trains and in a step: gated 2,048 x 24,576 x 4,096 294 and 291, 306 and 299, 303 and 286; 2,048 x 16,384 x 2,048 118 and 111, 120 and 110, 119
+# and 104; 544 x 34,816 x 5,120 195 and 186, 200 and 189, 194 and 182; relu2 4,096 x 8,192 x 2,048 125 and 130, 124 and 116, 120 and 117. Three
+# processes with files of their own took the same side at 27 of 28 shapes (512 rows 98 and 96 tile, 1,024 rows 180 and 181 pass; 256 rows, 67
+# and 65 to 66, differed).
+TRAIN_MS = 5.0                # of one form until its clock has settled, and as long again timed (trains of 3 in turn share a clock: 300 and 301 at the first)
+TRAINS = 2                    # of each form
+TRAIN_TIE = 0.015             # the product and its pass run where they are within this of the fastest (trains repeat within 1 %)
+TRAIN_TILES = 2               # of the tiles, the fastest alone
 
 _HIP_R_32F, _HIP_R_16BF = 0, 14
 _OP_N, _OP_T = 111, 112
@@ -124,7 +129,7 @@ def _plan_path(dev):
         if f is None:
             from ..csrc import build
             import hashlib
-            ident = f"{torch.cuda.get_device_name(dev)}|{torch.version.hip}|{CANDIDATES}|{WORKSPACE_BYTES}|tiles"
+            ident = f"{torch.cuda.get_device_name(dev)}|{torch.version.hip}|{CANDIDATES}|{WORKSPACE_BYTES}|trains"
             f = str(build.lib_dir() / f"blaslt_plans_{hashlib.sha256(ident.encode()).hexdigest()[:12]}.json")
         _stored_path = f
     return _stored_path
@@ -286,14 +291,18 @@ def _run(handle, plan, algo, a, w, out, workspace, beta=_zero, rows=None) -> Non
                              WORKSPACE_BYTES, stream), "matmul")
 
 
+def _flush_buffer(dev) -> torch.Tensor:
+    flush = _flush.get(dev)
+    if flush is None:
+        flush = _flush[dev] = torch.zeros(FLUSH_BYTES // 4, dtype=torch.float32, device=dev)   # summed as it is: no widened copy
+    return flush
+
+
 def flush_caches(dev) -> None:
     """Reads FLUSH_BYTES of other memory, so that what runs next finds its operands in HBM, as a weight is found
     in a model whose other layers have passed through the caches since. Read, not written: lines written here
     would still be on their way out while the timed kernel runs, and compete with it."""
-    flush = _flush.get(dev)
-    if flush is None:
-        flush = _flush[dev] = torch.zeros(FLUSH_BYTES // 4, dtype=torch.float32, device=dev)   # summed as it is: no widened copy
-    flush.sum()
+    _flush_buffer(dev).sum()
 
 
 def _least_of_three(a, m, run) -> float:
@@ -317,10 +326,36 @@ def _least_of_three(a, m, run) -> float:
     return t
 
 
-def _first_near(times) -> int:
-    """The first within TIE of the fastest: two measurements a per cent apart choose the same one."""
+def _first_near(times, tie=TIE) -> int:
+    """The first within `tie` of the fastest: two measurements a per cent apart choose the same one."""
     fastest = min(times)
-    return next(i for i, t in enumerate(times) if t <= fastest * (1.0 + TIE)) if fastest < float("inf") else 0
+    return next(i for i, t in enumerate(times) if t <= fastest * (1.0 + tie)) if fastest < float("inf") else 0
+
+
+def _in_trains(w, forms, alone) -> list:
+    """Milliseconds a launch of each form(weight) in trains with copies of w in turn; alone: what a launch takes about. Nothing waits in
+    between, so the chip stays as busy as a step keeps it."""
+    room = _flush_buffer(w.device).view(w.dtype)
+    n, k = w.shape
+    step = -(-((n - 1) * w.stride(0) + k) // 64) * 64       # elements between copies, whole lines
+    copies = [w]
+    for i in range(min(FLUSH_BYTES // (2 * step), 63)):
+        copies.append(room.as_strided((n, k), (w.stride(0), 1), i * step))
+        copies[-1].copy_(w)
+    launches = [max(4, min(128, round(TRAIN_MS / t))) for t in alone]
+    marks, at = [[] for _ in forms], 0
+    for _ in range(TRAINS):
+        for form, count, mine in zip(forms, launches, marks):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            for i in range(2 * count):
+                if i == count:
+                    start.record()
+                form(copies[at % len(copies)])
+                at += 1
+            end.record()
+            mine.append((start, end))
+    torch.cuda.synchronize(w.device)
+    return [min(start.elapsed_time(end) for start, end in mine) / count for mine, count in zip(marks, launches)]
 
 
 def _tune(handle, plan, m, a, w, out, workspace, beta=_zero) -> None:
@@ -436,10 +471,12 @@ class _End:
 _ends: dict = {}
 
 
-def with_end(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, end: str, rows: int, separate: Callable[[], None]) -> bool:
+def with_end(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, end: str, rows: int,
+             separate: Callable[[torch.Tensor], None]) -> bool:
     """out[:rows] = end(a @ w.T) in one kernel, bfloat16: end "gated" (w = [wg; wu] stacked, silu(a @ wg.T) * (a @ wu.T)) or an
-    activation of ops.GEMM_TILE_ACTS. m: the row count the choice goes by. False, and nothing done, where `separate`, which does the same
-    by a product and a pass of its own, was measured to be as fast, or nothing was measured."""
+    activation of ops.GEMM_TILE_ACTS. m: the row count the choice goes by; while measuring, out's rows up to m are written. False, and nothing
+    done, where `separate`, which does the same with the weight it is given by a product and a pass of its own, was measured to be as
+    fast (TRAIN_TIE), or nothing was measured."""
     global _stored_dirty, worth_measuring_met
     gated = end == "gated"
     n, k = w.shape
@@ -480,15 +517,17 @@ def _choose_end(plan, shape, a, w, out, separate, gated) -> None:
     m, n, k = shape[:3]
     found = [_Tile(i) for i in tiles.candidates(m, n, k, gated)]
     end = shape[-1]
-    times = [_least_of_three(a, m, separate)]
-    times += [_least_of_three(a, m, lambda: ops.gemm_tile(a, w, out, m, t.shape, gated=gated, act=None if gated else end)) for t in found]
-    best = _first_near(times[1:]) if found else 0
-    allowed = next(f for least, f in END_ALLOWANCE if times[0] >= least)
+    forms = [separate, *(lambda weight, t=t: ops.gemm_tile(a, weight, out, m, t.shape, gated=gated, act=None if gated else end) for t in found)]
+    alone = [_least_of_three(a, m, lambda: form(w)) for form in forms]
     plan.tuned = True
-    if min(times) == float("inf"):
+    if min(alone) == float("inf"):
         return      # nothing could be timed: a pass of its own, and no choice in the file
-    plan.tile = found[best] if found and times[1 + best] <= times[0] * allowed else None
-    plan.times = [round(t * 1e3, 1) if t < float("inf") else None for t in times]
+    last = sorted(alone[1:])[:TRAIN_TILES][-1:]
+    tried = [i for i, t in enumerate(alone) if t < float("inf") and (i == 0 or t <= last[0])]
+    trains = _in_trains(w, [forms[i] for i in tried], [alone[i] for i in tried])
+    best = tried[_first_near(trains, TRAIN_TIE)]
+    plan.tile = found[best - 1] if best else None
+    plan.times = [round(t * 1e3, 1) if t < float("inf") else None for t in alone], {i: round(t * 1e3, 1) for i, t in zip(tried, trains)}
     if _settings["log"]:
         print(f"[dinfer_amd] product {m} x {n} x {k} and {end}: {plan.tile.name() if plan.tile else 'a pass of its own'} of {plan.times} (us)",
               file=sys.stderr, flush=True)

@@ -157,13 +157,13 @@ def gated_nt(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, scratch: torch
     if a.dtype == torch.bfloat16 and act == "silu" and m <= SMALL_M and w.shape[1] % 8 == 0:
         return ops.gemm_small_m_gated(a, w, out, m)
 
-    def separate():
+    def separate(w):
         matmul_nt(a, w, scratch, m, may_pad=True)
         ops.gated_act(scratch, out, m, act)
 
     if not (a.dtype == torch.bfloat16 and act == "silu" and m > SMALL_M
             and blaslt.with_end(a, w, out, min(a.shape[0], out.shape[0], row_bucket(m)), "gated", m, separate)):
-        separate()
+        separate(w)
     return out
 
 
@@ -172,13 +172,13 @@ def act_nt(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, act: str
     if m <= 0:
         return out
 
-    def separate():
+    def separate(w):
         matmul_nt(a, w, out, m, may_pad=True)
         ops.act(out, out, m, act)
 
     if not (a.dtype == torch.bfloat16 and act in ops.GEMM_TILE_ACTS and m > SMALL_M
             and blaslt.with_end(a, w, out, min(a.shape[0], out.shape[0], row_bucket(m)), act, m, separate)):
-        separate()
+        separate(w)
     return out
 
 

@@ -30,6 +30,7 @@ def choices(monkeypatch, tmp_path):
 
     monkeypatch.setattr(blaslt, "_tune", tune)
     monkeypatch.setattr(blaslt, "_least_of_three", lambda a, m, run: 10.0)
+    monkeypatch.setattr(blaslt, "_in_trains", lambda w, forms, alone: [10.0] * len(forms), raising=False)
     blaslt.configure(tuning="measured", plan_file=str(tmp_path / "first.json"))
     return SimpleNamespace(ran=ran, folder=tmp_path)
 
@@ -38,7 +39,7 @@ A, W, OUT = (torch.zeros(s, dtype=torch.bfloat16) for s in ((320, 512), (1024, 5
 
 
 def _end():
-    return blaslt.with_end(A, W, OUT, 320, "gated", 300, lambda: None)
+    return blaslt.with_end(A, W, OUT, 320, "gated", 300, lambda w: None)
 
 
 def _product():
@@ -79,6 +80,25 @@ def test_no_tile_where_nothing_could_be_timed(choices, monkeypatch):
     with blaslt.measuring():
         assert not _end()
     assert not choices.ran and not (choices.folder / "first.json").exists()
+
+
+@pytest.mark.parametrize("alone,trains,tile", [
+    ((10.0, 11.0, 11.2), (10.0, 10.5, 11.0), None),      # the tiles lose by less than a single launch's error: the product and its pass
+    ((10.0, 9.9, 9.8), (10.0, 9.9, 9.9), None),          # they win by less than trains repeat
+    ((10.0, 11.0, 11.2), (10.0, 9.8, 9.4), 2),           # they win in trains, the second of them
+    ((10.0, 11.0, 11.2), (10.0, 9.4, 9.3), 1)])          # both alike: the first
+def test_ends_are_chosen_as_they_run_in_a_step(choices, monkeypatch, alone, trains, tile):
+    """By trains, without an allowance for either side, and the product and its pass where they are as fast; the forms are the pass first, then the
+    tiles in the order of their estimate."""
+    left = list(alone)
+    monkeypatch.setattr(blaslt, "_least_of_three", lambda a, m, run: left.pop(0))
+    monkeypatch.setattr(blaslt, "_in_trains", lambda w, forms, alone: list(trains), raising=False)
+    monkeypatch.setattr(tiles, "candidates", lambda m, n, k, gated: [1, 2])
+    with blaslt.measuring():
+        assert _end() == (tile is not None)
+    stored = json.loads((choices.folder / "first.json").read_text())
+    assert [v["tile"] for v in stored.values()] == [None if tile is None else list(tiles.shapes()[tile][:2])]
+    assert choices.ran == ([] if tile is None else [tile])
 
 
 def test_a_timed_run_finds_its_own_rows_in_the_caches(monkeypatch):
