@@ -466,6 +466,9 @@ FLASH_CASES = [
     (8, 1, 128, 16, 70, 12, True, 8.0, [(300, 100), (300, 1), (75, 2), (12, 12)]),
     (3, 3, 48, 8, 0, 0, True, 0.0, [(100, 17), (64, 1)]),
     (16, 4, 128, 16, 33, 40, True, 0.0, [(520, 130), (71, 1)]),     # keeps more than it sees; rows of three tiles
+    # heads of 128 with more tiles of 16 rows (longest x requests) than two a CU: 32 rows a tile, pages of a power of two and not
+    (32, 8, 128, 16, 70, 12, True, 8.0, [(300, 150), (75, 2)]),
+    (64, 8, 128, 24, 33, 40, True, 0.0, [(200, 97), (64, 17)]),
 ]
 
 

@@ -225,11 +225,28 @@ def test_attention_plain_kernel(dtype, window):
     torch.testing.assert_close(out.double().cpu().view(-1, H, D), want, **tol(dtype))
 
 
+def flash_rows(H, Hkv, D, page, window, new):
+    """The rows of a tile that attn_flash takes for a step, and the waves that share its keys (csrc/attention.hip, launch_flash); 0 rows: the
+    kernel of paired waves."""
+    cus, total, longest = torch.cuda.get_device_properties(0).multi_processor_count, sum(new), max(new)
+    if D == 128:
+        if window == 0 and ops().attn_flash_form(total, len(new), longest, H, Hkv, page):
+            return 0, 8
+        rounds = lambda rows: -(-(total // rows * H) // (2 * cus))
+        wide = total // 48 * H >= 1300 if len(new) == 1 else -(-longest // 48) * len(new) * H >= 2000 and rounds(48) < rounds(32)
+        if longest > 32 and wide:
+            return 48, 4
+    small = min(-(-longest // 16) * len(new), total // 16 + len(new)) * H
+    if D <= 128 and small <= cus and longest <= 128:
+        return 16, 8
+    return (32 if D <= 128 and longest > 16 and small > 2 * cus else 16), 4
+
+
 @pytest.mark.parametrize("window", [0, 50])
 @pytest.mark.parametrize("H,Hkv,D,page", GEOS)
 def test_attention_flash(H, Hkv, D, page, window):
     # prompts without history (70 / 33 / 5: several tiles, ragged tail, idle waves), portions with
-    # history that ends inside a page, single rows, and a long run that needs the two-tile kernel
+    # history that ends inside a page, single rows, and a longer run (all sizes in tiles of 16 rows)
     hist, new = [0, 0, 0, 40, 70, 300, 129, 7], [70, 33, 5, 5, 1, 1, 150, 64]
     q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=3)
     out = torch.zeros(sum(new), H * D, device=DEV, dtype=torch.bfloat16)
@@ -246,8 +263,23 @@ def test_attention_flash(H, Hkv, D, page, window):
 def test_attention_flash_few_tiles(H, Hkv, D, page, window, hist, new):
     """So few rows that tiles of 16 leave no CU more than two: their own kernels, a tile's keys shared by four waves or eight, some of which
     have none."""
-    cus, tiles = torch.cuda.get_device_properties(0).multi_processor_count, min(-(-max(new) // 16) * len(new), sum(new) // 16 + len(new))
-    assert tiles * H <= 2 * cus and (max(new) > 128 or tiles * H <= cus)
+    assert flash_rows(H, Hkv, D, page, window, new) == (16, 4 if max(new) > 128 else 8)
+    q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=3)
+    out = torch.full((sum(new) + 1, H * D), 7.0, device=DEV, dtype=torch.bfloat16)
+    ops().attn_flash(q, out, kc, vc, m["bt"], m["cu"], m["sl"], len(hist), sum(new), max(new), scale=D ** -0.5,
+                     window=window, heads=H, kv_heads=Hkv, head_dim=D, page_size=page)
+    want = expected_attention(outs, hist, D ** -0.5, window)
+    torch.testing.assert_close(out[:-1].double().cpu().view(-1, H, D), want, rtol=2e-2, atol=2e-2)
+    assert (out[-1] == 7.0).all()
+
+
+@pytest.mark.parametrize("H,Hkv,D,page,window,hist,new", [
+    (24, 8, 32, 8, 0, [0, 200, 31], [300, 129, 33]), (16, 4, 48, 16, 70, [0, 40, 7], [700, 300, 17]), (32, 4, 64, 16, 0, [1000, 5], [290, 70]),
+    (12, 4, 96, 24, 100, [0, 333, 0, 77], [700, 300, 5, 130]), (16, 4, 128, 24, 0, [0, 333, 0, 77], [700, 300, 5, 130]),
+    (16, 8, 128, 16, 50, [0, 64, 300], [520, 31, 33]), (40, 8, 128, 16, 0, [3000], [300])])
+def test_attention_flash_32_rows_a_tile(H, Hkv, D, page, window, hist, new):
+    """More tiles of 16 than two a CU: 32 rows a tile, two row tiles that share every key and value fragment, at every head size that has them."""
+    assert flash_rows(H, Hkv, D, page, window, new) == (32, 4)
     q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=3)
     out = torch.full((sum(new) + 1, H * D), 7.0, device=DEV, dtype=torch.bfloat16)
     ops().attn_flash(q, out, kc, vc, m["bt"], m["cu"], m["sl"], len(hist), sum(new), max(new), scale=D ** -0.5,
@@ -259,17 +291,18 @@ def test_attention_flash_few_tiles(H, Hkv, D, page, window, hist, new):
 
 @pytest.mark.parametrize("skip", [False, True])
 @pytest.mark.parametrize("H,Hkv,D,page,window,tile,new", [
-    (4, 2, 64, 16, 0, 32, [1] * 20 + [290, 1, 33] + [1] * 20), (4, 1, 128, 16, 0, 32, [1] * 80 + [130, 1, 65]),
-    (2, 1, 32, 8, 0, 32, [1] * 20 + [161, 1, 160] + [1] * 40), (2, 2, 96, 24, 50, 32, [1] * 40 + [257, 31]),
-    (64, 8, 128, 16, 0, 48, [1] * 30 + [1000] + [1] * 8), (32, 8, 128, 24, 100, 48, [1] * 50 + [1500, 500] + [1] * 20),
-    (2, 2, 48, 16, 0, 32, [300] + [1] * 66 + [17]), (3, 1, 256, 16, 0, 16, [1] * 66 + [150, 1, 15, 17])])
+    (4, 2, 64, 16, 0, 16, [1] * 20 + [290, 1, 33] + [1] * 20), (4, 1, 128, 16, 0, 16, [1] * 80 + [130, 1, 65]),
+    (2, 1, 32, 8, 0, 16, [1] * 20 + [161, 1, 160] + [1] * 40), (2, 2, 96, 24, 50, 16, [1] * 40 + [257, 31]),
+    (16, 4, 32, 8, 0, 32, [1] * 20 + [161, 1, 160] + [1] * 40), (16, 2, 48, 16, 0, 32, [300] + [1] * 66 + [17]),
+    (16, 4, 64, 16, 0, 32, [1] * 20 + [290, 1, 33] + [1] * 20), (16, 2, 96, 24, 50, 32, [1] * 40 + [257, 31]),
+    (8, 1, 128, 16, 0, 32, [1] * 80 + [130, 1, 65]),
+    (64, 8, 128, 16, 400, 48, [1] * 30 + [1000] + [1] * 8), (32, 8, 128, 24, 100, 48, [1] * 50 + [1500, 500] + [1] * 20),
+    (2, 2, 48, 16, 0, 16, [300] + [1] * 66 + [17]), (3, 1, 256, 16, 0, 16, [1] * 66 + [150, 1, 15, 17])])
 def test_attention_flash_counts_the_tiles_of_few_portions(H, Hkv, D, page, window, tile, new, skip):
     """A few portions among many single rows: workgroups for the tiles that exist only, over more requests than a wave counts at
     once, at 16, 32 and 48 rows a tile; single rows are served or left as they are."""
     assert -(-max(new) // tile) * len(new) >= 4 * (sum(new) // tile + len(new))     # where the tiles are counted
-    if D == 128:    # 48 rows a tile where that saves a round of two workgroups a CU
-        places = 2 * torch.cuda.get_device_properties(0).multi_processor_count
-        assert (tile == 48) == (-(-(sum(new) // 48 * H) // places) < -(-(sum(new) // 32 * H) // places))
+    assert flash_rows(H, Hkv, D, page, window, new)[0] == tile
     hist = [(7 * i + 3) % 90 for i in range(len(new))]
     q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=13)
     out = torch.full((sum(new) + 1, H * D), 7.0, device=DEV, dtype=torch.bfloat16)
@@ -763,11 +796,13 @@ def test_attention_flash_a_prompt_of_thousands_of_rows(page, rows, windowed, sid
 @pytest.mark.parametrize("side", [0, 1], ids=["spike_before_the_line", "spike_behind_the_line"])
 @pytest.mark.parametrize("window", [0, 4200])
 @pytest.mark.parametrize("page", [16, 8])
-def test_attention_flash_a_portion_behind_thousands_of_keys(page, window, side):
-    """600 rows behind 4,000 keys (32 rows a workgroup: every wave walks 1,150 keys), beside a short request."""
-    H, Hkv, D = 8, 2, 128
+@pytest.mark.parametrize("H,rows", [(8, 16), (16, 32)])
+def test_attention_flash_a_portion_behind_thousands_of_keys(H, rows, page, window, side):
+    """600 rows behind 4,000 keys (16 or 32 rows a workgroup: every wave walks 1,150 keys), beside a short request."""
+    Hkv, D = 2, 128
     hist, new = [4000, 20], [600, 40]
-    lines = [l for lo, hi in flash_wave_runs(hist[0], new[0], window, 32) for l in table_refetches(lo, hi, page)]
+    assert flash_rows(H, Hkv, D, page, window, new) == (rows, 4)
+    lines = [l for lo, hi in flash_wave_runs(hist[0], new[0], window, rows) for l in table_refetches(lo, hi, page)]
     assert lines
     key = lines[len(lines) // 2] - 1 + side
     q, kc, vc, m, outs = paged_case(torch.bfloat16, H, Hkv, D, page, hist, new, seed=29, spike={0: (key, 3.0)}, sharp=3.0)
