@@ -1148,10 +1148,10 @@ def test_library_gemm_with_measured_algorithm(tmp_path):
     stored = json.loads((tmp_path / "plans.json").read_text())
     assert any(k.startswith("520,1000,1096,") for k in stored) and all(0 <= v["index"] < 32 for v in stored.values())
     # a process that starts with the file takes its choices without measuring: forget the plans, keep the file
-    measured = {k: p.index for k, p in blaslt._plans.items() if p and p.tuned}
+    measured = {k: (p.index, p.tile and p.tile.shape) for k, p in blaslt._plans.items() if p and p.tuned}
     blaslt._plans.clear()
     _library_gemm_cases(gemm)
-    again = {k: p.index for k, p in blaslt._plans.items() if p and p.tuned}
+    again = {k: (p.index, p.tile and p.tile.shape) for k, p in blaslt._plans.items() if p and p.tuned}
     assert again == measured and all(p.times is None for p in blaslt._plans.values() if p)
     blaslt.configure(plan_file=None)
 

@@ -31,15 +31,15 @@ def _close(got, want, name):
     assert bool((err <= 2.0 ** -8 * want.abs() + 1e-4).all()), f"{name}: {float(err.max())}"
 
 
-def _shapes():
-    try:
-        from dinfer_amd.kernels import tiles
-        return range(len(tiles.shapes()))
-    except Exception:       # no library can be built here: nothing to collect
-        return range(1)
+SHAPES = 13
 
 
-@pytest.mark.parametrize("shape", _shapes())
+def test_every_shape_is_tested():
+    from dinfer_amd.kernels import tiles
+    assert len(tiles.shapes()) == SHAPES
+
+
+@pytest.mark.parametrize("shape", range(SHAPES))
 def test_every_shape_at_its_edges(shape):
     """Rows and columns one below, at and one above a tile, the least depth, one more step, and more tiles than workgroups (several
     rounds of a walk); nothing outside of the product is written."""
@@ -114,7 +114,7 @@ def test_products_with_ends_choose_and_remember(tmp_path):
         stored = json.loads((tmp_path / "plans.json").read_text())
         assert any(k.endswith(",gated") for k in stored) and any(k.endswith(",relu2") for k in stored)
         chosen = {k: p.tile and p.tile.shape for k, p in blaslt._ends.items() if p.tuned}
-        assert chosen
+        assert any(p.times for p in blaslt._ends.values())
         blaslt._plans.clear()
         blaslt._ends.clear()
         run()
@@ -132,3 +132,72 @@ def test_products_with_ends_choose_and_remember(tmp_path):
         blaslt.configure(plan_file=None)
         blaslt._plans.clear()
         blaslt._ends.clear()
+
+
+@pytest.mark.parametrize("end", ["gated", "relu2", "add", "floats", None])
+def test_a_tile_chosen_for_a_product_runs_it(tmp_path, monkeypatch, end):
+    """Where tiles time faster, by measuring and then by another process's plan file: the tile runs, the result is right, and rows between the
+    product's and the size it was chosen for are left alone."""
+    from dinfer_amd.kernels import blaslt, gemm, ops
+    m, n, k = 300, 512, 1024
+    assert gemm.row_bucket(m) == 320
+    ran = []
+    tile = ops.gemm_tile
+
+    def watched(a, w, out, rows, shape, **kw):
+        ran.append((rows, shape, "gated" if kw.get("gated") else kw.get("act")))
+        return tile(a, w, out, rows, shape, **kw)
+
+    def timed(run):     # (a pass of its own has a product before it, which a tile may run)
+        ran.clear()
+        run()
+        return 1.0 if ran and ran[-1][2] == (end if end in ("gated", "relu2") else None) else 2.0
+
+    monkeypatch.setattr(ops, "gemm_tile", watched)
+
+    monkeypatch.setattr(blaslt, "_least_of_three", lambda a, m, run: timed(run))
+    monkeypatch.setattr(blaslt, "_in_trains", lambda w, forms, alone: [timed(lambda: form(w)) for form in forms])
+    a, w = _inputs(m + 40, n, k, end == "gated", seed=4)
+    scratch = torch.empty(m + 40, 2 * n, device=DEV, dtype=torch.bfloat16)
+    start = torch.randn(m + 40, n, device=DEV).to(torch.bfloat16)
+
+    def run():
+        out = start.clone() if end == "add" else torch.full((m + 40, n), 7.0, device=DEV, dtype=torch.float32 if end == "floats" else torch.bfloat16)
+        if end == "gated":
+            gemm.gated_nt(a, w, out, scratch, m, "silu")
+        elif end == "relu2":
+            gemm.act_nt(a, w, out, m, "relu2")
+        elif end == "add":
+            assert gemm.add_nt(a, w, out, m)
+        else:
+            gemm.matmul_nt(a, w, out, m, may_pad=True)
+        return out
+
+    def forget():
+        blaslt._plans.clear()
+        blaslt._ends.clear()
+
+    forget()
+    blaslt.configure(tuning="measured", plan_file=str(tmp_path / "plans.json"))
+    try:
+        with blaslt.measuring():
+            run()
+        plans = lambda: [p for p in (*blaslt._plans.values(), *blaslt._ends.values()) if p and p.tile is not None]
+        chosen = [p.tile.shape for p in plans()]
+        assert chosen and any(e.get("tile") for e in json.loads((tmp_path / "plans.json").read_text()).values())
+        forget()
+        blaslt.configure(plan_file="")
+        blaslt.configure(plan_file=str(tmp_path / "plans.json"))
+        ran.clear()
+        out = run()
+        assert [r[:2] for r in ran] == [(m, plans()[0].tile.shape)] and [p.tile.shape for p in plans()] == chosen[-1:]
+        assert all(p.times is None for p in plans())
+        z = _want(a[:m], w, n, None if end == "floats" else end, start[:m])
+        if end == "floats":
+            torch.testing.assert_close(out[:m].double(), z, rtol=0, atol=4 * k ** 0.5 * 2.0 ** -24 * 8)    # (as above)
+        else:
+            _close(out[:m], z, str(end))
+        assert torch.equal(out[m:], start[m:]) if end == "add" else bool((out[m:] == 7).all())
+    finally:
+        blaslt.configure(plan_file=None)
+        forget()
