@@ -27,8 +27,8 @@ token ids back on the host). On the same line:
   phases    where a decode step's time goes (ms a step, from a second, instrumented run of the same steps that
             is not the one timed): the host's schedule, fill, launch, sample, wait and update, and the model's
             kernels on the device between two events (`gpu`);
-  gemm      which of the library's algorithms the products of many rows run with (index in its list per shape),
-            and how each was chosen.
+  gemm      which of the library's algorithms the products of many rows run with (index in its list per shape), or which
+            tiles of the kernel written here, and how each was chosen.
 
 All data is synthetic: weights N(0, 0.02) / gains 1 + N(0, 0.1) drawn on the device, token
 ids uniform in the vocabulary. The reference publishes no number for this size or
@@ -71,9 +71,11 @@ def model_numbers(c, dtype_bytes):
 
 
 def gemm_summary(chosen):
-    """The library's algorithm per product shape, short: 'rows x n x k[+]' -> index in its list ('+': adds into its output)."""
+    """The algorithm per product shape, short: 'rows x n x k[+]' -> index in the library's list, or 'rows x columns' of the tile kernel's
+    ('+': adds into its output; with the name of what a tile runs in its end)."""
     measured = sum(1 for c in chosen if c["chosen"] == "measured")
-    picks = {f"{c['m']}x{c['n']}x{c['k']}{'+' if c['accumulate'] else ''}": c["algorithm"]
+    picks = {f"{c['m']}x{c['n']}x{c['k']}{'+' if c['accumulate'] else ''}{' ' + c['end'] if 'end' in c else ''}":
+             c["algorithm"] if c["algorithm"] is not None else "x".join(map(str, c["tile"]))
              for c in chosen if c["m"] in (64, 2048)}
     return {"shapes": len(chosen), "measured": measured, "algorithm_of": picks}
 

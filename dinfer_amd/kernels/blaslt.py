@@ -382,16 +382,19 @@ def _shape_key(m, n, k, lda, ldw, ldc, out_dtype, aligned, accumulate) -> str:
 
 
 def chosen() -> list:
-    """What every shape met so far runs with: rows, columns, depth, index in the library's list ("tile": the rows and columns of the
-    tile kernel that runs it instead), how it was chosen."""
+    """What every shape met so far runs with: rows, columns, depth, index in the library's list (None: "tile", the rows and columns of
+    the tile kernel that runs it instead), how it was chosen. Products that a tile runs together with what follows them are named by their "end"."""
     out = []
     for key, plan in _plans.items():
         if plan:
             _, m, n, k = key[:4]
-            out.append({"m": m, "n": n, "k": k, "accumulate": bool(key[-1]), "algorithm": plan.index,
+            out.append({"m": m, "n": n, "k": k, "accumulate": bool(key[-1]), "algorithm": plan.index if plan.tile is None else None,
                         "chosen": "measured" if plan.tuned else "first suggestion"})
             if plan.tile is not None:
                 out[-1]["tile"] = plan.tile.name()
+    for (_, m, n, k, *_, end), plan in _ends.items():
+        if plan.tile is not None:
+            out.append({"m": m, "n": n, "k": k, "accumulate": False, "algorithm": None, "chosen": "measured", "tile": plan.tile.name(), "end": end})
     return out
 
 

@@ -118,3 +118,15 @@ def test_a_timed_run_finds_its_own_rows_in_the_caches(monkeypatch):
     monkeypatch.setattr(blaslt, "flush_caches", lambda dev: None)
     assert blaslt._least_of_three(Buffer(), 64, lambda: None) == 1.0
     assert read == [slice(None, 64)] * 3
+
+
+def test_what_was_chosen_names_the_tiles_that_run(choices, monkeypatch):
+    """No library algorithm is named for a product that a tile runs, and products with their ends are listed."""
+    import bench
+    plan = _product()
+    plan.tuned, plan.tile = True, blaslt._Tile(1)
+    blaslt._plans[torch.device("cpu"), 2048, 512, 512, 512, 512, 512, torch.bfloat16, True, False] = blaslt._plans.pop("p")
+    end = blaslt._ends[torch.device("cpu"), 2048, 1024, 512, 512, 512, 512, "gated"] = blaslt._End()
+    end.tuned, end.tile = True, blaslt._Tile(2)
+    assert bench.gemm_summary(blaslt.chosen()) == {"shapes": 2, "measured": 2, "algorithm_of": {
+        "2048x512x512": "128x128", "2048x1024x512 gated": "256x256"}}
