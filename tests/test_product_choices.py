@@ -130,3 +130,19 @@ def test_what_was_chosen_names_the_tiles_that_run(choices, monkeypatch):
     end.tuned, end.tile = True, blaslt._Tile(2)
     assert bench.gemm_summary(blaslt.chosen()) == {"shapes": 2, "measured": 2, "algorithm_of": {
         "2048x512x512": "128x128", "2048x1024x512 gated": "256x256"}}
+
+
+def test_the_warm_up_measures_on_rows_that_differ(choices, monkeypatch):
+    """Rows that are all alike take the matrix cores less power, and the kernels that they bound seem faster than in any real step."""
+    from dinfer_amd.engine import runner
+    monkeypatch.setattr(blaslt, "available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    steps = []
+    made_up = SimpleNamespace(
+        options=SimpleNamespace(gemm_tuning="measured", max_num_seqs=4, max_model_len=600), dtype=torch.bfloat16, group_specs=[None], max_tokens=1024,
+        num_blocks=100, page_size=16, max_rows=4, device=None, model=SimpleNamespace(spec=SimpleNamespace(vocab_size=500)),
+        reserve=lambda *a: True, finish=lambda rid: None, step=steps.append)
+    monkeypatch.setattr(blaslt, "worth_measuring_met", 0)
+    runner.ModelRunner.warm_up(made_up)
+    tokens = [t for e in steps[0] for t in e.tokens]
+    assert len(tokens) == 1024 and set(tokens) == set(range(500))
