@@ -53,7 +53,8 @@ TIE = 0.03                    # candidates within this fraction of the fastest c
 TRAIN_MS = 5.0                # of one form until its clock has settled, and as long again timed (trains of 3 in turn share a clock: 300 and 301 at the first)
 TRAINS = 2                    # of each form
 TRAIN_TIE = 0.015             # the product and its pass run where they are within this of the fastest (trains repeat within 1 %)
-TRAIN_TILES = 2               # of the tiles, the fastest alone
+TRAIN_TILES = 2               # the fastest tile alone, and the next one within 5 % of it
+TRAIN_CLEAR = 1.25            # a form this far above the fastest alone is left out (alone and in trains the two sides moved by up to 16 %)
 
 _HIP_R_32F, _HIP_R_16BF = 0, 14
 _OP_N, _OP_T = 111, 112
@@ -525,9 +526,9 @@ def _choose_end(plan, shape, a, w, out, separate, gated) -> None:
     plan.tuned = True
     if min(alone) == float("inf"):
         return      # nothing could be timed: a pass of its own, and no choice in the file
-    last = sorted(alone[1:])[:TRAIN_TILES][-1:]
-    tried = [i for i, t in enumerate(alone) if t < float("inf") and (i == 0 or t <= last[0])]
-    trains = _in_trains(w, [forms[i] for i in tried], [alone[i] for i in tried])
+    near = sorted(alone[1:])[:TRAIN_TILES]
+    tried = [i for i, t in enumerate(alone) if t < min(alone) * TRAIN_CLEAR and (i == 0 or (t <= near[-1] and t <= near[0] * 1.05))]
+    trains = _in_trains(w, [forms[i] for i in tried], [alone[i] for i in tried]) if len(tried) > 1 else [alone[tried[0]]]
     best = tried[_first_near(trains, TRAIN_TIE)]
     plan.tile = found[best - 1] if best else None
     plan.times = [round(t * 1e3, 1) if t < float("inf") else None for t in alone], {i: round(t * 1e3, 1) for i, t in zip(tried, trains)}

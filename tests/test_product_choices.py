@@ -101,6 +101,20 @@ def test_ends_are_chosen_as_they_run_in_a_step(choices, monkeypatch, alone, trai
     assert choices.ran == ([] if tile is None else [tile])
 
 
+@pytest.mark.parametrize("alone,forms,tile", [
+    ((10.0, 13.0, 14.0), 0, None), ((13.0, 10.0, 14.0), 0, 1),      # one is far ahead: no trains
+    ((10.0, 11.0, 12.0), 2, 1), ((10.0, 11.0, 11.4), 3, 1),         # the second tile only where it is near the first
+    ((float("inf"), 11.0, 12.0), 0, 1), ((10.0, float("inf"), 11.0), 2, 2)])     # what failed is left out
+def test_trains_only_of_forms_that_may_win(choices, monkeypatch, alone, forms, tile):
+    left, tried = list(alone), []
+    monkeypatch.setattr(blaslt, "_least_of_three", lambda a, m, run: left.pop(0))
+    monkeypatch.setattr(blaslt, "_in_trains", lambda w, f, alone: (tried.append(len(f)), [10.0, 9.0, 9.0][:len(f)])[1])
+    monkeypatch.setattr(tiles, "candidates", lambda m, n, k, gated: [1, 2])
+    with blaslt.measuring():
+        assert _end() == (tile is not None)
+    assert tried == ([forms] if forms else []) and choices.ran == ([] if tile is None else [tile])
+
+
 def test_a_timed_run_finds_its_own_rows_in_the_caches(monkeypatch):
     """Of an activation buffer as long as the engine's budget only the product's rows are read before a timed run."""
     read = []
