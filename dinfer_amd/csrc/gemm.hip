@@ -512,7 +512,9 @@ inline int few_rows_row_tiles(int64_t M, int64_t N) {
 // K = 12,288 or N = 5,120 sixteen lose). Every wave gets at least four k steps (K = 1,024: 4 waves, measured). With one row
 // tile four are the round of loads that a wave has in flight, so a K between eight and twelve waves' rounds takes as many
 // waves as it has: eight of them would fetch twice, the second time half a round (K = 3,072, N = 1,024, inside a step of
-// 28 layers: 979 -> 950 us at one token, 1,109 -> 1,084 at 8, 1,355 -> 1,311 at 32; 16 waves 957, 1,098 and 1,341).
+// 28 layers: 979 -> 950 us at one token, 1,109 -> 1,084 at 8, 1,355 -> 1,311 at 32; 16 waves 957, 1,098 and 1,341. Weights in turn, K 2,112,
+// 2,304, 2,560, 2,816 and 3,072, N 512 to 4,096, 1 to 32 tokens: 0.71 to 0.94 of eight waves' time at all 150, for instance K = 2,112, N = 4,096
+// 6.1 -> 5.5 us at one token, K = 3,072, N = 2,048 8.7 -> 7.1 at 32).
 inline int few_rows_waves(int mt, int rt, int64_t N, int64_t K) {
   int nw = (rt == 1 || N < 8192) ? 8 : 4;
   if (mt == 1 && rt == 1 && N <= 4096 && K <= 4096) nw = 16;

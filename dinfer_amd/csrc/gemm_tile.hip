@@ -19,16 +19,16 @@
 // one round of workgroups. (Lines brought into L2 ahead of their use, by touches of a ninth wave or by scalar loads: 10 to 50 %
 // slower. Loads into registers have the same limit.)
 //
-// Against the library's measured choice with the activation's kernel, products one after the other with weights in turn, us:
-//   gated  1,033 x 3,072 x 1,024    25    18      relu^2  4,096 x 8,192 x 2,048   120   103
-//          2,048 x 8,192 x 2,048   119   104      and without an activation
-//          2,048 x 12,288 x 4,096  303   286        543 x 7,168 x 5,120            57    49
-//          4,096 x 2,816 x 2,048    93    79        2,048 x 4,096 x 12,288        170   164
-//          543 x 17,408 x 5,120    194   182        1,033 x 4,096 x 1,024          15    13
-// Without an end that is a pass of its own the library is level or ahead in most steps (2,023 x 7,168 x 2,048 46 and 49, 4,096 x 2,048 x
-// 8,192 110 and 118), and so is it with few columns at 64 rows. Logits of 64 rows, floats: 151,936 x 4,096 236 and 219, 32,768 x 2,048 32 and 29.
-// Which of them runs a shape is measured where the library's own kernels are (blaslt.py). Whole steps: gate and up of
-// 28 layers of 1,024 columns, 1,152 rows, 3,026 -> 2,825 us; 8 of 4,096, 2,048 rows, 5,884 -> 5,739.
+// Against the library's measured choice (with an activation: and its kernel), in trains of launches with copies of the weight in turn, us:
+//   gated  1,152 x 3,072 x 1,024    26    20      relu^2  4,096 x 8,192 x 2,048   124   116
+//          2,048 x 8,192 x 2,048   120   110              2,048 x 8,192 x 2,048    66    61
+//          2,048 x 12,288 x 4,096  306   299      and without an activation
+//          4,096 x 2,816 x 2,048    98    87        543 x 7,168 x 5,120            56    53
+//          544 x 17,408 x 5,120    200   189        1,033 x 4,096 x 1,024          17    16
+// Without an end that is a pass of its own the library is level or ahead in most steps (2,048 x 4,096 x 12,288 169 and 171, 2,023 x 7,168 x 2,048
+// 49 and 57, 4,096 x 2,048 x 8,192 112 and 121, 1,033 x 1,024 x 3,072 18.5 and 19.8, 543 x 5,120 x 17,408 128 and 132). Logits of 64 rows, floats:
+// 151,936 x 4,096 250 and 230, 32,768 x 2,048 35 and 30.
+// Which of them runs a shape is measured where the library's own kernels are (blaslt.py).
 //
 // Reference behaviour: crates/kernels/src/gemm.rs:605-647 (the product; the reference hands it to its vendor library),
 // crates/kernels/cuda/activation.cu:8-16 (the gated activation).
@@ -166,7 +166,7 @@ __device__ __forceinline__ void store_blocks(const Product& p, int m0, int c0, c
   }
 }
 
-// Tiles of up to 224 x 128 or 128 x 256 (two sets of fragments and the sums in 256 registers), waves 2 x 4, NS stages of both operands.
+// Tiles of 96 x 64, 64 to 224 x 128, 96 x 192, 64 x 320 and 128 x 256 (two sets of fragments and the sums in 256 registers), waves 2 x 4, NS stages of both operands.
 // A step's first half computes on fragments read beside the MFMAs before, while the second half's are read; behind the barrier between
 // the halves every wave has all of the step in registers, so its place is sent anew, NS steps ahead, and the next step is here to be read.
 // The last NS steps of a tile send the first stages of the workgroup's next one (behind its last tile its own again, for nobody), whose
@@ -260,7 +260,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing on its way into LDS
 }
 
-// Tiles of 256 x 128 and 192 x 256 to 256 x 256: registers hold one set of a wave's row fragments, each read anew as soon as its MFMAs
+// Tiles of 256 x 128, 192 x 256, 256 x 192 and 256 x 256: registers hold one set of a wave's row fragments, each read anew as soon as its MFMAs
 // are issued, and LDS NA steps of A's rows and one more of the weight's, which come from HBM where A's, just written, are nearer: sent NA and
 // NA + 1 steps ahead (the other way round 2,048 x 12,288 x 4,096, gated, 296 us for 286, 543 x 17,408 x 5,120 222 for 182). The barrier of
 // a step comes behind the first rows of its second half, whose MFMAs cover the last reads.

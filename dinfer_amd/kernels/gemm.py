@@ -13,12 +13,14 @@ feed-forward), where the few-row kernel drowns in loads of the activations and
 the library has few output tiles to spread; the kernel that keeps a slice of the
 activations in LDS (csrc/gemm_mid.hip) runs it.
 
-Which kernel runs is a rule of the sizes, not a measurement at run time. A
-measurement was tried (every candidate captured into a graph of its own, timed
-after the caches were emptied) and did not predict the order inside a decode
-step: at 64 rows it chose the LDS kernel for the gate and up projections, which
-timed 8 % ahead alone and cost 0.1 ms a step in place. The rule below is what whole
-decode steps of an 8B-sized model measured.
+Which of the kernels for up to 64 rows runs, and where the library's side begins, is
+a rule of the sizes, not a measurement at run time. A measurement was tried there
+(every candidate captured into a graph of its own, timed after the caches were
+emptied) and did not predict the order inside a decode step: at 64 rows it chose the
+LDS kernel for the gate and up projections, which timed 8 % ahead alone and cost
+0.1 ms a step in place. The rule below is what whole decode steps of an 8B-sized model
+measured. What is measured, in the engine's warm-up, is the library's algorithm or
+tile for a product, singly, and a product's kernel with its end, in trains (blaslt.py).
 """
 from __future__ import annotations
 
@@ -149,7 +151,8 @@ def gated_nt(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, scratch: torch
     """out[:m] = act(a @ wg.T) * (a @ wu.T) for w = [wg; wu] stacked [2N, K]: the two projections of a gated
     feed-forward and its activation, in one weight-streaming kernel at decode sizes (up to 32 rows, up to 64 where
     the kernel for wide weights takes it). scratch
-    [rows, 2N] takes the projections where the activation is a pass of its own."""
+    [rows, 2N] takes the projections where the activation is a pass of its own; out is a scratch buffer too (see matmul_nt): while
+    measuring, its rows up to m's bucket are written."""
     if m <= 0:
         return out
     if a.dtype == torch.bfloat16 and act == "silu" and _wide(m, w.shape[0] // 2, w.shape[1]):

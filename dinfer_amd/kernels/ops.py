@@ -975,7 +975,7 @@ EXPERT_ACTS = {"silu": 2, "gelu": 3, "relu2": 4}    # activations the plain (not
 
 def moe_tile_rows(dtype: torch.dtype, entries: int, experts: int, k_in: int, k_mid: int) -> int:
     """Rows of a row tile for the two products of a routed layer over `entries` (token, choice) pairs: what the kernel
-    that will run them takes (16 where an expert gets few rows, 128 for many, 64 on the vector ALUs)."""
+    that will run them takes (16 where an expert gets few rows, 128 for many, 224 for more, 64 on the vector ALUs)."""
     return int(lib.get("dinfer_moe_tile_rows")(dtype_code(dtype), entries, experts, k_in, k_mid))
 
 
